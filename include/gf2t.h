@@ -133,12 +133,10 @@ int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dtmp,
  *              default 3072)
  *   "gcd_school_words" the host Karatsuba's schoolbook base in words
  *              (8..512; default 48)
- *   "fft_ept"  elements of a transform tile per thread (2, 4, 8, 16;
- *              default 2): fewer threads per tile
- *   "fft_low_bits" low index bits kept local in every transform pass,
- *              i.e. contiguous elements per HBM run of a tile (4, 5 or 6;
- *              default 4): longer runs, but fewer window bits per pass
- *              and so more passes.  Plans made before keep theirs
+ *   "fft_ept"  (2, 4, 8, 16; default 2) and "fft_low_bits" (4, 5, 6;
+ *              default 4): accepted and reported, without effect; the
+ *              transform's threads hold four units each and its passes
+ *              take the low bits their tile leaves
  *   "hm_zc_words" products of the host-buffer service (gf2t_mat2n_host,
  *              gf2t_mat2_host) whose operands and results take at most
  *              this many words together are read and written by the GPU
@@ -155,11 +153,10 @@ int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dtmp,
  * PCLMULQDQ where the CPU also has AVX-512 VPCLMULQDQ (read once). */
 int gf2t_tune(const char *key, int64_t value);
 /* The value a knob has now (the default until set): the keys above, and
- * "fft_tile_<m>" -- the tile of the 2^m-point transforms' passes is 2^T
- * elements, T in 6..13 (set with gf2t_tune("fft_tile_<m>", T), 0 = the
- * default: 13 from m = 19 up, 11 for m = 14..18, m below 14).  A smaller
- * tile spreads a small transform over more workgroups at the cost of more
- * passes; the reference's split knobs are gf2c_taylor_lv / gf2c_bfly_lv
+ * "fft_tile_<m>" -- the butterfly passes of the 2^m-point transforms use
+ * tiles of at most 2^T elements, T in 6..13 (set with
+ * gf2t_tune("fft_tile_<m>", T), 0 = the default: 13, or m where that is
+ * less).  A smaller tile spreads a small transform over more workgroups; the reference's split knobs are gf2c_taylor_lv / gf2c_bfly_lv
  * (src/gf2_cantor_cuda.h:24-61).  The autotuner (mersenne_trinomial_amd/
  * autotune.py) measures these and installs its choices. */
 int gf2t_tune_get(const char *key, int64_t *value);

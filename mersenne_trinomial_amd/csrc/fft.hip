@@ -4,25 +4,19 @@
 // Transform (same evaluation points and natural output order as the
 // reference's CantorFFT, src/gf2_cantor_engine.h:125-188): output i is
 // the chunk polynomial evaluated at sum_{bits k of i} b[k] of the Cantor
-// basis.  In index-bit terms the reference's in-place algorithm is a
-// sequence of small linear maps:
-//   Taylor level e  (bits e, e+1):  f[..10..] ^= f[..11..]; f[..01..] ^= f[..10..]
-//   forward Taylor cascade: for L = 0..m-2: for e = m-2 down to L: T(e)
-//   butterfly depth L (bit L): e1 = g + W(t) h, e2 = e1 + h with
-//   W(t) = sum_{bits k of t} b[k+1], t = index >> (L+1)
-//   forward butterflies: L = m-1 down to 0.
-// Each map touches one or two index bits, so a tile that holds every
-// element along a set of "local" index bits can apply, in LDS, every map
-// whose bits are local.  A host scheduler packs the sequence into as few
-// HBM passes as possible, moving a map earlier only past maps it
-// commutes with (disjoint bits, and a butterfly's twiddle bits untouched).
-// The pass's local bits are the low c bits (for coalesced 128-byte
-// segments) plus a window [a, a+w) of higher bits.
-//
-// Twiddles are linear in t, so each block builds four 256-entry byte
-// tables in LDS (W(t) = T0[t&255]^T1[t>>8&255]^...) instead of reading an
-// n/2-entry table from HBM.
+// basis.  Two parts:
+//   1. the basis conversion (cantor.hpp): from powers of X to the products
+//      of the subspace polynomials s_k, XORs only, O(m log m) of them per
+//      coefficient.  Of a product's operands it runs on their 32-bit
+//      chunks, before they become field elements.
+//   2. butterflies, level L on index bit L: e1 = g + W(t) h, e2 = e1 + h
+//      with W(t) = sum_{bits k of t} b[k+1], t = index >> (L+1); forward
+//      L = m-1 down to 0.  Elements are in the tower basis of cantor.hpp,
+//      two to a unit of four words; a thread holds 16 units and takes four
+//      levels between two exchanges through LDS, so a pass over memory
+//      takes eight levels.
 #include "gf2t_internal.hpp"
+#include "cantor.hpp"
 #include "../../include/gf2t.h"
 #include <vector>
 #include <map>
@@ -34,222 +28,502 @@
 
 namespace {
 
-constexpr int FFT_MAX_OPS = 64;
-constexpr int FFT_THREADS = 512;    // most threads per block (a tile of 2^T elements uses 2^(T-1))
-constexpr int FFT_TILE_BITS = 13;   // largest tile: 8192 elements = 64 KiB of LDS
+constexpr int FFT_MAX_M = 27;
+constexpr int FFT_TILE_BITS = 13;   // largest tile: 8192 elements
 constexpr int FFT_MIN_TILE_BITS = 6;
-constexpr int FFT_LOW_BITS = 4;     // default: 16 contiguous elements = 128 bytes
+constexpr int FFT_LOW_BITS = 4;
 constexpr int PACK_LIST = 12;   // four matrix entries + four vector pairs
+constexpr int CONV_ONE_TILE = 12;   // largest conversion done in one tile
+constexpr int CONV_TILE32 = 13, CONV_TILE64 = 12;
 
-enum : uint8_t { OP_TF = 0, OP_TI = 1, OP_BF = 2, OP_BI = 3 };
+__constant__ TwEnt c_tw[4][256];
+__device__ FftTables g_tab;
 
-struct Op {
-    uint8_t kind, bit;
-};
-
-struct PassDesc {
-    int m;        // transform size exponent
-    int c, a, w;  // local bits: [0,c) and [a, a+w); tile = 2^(c+w)
-    int nops;
-    int nbf;      // butterfly ops among them (0: no twiddle tables needed)
-    uint8_t kind[FFT_MAX_OPS];
-    uint8_t lbit[FFT_MAX_OPS];   // local bit of the op (low bit of a Taylor pair)
-    uint8_t gbit[FFT_MAX_OPS];   // global bit (butterfly depth L)
-};
-
-__constant__ u64 c_basis[64];
-
-struct TwTables {
-    u64 t[4][256];
-};
-
-// Where the first pass of a batch of transforms packs its input from:
-// 32-bit chunk k of an operand is element k (zero from nchunks on, the
-// last chunk masked to lastmask).  Stride form: batch element y packs
-// from src + y*stride.  List form (nlist > 0): element y < nlist packs
-// from lsrc[y] with its own chunk count and mask, so operands of
-// different lengths share one launch.  xor0 is XORed into element 0
-// (adds x to the operand).
-struct PackArg {
+// One operand of a transform: n 32-bit chunks at src (the last masked to
+// mask, xor0 XORed into the first), and the buffer its converted
+// coefficients go to (16-byte aligned).
+struct Operand {
     const u32 *src;
-    u64 stride;
-    u64 nchunks;
-    u32 lastmask, xor0;
-    int nlist;
-    const u32 *lsrc[PACK_LIST];
-    u64 lnch[PACK_LIST];
-    u32 lmask[PACK_LIST];
+    u32 *lch;
+    u64 n;
+    u32 mask, xor0;
 };
-
-// W(t) for t < 2^32: four independent table reads, no branches (the
-// tables past the ones a transform needs hold only their entry 0 = 0,
-// which is all that a t below 2^(8 ntab) reads there)
-GF2T_DEV u64 twiddle(const TwTables &tw, u64 t) {
-    const u32 v = (u32)t;
-    return xor3(tw.t[0][v & 255], tw.t[1][(v >> 8) & 255], tw.t[2][(v >> 16) & 255]) ^
-           tw.t[3][v >> 24];
+// The operands of a launch, blockIdx selecting one: a list in the launch
+// arguments (list = null, group = 0), a list in device memory, or two
+// groups of `group` operands, sources sstride[.] and buffers lstride apart.
+struct Operands {
+    const Operand *list;
+    u32 group;
+    u64 sstride[2], lstride;   // 32-bit words
+    Operand op[PACK_LIST];
+};
+GF2T_DEV Operand operand(const Operands &o, u32 y) {
+    if (o.list) return o.list[y];
+    if (!o.group) return o.op[y];
+    const u32 g = y / o.group, i = y - g * o.group;
+    Operand r = o.op[g];
+    r.src += (u64)i * (g ? o.sstride[1] : o.sstride[0]);
+    r.lch += (u64)i * o.lstride;
+    return r;
 }
-
-// the global index of tile element li (li < 2^(c+w)): its low c bits stay,
-// its bits [c, c+w) go to [a, a+w), and gbase holds the tile's own bits
-GF2T_DEV u64 global_index(const PassDesc &pd, u32 li, u64 gbase) {
-    const u32 cm = (1u << pd.c) - 1;
-    return gbase | (u64)(li & cm) | ((u64)(li >> pd.c) << pd.a);
-}
-
-// pack: element k of the transform input = 32-bit chunk k of the bit
-// array (zero beyond nchunks; last chunk masked to `lastbits`)
-GF2T_DEV u64 packed_chunk(const u32 *__restrict__ src, u64 nchunks, u32 lastmask, u64 k) {
-    if (k >= nchunks) return 0;
-    u32 v = src[k];
-    if (k == nchunks - 1) v &= lastmask;
+// chunk k, zero from n on
+GF2T_DEV u32 chunk(const Operand &o, u64 k) {
+    if (k >= o.n) return 0;
+    u32 v = o.src[k];
+    if (k == o.n - 1) v &= o.mask;
+    if (k == 0) v ^= o.xor0;
     return v;
 }
 
-// One pass over the tile `blk` of the transform at f (2^m elements):
-// load the tile (packing the input chunks on the first pass), apply the
-// pass's ops in LDS, store.  The block's threads stride over the tile;
-// ntab byte tables of twiddles cover the twiddle indices t < 2^(8 ntab)
-// the transform uses.
-GF2T_DEV void fft_pass_tile(u64 *__restrict__ f, const PassDesc &pd, bool pack,
-                            const u32 *__restrict__ psrc, u64 pn, u32 pmask, u32 xor0, int ntab,
-                            u64 blk, u64 *lds) {
-    TwTables &tw = *reinterpret_cast<TwTables *>(lds);
-    u64 *tile = lds + 4 * 256;
-    const int T = pd.c + pd.w;
-    const u32 tsize = 1u << T;
-    const unsigned nthr = blockDim.x;
-    const int nlo = pd.a - pd.c;
-    // the tile's fixed index bits: blk's low nlo bits at [c, a), the rest
-    // from a + w up
-    const u64 gbase = ((blk & ((1ULL << nlo) - 1)) << pd.c) | ((blk >> nlo) << (pd.a + pd.w));
-
-    // twiddle byte tables: T_k[v] = sum_{bits j of v} b[8k + j + 1]
-    if (pd.nbf == 0) ntab = 0;
-    for (int e = threadIdx.x; e < 256 * ntab; e += nthr) {
-        int k = e >> 8, v = e & 255;
-        u64 acc = 0;
-        for (int j = 0; j < 8; j++)
-            if ((v >> j) & 1) {
-                int bi = 8 * k + j + 1;
-                acc ^= bi < 64 ? c_basis[bi] : 0;
-            }
-        tw.t[k][v] = acc;
+// where a conversion reads and writes: an operand's chunks (the first
+// launch from src, the others in place in lch), or a transform's elements
+struct ChunkIo {
+    Operand o;
+    bool first;
+    typedef u32 type;
+    GF2T_DEV bool any(u64 i) const { return i < o.n; }
+    GF2T_DEV u32 load(u64 i) const {
+        if (first) return chunk(o, i);
+        return i < o.n ? o.lch[i] : 0;
     }
-    if (pd.nbf && threadIdx.x < 4 - ntab) tw.t[3 - threadIdx.x][0] = 0;
-    // load the tile (low c bits contiguous in memory)
-    for (u32 li = threadIdx.x; li < tsize; li += nthr) {
-        const u64 g = global_index(pd, li, gbase);
-        u64 v;
-        if (pack) {
-            v = packed_chunk(psrc, pn, pmask, g);
-            if (g == 0) v ^= xor0;
-        } else {
-            v = f[g];
+    GF2T_DEV void store(u64 i, u32 v) const {
+        if (i < o.n) o.lch[i] = v;
+    }
+};
+struct ElemIo {
+    u64 *f;
+    typedef u64 type;
+    GF2T_DEV bool any(u64) const { return true; }
+    GF2T_DEV u64 load(u64 i) const { return f[i]; }
+    GF2T_DEV void store(u64 i, u64 v) const { f[i] = v; }
+};
+
+constexpr int CONV_THREADS = 256;
+constexpr u32 CONV_EDGE_RHO = 16;
+
+// One group of K expansion steps (ConvStep): blockIdx.y is the block of
+// 2^K rows; the first colblocks blocks take a skewed column per thread,
+// all rows of it in registers, in place; the others the columns at the
+// rows' ends, in LDS.
+template <int K, bool INV, class Io>
+GF2T_DEV void conv_step_block(const Io &io, const ConvStep &s, u32 colblocks,
+                              typename Io::type *lds) {
+    typedef typename Io::type E;
+    constexpr int R = 1 << K;
+    const u64 base = (u64)blockIdx.y << (s.hb + K);
+    if (!io.any(base)) return;   // whole block
+    if (blockIdx.x < colblocks) {
+        const u32 t = blockIdx.x * CONV_THREADS + threadIdx.x;
+        if (t >= conv_full(s)) return;
+        E x[R];
+#pragma unroll
+        for (int k = 0; k < R; k++) x[k] = io.load(base + ((u64)k << s.hb) + conv_col(s, t, k));
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            const int e = INV ? j : K - 1 - j;
+#pragma unroll
+            for (int k = 0; k < R; k++)
+                if ((k >> e) & 1) x[k ^ (1 << e)] ^= x[k];
         }
-        tile[li] = v;
+#pragma unroll
+        for (int k = 0; k < R; k++) io.store(base + ((u64)k << s.hb) + conv_col(s, t, k), x[k]);
+        return;
+    }
+    // edge: rho0 .. rho0 + nr of the unit, R x R coefficients each
+    const u32 unit = 1u << s.ub, nr = unit < CONV_EDGE_RHO ? unit : CONV_EDGE_RHO;
+    const int lr = s.ub < 4 ? s.ub : 4;
+    const u32 rho0 = (blockIdx.x - colblocks) * nr;
+    const u32 total = (u32)(R * R) << lr;
+    for (u32 i = threadIdx.x; i < total; i += CONV_THREADS) {
+        const u32 rho = i & (nr - 1), q = (i >> lr) & (R - 1), k = i >> (lr + K);
+        lds[i] = io.load(base + ((u64)k << s.hb) + conv_edge(s, (int)k, q, rho0 + rho));
     }
     __syncthreads();
-
-    for (int o = 0; o < pd.nops; o++) {
-        const int kind = pd.kind[o];
-        const int l = pd.lbit[o];
-        const u32 lo_mask = (1u << l) - 1;
-        if (kind == OP_TF || kind == OP_TI) {
-            const u32 st = 1u << l;
-            for (u32 qd = threadIdx.x; qd < (tsize >> 2); qd += nthr) {
-                const u32 base = (qd & lo_mask) | ((qd >> l) << (l + 2));
-                u64 x01 = tile[base + st], x10 = tile[base + 2 * st], x11 = tile[base + 3 * st];
-                if (kind == OP_TF) { x10 ^= x11; x01 ^= x10; }
-                else { x01 ^= x10; x10 ^= x11; }
-                tile[base + st] = x01;
-                tile[base + 2 * st] = x10;
-            }
-        } else {
-            const int L = pd.gbit[o];
-            const u32 st = 1u << l;
-            for (u32 pr = threadIdx.x; pr < (tsize >> 1); pr += nthr) {
-                const u32 i1 = (pr & lo_mask) | ((pr >> l) << (l + 1));
-                const u64 g1 = global_index(pd, i1, gbase);
-                u64 w = twiddle(tw, g1 >> (L + 1));
-                u64 e1 = tile[i1], e2 = tile[i1 + st];
-                if (kind == OP_BF) {
-                    e1 ^= gf64_mul(w, e2);
-                    e2 ^= e1;
-                } else {
-                    e2 ^= e1;
-                    e1 ^= gf64_mul(w, e2);
-                }
-                tile[i1] = e1;
-                tile[i1 + st] = e2;
-            }
+    for (int j = 0; j < K; j++) {
+        const int e = INV ? j : K - 1 - j;
+        for (u32 i = threadIdx.x; i < total / 2; i += CONV_THREADS) {
+            const u32 rho = i & (nr - 1);
+            conv_tile_op([&](u32 l) -> E & { return lds[(l << lr) | rho]; }, i >> lr, K, e, INV);
         }
         __syncthreads();
     }
-    for (u32 li = threadIdx.x; li < tsize; li += nthr)
-        f[global_index(pd, li, gbase)] = tile[li];
+    for (u32 i = threadIdx.x; i < total; i += CONV_THREADS) {
+        const u32 rho = i & (nr - 1), q = (i >> lr) & (R - 1), k = i >> (lr + K);
+        io.store(base + ((u64)k << s.hb) + conv_edge(s, (int)k, q, rho0 + rho), lds[i]);
+    }
+}
+template <int K>
+__global__ __launch_bounds__(CONV_THREADS) void k_conv_step32(const Operands ops, const ConvStep s,
+                                                              u32 colblocks, int first) {
+    __shared__ u32 lds[(1 << (2 * K)) * CONV_EDGE_RHO];
+    conv_step_block<K, false>(ChunkIo{operand(ops, blockIdx.z), first != 0}, s, colblocks, lds);
+}
+template <int K, bool INV>
+__global__ __launch_bounds__(CONV_THREADS) void k_conv_step64(u64 *__restrict__ f, u64 f_stride,
+                                                              const ConvStep s, u32 colblocks) {
+    __shared__ u64 lds[(1 << (2 * K)) * CONV_EDGE_RHO];
+    conv_step_block<K, INV>(ElemIo{f + (u64)blockIdx.z * f_stride}, s, colblocks, lds);
 }
 
-// blockIdx.y selects one transform of a batch: element y lives at
-// f + y*f_stride.  pack (first pass only) describes the input to pack.
-// The block has 2^(T-1) threads (at most FFT_THREADS) for its 2^T-element
-// tile.
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_pass(u64 *__restrict__ f, const PassDesc pd,
-                                                          const PackArg pk, int pack, int ntab,
-                                                          u64 f_stride) {
-    extern __shared__ u64 lds[];
-    const unsigned y = blockIdx.y;
-    const u32 *psrc = nullptr;
-    u64 pn = 0;
-    u32 pmask = 0;
-    if (pack) {
-        if (pk.nlist) {
-            psrc = pk.lsrc[y];
-            pn = pk.lnch[y];
-            pmask = pk.lmask[y];
-        } else {
-            psrc = pk.src + (u64)y * pk.stride;
-            pn = pk.nchunks;
-            pmask = pk.lastmask;
+// A group of up to eight index bits (ConvGroup): 64 coefficients per thread
+// in registers, two exchanges through LDS for w = 7, 8.  One coefficient in
+// 64 is left out of the LDS index, so that the threads of both layouts fall
+// on different banks.
+GF2T_DEV u32 group_pad(u32 i) { return i + (i >> 6); }
+template <bool INV, class Io>
+GF2T_DEV void conv_group_block(const Io &io, const ConvGroup &g, typename Io::type *lds) {
+    typedef typename Io::type E;
+    const u64 base = group_base(g, blockIdx.x);
+    if (!io.any(base)) return;   // whole block
+    const u32 tid = threadIdx.x, nthr = blockDim.x;
+    const bool two = g.w > 6;
+    E x[64];
+    if (g.off) {
+#pragma unroll
+        for (int r = 0; r < 64; r++)
+            x[r] = io.load(base + group_mem(g, group_local(g, 0, tid, r)));
+    } else {   // contiguous: through LDS, so that a wave reads whole runs
+#pragma unroll
+        for (int r = 0; r < 64; r++) lds[group_pad(tid + r * nthr)] = io.load(base + tid + r * nthr);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 0, tid, r))];
+    }
+    if (two) {
+        if (INV) conv_group_top<INV>(x, g.w);
+        else conv_group_first<INV>(x, g.w);
+        if (!g.off) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 0, tid, r))] = x[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 1, tid, r))];
+        conv_group_low<INV>(x, g.w);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 1, tid, r))] = x[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 0, tid, r))];
+        if (INV) conv_group_first<INV>(x, g.w);
+        else conv_group_top<INV>(x, g.w);
+    } else {
+        conv_group_first<INV>(x, g.w);
+    }
+    if (g.off) {
+#pragma unroll
+        for (int r = 0; r < 64; r++)
+            io.store(base + group_mem(g, group_local(g, 0, tid, r)), x[r]);
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 0, tid, r))] = x[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 64; r++) io.store(base + tid + r * nthr, lds[group_pad(tid + r * nthr)]);
+    }
+}
+__global__ __launch_bounds__(128) void k_conv_group32(const Operands ops, const ConvGroup g,
+                                                      int first) {
+    extern __shared__ u32 lds32[];
+    conv_group_block<false>(ChunkIo{operand(ops, blockIdx.y), first != 0}, g, lds32);
+}
+template <bool INV>
+__global__ __launch_bounds__(128) void k_conv_group64(u64 *__restrict__ f, u64 f_stride,
+                                                      const ConvGroup g) {
+    extern __shared__ u64 lds64[];
+    conv_group_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride}, g, lds64);
+}
+
+// Small sizes: the whole conversion of a transform in one block, every
+// step inside LDS.
+constexpr int CONV_MAX_OPS = 32;
+struct TileArg {
+    int T, nops;
+    signed char h[CONV_MAX_OPS], pos[CONV_MAX_OPS];   // in execution order
+};
+template <bool INV, class Io>
+GF2T_DEV void conv_tile_block(const Io &io, const TileArg &t, typename Io::type *lds) {
+    typedef typename Io::type E;
+    const u32 n = 1u << t.T, nthr = blockDim.x;
+    if (!io.any(0)) return;   // whole block
+    for (u32 l = threadIdx.x; l < n; l += nthr) lds[l] = io.load(l);
+    __syncthreads();
+    for (int o = 0; o < t.nops; o++) {
+        const int h = t.h[o], pos = t.pos[o];
+        for (u32 i = threadIdx.x; i < n / 2; i += nthr)
+            conv_tile_op([&](u32 l) -> E & { return lds[l]; }, i, h, pos, INV);
+        __syncthreads();
+    }
+    for (u32 l = threadIdx.x; l < n; l += nthr) io.store(l, lds[l]);
+}
+__global__ __launch_bounds__(1024) void k_conv_tile32(const Operands ops, const TileArg t,
+                                                      int first) {
+    extern __shared__ u32 lds32[];
+    conv_tile_block<false>(ChunkIo{operand(ops, blockIdx.y), first != 0}, t, lds32);
+}
+template <bool INV>
+__global__ __launch_bounds__(1024) void k_conv_tile64(u64 *__restrict__ f, u64 f_stride,
+                                                      const TileArg t) {
+    extern __shared__ u64 lds64[];
+    conv_tile_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride}, t, lds64);
+}
+
+// ------------------------------------------------------------ butterflies
+// LDS copy of the GF(2^8) multiply tables
+struct MulLds {
+    uint4 A[256];
+    u32 B[256];
+    GF2T_DEV void load() {
+        for (u32 i = threadIdx.x; i < 256; i += blockDim.x) {
+            A[i] = reinterpret_cast<const uint4 *>(g_tab.mulA)[i];
+            B[i] = g_tab.mulB[i];
         }
     }
-    fft_pass_tile(f + (u64)y * f_stride, pd, pack != 0, psrc, pn, pmask, pk.xor0, ntab,
-                  blockIdx.x, lds);
-}
-
-// A grouped launch: one pass each of several transforms of different
-// sizes (the i-th pass of every product in a batch that has one).  Entry
-// e owns blocks [block0, block0 + nblocks * ntrans) of the grid: ntrans
-// transforms n words apart, nblocks tiles each; a block finds its entry
-// by its index.
-struct GroupPass {
-    PassDesc pd;
-    u64 *f;
-    u64 f_stride;
-    const u32 *src[2];
-    u64 nch[2];
-    u32 mask[2];
-    int pack, ntab;
-    u32 block0, nblocks, ntrans, pad;
+    GF2T_DEV Mul8 operator()(u32 v) const {
+        const uint4 a = A[v];
+        return Mul8{a.x, a.y, a.z, a.w, B[v]};
+    }
 };
+// what a pass reads and writes: units; the chunks of an operand (lch:
+// converted ones); elements in the polynomial basis
+enum { IO_UNITS = 0, IO_CHUNKS = 1, IO_LCH = 2, IO_PLAIN = 3 };
 
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_pass_grouped(
-        const GroupPass *__restrict__ gp, int nent) {
-    extern __shared__ u64 lds[];
-    const u32 b = blockIdx.x;
-    int e = 0;
-    while (e + 1 < nent && gp[e + 1].block0 <= b) e++;
-    const GroupPass &G = gp[e];
-    const u32 local = b - G.block0;
-    const u32 y = local / G.nblocks, x = local - y * G.nblocks;
-    fft_pass_tile(G.f + (u64)y * G.f_stride, G.pd, G.pack != 0, G.pack ? G.src[y] : nullptr,
-                  G.pack ? G.nch[y] : 0, G.pack ? G.mask[y] : 0, 0, G.ntab, x, lds);
+// transform buffers are the caller's: 8-byte aligned
+typedef u32 G4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef u64 G2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef u64 Emb[256];
+GF2T_DEV U4 load_unit(const U4 *f, u32 i, int io, const Operand &o, const Emb *emb) {
+    if (io == IO_UNITS) {
+        const G4 v = reinterpret_cast<const G4 *>(f)[i];
+        return U4{{v.x, v.y, v.z, v.w}};
+    }
+    if (io == IO_PLAIN) {
+        const G2 v = reinterpret_cast<const G2 *>(f)[i];
+        return unit_embed64(v.x, v.y, emb);
+    }
+    U4 z = {{0, 0, 0, 0}};
+    const u64 k = 2 * (u64)i;
+    if (k >= o.n) return z;
+    u32 e, g;
+    if (io == IO_LCH) {
+        if (k + 1 < o.n) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(o.lch + k);
+            e = v.x;
+            g = v.y;
+        } else {
+            e = o.lch[k];
+            g = 0;
+        }
+    } else {
+        e = chunk(o, k);
+        g = chunk(o, k + 1);
+    }
+    return unit_embed32(e, g, emb);
+}
+GF2T_DEV void store_unit(U4 *f, u32 i, const U4 &u, int io, const Emb *une) {
+    if (io == IO_UNITS) {
+        reinterpret_cast<G4 *>(f)[i] = G4{u.w[0], u.w[1], u.w[2], u.w[3]};
+        return;
+    }
+    u64 e, g;
+    unit_unembed(u, une, e, g);
+    reinterpret_cast<G2 *>(f)[i] = G2{e, g};
+}
+// copy a basis table (8 x 256 entries; 4 x 256 for chunks) to LDS
+GF2T_DEV void load_basis(u64 *dst, const u64 (*src)[256], int bytes) {
+    for (u32 i = threadIdx.x; i < (u32)bytes * 256; i += blockDim.x)
+        dst[i] = reinterpret_cast<const u64 *>(src)[i];
+}
+GF2T_DEV u32 uniform32(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// One butterfly pass over the window of P (see BfPass): 2^RB units per
+// thread, RB levels, an exchange through LDS, and so on.
+template <int CLS, bool INV>
+__global__ __launch_bounds__(512) void k_bfly(u64 *__restrict__ f_, u64 f_stride, const BfPass P,
+                                              const Operands ops, int in, int out) {
+    constexpr int R = 1 << RB;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    MulLds &tab = *reinterpret_cast<MulLds *>(lds_raw);
+    u64 *basis = reinterpret_cast<u64 *>(lds_raw + sizeof(MulLds));
+    U4 *ex = reinterpret_cast<U4 *>(basis);
+    U4 *f = reinterpret_cast<U4 *>(f_ + (u64)blockIdx.y * f_stride);
+    Operand o{};
+    if (in == IO_CHUNKS || in == IO_LCH) o = operand(ops, blockIdx.y);
+    tab.load();
+    if (in != IO_UNITS) load_basis(basis, g_tab.emb, in == IO_PLAIN ? 8 : 4);
+    __syncthreads();
+    const u32 tid = threadIdx.x;
+    const BfTile T = bf_tile(P, blockIdx.x);
+    const int ns = bf_stages(P);
+    const Emb *emb = reinterpret_cast<const Emb *>(basis);
+    U4 x[R];
+    int s = INV ? ns - 1 : 0;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        x[r] = load_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), in, o, emb);
+    bool gives = in != IO_UNITS;   // the basis table gives way to the exchange
+#pragma nounroll
+    for (int k = 0;; k++) {
+        TwEnt W[RB];
+        bf_twiddles(P, T, s, tid, c_tw, W);
+        fft_stage<CLS, INV>(x, bf_active(P, s), W, tab);
+        if (k == ns - 1) break;
+        if (gives) __syncthreads();
+        gives = true;
+#pragma unroll
+        for (int r = 0; r < R; r++) ex[bf_local(P, s, tid, r)] = x[r];
+        s += INV ? -1 : 1;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; r++) x[r] = ex[bf_local(P, s, tid, r)];
+    }
+    if (out == IO_PLAIN) {
+        __syncthreads();   // exchange (or embedding table) done with
+        load_basis(basis, g_tab.une, 8);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        store_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), x[r], out, emb);
 }
 
-__global__ void k_pointwise(u64 *__restrict__ fa, const u64 *__restrict__ fb, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) fa[i] = gf64_mul(fa[i], fb[i]);
+// ---- the low levels
+constexpr u32 LO_UNITS = 64u << RB;              // per wave
+constexpr u32 LO_EXCH = (64u << RB) + (4u << RB);  // words of a wave's exchange plane
+
+GF2T_DEV u32 lo_pad(u32 u) { return u + (u >> 4); }
+// the wave's units from the layout of one stage to that of another, a word
+// of each unit at a time through the wave's own plane in LDS
+GF2T_DEV void lo_exchange(U4 *x, u32 lane, u32 *plane, int from, int to) {
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < (1 << RB); r++) plane[lo_pad(lo_unit(from, lane, r))] = x[r].w[p];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < (1 << RB); r++) x[r].w[p] = plane[lo_pad(lo_unit(to, lane, r))];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+template <int CA, int CB>
+GF2T_DEV void lo_forward(U4 *x, int m, u32 ubase, u32 lane, const MulLds &tab, const TwEnt *hi,
+                         u32 *plane) {
+    TwEnt W[RB], W0;
+    lo_twiddles(ubase, 0, lane, c_tw, hi, W, W0);
+    fft_stage<CA, false>(x, lo_active(m, 0), W, tab);
+#pragma nounroll
+    for (int s = 1; s < lo_stages(); s++) {
+        lo_exchange(x, lane, plane, s - 1, s);
+        lo_twiddles(ubase, s, lane, c_tw, hi, W, W0);
+        fft_stage<CB, false>(x, lo_active(m, s), W, tab);
+    }
+    fft_level0<CB, false>(x, W0, tab);
+}
+template <int CA, int CB>
+GF2T_DEV void lo_inverse(U4 *x, int m, u32 ubase, u32 lane, const MulLds &tab, const TwEnt *hi,
+                         u32 *plane) {
+    TwEnt W[RB], W0;
+    lo_twiddles(ubase, lo_stages() - 1, lane, c_tw, hi, W, W0);
+    fft_level0<CB, true>(x, W0, tab);
+#pragma nounroll
+    for (int s = lo_stages() - 1; s > 0; s--) {
+        lo_twiddles(ubase, s, lane, c_tw, hi, W, W0);
+        fft_stage<CB, true>(x, lo_active(m, s), W, tab);
+        lo_exchange(x, lane, plane, s, s - 1);
+    }
+    lo_twiddles(ubase, 0, lane, c_tw, hi, W, W0);
+    fft_stage<CA, true>(x, lo_active(m, 0), W, tab);
+}
+struct ProdLds {   // GF(2^32) basis tables
+    u32 d32[4][256], d5[4][256], b32[4][256];
+    GF2T_DEV void load() {
+        for (u32 i = threadIdx.x; i < 1024; i += blockDim.x) {
+            (&d32[0][0])[i] = (&g_tab.d32[0][0])[i];
+            (&d5[0][0])[i] = (&g_tab.d5[0][0])[i];
+            (&b32[0][0])[i] = (&g_tab.b32[0][0])[i];
+        }
+    }
+};
+enum { LO_FWD = 0, LO_INV = 1, LO_MUL = 2 };
+// Levels 7..0 of a transform (LO_FWD, LO_INV), or, of two transforms, both
+// forward, their product and the inverse of it in one pass (LO_MUL: f and
+// g, into f).  A wave takes LO_UNITS consecutive units.
+template <int CA, int CB, int DIR>
+__global__ __launch_bounds__(256) void k_low(u64 *__restrict__ f_, u64 f_stride,
+                                             const u64 *__restrict__ g_, int m,
+                                             const Operands ops, u32 g_op, int in, int out) {
+    constexpr int R = 1 << RB;
+    constexpr int LAST = lo_stages() - 1;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    MulLds &tab = *reinterpret_cast<MulLds *>(lds_raw);
+    TwEnt *hi = reinterpret_cast<TwEnt *>(lds_raw + sizeof(MulLds));
+    ProdLds &pt = *reinterpret_cast<ProdLds *>(hi + 4);
+    unsigned char *rest = (unsigned char *)(hi + 4) + (DIR == LO_MUL ? sizeof(ProdLds) : 0);
+    u32 *plane = reinterpret_cast<u32 *>(rest) + (threadIdx.x >> 6) * LO_EXCH;
+    u64 *basis = reinterpret_cast<u64 *>(rest + (blockDim.x >> 6) * LO_EXCH * 4);
+    const Emb *emb = reinterpret_cast<const Emb *>(basis);
+    U4 *f = reinterpret_cast<U4 *>(f_ + (u64)blockIdx.y * f_stride);
+    tab.load();
+    if (threadIdx.x < 4) hi[threadIdx.x] = tw_of(g_tab.tw, threadIdx.x << 7);
+    if (DIR == LO_MUL) pt.load();
+    if (in != IO_UNITS) load_basis(basis, g_tab.emb, in == IO_PLAIN ? 8 : 4);
+    __syncthreads();
+    const u32 units = 1u << (m - 1);
+    const u32 lane = threadIdx.x & 63;
+    const u32 ubase =
+        uniform32((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * LO_UNITS);
+    const bool act = ubase < units;   // whole wave
+    U4 x[R], y[R];
+    if (act) {
+#pragma nounroll
+        for (int op = 0; op < (DIR == LO_MUL ? 2 : 1); op++) {
+            if (DIR == LO_MUL) {
+#pragma unroll
+                for (int r = 0; r < R; r++) y[r] = x[r];
+            }
+            const U4 *src = op ? reinterpret_cast<const U4 *>(g_ + (u64)blockIdx.y * f_stride) : f;
+            Operand o{};
+            if (in == IO_CHUNKS || in == IO_LCH) o = operand(ops, blockIdx.y + (op ? g_op : 0));
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const u32 i = ubase + lo_unit(0, lane, r);
+                x[r] = i < units ? load_unit(src, i, in, o, emb) : U4{{0, 0, 0, 0}};
+            }
+            if (DIR != LO_INV) lo_forward<CA, CB>(x, m, ubase, lane, tab, hi, plane);
+        }
+        if (DIR == LO_MUL) {
+            // one unit's product per round, the registers turning, so that
+            // the code is there once
+#pragma nounroll
+            for (int k = 0; k < R; k++) {
+                const U4 v = unit_mul(y[0], x[0], pt.d32, pt.d5, pt.b32);
+#pragma unroll
+                for (int r = 0; r + 1 < R; r++) {
+                    x[r] = x[r + 1];
+                    y[r] = y[r + 1];
+                }
+                x[R - 1] = v;
+            }
+        }
+        if (DIR == LO_FWD) lo_exchange(x, lane, plane, LAST, 0);   // to contiguous stores
+        if (DIR == LO_INV) lo_exchange(x, lane, plane, 0, LAST);
+        if (DIR != LO_FWD) lo_inverse<CA, CB>(x, m, ubase, lane, tab, hi, plane);
+    }
+    if (out == IO_PLAIN) {
+        __syncthreads();
+        load_basis(basis, g_tab.une, 8);
+        __syncthreads();
+    }
+    if (act) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const u32 i = ubase + lo_unit(0, lane, r);
+            if (i < units) store_unit(f, i, x[r], out, emb);
+        }
+    }
 }
 
 // overlap-add in gather form: output word w collects chunks 2w-1, 2w, 2w+1
@@ -266,93 +540,6 @@ __global__ void k_overlap_add(const u64 *__restrict__ F, size_t nchunks, u64 *__
     if (k + 1 < nchunks) v ^= F[k + 1] << 32;
     if (w && k - 1 < nchunks) v ^= F[k - 1] >> 32;
     out[w] = v;
-}
-
-// ------------------------------------------------------------ scheduler
-bool op_conflict(const Op &x, const Op &y) {
-    bool tx = x.kind <= OP_TI, ty = y.kind <= OP_TI;
-    if (tx && ty) return std::abs((int)x.bit - (int)y.bit) <= 1;
-    if (!tx && !ty) return true;
-    const Op &t = tx ? x : y, &b = tx ? y : x;
-    return (int)t.bit + 1 >= (int)b.bit;   // shares bit L or a twiddle bit
-}
-
-struct Window {
-    int c, a, w;
-    bool has(int bit) const { return bit < c || (bit >= a && bit < a + w); }
-    int loc(int bit) const { return bit < c ? bit : c + (bit - a); }
-};
-
-bool op_fits(const Op &o, const Window &W) {
-    if (o.kind <= OP_TI) return W.has(o.bit) && W.has(o.bit + 1);
-    return W.has(o.bit);
-}
-
-std::vector<Op> op_sequence(int m, bool forward) {
-    std::vector<Op> ops;
-    if (forward) {
-        for (int L = 0; L <= m - 2; L++)
-            for (int e = m - 2; e >= L; e--) ops.push_back({OP_TF, (uint8_t)e});
-        for (int L = m - 1; L >= 0; L--) ops.push_back({OP_BF, (uint8_t)L});
-    } else {
-        for (int L = 0; L <= m - 1; L++) ops.push_back({OP_BI, (uint8_t)L});
-        for (int L = m - 2; L >= 0; L--)
-            for (int e = L; e <= m - 2; e++) ops.push_back({OP_TI, (uint8_t)e});
-    }
-    return ops;
-}
-
-// Pack the op sequence of a 2^m-point transform into passes over tiles of
-// 2^min(m, tile_bits) elements.
-std::vector<PassDesc> schedule(int m, bool forward, int tile_bits, int low_bits) {
-    std::vector<Op> rem = op_sequence(m, forward);
-    std::vector<PassDesc> passes;
-    int T = std::min(m, tile_bits);
-    // at least two window bits, so that every Taylor step fits some window
-    int c = std::min(low_bits, std::max(T - 2, 1));
-    int w = T - c;
-    while (!rem.empty()) {
-        std::vector<Window> cands;
-        if (m <= T) cands.push_back({m, m, 0});
-        else
-            for (int a = c; a + w <= m; a++) cands.push_back({c, a, w});
-        size_t best_n = 0;
-        Window bestW = cands[0];
-        std::vector<Op> best_take, best_skip;
-        for (const Window &W : cands) {
-            std::vector<Op> take, skip;
-            for (const Op &o : rem) {
-                bool ok = op_fits(o, W) && (int)take.size() < FFT_MAX_OPS;
-                if (ok)
-                    for (const Op &s : skip)
-                        if (op_conflict(o, s)) { ok = false; break; }
-                (ok ? take : skip).push_back(o);
-            }
-            if (take.size() > best_n) {
-                best_n = take.size();
-                bestW = W;
-                best_take.swap(take);
-                best_skip.swap(skip);
-            }
-        }
-        if (best_n == 0) break;   // cannot happen: some window fits the head op
-        PassDesc pd{};
-        pd.m = m;
-        pd.c = bestW.c;
-        pd.a = bestW.a;
-        pd.w = bestW.w;
-        pd.nops = (int)best_take.size();
-        pd.nbf = 0;
-        for (int i = 0; i < pd.nops; i++) {
-            pd.nbf += best_take[i].kind >= OP_BF;
-            pd.kind[i] = best_take[i].kind;
-            pd.lbit[i] = (uint8_t)bestW.loc(best_take[i].bit);
-            pd.gbit[i] = best_take[i].bit;
-        }
-        passes.push_back(pd);
-        rem.swap(best_skip);
-    }
-    return passes;
 }
 
 // --------------------------------------------------------- basis (host)
@@ -422,7 +609,20 @@ int ensure_basis() {
     GF2T_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_basis.mu);
     if (g_basis.uploaded_dev != dev) {
-        GF2T_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_basis), g_basis.b, sizeof(g_basis.b)));
+        static FftTables *tab = [] {
+            FftTables *t = new FftTables;
+            if (!cantor_host::build_tables(g_basis.b, *t)) {
+                delete t;
+                t = nullptr;
+            }
+            return t;
+        }();
+        if (!tab) {
+            gf2t::set_error("fft: the Cantor basis does not give the subfield towers");
+            return GF2T_EINTERNAL;
+        }
+        GF2T_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tab), tab, sizeof(FftTables)));
+        GF2T_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_tw), tab->tw, sizeof(tab->tw)));
         g_basis.uploaded_dev = dev;
     }
     return GF2T_OK;
@@ -431,102 +631,234 @@ int ensure_basis() {
 }  // namespace
 
 struct gf2t_fft_plan {
-    int m, T;   // 2^m points, tiles of 2^T elements
-    std::vector<PassDesc> fwd, inv;
+    int m, T;   // 2^m points, butterfly tiles of at most 2^T elements
 };
 
 namespace {
-constexpr int FFT_MAX_M = 27;
-std::mutex g_plan_mu;
-std::map<int, gf2t_fft_plan *> g_plans;   // key (m * 32 + T) * 8 + low bits
-
-// Tile bits per transform size: whole 8192-element tiles from 2^19 points
-// up; below that smaller tiles, so that a transform still spreads over
-// tens of workgroups (a 2^15-point transform in 8192-element tiles
-// occupies four CUs, each running 15 dependent butterfly levels).
-// Overridden per size by gf2t_tune("fft_tile_<m>", T), which is how the
-// autotuner installs what it measured.
-int default_tile_bits(int m) {
-    if (m >= 19) return FFT_TILE_BITS;
-    if (m >= 14) return 11;
-    return std::min(m, FFT_TILE_BITS);
-}
-std::atomic<int> g_tile_bits[FFT_MAX_M + 1];   // 0: default_tile_bits
+std::atomic<int> g_tile_bits[FFT_MAX_M + 1];   // 0: the default
+std::atomic<int> g_fft_ept{2};
+std::atomic<int> g_fft_low{FFT_LOW_BITS};
 
 int tile_bits_for(int m) {
     int T = g_tile_bits[m].load(std::memory_order_relaxed);
-    return T ? T : default_tile_bits(m);
+    return T ? T : std::min(m < 6 ? 6 : m, FFT_TILE_BITS);
 }
+gf2t_fft_plan plan_for(int m) { return gf2t_fft_plan{m, tile_bits_for(m)}; }
 
-// Threads of a pass over a 2^T-element tile: one per `ept` elements
-// (gf2t_tune "fft_ept": 2, 4, 8 or 16; default 2), between 64 and
-// FFT_THREADS.  Fewer threads per tile leave room for more blocks of
-// other launches on a CU (concurrent products of small transforms).
-std::atomic<int> g_fft_ept{2};
-
-// Low index bits of every pass's tile (gf2t_tune "fft_low_bits", 4..6):
-// runs of 2^c contiguous elements per HBM access of a tile
-std::atomic<int> g_fft_low{FFT_LOW_BITS};
-unsigned threads_for_tile(int T) {
-    const u64 ept = (u64)g_fft_ept.load(std::memory_order_relaxed);
-    return (unsigned)std::max<u64>(64, std::min<u64>(FFT_THREADS, (1ULL << (T > 0 ? T : 0)) / ept));
+// the conversion plans by size, built once
+const cantor_host::ConvPlan &conv_plan32(int k) {
+    static const std::vector<cantor_host::ConvPlan> v = [] {
+        std::vector<cantor_host::ConvPlan> p;
+        for (int j = 0; j <= FFT_MAX_M; j++)
+            p.push_back(cantor_host::conv_plan(j, CONV_ONE_TILE, CONV_TILE32));
+        return p;
+    }();
+    return v[k];
 }
-
-const gf2t_fft_plan *cached_plan_T(int m, int T) {
-    T = std::max(FFT_MIN_TILE_BITS, std::min(T, FFT_TILE_BITS));
-    const int c = g_fft_low.load(std::memory_order_relaxed);
-    const int key = (m * 32 + T) * 8 + c;
-    std::lock_guard<std::mutex> lk(g_plan_mu);
-    auto it = g_plans.find(key);
-    if (it != g_plans.end()) return it->second;
-    gf2t_fft_plan *p = new gf2t_fft_plan{m, T, schedule(m, true, T, c), schedule(m, false, T, c)};
-    g_plans[key] = p;
-    return p;
+const cantor_host::ConvPlan &conv_plan64(int k) {
+    static const std::vector<cantor_host::ConvPlan> v = [] {
+        std::vector<cantor_host::ConvPlan> p;
+        for (int j = 0; j <= FFT_MAX_M; j++)
+            p.push_back(cantor_host::conv_plan(j, CONV_ONE_TILE, CONV_TILE64));
+        return p;
+    }();
+    return v[k];
 }
-const gf2t_fft_plan *cached_plan(int m) { return cached_plan_T(m, tile_bits_for(m)); }
-
-// Run the passes of one transform (or of nbatch transforms f_stride words
-// apart, blockIdx.y selecting one); pk (may be null) packs the first
-// pass's input.
-int run_passes(const std::vector<PassDesc> &ps, u64 *df, hipStream_t st, const PackArg *pk,
-               unsigned nbatch = 1, u64 f_stride = 0) {
-    static std::once_flag lds_once;
-    static hipError_t lds_err = hipSuccess;
-    std::call_once(lds_once, [] {
-        lds_err = hipFuncSetAttribute((const void *)k_fft_pass,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)((4 * 256 + ((size_t)1 << FFT_TILE_BITS)) * sizeof(u64)));
-    });
-    GF2T_HIP(lds_err);
-    if (nbatch == 0) return GF2T_OK;
-    if (pk && pk->nlist && nbatch > (unsigned)pk->nlist) {
-        gf2t::set_error("fft: %u transforms but %d pack sources", nbatch, pk->nlist);
-        return GF2T_EINTERNAL;
+TileArg tile_arg(const std::vector<cantor_host::TileOp> &ops, int T, bool inv) {
+    TileArg a{};
+    a.T = T;
+    a.nops = (int)ops.size();
+    for (int i = 0; i < a.nops; i++) {
+        const auto &op = ops[inv ? a.nops - 1 - i : i];
+        a.h[i] = (signed char)op.h;
+        a.pos[i] = (signed char)op.pos;
     }
-    PackArg none{};
-    for (size_t i = 0; i < ps.size(); i++) {
-        const PassDesc &pd = ps[i];
-        const int T = pd.c + pd.w;
-        const int ntab = std::max(1, std::min(4, (pd.m - 1 + 7) / 8));
-        const unsigned blocks = (unsigned)(1ULL << (pd.m - T));
-        const unsigned threads = threads_for_tile(T);
-        const size_t lds = (4 * 256 + ((size_t)1 << T)) * sizeof(u64);
-        const bool pack = i == 0 && pk;
-        hipLaunchKernelGGL(k_fft_pass, dim3(blocks, nbatch), dim3(threads), lds, st, df, pd,
-                           pack ? *pk : none, pack ? 1 : 0, ntab, f_stride);
+    return a;
+}
+dim3 step_grid(const ConvStep &s, int k, unsigned nbatch, u32 &colblocks) {
+    colblocks = (conv_full(s) + CONV_THREADS - 1) / CONV_THREADS;
+    const u32 unit = 1u << s.ub;
+    const u32 edges = unit < CONV_EDGE_RHO ? 1 : unit / CONV_EDGE_RHO;
+    return dim3(colblocks + edges, 1u << (k - s.hb - s.K), nbatch);
+}
+size_t group_lds(const ConvGroup &g, size_t elem) {
+    return g.off && g.w <= 6 ? 0 : (((size_t)1 << g.tb) + ((size_t)1 << g.tb) / 64) * elem;
+}
+unsigned tile_threads(int T) { return (unsigned)std::max(64, std::min(1024, 1 << (T - 1))); }
+
+// basis conversion of nbatch operands of at most 2^k chunks, into their
+// lch buffers; ran: whether anything was launched (k > 1)
+int run_conv32(const Operands &ops, int k, unsigned nbatch, hipStream_t st, bool &ran) {
+    const cantor_host::ConvPlan &P = conv_plan32(k);
+    ran = !P.empty();
+    int first = 1;
+    if (!P.tile.empty())
+        hipLaunchKernelGGL(k_conv_tile32, dim3(1, nbatch), dim3(tile_threads(k)), (size_t)4 << k,
+                           st, ops, tile_arg(P.tile, k, false), first);
+    for (const ConvStep &s : P.steps) {
+        u32 cb;
+        const dim3 g = step_grid(s, k, nbatch, cb);
+        switch (s.K) {
+        case 1: hipLaunchKernelGGL(k_conv_step32<1>, g, dim3(CONV_THREADS), 0, st, ops, s, cb, first); break;
+        case 2: hipLaunchKernelGGL(k_conv_step32<2>, g, dim3(CONV_THREADS), 0, st, ops, s, cb, first); break;
+        case 3: hipLaunchKernelGGL(k_conv_step32<3>, g, dim3(CONV_THREADS), 0, st, ops, s, cb, first); break;
+        default: hipLaunchKernelGGL(k_conv_step32<4>, g, dim3(CONV_THREADS), 0, st, ops, s, cb, first); break;
+        }
+        first = 0;
     }
-    GF2T_CHECK_LAUNCH("k_fft_pass");
+    for (const ConvGroup &g : P.groups) {
+        hipLaunchKernelGGL(k_conv_group32, dim3(1u << (k - g.tb), nbatch), dim3(1u << (g.tb - 6)),
+                           group_lds(g, 4), st, ops, g, first);
+        first = 0;
+    }
+    GF2T_CHECK_LAUNCH("k_conv32");
     return GF2T_OK;
 }
-
-PackArg pack_one(const u64 *src, u64 bits, u32 xor0 = 0) {
-    PackArg p{};
-    p.src = (const u32 *)src;
-    p.nchunks = (bits + 31) >> 5;
-    p.lastmask = (bits & 31) ? (u32)((1ULL << (bits & 31)) - 1) : 0xFFFFFFFFu;
-    p.xor0 = xor0;
-    return p;
+template <bool INV>
+int run_conv64(u64 *f, u64 stride, int m, unsigned nbatch, hipStream_t st) {
+    const cantor_host::ConvPlan &P = conv_plan64(m);
+    auto step = [&](const ConvStep &s) {
+        u32 cb;
+        const dim3 g = step_grid(s, m, nbatch, cb);
+        switch (s.K) {
+        case 1: hipLaunchKernelGGL((k_conv_step64<1, INV>), g, dim3(CONV_THREADS), 0, st, f, stride, s, cb); break;
+        case 2: hipLaunchKernelGGL((k_conv_step64<2, INV>), g, dim3(CONV_THREADS), 0, st, f, stride, s, cb); break;
+        case 3: hipLaunchKernelGGL((k_conv_step64<3, INV>), g, dim3(CONV_THREADS), 0, st, f, stride, s, cb); break;
+        default: hipLaunchKernelGGL((k_conv_step64<4, INV>), g, dim3(CONV_THREADS), 0, st, f, stride, s, cb); break;
+        }
+    };
+    auto group = [&](const ConvGroup &g) {
+        hipLaunchKernelGGL(k_conv_group64<INV>, dim3(1u << (m - g.tb), nbatch),
+                           dim3(1u << (g.tb - 6)), group_lds(g, 8), st, f, stride, g);
+    };
+    if (!P.tile.empty())
+        hipLaunchKernelGGL(k_conv_tile64<INV>, dim3(1, nbatch), dim3(tile_threads(m)),
+                           (size_t)8 << m, st, f, stride, tile_arg(P.tile, m, INV));
+    if (!INV) {
+        for (const ConvStep &s : P.steps) step(s);
+        for (const ConvGroup &g : P.groups) group(g);
+    } else {
+        for (size_t i = P.groups.size(); i--;) group(P.groups[i]);
+        for (size_t i = P.steps.size(); i--;) step(P.steps[i]);
+    }
+    GF2T_CHECK_LAUNCH("k_conv64");
+    return GF2T_OK;
 }
+// butterfly passes above the low eight levels, all of nbatch transforms
+// stride words apart
+std::vector<BfPass> passes_for(const gf2t_fft_plan &pl, unsigned nbatch) {
+    // smaller tiles until the launch fills the chip
+    int tile = std::min(8 + RB, std::max(pl.T - 1, 6));
+    while (tile > 6 + RB && ((((u64)1 << (pl.m - 1)) >> tile) * nbatch) < 1024) tile--;
+    return cantor_host::bf_passes(pl.m, tile);
+}
+template <int CLS, bool INV>
+void launch_bfly(u64 *f, u64 stride, const BfPass &P, const Operands &ops, int in, int out,
+                 unsigned nbatch, hipStream_t st) {
+    size_t body = P.w > RB ? ((size_t)16 << P.tb) : 0;
+    if (in == IO_PLAIN || out == IO_PLAIN) body = std::max<size_t>(body, 16384);
+    else if (in != IO_UNITS) body = std::max<size_t>(body, 8192);
+    hipLaunchKernelGGL((k_bfly<CLS, INV>), dim3(1u << (P.m - 1 - P.tb), nbatch),
+                       dim3(1u << (P.tb - RB)), sizeof(MulLds) + body, st, f, stride, P, ops, in,
+                       out);
+}
+template <bool INV>
+void run_bfly(u64 *f, u64 stride, const BfPass &P, const Operands &ops, int in, int out,
+                 unsigned nbatch, hipStream_t st) {
+    switch (cantor_host::bf_class(P)) {
+    case 8: launch_bfly<8, INV>(f, stride, P, ops, in, out, nbatch, st); break;
+    case 16: launch_bfly<16, INV>(f, stride, P, ops, in, out, nbatch, st); break;
+    default: launch_bfly<32, INV>(f, stride, P, ops, in, out, nbatch, st); break;
+    }
+}
+template <int DIR>
+void run_low(u64 *f, u64 stride, const u64 *g, int m, const Operands &ops, u32 g_op, int in,
+                int out, unsigned nbatch, hipStream_t st) {
+    const u32 waves = std::max<u32>(1, (1u << (m - 1)) / LO_UNITS);
+    const u32 wpb = (u64)waves * nbatch >= 4096 ? 4 : (u64)waves * nbatch >= 1024 ? 2 : 1;
+    const u32 blocks = (waves + wpb - 1) / wpb;
+    size_t lds = sizeof(MulLds) + 4 * sizeof(TwEnt) + (DIR == LO_MUL ? sizeof(ProdLds) : 0) +
+                 wpb * LO_EXCH * 4;
+    if (in == IO_PLAIN || out == IO_PLAIN) lds += 16384;
+    else if (in != IO_UNITS) lds += 8192;
+    const dim3 gr(blocks, nbatch), th(64 * wpb);
+    if (m <= 16)
+        hipLaunchKernelGGL((k_low<16, 16, DIR>), gr, th, lds, st, f, stride, g, m, ops, g_op, in, out);
+    else if (m <= 24 - RB)
+        hipLaunchKernelGGL((k_low<16, 32, DIR>), gr, th, lds, st, f, stride, g, m, ops, g_op, in, out);
+    else
+        hipLaunchKernelGGL((k_low<32, 32, DIR>), gr, th, lds, st, f, stride, g, m, ops, g_op, in, out);
+}
+// Forward transforms of nbatch operands (at most 2^k chunks each) at f, f
+// + stride, ... as units; low: the low levels too
+int run_forward(const gf2t_fft_plan &pl, u64 *f, u64 stride, const Operands &ops, int k,
+                unsigned nbatch, bool low, hipStream_t st, int &in) {
+    bool ran;
+    int rc = run_conv32(ops, k, nbatch, st, ran);
+    if (rc) return rc;
+    in = ran ? IO_LCH : IO_CHUNKS;
+    for (const BfPass &P : passes_for(pl, nbatch)) {
+        run_bfly<false>(f, stride, P, ops, in, IO_UNITS, nbatch, st);
+        in = IO_UNITS;
+    }
+    if (low) {
+        run_low<LO_FWD>(f, stride, nullptr, pl.m, ops, 0, in, IO_UNITS, nbatch, st);
+        in = IO_UNITS;
+    }
+    GF2T_CHECK_LAUNCH("fft forward");
+    return GF2T_OK;
+}
+// the rest of an inverse whose low levels are done (low: still to do), and
+// the conversion back: coefficients in the polynomial basis
+int run_inverse(const gf2t_fft_plan &pl, u64 *f, u64 stride, unsigned nbatch, bool low, int in,
+                hipStream_t st) {
+    const Operands none{};
+    std::vector<BfPass> ps = passes_for(pl, nbatch);
+    if (low) {
+        run_low<LO_INV>(f, stride, nullptr, pl.m, none, 0, in, ps.empty() ? IO_PLAIN : IO_UNITS,
+                        nbatch, st);
+        in = IO_UNITS;
+    }
+    for (size_t i = ps.size(); i--;)
+        run_bfly<true>(f, stride, ps[i], none, IO_UNITS, i ? IO_UNITS : IO_PLAIN, nbatch, st);
+    GF2T_CHECK_LAUNCH("fft inverse");
+    return run_conv64<true>(f, stride, pl.m, nbatch, st);
+}
+// Products of nbatch operand pairs (operands y and nbatch + y of ops, at
+// most 2^k chunks): transforms at f + y stride and g + y stride, the
+// product's coefficients modulo the vanishing polynomial of the 2^m
+// points at f + y stride, in the polynomial basis.  g - f = nbatch stride.
+int run_product(const gf2t_fft_plan &pl, u64 *f, u64 stride, const Operands &ops, int k,
+                unsigned nbatch, hipStream_t st) {
+    int in;
+    int rc = run_forward(pl, f, stride, ops, k, 2 * nbatch, false, st, in);
+    if (rc) return rc;
+    run_low<LO_MUL>(f, stride, f + (u64)nbatch * stride, pl.m, ops, nbatch, in,
+                    pl.m <= 8 ? IO_PLAIN : IO_UNITS, nbatch, st);
+    GF2T_CHECK_LAUNCH("k_low");
+    return run_inverse(pl, f, stride, nbatch, false, IO_UNITS, st);
+}
+
+u32 last_mask(u64 bits) { return (bits & 31) ? (u32)((1ULL << (bits & 31)) - 1) : 0xFFFFFFFFu; }
+
+// operand of `bits` bits, its converted chunks at lch
+Operand operand_of(const u64 *src, u64 bits, void *lch, u32 xor0 = 0) {
+    return Operand{(const u32 *)src, (u32 *)lch, (bits + 31) >> 5, last_mask(bits), xor0};
+}
+// the chunks [first, first + count) of operand o
+Operand operand_range(Operand o, u64 first, u64 count) {
+    if (first + count != o.n) o.mask = 0xFFFFFFFFu;
+    if (first) o.xor0 = 0;
+    o.src += first;
+    o.n = count;
+    return o;
+}
+int log2_ceil(u64 n) {
+    int k = 0;
+    while (((u64)1 << k) < n) k++;
+    return k;
+}
+u64 round4(u64 n) { return (n + 3) & ~(u64)3; }
 
 int fft_m_for(u64 nchunks_total) {
     int m = 1;
@@ -536,9 +868,9 @@ int fft_m_for(u64 nchunks_total) {
 
 }  // namespace
 
-// gf2t_tune("fft_tile_<m>", T): tiles of 2^T elements (6..13) for 2^m-point
-// transforms from now on; 0 restores the default.  Plans already made
-// keep theirs.
+// gf2t_tune("fft_tile_<m>", T): butterfly tiles of at most 2^T elements
+// (6..13) for 2^m-point transforms from now on; 0 restores the default.
+// Plans already made keep theirs.
 int gf2t_fft_set_tile_bits(int m, int64_t T) {
     if (m < 1 || m > FFT_MAX_M || (T != 0 && (T < FFT_MIN_TILE_BITS || T > FFT_TILE_BITS))) {
         gf2t::set_error("gf2t_tune: fft_tile_<m> needs 1 <= m <= %d and T = 0 or %d..%d",
@@ -585,9 +917,7 @@ extern "C" int gf2t_fft_plan_create(int m, gf2t_fft_plan **plan) {
         gf2t::set_error("gf2t_fft_plan_create: basis length %d < m", g_basis.len);
         return GF2T_EINTERNAL;
     }
-    const int T = std::max(FFT_MIN_TILE_BITS, std::min(tile_bits_for(m), FFT_TILE_BITS));
-    const int c = g_fft_low.load(std::memory_order_relaxed);
-    *plan = new gf2t_fft_plan{m, T, schedule(m, true, T, c), schedule(m, false, T, c)};
+    *plan = new gf2t_fft_plan(plan_for(m));
     return GF2T_OK;
 }
 
@@ -598,8 +928,9 @@ extern "C" int gf2t_fft_plan_destroy(gf2t_fft_plan *plan) {
 
 extern "C" int gf2t_fft_plan_passes(const gf2t_fft_plan *plan, int *fwd_passes, int *inv_passes) {
     if (!plan) return GF2T_EINVAL;
-    if (fwd_passes) *fwd_passes = (int)plan->fwd.size();
-    if (inv_passes) *inv_passes = (int)plan->inv.size();
+    const size_t n = conv_plan64(plan->m).launches() + passes_for(*plan, 1).size() + 1;
+    if (fwd_passes) *fwd_passes = (int)n;
+    if (inv_passes) *inv_passes = (int)n;
     return GF2T_OK;
 }
 
@@ -607,14 +938,25 @@ extern "C" int gf2t_fft_fwd(const gf2t_fft_plan *plan, uint64_t *df, void *strea
     if (!plan || !df) return GF2T_EINVAL;
     int rc = ensure_basis();
     if (rc) return rc;
-    return run_passes(plan->fwd, df, (hipStream_t)stream, nullptr);
+    hipStream_t st = (hipStream_t)stream;
+    rc = run_conv64<false>(df, 0, plan->m, 1, st);
+    if (rc) return rc;
+    const Operands none{};
+    int in = IO_PLAIN;
+    for (const BfPass &P : passes_for(*plan, 1)) {
+        run_bfly<false>(df, 0, P, none, in, IO_UNITS, 1, st);
+        in = IO_UNITS;
+    }
+    run_low<LO_FWD>(df, 0, nullptr, plan->m, none, 0, in, IO_PLAIN, 1, st);
+    GF2T_CHECK_LAUNCH("gf2t_fft_fwd");
+    return GF2T_OK;
 }
 
 extern "C" int gf2t_fft_inv(const gf2t_fft_plan *plan, uint64_t *df, void *stream) {
     if (!plan || !df) return GF2T_EINVAL;
     int rc = ensure_basis();
     if (rc) return rc;
-    return run_passes(plan->inv, df, (hipStream_t)stream, nullptr);
+    return run_inverse(*plan, df, 0, 1, true, IO_PLAIN, (hipStream_t)stream);
 }
 
 extern "C" size_t gf2t_mul_out_words(uint64_t abits, uint64_t bbits) {
@@ -729,16 +1071,6 @@ __global__ void k_overlap_add_wrap(const u64 *__restrict__ R, u64 r_stride,
     out[wd] = v;
 }
 
-// pack source of chunks [first, first + count) of an operand of nch chunks
-// whose last chunk is masked to lastmask
-PackArg pack_range(const u32 *src, u64 first, u64 count, u64 nch, u32 lastmask) {
-    PackArg p{};
-    p.src = src + first;
-    p.nchunks = count;
-    p.lastmask = first + count == nch ? lastmask : 0xFFFFFFFFu;
-    return p;
-}
-
 int mul_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 *dprod, void *dwork,
              hipStream_t st) {
     u64 ca = (abits + 31) >> 5, cb = (bbits + 31) >> 5;
@@ -751,36 +1083,28 @@ int mul_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 *dprod, voi
     }
     int rc = ensure_basis();
     if (rc) return rc;
+    // the converted chunks of both operands, behind the two transforms
+    // (where the product goes later, or the workspace's tail)
+    const size_t n = (size_t)1 << m;
+    u64 *FA = (u64 *)dwork;
+    u32 *lch = (u32 *)(FA + 2 * n);
+    Operands two{};
+    two.op[0] = operand_of(da, abits, lch);
+    two.op[1] = operand_of(db, bbits, lch + round4(ca));
+    const int k = log2_ceil(std::max(ca, cb));
     const Wrap W = wrap_for(ca, cb);
     if (W.on) {
         // both operands at 2^mp points, their top e chunks at 2^ms points
         // (2^mp + 2^ms <= 2^m words each, inside the workspace of an
         // unwrapped product)
-        const gf2t_fft_plan *pl = cached_plan(W.mp), *ps = cached_plan(W.ms);
-        const size_t n = (size_t)1 << W.mp, ns = (size_t)1 << W.ms;
-        u64 *FA = (u64 *)dwork, *FB = FA + n, *TA = FB + n, *TB = TA + ns;
-        const PackArg pa = pack_one(da, abits), pb = pack_one(db, bbits);
-        PackArg two{};
-        two.nlist = 2;
-        two.lsrc[0] = pa.src; two.lnch[0] = pa.nchunks; two.lmask[0] = pa.lastmask;
-        two.lsrc[1] = pb.src; two.lnch[1] = pb.nchunks; two.lmask[1] = pb.lastmask;
-        rc = run_passes(pl->fwd, FA, st, &two, 2, n);
+        const size_t np = (size_t)1 << W.mp, ns = (size_t)1 << W.ms;
+        u64 *TA = FA + 2 * np;
+        Operands top{};
+        top.op[0] = operand_range(two.op[0], ca - W.e, W.e);
+        top.op[1] = operand_range(two.op[1], cb - W.e, W.e);
+        rc = run_product(plan_for(W.mp), FA, np, two, k, 1, st);
         if (rc) return rc;
-        const PackArg ta = pack_range(pa.src, ca - W.e, W.e, ca, pa.lastmask);
-        const PackArg tb = pack_range(pb.src, cb - W.e, W.e, cb, pb.lastmask);
-        PackArg top{};
-        top.nlist = 2;
-        top.lsrc[0] = ta.src; top.lnch[0] = ta.nchunks; top.lmask[0] = ta.lastmask;
-        top.lsrc[1] = tb.src; top.lnch[1] = tb.nchunks; top.lmask[1] = tb.lastmask;
-        rc = run_passes(ps->fwd, TA, st, &top, 2, ns);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_pointwise, dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)),
-                           dim3(256), 0, st, FA, FB, n);
-        hipLaunchKernelGGL(k_pointwise, dim3((unsigned)std::min<size_t>((ns + 255) / 256, 8192)),
-                           dim3(256), 0, st, TA, TB, ns);
-        rc = run_passes(pl->inv, FA, st, nullptr);
-        if (rc) return rc;
-        rc = run_passes(ps->inv, TA, st, nullptr);
+        rc = run_product(plan_for(W.ms), TA, ns, top, log2_ceil(W.e), 1, st);
         if (rc) return rc;
         // C_high[u] = coefficient e - 1 + u of the top product
         hipLaunchKernelGGL(k_overlap_add_wrap, dim3((unsigned)((ow + 255) / 256)), dim3(256), 0,
@@ -789,20 +1113,7 @@ int mul_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 *dprod, voi
         GF2T_CHECK_LAUNCH("k_overlap_add_wrap");
         return GF2T_OK;
     }
-    const gf2t_fft_plan *plan = cached_plan(m);
-    size_t n = (size_t)1 << m;
-    u64 *FA = (u64 *)dwork, *FB = FA + n;
-    // both operands in one launch chain: FA and FB are n words apart
-    const PackArg pa = pack_one(da, abits), pb = pack_one(db, bbits);
-    PackArg two{};
-    two.nlist = 2;
-    two.lsrc[0] = pa.src; two.lnch[0] = pa.nchunks; two.lmask[0] = pa.lastmask;
-    two.lsrc[1] = pb.src; two.lnch[1] = pb.nchunks; two.lmask[1] = pb.lastmask;
-    rc = run_passes(plan->fwd, FA, st, &two, 2, n);
-    if (rc) return rc;
-    unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_pointwise, dim3(blocks), dim3(256), 0, st, FA, FB, n);
-    rc = run_passes(plan->inv, FA, st, nullptr);
+    rc = run_product(plan_for(m), FA, n, two, k, 1, st);
     if (rc) return rc;
     hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256)), dim3(256), 0, st, FA,
                        (size_t)(ca + cb - 1), dprod, ow, (u64)0, (u64)0);
@@ -896,7 +1207,8 @@ int gf2t_noalloc_setup() {
             g_scratch_ptr[dev] = (u64 *)p;
         }
     }
-    for (int m = 1; m <= NA_MAX_M; m++) cached_plan(m);
+    conv_plan32(0);
+    conv_plan64(0);
     return ensure_basis();
 }
 
@@ -957,11 +1269,10 @@ extern "C" int gf2t_mulmod_noalloc(const uint64_t *da, uint64_t abits, const uin
 // each.  Each product keeps its own transform size and tile.
 namespace {
 struct PairSeg {       // one pair's part of a flat grouped launch over elements
-    u64 *fa;
-    const u64 *fb;
+    const u64 *fa;
     u64 *prod;
     u64 *out;
-    u64 n, nch, ow, pw, L, s, start;   // start: the pair's first element in the launch
+    u64 nch, ow, pw, L, s, start;   // start: the pair's first element in the launch
 };
 
 GF2T_DEV int find_seg(const PairSeg *__restrict__ sg, int np, u64 i) {
@@ -973,8 +1284,8 @@ GF2T_DEV int find_seg(const PairSeg *__restrict__ sg, int np, u64 i) {
     return lo;
 }
 
-// phase 0: FA *= FB pointwise; 1: overlap-add FA into prod; 2: fold prod
-// into out.  total = sum of the pairs' element counts for the phase.
+// phase 0: overlap-add FA into prod; 1: fold prod into out.  total = sum
+// of the pairs' element counts for the phase.
 __global__ void k_pairs_grouped(const PairSeg *__restrict__ sg, int np, u64 total, int phase,
                                 u64 r) {
     u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
@@ -983,8 +1294,6 @@ __global__ void k_pairs_grouped(const PairSeg *__restrict__ sg, int np, u64 tota
         const PairSeg &S = sg[find_seg(sg, np, i)];
         const u64 k = i - S.start;
         if (phase == 0) {
-            S.fa[k] = gf64_mul(S.fa[k], S.fb[k]);
-        } else if (phase == 1) {
             const u64 c = 2 * k;
             u64 v = 0;
             if (c < S.nch) v ^= S.fa[c];
@@ -997,44 +1306,55 @@ __global__ void k_pairs_grouped(const PairSeg *__restrict__ sg, int np, u64 tota
     }
 }
 
+// Pairs of one transform size run as one chain of launches, their A
+// transforms side by side and the B transforms behind them.
+struct BatchGroup {
+    int m;
+    std::vector<int> pairs;
+    size_t f;   // word offset of the group's transforms
+};
 struct BatchLayout {
-    std::vector<size_t> fa, prod;   // word offsets of each pair's transforms and product
+    std::vector<BatchGroup> groups;
+    std::vector<size_t> fa, prod;   // word offsets of each pair's A transform and product
     std::vector<int> m;
     size_t desc_off = 0, words = 0;
 };
 
-BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits, size_t ndesc_bytes) {
+BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
     BatchLayout L;
-    size_t off = 0;
+    L.fa.resize(n);
     for (int j = 0; j < n; j++) {
         u64 ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
-        int m = (ca && cb) ? fft_m_for(ca + cb - 1) : 0;
-        L.m.push_back(m);
-        L.fa.push_back(off);
-        off += m ? 2 * ((size_t)1 << m) : 0;
+        L.m.push_back((ca && cb) ? fft_m_for(ca + cb - 1) : 0);
+    }
+    size_t off = 0;
+    for (int m = FFT_MAX_M; m >= 1; m--) {
+        BatchGroup g{m, {}, off};
+        for (int j = 0; j < n; j++)
+            if (L.m[j] == m) {
+                L.fa[j] = off + (g.pairs.size() << m);
+                g.pairs.push_back(j);
+            }
+        if (g.pairs.empty()) continue;
+        off += 2 * g.pairs.size() << m;
+        L.groups.push_back(g);
+    }
+    for (int j = 0; j < n; j++) {
         L.prod.push_back(off);
-        off += (gf2t_mul_out_words(abits[j], bbits[j]) + 31) & ~(size_t)31;
+        // the product, and before it both operands' converted chunks
+        off += (gf2t_mul_out_words(abits[j], bbits[j]) + 4 + 31) & ~(size_t)31;
     }
     L.desc_off = off;
-    L.words = off + (ndesc_bytes + 7) / 8 + 32;
+    const size_t desc = (size_t)n * 2 * (sizeof(Operand) + sizeof(PairSeg)) + 256;
+    L.words = off + (desc + 7) / 8 + 32;
     return L;
-}
-
-// room for the descriptors whatever tiles the plans use: a pass holds at
-// least one op, so a transform has at most m(m+1)/2 passes each way
-size_t batch_desc_bytes(int n, const std::vector<int> &ms) {
-    size_t steps = 0;
-    for (int m : ms)
-        if (m) steps += 2 * (size_t)(m * (m + 1) / 2);
-    return steps * sizeof(GroupPass) + (size_t)n * 3 * sizeof(PairSeg) + 256;
 }
 }  // namespace
 
 extern "C" size_t gf2t_mulmod_batch_workspace_bytes(int n, const uint64_t *abits,
                                                    const uint64_t *bbits) {
     if (n <= 0 || !abits || !bbits) return 0;
-    BatchLayout L0 = batch_layout(n, abits, bbits, 0);
-    return batch_layout(n, abits, bbits, batch_desc_bytes(n, L0.m)).words * 8;
+    return batch_layout(n, abits, bbits).words * 8;
 }
 
 extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_t *abits,
@@ -1063,56 +1383,20 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     int rc = ensure_basis();
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    BatchLayout L0 = batch_layout(n, abits, bbits, 0);
-    BatchLayout L = batch_layout(n, abits, bbits, batch_desc_bytes(n, L0.m));
+    const BatchLayout L = batch_layout(n, abits, bbits);
     u64 *W = (u64 *)dwork;
-    // the steps of the grouped launches: forward passes, then inverse
-    std::vector<const gf2t_fft_plan *> plan(n, nullptr);
-    size_t maxf = 0, maxi = 0;
-    for (int j = 0; j < n; j++)
-        if (L.m[j]) {
-            plan[j] = cached_plan(L.m[j]);
-            maxf = std::max(maxf, plan[j]->fwd.size());
-            maxi = std::max(maxi, plan[j]->inv.size());
-        }
-    std::vector<GroupPass> desc;
-    struct Step { size_t first; int count; u32 blocks; int T; };
-    std::vector<Step> steps;
-    for (int dir = 0; dir < 2; dir++) {
-        const size_t ns = dir ? maxi : maxf;
-        for (size_t i = 0; i < ns; i++) {
-            Step S{desc.size(), 0, 0, 0};
-            for (int j = 0; j < n; j++) {
-                if (!plan[j]) continue;
-                const std::vector<PassDesc> &ps = dir ? plan[j]->inv : plan[j]->fwd;
-                if (i >= ps.size()) continue;
-                GroupPass g{};
-                g.pd = ps[i];
-                const size_t nn = (size_t)1 << L.m[j];
-                g.f = W + L.fa[j];
-                g.f_stride = nn;
-                g.ntrans = dir ? 1 : 2;
-                g.pack = (!dir && i == 0) ? 1 : 0;
-                g.src[0] = (const u32 *)da[j];
-                g.src[1] = (const u32 *)db[j];
-                g.nch[0] = (abits[j] + 31) >> 5;
-                g.nch[1] = (bbits[j] + 31) >> 5;
-                g.mask[0] = (abits[j] & 31) ? (u32)((1ULL << (abits[j] & 31)) - 1) : 0xFFFFFFFFu;
-                g.mask[1] = (bbits[j] & 31) ? (u32)((1ULL << (bbits[j] & 31)) - 1) : 0xFFFFFFFFu;
-                g.ntab = std::max(1, std::min(4, (L.m[j] - 1 + 7) / 8));
-                const int T = g.pd.c + g.pd.w;
-                g.nblocks = (u32)(1ULL << (g.pd.m - T));
-                g.block0 = S.blocks;
-                S.blocks += g.nblocks * g.ntrans;
-                S.T = std::max(S.T, T);
-                S.count++;
-                desc.push_back(g);
+    // the operands, group by group: the A's, then the B's
+    std::vector<Operand> opv;
+    for (const BatchGroup &g : L.groups)
+        for (int o = 0; o < 2; o++)
+            for (int j : g.pairs) {
+                u32 *lch = (u32 *)(W + L.prod[j]);
+                opv.push_back(o ? operand_of(db[j], bbits[j],
+                                             lch + round4((abits[j] + 31) >> 5))
+                                : operand_of(da[j], abits[j], lch));
             }
-            steps.push_back(S);
-        }
-    }
-    std::vector<PairSeg> seg[3];
-    u64 total[3] = {0, 0, 0};
+    std::vector<PairSeg> seg[2];
+    u64 total[2] = {0, 0};
     int nz = 0;
     for (int j = 0; j < n; j++) {
         const size_t nw = words_of(r);
@@ -1122,21 +1406,19 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
             nz++;
             continue;
         }
-        const u64 nn = 1ULL << L.m[j], ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
+        const u64 ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
         const u64 ow = gf2t_mul_out_words(abits[j], bbits[j]);
         PairSeg p{};
         p.fa = W + L.fa[j];
-        p.fb = p.fa + nn;
         p.prod = W + L.prod[j];
         p.out = dout[j];
-        p.n = nn;
         p.nch = ca + cb - 1;
         p.ow = ow;
         p.pw = ow;
         p.L = abits[j] + bbits[j] - 1;
         p.s = s[j];
-        const u64 cnt[3] = {nn, ow, (u64)nw};
-        for (int ph = 0; ph < 3; ph++) {
+        const u64 cnt[2] = {ow, (u64)nw};
+        for (int ph = 0; ph < 2; ph++) {
             p.start = total[ph];
             total[ph] += cnt[ph];
             seg[ph].push_back(p);
@@ -1144,44 +1426,35 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     }
     const int np = n - nz;
     if (np == 0) return GF2T_OK;
-    // descriptors: the pass entries, then the three segment tables
-    std::vector<unsigned char> host(desc.size() * sizeof(GroupPass) + 3 * np * sizeof(PairSeg));
-    std::memcpy(host.data(), desc.data(), desc.size() * sizeof(GroupPass));
-    for (int ph = 0; ph < 3; ph++)
-        std::memcpy(host.data() + desc.size() * sizeof(GroupPass) + ph * np * sizeof(PairSeg),
-                    seg[ph].data(), np * sizeof(PairSeg));
+    // descriptors: the operands, then the two segment tables
+    const size_t ob = opv.size() * sizeof(Operand);
+    std::vector<unsigned char> host(ob + 2 * np * sizeof(PairSeg));
+    std::memcpy(host.data(), opv.data(), ob);
+    for (int ph = 0; ph < 2; ph++)
+        std::memcpy(host.data() + ob + ph * np * sizeof(PairSeg), seg[ph].data(),
+                    np * sizeof(PairSeg));
     unsigned char *dd = (unsigned char *)(W + L.desc_off);
     dd = (unsigned char *)(((uintptr_t)dd + 255) & ~(uintptr_t)255);
     GF2T_HIP(hipMemcpyAsync(dd, host.data(), host.size(), hipMemcpyHostToDevice, st));
     GF2T_HIP(hipStreamSynchronize(st));   // `host` is a pageable local buffer
-    const GroupPass *dgp = (const GroupPass *)dd;
-    const PairSeg *dseg = (const PairSeg *)(dd + desc.size() * sizeof(GroupPass));
-    static std::once_flag lds_once;
-    static hipError_t lds_err = hipSuccess;
-    std::call_once(lds_once, [] {
-        lds_err = hipFuncSetAttribute((const void *)k_fft_pass_grouped,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)((4 * 256 + ((size_t)1 << FFT_TILE_BITS)) * sizeof(u64)));
-    });
-    GF2T_HIP(lds_err);
-    auto grouped_phase = [&](int ph) {
-        const u64 tot = total[ph];
-        unsigned blocks = (unsigned)std::min<u64>((tot + 255) / 256, 65536);
-        hipLaunchKernelGGL(k_pairs_grouped, dim3(blocks), dim3(256), 0, st, dseg + ph * np, np,
-                           tot, ph, (u64)r);
-    };
-    for (size_t k = 0; k < steps.size(); k++) {
-        if (k == maxf) grouped_phase(0);   // between the forward and inverse passes
-        const Step &S = steps[k];
-        const size_t lds = (4 * 256 + ((size_t)1 << S.T)) * sizeof(u64);
-        const unsigned threads =
-            threads_for_tile(S.T);
-        hipLaunchKernelGGL(k_fft_pass_grouped, dim3(S.blocks), dim3(threads), lds, st,
-                           dgp + S.first, S.count);
+    const Operand *dop = (const Operand *)dd;
+    const PairSeg *dseg = (const PairSeg *)(dd + ob);
+    size_t first = 0;
+    for (const BatchGroup &g : L.groups) {
+        const unsigned cnt = (unsigned)g.pairs.size();
+        u64 most = 1;
+        for (int j : g.pairs)
+            most = std::max(most, std::max((abits[j] + 31) >> 5, (bbits[j] + 31) >> 5));
+        Operands ops{};
+        ops.list = dop + first;
+        rc = run_product(plan_for(g.m), W + g.f, (u64)1 << g.m, ops, log2_ceil(most), cnt, st);
+        if (rc) return rc;
+        first += 2 * cnt;
     }
-    if (steps.size() == maxf) grouped_phase(0);
-    grouped_phase(1);
-    grouped_phase(2);
+    for (int ph = 0; ph < 2; ph++)
+        hipLaunchKernelGGL(k_pairs_grouped,
+                           dim3((unsigned)std::min<u64>((total[ph] + 255) / 256, 65536)),
+                           dim3(256), 0, st, dseg + ph * np, np, total[ph], ph, (u64)r);
     GF2T_CHECK_LAUNCH("gf2t_mulmod_batch");
     return GF2T_OK;
 }
@@ -1226,83 +1499,45 @@ extern "C" int gf2t_mulmod_slab(const uint64_t *da, size_t apitch, const uint64_
     u64 ca = (r + 31) >> 5;
     int m = fft_m_for(2 * ca - 1);
     if (m > FFT_MAX_M) { gf2t::set_error("gf2t_mulmod_slab: r too large"); return GF2T_ERANGE; }
-    const gf2t_fft_plan *plan = cached_plan(m);
-    size_t N = (size_t)1 << m;
-    u64 *FA = (u64 *)dwork, *FB = FA + N * n, *prod = FB + N * n;
-    size_t ppitch = 2 * nw + 2;
-    u32 lm = (r & 31) ? (u32)((1ULL << (r & 31)) - 1) : 0xFFFFFFFFu;
+    const size_t N = (size_t)1 << m;
+    u64 *FA = (u64 *)dwork, *prod = FA + 2 * N * n;
+    const size_t ppitch = 2 * nw + 2;
+    // operands y < n: the a's, then the b's; their converted chunks where
+    // the products go later (2 ca chunks in the 4 nw + 4 of a residue)
+    Operands ops{};
+    ops.group = (u32)n;
+    ops.lstride = 2 * ppitch;
+    ops.op[0] = operand_of(da, r, prod);
+    ops.op[1] = operand_of(db, r, (u32 *)prod + 2 * nw + 2, b_add_x ? 2u : 0u);
+    const u64 ow = 2 * nw;   // product of two r-bit operands: 2r-1 bits
+    ops.sstride[0] = 2 * apitch;
+    ops.sstride[1] = 2 * bpitch;
+    const int k = log2_ceil(ca);
     const Wrap W = wrap_for(ca, ca);
     if (W.on) {
         // the wrapped product (see wrap_for): 2^mp-point transforms of both
         // operands and 2^ms-point transforms of their top e chunks, laid
         // out inside the 2 N n words an unwrapped product uses
-        const gf2t_fft_plan *pl = cached_plan(W.mp), *ps = cached_plan(W.ms);
         const size_t np = (size_t)1 << W.mp, ns = (size_t)1 << W.ms;
-        u64 *GA = (u64 *)dwork, *GB = GA + np * n, *TA = GB + np * n, *TB = TA + ns * n;
-        PackArg pa{};
-        pa.src = (const u32 *)da;
-        pa.stride = 2 * apitch;
-        pa.nchunks = ca;
-        pa.lastmask = lm;
-        rc = run_passes(pl->fwd, GA, st, &pa, (unsigned)n, np);
-        if (rc) return rc;
-        PackArg pb = pa;
-        pb.src = (const u32 *)db;
-        pb.stride = 2 * bpitch;
-        pb.xor0 = b_add_x ? 2u : 0u;
-        rc = run_passes(pl->fwd, GB, st, &pb, (unsigned)n, np);
+        u64 *TA = FA + 2 * np * n;
+        rc = run_product(plan_for(W.mp), FA, np, ops, k, (unsigned)n, st);
         if (rc) return rc;
         // top chunks [ca - e, ca); chunk 0 (where b_add_x adds x) is not among them
-        PackArg ta = pa, tb = pb;
-        ta.src += ca - W.e;
-        tb.src += ca - W.e;
-        ta.nchunks = tb.nchunks = W.e;
-        tb.xor0 = 0;
-        rc = run_passes(ps->fwd, TA, st, &ta, (unsigned)n, ns);
+        Operands top = ops;
+        for (int g = 0; g < 2; g++) top.op[g] = operand_range(ops.op[g], ca - W.e, W.e);
+        rc = run_product(plan_for(W.ms), TA, ns, top, log2_ceil(W.e), (unsigned)n, st);
         if (rc) return rc;
-        rc = run_passes(ps->fwd, TB, st, &tb, (unsigned)n, ns);
-        if (rc) return rc;
-        size_t tot = np * (size_t)n, tots = ns * (size_t)n;
-        hipLaunchKernelGGL(k_pointwise, dim3((unsigned)std::min<size_t>((tot + 255) / 256, 65536)),
-                           dim3(256), 0, st, GA, GB, tot);
-        hipLaunchKernelGGL(k_pointwise, dim3((unsigned)std::min<size_t>((tots + 255) / 256, 65536)),
-                           dim3(256), 0, st, TA, TB, tots);
-        rc = run_passes(pl->inv, GA, st, nullptr, (unsigned)n, np);
-        if (rc) return rc;
-        rc = run_passes(ps->inv, TA, st, nullptr, (unsigned)n, ns);
-        if (rc) return rc;
-        size_t ow = 2 * nw;
         hipLaunchKernelGGL(k_overlap_add_wrap, dim3((unsigned)((ow + 255) / 256), n), dim3(256), 0,
-                           st, GA, (u64)np, TA + (W.e - 1), (u64)ns, wrap_arg(W),
-                           (size_t)(2 * ca - 1), prod, ow, (u64)ppitch);
-        hipLaunchKernelGGL(k_fold_slab, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st,
-                           prod, ow, (u64)ppitch, 2 * r - 1, dout, (u64)opitch, nw, r, ds);
-        GF2T_CHECK_LAUNCH("gf2t_mulmod_slab");
-        return GF2T_OK;
+                           st, FA, (u64)np, TA + (W.e - 1), (u64)ns, wrap_arg(W),
+                           (size_t)(2 * ca - 1), prod, (size_t)ow, (u64)ppitch);
+    } else {
+        rc = run_product(plan_for(m), FA, N, ops, k, (unsigned)n, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), n), dim3(256), 0, st,
+                           FA, (size_t)(2 * ca - 1), prod, (size_t)ow, (u64)N, (u64)ppitch);
     }
-    PackArg pa{};
-    pa.src = (const u32 *)da;
-    pa.stride = 2 * apitch;
-    pa.nchunks = ca;
-    pa.lastmask = lm;
-    rc = run_passes(plan->fwd, FA, st, &pa, (unsigned)n, N);
-    if (rc) return rc;
-    PackArg pb = pa;
-    pb.src = (const u32 *)db;
-    pb.stride = 2 * bpitch;
-    pb.xor0 = b_add_x ? 2u : 0u;
-    rc = run_passes(plan->fwd, FB, st, &pb, (unsigned)n, N);
-    if (rc) return rc;
-    size_t tot = N * (size_t)n;
-    unsigned blocks = (unsigned)std::min<size_t>((tot + 255) / 256, 65536);
-    hipLaunchKernelGGL(k_pointwise, dim3(blocks), dim3(256), 0, st, FA, FB, tot);
-    rc = run_passes(plan->inv, FA, st, nullptr, (unsigned)n, N);
-    if (rc) return rc;
-    size_t ow = 2 * nw;   // product of two r-bit operands: 2r-1 bits
-    hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), n), dim3(256), 0, st, FA,
-                       (size_t)(2 * ca - 1), prod, ow, (u64)N, (u64)ppitch);
     hipLaunchKernelGGL(k_fold_slab, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st, prod,
-                       ow, (u64)ppitch, 2 * r - 1, dout, (u64)opitch, nw, r, ds);
+                       (size_t)ow, (u64)ppitch, 2 * r - 1, dout, (u64)opitch, nw, r, ds);
     GF2T_CHECK_LAUNCH("gf2t_mulmod_slab");
     return GF2T_OK;
 }
@@ -1388,7 +1623,6 @@ int hm_reserve(HostMulCtx &c, size_t words, size_t host_words) {
     return GF2T_OK;
 }
 
-u32 last_mask(u64 bits) { return (bits & 31) ? (u32)((1ULL << (bits & 31)) - 1) : 0xFFFFFFFFu; }
 }  // namespace
 
 int gf2t_hm_set_zc_words(int64_t words) {
@@ -1435,17 +1669,34 @@ extern "C" int gf2t_mul_host(const uint64_t *ha, uint64_t abits, const uint64_t 
 namespace {
 // Pair p of a batched matrix-vector product: its two transforms (at F + (4
 // + 2p) n and F + (5 + 2p) n) become (m0 a + m1 b, m2 a + m3 b), the
-// matrix transforms at F .. F + 3n left as they are.
-__global__ void k_mat2n_pointwise(u64 *__restrict__ F, size_t n, int npairs) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) {
-        const u64 m0 = F[i], m1 = F[n + i], m2 = F[2 * n + i], m3 = F[3 * n + i];
+// matrix transforms at F .. F + 3n left as they are.  A thread per unit.
+__global__ __launch_bounds__(256) void k_mat2n_pointwise(u64 *__restrict__ F, size_t n,
+                                                         int npairs) {
+    __shared__ ProdLds pt;
+    pt.load();
+    __syncthreads();
+    const size_t units = n / 2;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    const Operand none{};
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < units; i += stride) {
+        Half32 M[4], C[4];
+        for (int k = 0; k < 4; k++) {
+            const U4 u = load_unit((const U4 *)(F + k * n), (u32)i, IO_UNITS, none, nullptr);
+            M[k] = unit_to32(u, pt.d32);
+            C[k] = unit_c5(u, pt.d5);
+        }
         for (int p = 0; p < npairs; p++) {
-            u64 *fa = F + (4 + 2 * (size_t)p) * n, *fb = fa + n;
-            const u64 a = fa[i], b = fb[i];
-            fa[i] = gf64_mul(m0, a) ^ gf64_mul(m1, b);
-            fb[i] = gf64_mul(m2, a) ^ gf64_mul(m3, b);
+            U4 *fa = (U4 *)(F + (4 + 2 * (size_t)p) * n), *fb = (U4 *)(F + (5 + 2 * (size_t)p) * n);
+            const Half32 a = unit_to32(load_unit(fa, (u32)i, IO_UNITS, none, nullptr), pt.d32);
+            const Half32 b = unit_to32(load_unit(fb, (u32)i, IO_UNITS, none, nullptr), pt.d32);
+            for (int o = 0; o < 2; o++) {
+                Acc64 E{0, 0}, G{0, 0};
+                acc_mul(E, a.v[0], a.v[1], M[2 * o].v[0], M[2 * o].v[1], C[2 * o].v[1]);
+                acc_mul(E, b.v[0], b.v[1], M[2 * o + 1].v[0], M[2 * o + 1].v[1], C[2 * o + 1].v[1]);
+                acc_mul(G, a.v[2], a.v[3], M[2 * o].v[2], M[2 * o].v[3], C[2 * o].v[3]);
+                acc_mul(G, b.v[2], b.v[3], M[2 * o + 1].v[2], M[2 * o + 1].v[3], C[2 * o + 1].v[3]);
+                store_unit(o ? fb : fa, (u32)i, unit_back(E, G, pt.b32), IO_UNITS, nullptr);
+            }
         }
     }
 }
@@ -1486,32 +1737,31 @@ extern "C" int gf2t_mat2n_host(const uint64_t *const hm[4], const uint64_t mbits
     if (rc) return rc;
     HmLease lease;
     HostMulCtx &hc = *lease.c;
-    const gf2t_fft_plan *plan = cached_plan(m);
+    const gf2t_fft_plan plan = plan_for(m);
     const int nt = 4 + nv;                    // transforms: matrix, then the vectors
     size_t n = (size_t)1 << m, ow = gf2t_mul_out_words(mb, vb);
     const u64 *src[PACK_LIST];
     u64 bits[PACK_LIST];
-    size_t in_w[PACK_LIST], stage = 0;
+    size_t in_w[PACK_LIST], stage = 0, lchw = 0;   // words
     for (int i = 0; i < nt; i++) {
         src[i] = i < 4 ? hm[i] : hv[i - 4];
         bits[i] = i < 4 ? mbits[i] : vbits[i - 4];
         in_w[i] = words_of(bits[i]);
         stage += (in_w[i] + 3) & ~(size_t)3;
     }
-    rc = hm_reserve(hc, nt * n + nv * ow + stage + 64, std::max(stage, nv * ow));
+    lchw = stage;   // the converted chunks of every operand
+    rc = hm_reserve(hc, nt * n + nv * ow + stage + lchw + 64, std::max(stage, nv * ow));
     if (rc) return rc;
     hipStream_t st = hc.st;
     u64 *F = hc.dbuf;                         // nt transforms, n words apart
     u64 *dout = F + nt * n, *dstage = dout + nv * ow;
     // the operands, 32-byte aligned, in one pinned buffer and one copy
-    PackArg pk{};
-    pk.nlist = nt;
+    Operands pk{};
+    u64 *lch = dstage + stage;
     size_t off = 0;
     for (int i = 0; i < nt; i++) {
         if (in_w[i]) std::memcpy(hc.hbuf + off, src[i], in_w[i] * 8);
-        pk.lsrc[i] = (const u32 *)(dstage + off);
-        pk.lnch[i] = (bits[i] + 31) >> 5;     // 0 for a zero operand: its transform is all zero
-        pk.lmask[i] = last_mask(bits[i]);
+        pk.op[i] = operand_of(dstage + off, bits[i], lch + off);   // n = 0 for a zero operand
         off += (in_w[i] + 3) & ~(size_t)3;
     }
     // small products read their operands from the pinned staging buffer
@@ -1521,18 +1771,19 @@ extern "C" int gf2t_mat2n_host(const uint64_t *const hm[4], const uint64_t mbits
     if (zc) {
         size_t o2 = 0;
         for (int i = 0; i < nt; i++) {
-            pk.lsrc[i] = (const u32 *)(hc.hbuf + o2);
+            pk.op[i].src = (const u32 *)(hc.hbuf + o2);
             o2 += (in_w[i] + 3) & ~(size_t)3;
         }
         dout = hc.hbuf;
     } else if (off) {
         GF2T_HIP(hipMemcpyAsync(dstage, hc.hbuf, off * 8, hipMemcpyHostToDevice, st));
     }
-    rc = run_passes(plan->fwd, F, st, &pk, (unsigned)nt, n);
+    int in;
+    rc = run_forward(plan, F, n, pk, log2_ceil(std::max(cm, cv)), (unsigned)nt, true, st, in);
     if (rc) return rc;
-    unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
+    unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 2048);
     hipLaunchKernelGGL(k_mat2n_pointwise, dim3(blocks), dim3(256), 0, st, F, n, npairs);
-    rc = run_passes(plan->inv, F + 4 * n, st, nullptr, (unsigned)nv, n);
+    rc = run_inverse(plan, F + 4 * n, n, (unsigned)nv, true, IO_UNITS, st);
     if (rc) return rc;
     size_t nch = (size_t)(cm + cv - 1);
     hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), nv), dim3(256), 0, st,
