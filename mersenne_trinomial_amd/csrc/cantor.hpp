@@ -23,27 +23,41 @@
 struct alignas(16) U4 {
     u32 w[4];
 };
-// bytes of a twiddle W = Wa + Wb u4 (Wa, Wb in GF(2^16)): p for the
-// product with Wa, q with c4 Wb, r with Wa + Wb; each as the three byte
-// factors of a Karatsuba product over GF(2^8): v0, c3 v1, v0 + v1.  Every
-// entry is linear in W.
-struct TwEnt {
-    u32 p, q, r, pad;
+// A twiddle W = Wa + Wb u4 (Wa, Wb in GF(2^16)) as the bytes its product
+// needs: p for the product with Wa, q with c4 Wb, r with Wa + Wb, each as
+// the three byte factors of a Karatsuba product over GF(2^8), v0, c3 v1 and
+// v0 + v1.  Every byte is linear in W.  Two to a word, each times 16, the
+// byte offset of its entry in the first multiply table (a quarter of it in
+// the second).
+struct alignas(16) TwEnt {
+    u32 p02, r02;   // bytes 0 (low half) and 2 of p, r: an element v of
+                    // GF(2^8) added to W adds v to all four
+    u32 p1r1, q01, q2;
+    u32 pad[3];
 };
+GF2T_HD u32 tw_lo(u32 w) { return w & 0xFF0u; }
+GF2T_HD u32 tw_hi(u32 w) { return w >> 16; }
+GF2T_HD u32 tw_byte(u32 v) { return (v << 4) | (v << 20); }
+GF2T_HD TwEnt tw_xor(const TwEnt &a, const TwEnt &b) {
+    return TwEnt{a.p02 ^ b.p02, a.r02 ^ b.r02, a.p1r1 ^ b.p1r1, a.q01 ^ b.q01, a.q2 ^ b.q2, {}};
+}
 // multiply-by-v tables: a = images of the byte's bits 0..2 (8 bytes), b of
 // bits 3..5, c of bits 6, 7 (4 bytes)
 struct Mul8 {
     u32 a0, a1, b0, b1, c;
 };
-struct FftTables {
+struct alignas(16) FftTables {
+    // the first two runs are copied to LDS as they stand
     u32 mulA[256][4];   // a0, a1, b0, b1 of the product with v
-    u32 mulB[256];      // c
-    TwEnt tw[4][256];   // W(t) for byte k of t: sum of b[8k + j + 1] over its bits j
-    u64 emb[8][256];    // polynomial-basis byte k -> tower halfwords
-    u64 une[8][256];    // tower byte k -> polynomial basis
+    u32 mulB[256];      // c (apart: rows of 16 bytes spread over all LDS
+                        // banks; with rows of 32, the low pass of a 2^23-
+                        // point product took 360 us instead of 267)
     u32 d32[4][256];    // GF(2^32): tower byte p -> basis of powers of rho
     u32 d5[4][256];     // the same times c5
     u32 b32[4][256];    // back: byte k -> the four tower bytes
+    u64 emb[8][256];    // polynomial-basis byte k -> tower halfwords
+    u64 une[8][256];    // tower byte k -> polynomial basis
+    TwEnt tw[4][256];   // W(t) for byte k of t: sum of b[8k + j + 1] over its bits j
 };
 
 // rho: a root of x^32 + x^7 + x^3 + x^2 + 1 in GF(2^64)
@@ -62,64 +76,68 @@ GF2T_HD Bits8 xor8(const Bits8 &x, const Bits8 &y) {
 GF2T_HD u32 map8(const Mul8 &t, const Bits8 &s) {
     return xor3_32(perm8(t.a1, t.a0, s.l), perm8(t.b1, t.b0, s.m), perm8(t.c, t.c, s.h));
 }
-GF2T_HD u32 addmap8(u32 y, const Mul8 &t, const Bits8 &s) {
-    return xor3_32(xor3_32(y, perm8(t.a1, t.a0, s.l), perm8(t.b1, t.b0, s.m)),
-                   perm8(t.c, t.c, s.h), 0);
-}
-
 // The factor tables of one twiddle, by the subfield it lies in: CLS 8 one
-// table, 16 three, 32 nine.  All of them but those of bytes 0 and 2 of p
-// and r stay the same when an element of GF(2^8) is added to W, so a
-// stage fetches those once per level.
+// table, 16 three, 32 nine; tab(off) reads the entry at byte offset off.
+// All of them but those of bytes 0 and 2 of p and r stay the same when an
+// element of GF(2^8) is added to W, so a stage fetches those once per
+// level.
 template <int CLS>
 struct TwTab {
     Mul8 p0, p1, p2, q0, q1, q2, r0, r1, r2;
     template <class Tab>
     GF2T_HDM void fixed(const TwEnt &w, const Tab &tab) {
-        if (CLS >= 16) p1 = tab((w.p >> 8) & 255);
+        if (CLS >= 16) p1 = tab(tw_lo(w.p1r1));
         if (CLS >= 32) {
-            q0 = tab(w.q & 255);
-            q1 = tab((w.q >> 8) & 255);
-            q2 = tab((w.q >> 16) & 255);
-            r1 = tab((w.r >> 8) & 255);
+            r1 = tab(tw_hi(w.p1r1));
+            q0 = tab(tw_lo(w.q01));
+            q1 = tab(tw_hi(w.q01));
+            q2 = tab(w.q2);
         }
     }
     template <class Tab>   // for W + v, v in GF(2^8)
     GF2T_HDM void add(const TwEnt &w, u32 v, const Tab &tab) {
-        p0 = tab((w.p & 255) ^ v);
-        if (CLS >= 16) p2 = tab(((w.p >> 16) & 255) ^ v);
+        const u32 p = w.p02 ^ tw_byte(v), r = w.r02 ^ tw_byte(v);
+        p0 = tab(tw_lo(p));
+        if (CLS >= 16) p2 = tab(tw_hi(p));
         if (CLS >= 32) {
-            r0 = tab((w.r & 255) ^ v);
-            r2 = tab(((w.r >> 16) & 255) ^ v);
+            r0 = tab(tw_lo(r));
+            r2 = tab(tw_hi(r));
         }
     }
 };
 
-// y += W x on units
+struct UnitBits {   // the bits of a unit's words
+    Bits8 b[4];
+};
+GF2T_HD UnitBits unit_bits(const U4 &x) {
+    return UnitBits{{split8(x.w[0]), split8(x.w[1]), split8(x.w[2]), split8(x.w[3])}};
+}
+// y += W x on units, x by its bits
 template <int CLS>
-GF2T_HD void unit_madd(U4 &y, const U4 &x, const TwTab<CLS> &t) {
+GF2T_HD void unit_madd(U4 &y, const UnitBits &x, const TwTab<CLS> &t) {
     if (CLS == 8) {
-        for (int k = 0; k < 4; k++) y.w[k] ^= map8(t.p0, split8(x.w[k]));
+#pragma unroll
+        for (int k = 0; k < 4; k++) y.w[k] ^= map8(t.p0, x.b[k]);
     } else if (CLS == 16) {
+#pragma unroll
         for (int k = 0; k < 4; k += 2) {
-            const Bits8 s0 = split8(x.w[k]), s1 = split8(x.w[k + 1]);
+            const Bits8 &s0 = x.b[k], &s1 = x.b[k + 1];
             const u32 P = map8(t.p0, s0);
             y.w[k] = xor3_32(y.w[k], P, map8(t.p1, s1));
             y.w[k + 1] = xor3_32(y.w[k + 1], P, map8(t.p2, xor8(s0, s1)));
         }
     } else {
-        const Bits8 a0 = split8(x.w[0]), a1 = split8(x.w[1]);
-        const Bits8 b0 = split8(x.w[2]), b1 = split8(x.w[3]);
+        const Bits8 &a0 = x.b[0], &a1 = x.b[1], &b0 = x.b[2], &b1 = x.b[3];
         const Bits8 c0 = xor8(a0, b0), c1 = xor8(a1, b1);
         const u32 P0 = map8(t.p0, a0);
         const u32 A = P0 ^ map8(t.p1, a1);             // Wa Xa, low and high
         const u32 B = P0 ^ map8(t.p2, xor8(a0, a1));
         const u32 Q0 = map8(t.q0, b0);
-        y.w[0] = xor3_32(y.w[0], A, Q0 ^ map8(t.q1, b1));
-        y.w[1] = xor3_32(y.w[1], B, Q0 ^ map8(t.q2, xor8(b0, b1)));
+        y.w[0] = xor3_32(y.w[0], A, Q0) ^ map8(t.q1, b1);
+        y.w[1] = xor3_32(y.w[1], B, Q0) ^ map8(t.q2, xor8(b0, b1));
         const u32 R0 = map8(t.r0, c0);
-        y.w[2] = xor3_32(y.w[2], A, R0 ^ map8(t.r1, c1));
-        y.w[3] = xor3_32(y.w[3], B, R0 ^ map8(t.r2, xor8(c0, c1)));
+        y.w[2] = xor3_32(y.w[2], A, R0) ^ map8(t.r1, c1);
+        y.w[3] = xor3_32(y.w[3], B, R0) ^ map8(t.r2, xor8(c0, c1));
     }
 }
 GF2T_HD void unit_xor(U4 &y, const U4 &x) {
@@ -139,30 +157,38 @@ constexpr int RB = 2;
 // unit index is a level, active when bit rb of act is set; W[rb] is the
 // twiddle of the rows whose bits above rb are clear, and the rows whose
 // bits above rb spell `up` add sum of b[j + 1] over the bits j of up, the
-// byte up << 1.
-template <int CLS, bool INV, class Tab>
-GF2T_HD void fft_stage(U4 *x, int act, const TwEnt *W, const Tab &tab) {
+// byte up << 1.  zero: the W[.] are all 0 (the topmost levels), so the rows
+// with up = 0 have no product.
+template <int rb, int CLS, bool INV, class Tab>
+GF2T_HD void fft_level(U4 *x, const TwEnt &W, bool zero, const Tab &tab) {
+    TwTab<CLS> t;
+    t.fixed(W, tab);
 #pragma unroll
-    for (int k = 0; k < RB; k++) {
-        const int rb = INV ? k : RB - 1 - k;
-        if (!((act >> rb) & 1)) continue;
-        TwTab<CLS> t;
-        t.fixed(W[rb], tab);
+    for (int up = 0; up < ((1 << (RB - 1)) >> rb); up++) {
+        const bool mul = up || !zero;
+        if (mul) t.add(W, (u32)up << 1, tab);
 #pragma unroll
-        for (int up = 0; up < ((1 << (RB - 1)) >> rb); up++) {
-            t.add(W[rb], (u32)up << 1, tab);
-#pragma unroll
-            for (int lo = 0; lo < (1 << rb); lo++) {
-                const int r0 = (up << (rb + 1)) | lo, r1 = r0 | (1 << rb);
-                if (INV) {
-                    unit_xor(x[r1], x[r0]);
-                    unit_madd<CLS>(x[r0], x[r1], t);
-                } else {
-                    unit_madd<CLS>(x[r0], x[r1], t);
-                    unit_xor(x[r1], x[r0]);
-                }
+        for (int lo = 0; lo < (1 << rb); lo++) {
+            const int r0 = (up << (rb + 1)) | lo, r1 = r0 | (1 << rb);
+            if (INV) {
+                unit_xor(x[r1], x[r0]);
+                if (mul) unit_madd<CLS>(x[r0], unit_bits(x[r1]), t);
+            } else {
+                if (mul) unit_madd<CLS>(x[r0], unit_bits(x[r1]), t);
+                unit_xor(x[r1], x[r0]);
             }
         }
+    }
+}
+template <int CLS, bool INV, class Tab>
+GF2T_HD void fft_stage(U4 *x, int act, const TwEnt *W, bool zero, const Tab &tab) {
+    static_assert(RB == 2, "two levels");
+    if (INV) {
+        if (act & 1) fft_level<0, CLS, true>(x, W[0], zero, tab);
+        if (act & 2) fft_level<1, CLS, true>(x, W[1], zero, tab);
+    } else {
+        if (act & 2) fft_level<1, CLS, false>(x, W[1], zero, tab);
+        if (act & 1) fft_level<0, CLS, false>(x, W[0], zero, tab);
     }
 }
 // Level 0, inside the units: rows r and r + 1 (r even) are taken together,
@@ -170,22 +196,27 @@ GF2T_HD void fft_stage(U4 *x, int act, const TwEnt *W, const Tab &tab) {
 // 0, row r adds the byte r << 1.
 template <int CLS, bool INV, class Tab>
 GF2T_HD void fft_level0(U4 *x, const TwEnt &W, const Tab &tab) {
-    const u32 LO = 0x05040100u, HI = 0x07060302u;
-    const Mul8 b1 = tab(2);
+    const u32 LO = 0x05040100u, HI = 0x07060302u, TOP = 0xFFFF0000u;
+    const Mul8 b1 = tab(2 << 4);
     TwTab<CLS> t;
     t.fixed(W, tab);
 #pragma unroll
     for (int r = 0; r < (1 << RB); r += 2) {
         t.add(W, (u32)r << 1, tab);
         U4 e, f;
+#pragma unroll
         for (int p = 0; p < 4; p++) {
             e.w[p] = perm8(x[r + 1].w[p], x[r].w[p], LO);
             f.w[p] = perm8(x[r + 1].w[p], x[r].w[p], HI);
         }
         if (INV) unit_xor(f, e);
-        unit_madd<CLS>(e, f, t);
-        for (int p = 0; p < 4; p++) e.w[p] ^= map8(b1, split8(f.w[p] & 0xFFFF0000u));
+        const UnitBits s = unit_bits(f);
+        unit_madd<CLS>(e, s, t);
+#pragma unroll
+        for (int p = 0; p < 4; p++)   // row r + 1: W + b[1]
+            e.w[p] ^= map8(b1, Bits8{s.b[p].l & TOP, s.b[p].m & TOP, s.b[p].h & TOP});
         if (!INV) unit_xor(f, e);
+#pragma unroll
         for (int p = 0; p < 4; p++) {
             x[r].w[p] = perm8(f.w[p], e.w[p], LO);
             x[r + 1].w[p] = perm8(f.w[p], e.w[p], HI);
@@ -196,15 +227,14 @@ GF2T_HD void fft_level0(U4 *x, const TwEnt &W, const Tab &tab) {
 // W(t) from the byte tables
 template <class TwT>
 GF2T_HD TwEnt tw_of(const TwT &tw, u32 t) {
-    const TwEnt a = tw[0][t & 255], b = tw[1][(t >> 8) & 255], c = tw[2][(t >> 16) & 255],
-                d = tw[3][t >> 24];
-    return TwEnt{xor3_32(a.p, b.p, c.p) ^ d.p, xor3_32(a.q, b.q, c.q) ^ d.q,
-                 xor3_32(a.r, b.r, c.r) ^ d.r, 0};
+    return tw_xor(tw_xor(tw[0][t & 255], tw[1][(t >> 8) & 255]),
+                  tw_xor(tw[2][(t >> 16) & 255], tw[3][t >> 24]));
 }
 // W + v for v in GF(2^8)
 GF2T_HD TwEnt tw_add8(TwEnt w, u32 v) {
-    w.p ^= v | (v << 16);
-    w.r ^= v | (v << 16);
+    const u32 b = tw_byte(v);
+    w.p02 ^= b;
+    w.r02 ^= b;
     return w;
 }
 
@@ -360,15 +390,15 @@ GF2T_HD void bf_twiddles(const BfPass &P, const BfTile &T, int s, u32 tid, const
     }
 }
 
+// the twiddles of the stage's row 0 are all 0: the top of the transform
+GF2T_HD bool bf_zero(const BfPass &P, const BfTile &T, int s) { return s == 0 && T.hi == 0; }
+
 // The last (lowest) levels 7..0: a wave's 64 lanes hold 64 << RB
 // consecutive units, in stage s the rows being the unit bits from
 // lo_pos(s) up: levels lo_pos + 1 + j on row bits j, level 0 inside the
 // units after the last stage: unit bits 6 and 5, 4 and 3, 2 and 1, 1 and 0
 // (only bit 0 a level there).
-GF2T_HD int lo_pos(int s) {
-    const int p = 7 - RB * (s + 1);
-    return p > 0 ? p : 0;
-}
+GF2T_HD constexpr int lo_pos(int s) { return 7 - RB * (s + 1) > 0 ? 7 - RB * (s + 1) : 0; }
 GF2T_HD constexpr int lo_stages() { return (7 + RB - 1) / RB; }
 GF2T_HD u32 lo_unit(int s, u32 lane, int r) { return spread_rows(lane, r, lo_pos(s), RB); }
 GF2T_HD int lo_active(int m, int s) {
@@ -379,32 +409,23 @@ GF2T_HD int lo_active(int m, int s) {
     }
     return act;
 }
-// twiddle of row 0 at level L of stage s, wave's first unit ubase: the
-// lane bits above the rows are t bits from RB - 1 - j up; t < 2^7 of them
-// is the byte t << 1, the two bits above go through the tables
-template <class TwC>
-GF2T_HD TwEnt lo_twiddle(u32 ubase, int L, u32 tlane, const TwC &tw) {
-    return tw_add8(tw_of(tw, (ubase << 1) >> (L + 1)), (tlane << 1) & 255);
-}
+// twiddle of row 0 at level L, wave's first unit ubase: t_lane are the lane
+// bits above the rows; those below 2^7 are the byte t << 1, the two bits
+// above go through the table hi
 template <class TwC, class TwG>
-GF2T_HD void lo_twiddles(u32 ubase, int s, u32 lane, const TwC &tw, const TwG &hi, TwEnt *W,
-                         TwEnt &W0) {
-    const int pos = lo_pos(s);
+GF2T_HD TwEnt lo_twiddle(u32 ubase, int L, u32 tlane, bool high, const TwC &tw, const TwG &hi) {
+    TwEnt w = tw_add8(tw_of(tw, (ubase << 1) >> (L + 1)), (tlane << 1) & 255);
+    if (high) w = tw_xor(w, hi[(tlane >> 7) & 3]);
+    return w;
+}
+template <int S, class TwC, class TwG>
+GF2T_HD void lo_twiddles(u32 ubase, u32 lane, const TwC &tw, const TwG &hi, TwEnt *W, TwEnt &W0) {
+    constexpr int pos = lo_pos(S);
 #pragma unroll
-    for (int j = 0; j < RB; j++) {
-        const u32 t = (lane >> pos) << (RB - 1 - j);
-        W[j] = lo_twiddle(ubase, pos + 1 + j, t, tw);
-        if (6 - pos + RB - 1 - j > 7) {   // t has bits from 7 on
-            const TwEnt &h = hi[(t >> 7) & 3];
-            W[j].p ^= h.p; W[j].q ^= h.q; W[j].r ^= h.r;
-        }
-    }
-    if (s == lo_stages() - 1) {
-        const u32 t = lane << RB;
-        W0 = lo_twiddle(ubase, 0, t, tw);
-        const TwEnt &h = hi[(t >> 7) & 3];
-        W0.p ^= h.p; W0.q ^= h.q; W0.r ^= h.r;
-    }
+    for (int j = 0; j < RB; j++)
+        W[j] = lo_twiddle(ubase, pos + 1 + j, (lane >> pos) << (RB - 1 - j),
+                          6 - pos + RB - 1 - j > 7, tw, hi);
+    if (S == lo_stages() - 1) W0 = lo_twiddle(ubase, 0, lane << RB, true, tw, hi);
 }
 
 // ------------------------------------------------- conversion of the basis
@@ -452,85 +473,6 @@ GF2T_HD void conv_nibble(T *x) {
         conv_regs<2, POS + 1, N, true>(x);
     }
 }
-// A group of w index bits (2 <= w <= 8) converted by threads of 64
-// coefficients: layout 0 has the top six bits of the window (with lower
-// bits of the tile for w < 6) in the registers, layout 1 the low six.  w =
-// 7, 8: expansion in powers of s_4 in both, then the low nibble in layout 1
-// and the top w - 4 bits in layout 0; w <= 6: all of it in layout 0.
-template <bool INV, class T>
-GF2T_HD void conv_group_first(T *x, int w) {   // layout 0, before any exchange (INV: after)
-    switch (w) {
-    case 8:
-    case 7:
-        if (!INV) { conv_regs<4, 1, 64, INV>(x); conv_regs<4, 0, 64, INV>(x); }
-        else { conv_regs<4, 0, 64, INV>(x); conv_regs<4, 1, 64, INV>(x); }
-        break;
-    case 6:
-        if (!INV) {
-            conv_regs<4, 1, 64, INV>(x); conv_regs<4, 0, 64, INV>(x);
-            conv_nibble<0, 64, INV>(x); conv_regs<1, 4, 64, INV>(x);
-        } else {
-            conv_regs<1, 4, 64, INV>(x); conv_nibble<0, 64, INV>(x);
-            conv_regs<4, 0, 64, INV>(x); conv_regs<4, 1, 64, INV>(x);
-        }
-        break;
-    case 5:
-        if (!INV) { conv_regs<4, 1, 64, INV>(x); conv_nibble<1, 64, INV>(x); }
-        else { conv_nibble<1, 64, INV>(x); conv_regs<4, 1, 64, INV>(x); }
-        break;
-    case 4: conv_nibble<2, 64, INV>(x); break;
-    case 3:
-        if (!INV) { conv_regs<2, 3, 64, INV>(x); conv_regs<1, 3, 64, INV>(x); }
-        else { conv_regs<1, 3, 64, INV>(x); conv_regs<2, 3, 64, INV>(x); }
-        break;
-    default: conv_regs<1, 4, 64, INV>(x); break;
-    }
-}
-template <bool INV, class T>
-GF2T_HD void conv_group_low(T *x, int w) {     // layout 1, w = 7, 8
-    if (INV) conv_nibble<0, 64, INV>(x);
-    if (w == 8) {
-        if (!INV) { conv_regs<4, 1, 64, INV>(x); conv_regs<4, 0, 64, INV>(x); }
-        else { conv_regs<4, 0, 64, INV>(x); conv_regs<4, 1, 64, INV>(x); }
-    } else {
-        conv_regs<4, 0, 64, INV>(x);
-    }
-    if (!INV) conv_nibble<0, 64, INV>(x);
-}
-template <bool INV, class T>
-GF2T_HD void conv_group_top(T *x, int w) {     // layout 0, w = 7, 8
-    if (w == 8) {
-        conv_nibble<2, 64, INV>(x);
-    } else if (!INV) {
-        conv_regs<2, 3, 64, INV>(x);
-        conv_regs<1, 3, 64, INV>(x);
-    } else {
-        conv_regs<1, 3, 64, INV>(x);
-        conv_regs<2, 3, 64, INV>(x);
-    }
-}
-// element bits [off, off + w), tiles of 2^tb coefficients: local bits
-// [0, tb - w) are memory's low bits, [tb - w, tb) the window (off > 0); a
-// contiguous tile, window lowest (off = 0)
-struct ConvGroup {
-    int off, w, tb;
-};
-GF2T_HD u64 group_base(const ConvGroup &g, u32 blk) {
-    if (!g.off) return (u64)blk << g.tb;
-    const int lc = g.tb - g.w, nlo = g.off - lc;
-    return ((u64)(blk & ((1u << nlo) - 1)) << lc) | ((u64)(blk >> nlo) << (g.off + g.w));
-}
-// register r of a thread: its local index in layout 0 and 1, and the
-// memory offset of a local index
-GF2T_HD u32 group_local(const ConvGroup &g, int layout, u32 tid, int r) {
-    if (g.off) return spread_rows(tid, r, layout ? g.tb - g.w : g.tb - 6, 6);
-    return spread_rows(tid, r, layout ? 0 : g.w - 6, 6);
-}
-GF2T_HD u64 group_mem(const ConvGroup &g, u32 local) {
-    if (!g.off) return local;
-    const int lc = g.tb - g.w;
-    return (local & ((1u << lc) - 1)) + ((u64)(local >> lc) << g.off);
-}
 // Steps e0 + K - 1 .. e0 of the expansion in powers of s_h, with unit =
 // 2^e0 (times 2^off inside a higher index part): 2^K rows of 2^hb
 // coefficients, hb = h + e0 + off, each step adding row k (bit e set) to
@@ -551,74 +493,192 @@ GF2T_HD u32 conv_edge(const ConvStep &s, int k, u32 q, u32 rho) {
     const u32 n = 1u << s.K;
     return q < n - (u32)k ? (q << s.ub) + rho : (1u << s.hb) - ((n - q) << s.ub) + rho;
 }
-// the same step inside a tile, on local index bits: pair number idx of
-// the 2^(T-1), T_h at local bit pos; x(i) is local coefficient i
+// step e on the 2^K x 2^K coefficients of an edge, x(row * 2^K + q): pair
+// number idx of half of them
 template <class X>
-GF2T_HD void conv_tile_op(X &&x, u32 idx, int h, int pos, bool inv) {
-    const u32 L = 1u << (h + pos), U = 1u << pos;
-    const u32 p = idx & (L - 1);
-    const u32 f0 = (idx >> (h + pos)) << (h + pos + 1), f1 = f0 + L;
-    auto v = x(f1 + p);
+GF2T_HD void conv_edge_pair(X &&x, int K, int e, bool inv, u32 idx) {
+    const u32 L = 1u << (K + e), U = 1u << e;
+    const u32 p = idx & (L - 1), f0 = idx + (idx & ~(L - 1)), f1 = f0 + L;
+    auto v = x(f1);
     if (!inv && p < U) {
-        v ^= x(f1 + L - U + p);
-        x(f1 + p) = v;
+        v ^= x(f1 + L - U);
+        x(f1) = v;
     }
-    if (p + U < L) x(f0 + p + U) ^= v;
-    if (inv && p < U) x(f1 + p) = v ^ x(f1 + L - U + p);
+    if (p + U < L) x(f0 + U) ^= v;
+    if (inv && p < U) x(f1) = v ^ x(f1 + L - U);
+}
+// Inside a tile the steps run on local index bits, 16 coefficients per
+// thread in registers between two passes through LDS; x(i) is local
+// coefficient i, q the thread of 2^(T-4).
+// One step (K = 1): eight pairs, T_h of s at local bit s.ub
+template <bool INV, class E, class X>
+GF2T_HD void conv_tile1(X &&x, u32 q, u32 threads, const ConvStep &s) {
+    const u32 L = 1u << s.hb, U = 1u << s.ub;
+    E v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const u32 idx = q + (u32)i * threads, p = idx & (L - 1), f1 = idx + (idx & ~(L - 1)) + L;
+        v[i] = x(f1);
+        if (!INV && p < U) {
+            v[i] ^= x(f1 + L - U);
+            x(f1) = v[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const u32 idx = q + (u32)i * threads, p = idx & (L - 1), f0 = idx + (idx & ~(L - 1));
+        if (p + U < L) x(f0 + U) ^= v[i];
+        if (INV && p < U) x(f0 + L) = v[i] ^ x(f0 + L + L - U);
+    }
+}
+// Two steps (K = 2): four skewed columns of four rows, or the 16
+// coefficients of an edge.  A block of four rows of 2^hb has 2^hb / 4
+// threads: (2^hb - 4 unit) / 4 for the columns, unit for the edges.
+template <bool INV, class E, class X>
+GF2T_HD void conv_tile2(X &&x, u32 q, const ConvStep &s) {
+    const u32 per = 1u << (s.hb - 2), cols = per - (1u << s.ub);
+    const u32 t = q & (per - 1), base = (q >> (s.hb - 2)) << (s.hb + 2);
+    E v[16];
+    if (t < cols) {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                v[4 * c + k] = x(base + ((u32)k << s.hb) + conv_col(s, t + (u32)c * cols, k));
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            E *y = v + 4 * c;
+            if (!INV) { y[0] ^= y[2]; y[1] ^= y[3]; }
+            y[0] ^= y[1];
+            y[2] ^= y[3];
+            if (INV) { y[0] ^= y[2]; y[1] ^= y[3]; }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)   // row 3 keeps its value
+                x(base + ((u32)k << s.hb) + conv_col(s, t + (u32)c * cols, k)) = v[4 * c + k];
+    } else {
+        const u32 rho = t - cols;
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            v[i] = x(base + ((u32)(i >> 2) << s.hb) + conv_edge(s, i >> 2, (u32)(i & 3), rho));
+        if (!INV) { conv_regs<2, 1, 16, INV>(v); conv_regs<2, 0, 16, INV>(v); }
+        else { conv_regs<2, 0, 16, INV>(v); conv_regs<2, 1, 16, INV>(v); }
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            x(base + ((u32)(i >> 2) << s.hb) + conv_edge(s, i >> 2, (u32)(i & 3), rho)) = v[i];
+    }
+}
+// all of the conversion of nb bits (2, 3 or 4) whose top is local bit
+// pos + 3, the registers being the local bits pos .. pos + 3
+template <bool INV, class E, class X>
+GF2T_HD void conv_tile_nibble(X &&x, u32 q, int pos, int nb) {
+    const u32 base = spread_rows(q, 0, pos, 4);
+    E v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = x(base + ((u32)r << pos));
+    if (nb == 4) {
+        conv_nibble<0, 16, INV>(v);
+    } else if (nb == 3) {
+        if (!INV) { conv_regs<2, 1, 16, INV>(v); conv_regs<1, 1, 16, INV>(v); }
+        else { conv_regs<1, 1, 16, INV>(v); conv_regs<2, 1, 16, INV>(v); }
+    } else {
+        conv_regs<1, 2, 16, INV>(v);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) x(base + ((u32)r << pos)) = v[r];
+}
+// a stage of a tile: K = 1, 2 steps s, or K = 0: nibble at s.ub, s.hb bits
+template <bool INV, class E, class X>
+GF2T_HD void conv_tile_stage(X &&x, u32 q, u32 threads, const ConvStep &s) {
+    if (s.K == 2) conv_tile2<INV, E>(x, q, s);
+    else if (s.K == 1) conv_tile1<INV, E>(x, q, threads, s);
+    else conv_tile_nibble<INV, E>(x, q, s.ub, s.hb);
+}
+// a tile: the local bits [0, c) are memory's, [c, c + w) the index bits
+// [a, a + w)
+constexpr int CONV_MAX_STAGES = 12;
+struct ConvTile {
+    int c, a, w, n;
+    ConvStep st[CONV_MAX_STAGES];   // forward order
+};
+GF2T_HD u64 tile_base(const ConvTile &t, u32 blk) {
+    const int nlo = t.a - t.c;
+    return ((u64)(blk & ((1u << nlo) - 1)) << t.c) | ((u64)(blk >> nlo) << (t.a + t.w));
+}
+GF2T_HD u64 tile_mem(const ConvTile &t, u32 l) {
+    return (l & ((1u << t.c) - 1)) + ((u64)(l >> t.c) << t.a);
 }
 
 // ------------------------------------------------------------- host side
 #include <vector>
 namespace cantor_host {
 // the plan of a basis conversion of 2^k coefficients, in forward order
-struct TileOp {
-    int h, pos;   // T_h at index bit pos
-};
 struct ConvPlan {
-    std::vector<TileOp> tile;        // small sizes: the whole of it in one tile
-    std::vector<ConvStep> steps;     // else: the expansions, then
-    std::vector<ConvGroup> groups;   // the groups
-    bool empty() const { return tile.empty() && steps.empty() && groups.empty(); }
-    size_t launches() const { return !tile.empty() + steps.size() + groups.size(); }
+    std::vector<ConvStep> steps;    // before the tiles
+    std::vector<ConvTile> tiles;
+    bool empty() const { return steps.empty() && tiles.empty(); }
+    size_t launches() const { return steps.size() + tiles.size(); }
 };
-// conversion of the bits [pos, pos + k), k <= 8
-inline void group_ops(std::vector<TileOp> &ops, int pos, int k) {
+// steps e = n - 1 .. 0 of the expansion in powers of s_h, at index bit off,
+// at most `most` to a group, the groups counted from the bottom
+template <class F>
+inline void conv_steps(int off, int h, int n, int most, F &&put) {
+    for (int lo = (n - 1) / most * most; lo >= 0; lo -= most)
+        put(ConvStep{n - lo < most ? n - lo : most, h + lo + off, lo + off});
+}
+// stages of the bits [pos, pos + k), k <= 8, of a tile of 2^T: the top one
+// of a k that is no multiple of four has the tile's top bits
+inline void tile_group(ConvTile &t, int pos, int k) {
+    auto put = [&](const ConvStep &s) { t.st[t.n++] = s; };
     if (k <= 1) return;
-    const int h = k > 4 ? 4 : k > 2 ? 2 : 1;
-    for (int e = k - h - 1; e >= 0; e--) ops.push_back({h, pos + e});
-    group_ops(ops, pos + h, k - h);
-    group_ops(ops, pos, h);
+    if (k <= 4) {
+        put(ConvStep{0, k, pos + k - 4 < 0 ? 0 : pos + k - 4});
+        return;
+    }
+    conv_steps(pos, 4, k - 4, 2, put);
+    tile_group(t, pos + 4, k - 4);
+    tile_group(t, pos, 4);
 }
-inline void conv_steps(std::vector<ConvStep> &st, int off, int h, int n) {
-    // steps e = n - 1 .. 0, in groups of four from the bottom
-    for (int lo = (n - 1) & ~3; lo >= 0; lo -= 4)
-        st.push_back(ConvStep{n - lo < 4 ? n - lo : 4, h + lo + off, lo + off});
-}
-// one_tile: the largest k converted in a single tile
+// one_tile: the largest k converted in a single tile; tile_bits: of the
+// others' tiles.  Tiles have at least 16 coefficients (k < 4: zeros above).
 inline ConvPlan conv_plan(int k, int one_tile, int tile_bits) {
     ConvPlan P;
     if (k <= 1) return P;
+    auto step = [&](const ConvStep &s) { P.steps.push_back(s); };
     if (k <= one_tile) {
+        ConvTile t{k < 4 ? 4 : k, k < 4 ? 4 : k, 0, 0, {}};
+        auto put = [&](const ConvStep &s) { t.st[t.n++] = s; };
         if (k > 8) {
-            for (int e = k - 9; e >= 0; e--) P.tile.push_back({8, e});
-            group_ops(P.tile, 8, k - 8);
+            conv_steps(0, 8, k - 8, 2, put);
+            tile_group(t, 8, k - 8);
         }
-        group_ops(P.tile, 0, k > 8 ? 8 : k);
+        tile_group(t, 0, k > 8 ? 8 : k < 4 ? 4 : k);
+        P.tiles.push_back(t);
         return P;
     }
     const int low = k < 16 ? k : 16;
     if (k > 16) {
-        const int top = k - 16;
-        conv_steps(P.steps, 0, 16, top);
-        if (top > 8) conv_steps(P.steps, 16, 8, top - 8);
+        conv_steps(0, 16, k - 16, 4, step);
+        if (k > 24) conv_steps(16, 8, k - 24, 4, step);
     }
-    conv_steps(P.steps, 0, 8, low - 8);
-    for (int off = 0; off < k; off += 8) {
+    // the low part's expansion in powers of s_8: its steps 3..0 run in the
+    // contiguous tiles
+    const int n8 = low - 8;
+    if (n8 > 4) P.steps.push_back(ConvStep{n8 - 4, 12, 4});
+    ConvTile lo{12, 12, 0, 0, {}};
+    conv_steps(0, 8, n8 < 4 ? n8 : 4, 2, [&](const ConvStep &s) { lo.st[lo.n++] = s; });
+    tile_group(lo, 0, 8);
+    P.tiles.push_back(lo);
+    for (int off = 8; off < k; off += 8) {
         const int w = k - off < 8 ? k - off : 8;
         if (w < 2) break;
-        int tb = tile_bits;
-        if (off && tb > off + w) tb = off + w;
-        P.groups.push_back(ConvGroup{off, w, tb});
+        int c = tile_bits - w;
+        if (c > off) c = off;
+        ConvTile g{c, off, w, 0, {}};
+        tile_group(g, c, w);
+        P.tiles.push_back(g);
     }
     return P;
 }
@@ -728,9 +788,11 @@ inline bool build_tables(const u64 *b, FftTables &T) {
         const u64 tq = apply(inv, gf64_mul(b[15], wb));   // c4 Wb
         const u32 q0 = (u32)tq & 255, q1 = (u32)(tq >> 16) & 255;
         const u32 r0 = a0 ^ b0, r1 = a1 ^ b1;
-        return TwEnt{a0 | (m8(c3, a1) << 8) | ((a0 ^ a1) << 16),
-                     q0 | (m8(c3, q1) << 8) | ((q0 ^ q1) << 16),
-                     r0 | (m8(c3, r1) << 8) | ((r0 ^ r1) << 16), 0};
+        const u32 p[3] = {a0, m8(c3, a1), a0 ^ a1}, q[3] = {q0, m8(c3, q1), q0 ^ q1},
+                  r[3] = {r0, m8(c3, r1), r0 ^ r1};
+        auto two = [](u32 x, u32 y) { return (x << 4) | (y << 20); };
+        return TwEnt{two(p[0], p[2]), two(r[0], r[2]), two(p[1], r[1]), two(q[0], q[1]),
+                     q[2] << 4, {}};
     };
     TwEnt bit[32] = {};
     for (int j = 0; j + 1 < 32; j++) {
@@ -739,13 +801,9 @@ inline bool build_tables(const u64 *b, FftTables &T) {
     }
     for (int k = 0; k < 4; k++)
         for (int v = 0; v < 256; v++) {
-            TwEnt e{0, 0, 0, 0};
+            TwEnt e{};
             for (int j = 0; j < 8; j++)
-                if ((v >> j) & 1) {
-                    e.p ^= bit[8 * k + j].p;
-                    e.q ^= bit[8 * k + j].q;
-                    e.r ^= bit[8 * k + j].r;
-                }
+                if ((v >> j) & 1) e = tw_xor(e, bit[8 * k + j]);
             T.tw[k][v] = e;
         }
     // GF(2^32): tower bytes (p = 0..3, u5^0) <-> powers of rho

@@ -25,6 +25,7 @@
 #include <cstring>
 #include <algorithm>
 #include <atomic>
+#include <cstddef>
 
 namespace {
 
@@ -33,7 +34,7 @@ constexpr int FFT_TILE_BITS = 13;   // largest tile: 8192 elements
 constexpr int FFT_MIN_TILE_BITS = 6;
 constexpr int FFT_LOW_BITS = 4;
 constexpr int PACK_LIST = 12;   // four matrix entries + four vector pairs
-constexpr int CONV_ONE_TILE = 12;   // largest conversion done in one tile
+constexpr int CONV_ONE_TILE = 13;   // largest conversion done in one tile
 constexpr int CONV_TILE32 = 13, CONV_TILE64 = 12;
 
 __constant__ TwEnt c_tw[4][256];
@@ -92,14 +93,17 @@ struct ChunkIo {
 };
 struct ElemIo {
     u64 *f;
+    u64 n;
     typedef u64 type;
     GF2T_DEV bool any(u64) const { return true; }
-    GF2T_DEV u64 load(u64 i) const { return f[i]; }
-    GF2T_DEV void store(u64 i, u64 v) const { f[i] = v; }
+    GF2T_DEV u64 load(u64 i) const { return i < n ? f[i] : 0; }
+    GF2T_DEV void store(u64 i, u64 v) const {
+        if (i < n) f[i] = v;
+    }
 };
 
 constexpr int CONV_THREADS = 256;
-constexpr u32 CONV_EDGE_RHO = 16;
+constexpr u32 CONV_EDGE_RHO = 4;   // columns of the edges per block
 
 // One group of K expansion steps (ConvStep): blockIdx.y is the block of
 // 2^K rows; the first colblocks blocks take a skewed column per thread,
@@ -131,25 +135,38 @@ GF2T_DEV void conv_step_block(const Io &io, const ConvStep &s, u32 colblocks,
     }
     // edge: rho0 .. rho0 + nr of the unit, R x R coefficients each
     const u32 unit = 1u << s.ub, nr = unit < CONV_EDGE_RHO ? unit : CONV_EDGE_RHO;
-    const int lr = s.ub < 4 ? s.ub : 4;
+    const int lr = s.ub < 2 ? s.ub : 2;
     const u32 rho0 = (blockIdx.x - colblocks) * nr;
     const u32 total = (u32)(R * R) << lr;
-    for (u32 i = threadIdx.x; i < total; i += CONV_THREADS) {
+    constexpr int PER = (R * R * CONV_EDGE_RHO + CONV_THREADS - 1) / CONV_THREADS;
+    E v[PER];
+    auto mem = [&](u32 i) {
         const u32 rho = i & (nr - 1), q = (i >> lr) & (R - 1), k = i >> (lr + K);
-        lds[i] = io.load(base + ((u64)k << s.hb) + conv_edge(s, (int)k, q, rho0 + rho));
+        return base + ((u64)k << s.hb) + conv_edge(s, (int)k, q, rho0 + rho);
+    };
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const u32 i = threadIdx.x + j * CONV_THREADS;
+        v[j] = i < total ? io.load(mem(i)) : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const u32 i = threadIdx.x + j * CONV_THREADS;
+        if (i < total) lds[i] = v[j];
     }
     __syncthreads();
     for (int j = 0; j < K; j++) {
         const int e = INV ? j : K - 1 - j;
         for (u32 i = threadIdx.x; i < total / 2; i += CONV_THREADS) {
             const u32 rho = i & (nr - 1);
-            conv_tile_op([&](u32 l) -> E & { return lds[(l << lr) | rho]; }, i >> lr, K, e, INV);
+            conv_edge_pair([&](u32 l) -> E & { return lds[(l << lr) | rho]; }, K, e, INV, i >> lr);
         }
         __syncthreads();
     }
-    for (u32 i = threadIdx.x; i < total; i += CONV_THREADS) {
-        const u32 rho = i & (nr - 1), q = (i >> lr) & (R - 1), k = i >> (lr + K);
-        io.store(base + ((u64)k << s.hb) + conv_edge(s, (int)k, q, rho0 + rho), lds[i]);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const u32 i = threadIdx.x + j * CONV_THREADS;
+        if (i < total) io.store(mem(i), lds[i]);
     }
 }
 template <int K>
@@ -162,129 +179,78 @@ template <int K, bool INV>
 __global__ __launch_bounds__(CONV_THREADS) void k_conv_step64(u64 *__restrict__ f, u64 f_stride,
                                                               const ConvStep s, u32 colblocks) {
     __shared__ u64 lds[(1 << (2 * K)) * CONV_EDGE_RHO];
-    conv_step_block<K, INV>(ElemIo{f + (u64)blockIdx.z * f_stride}, s, colblocks, lds);
+    conv_step_block<K, INV>(ElemIo{f + (u64)blockIdx.z * f_stride, ~0ULL}, s, colblocks, lds);
 }
 
-// A group of up to eight index bits (ConvGroup): 64 coefficients per thread
-// in registers, two exchanges through LDS for w = 7, 8.  One coefficient in
-// 64 is left out of the LDS index, so that the threads of both layouts fall
-// on different banks.
-GF2T_DEV u32 group_pad(u32 i) { return i + (i >> 6); }
+// The conversion's other part: a tile in LDS (one coefficient in 17 left
+// out, so that the threads' runs of sixteen fall on different banks),
+// 16 coefficients per thread, stage by stage in registers.
+GF2T_DEV u32 conv_pad(u32 i) { return i + (i >> 4); }
 template <bool INV, class Io>
-GF2T_DEV void conv_group_block(const Io &io, const ConvGroup &g, typename Io::type *lds) {
+GF2T_DEV void conv_tile_block(const Io &io, const ConvTile &t, typename Io::type *lds) {
     typedef typename Io::type E;
-    const u64 base = group_base(g, blockIdx.x);
+    const u64 base = tile_base(t, blockIdx.x);
     if (!io.any(base)) return;   // whole block
-    const u32 tid = threadIdx.x, nthr = blockDim.x;
-    const bool two = g.w > 6;
-    E x[64];
-    if (g.off) {
+    const u32 q = threadIdx.x, nthr = blockDim.x;   // 16 coefficients each
+    E v[16];
 #pragma unroll
-        for (int r = 0; r < 64; r++)
-            x[r] = io.load(base + group_mem(g, group_local(g, 0, tid, r)));
-    } else {   // contiguous: through LDS, so that a wave reads whole runs
+    for (int j = 0; j < 16; j++) v[j] = io.load(base + tile_mem(t, q + j * nthr));
 #pragma unroll
-        for (int r = 0; r < 64; r++) lds[group_pad(tid + r * nthr)] = io.load(base + tid + r * nthr);
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 0, tid, r))];
-    }
-    if (two) {
-        if (INV) conv_group_top<INV>(x, g.w);
-        else conv_group_first<INV>(x, g.w);
-        if (!g.off) __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 0, tid, r))] = x[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 1, tid, r))];
-        conv_group_low<INV>(x, g.w);
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 1, tid, r))] = x[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) x[r] = lds[group_pad(group_local(g, 0, tid, r))];
-        if (INV) conv_group_first<INV>(x, g.w);
-        else conv_group_top<INV>(x, g.w);
-    } else {
-        conv_group_first<INV>(x, g.w);
-    }
-    if (g.off) {
-#pragma unroll
-        for (int r = 0; r < 64; r++)
-            io.store(base + group_mem(g, group_local(g, 0, tid, r)), x[r]);
-    } else {
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) lds[group_pad(group_local(g, 0, tid, r))] = x[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 64; r++) io.store(base + tid + r * nthr, lds[group_pad(tid + r * nthr)]);
-    }
-}
-__global__ __launch_bounds__(128) void k_conv_group32(const Operands ops, const ConvGroup g,
-                                                      int first) {
-    extern __shared__ u32 lds32[];
-    conv_group_block<false>(ChunkIo{operand(ops, blockIdx.y), first != 0}, g, lds32);
-}
-template <bool INV>
-__global__ __launch_bounds__(128) void k_conv_group64(u64 *__restrict__ f, u64 f_stride,
-                                                      const ConvGroup g) {
-    extern __shared__ u64 lds64[];
-    conv_group_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride}, g, lds64);
-}
-
-// Small sizes: the whole conversion of a transform in one block, every
-// step inside LDS.
-constexpr int CONV_MAX_OPS = 32;
-struct TileArg {
-    int T, nops;
-    signed char h[CONV_MAX_OPS], pos[CONV_MAX_OPS];   // in execution order
-};
-template <bool INV, class Io>
-GF2T_DEV void conv_tile_block(const Io &io, const TileArg &t, typename Io::type *lds) {
-    typedef typename Io::type E;
-    const u32 n = 1u << t.T, nthr = blockDim.x;
-    if (!io.any(0)) return;   // whole block
-    for (u32 l = threadIdx.x; l < n; l += nthr) lds[l] = io.load(l);
+    for (int j = 0; j < 16; j++) lds[conv_pad(q + j * nthr)] = v[j];
     __syncthreads();
-    for (int o = 0; o < t.nops; o++) {
-        const int h = t.h[o], pos = t.pos[o];
-        for (u32 i = threadIdx.x; i < n / 2; i += nthr)
-            conv_tile_op([&](u32 l) -> E & { return lds[l]; }, i, h, pos, INV);
+    for (int i = 0; i < t.n; i++) {
+        const ConvStep s = t.st[INV ? t.n - 1 - i : i];
+        conv_tile_stage<INV, E>([&](u32 l) -> E & { return lds[conv_pad(l)]; }, q, nthr, s);
         __syncthreads();
     }
-    for (u32 l = threadIdx.x; l < n; l += nthr) io.store(l, lds[l]);
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+        io.store(base + tile_mem(t, q + j * nthr), lds[conv_pad(q + j * nthr)]);
 }
-__global__ __launch_bounds__(1024) void k_conv_tile32(const Operands ops, const TileArg t,
-                                                      int first) {
+__global__ __launch_bounds__(512) void k_conv_tile32(const Operands ops, const ConvTile t,
+                                                     int first) {
     extern __shared__ u32 lds32[];
     conv_tile_block<false>(ChunkIo{operand(ops, blockIdx.y), first != 0}, t, lds32);
 }
 template <bool INV>
-__global__ __launch_bounds__(1024) void k_conv_tile64(u64 *__restrict__ f, u64 f_stride,
-                                                      const TileArg t) {
+__global__ __launch_bounds__(512) void k_conv_tile64(u64 *__restrict__ f, u64 f_stride, u64 n,
+                                                     const ConvTile t) {
     extern __shared__ u64 lds64[];
-    conv_tile_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride}, t, lds64);
+    conv_tile_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride, n}, t, lds64);
 }
 
 // ------------------------------------------------------------ butterflies
-// LDS copy of the GF(2^8) multiply tables
+// n 16-byte words from memory to LDS, four loads in flight per thread
+GF2T_DEV void copy_lds(void *dst_, const void *src_, u32 n) {
+    uint4 *dst = (uint4 *)dst_;
+    const uint4 *src = (const uint4 *)src_;
+    const u32 nthr = blockDim.x;
+    for (u32 i = threadIdx.x; i < n; i += 4 * nthr) {
+        const u32 i1 = i + nthr, i2 = i1 + nthr, i3 = i2 + nthr, e = n - 1;
+        const uint4 v0 = src[i], v1 = src[i1 < e ? i1 : e], v2 = src[i2 < e ? i2 : e],
+                    v3 = src[i3 < e ? i3 : e];
+        dst[i] = v0;
+        if (i1 < n) dst[i1] = v1;
+        if (i2 < n) dst[i2] = v2;
+        if (i3 < n) dst[i3] = v3;
+    }
+}
+// LDS copies of the GF(2^8) multiply tables and, behind them, the GF(2^32)
+// basis tables (FftTables' first members)
 struct MulLds {
     uint4 A[256];
     u32 B[256];
-    GF2T_DEV void load() {
-        for (u32 i = threadIdx.x; i < 256; i += blockDim.x) {
-            A[i] = reinterpret_cast<const uint4 *>(g_tab.mulA)[i];
-            B[i] = g_tab.mulB[i];
-        }
-    }
-    GF2T_DEV Mul8 operator()(u32 v) const {
-        const uint4 a = A[v];
-        return Mul8{a.x, a.y, a.z, a.w, B[v]};
+    GF2T_DEV Mul8 operator()(u32 off) const {
+        const unsigned char *p = reinterpret_cast<const unsigned char *>(A);
+        const uint4 a = *reinterpret_cast<const uint4 *>(p + off);
+        return Mul8{a.x, a.y, a.z, a.w,
+                    *reinterpret_cast<const u32 *>(p + sizeof(A) + (off >> 2))};
     }
 };
+struct ProdLds {
+    u32 d32[4][256], d5[4][256], b32[4][256];
+};
+static_assert(sizeof(MulLds) + sizeof(ProdLds) == offsetof(FftTables, emb), "table layout");
 // what a pass reads and writes: units; the chunks of an operand (lch:
 // converted ones); elements in the polynomial basis
 enum { IO_UNITS = 0, IO_CHUNKS = 1, IO_LCH = 2, IO_PLAIN = 3 };
@@ -332,198 +298,341 @@ GF2T_DEV void store_unit(U4 *f, u32 i, const U4 &u, int io, const Emb *une) {
 }
 // copy a basis table (8 x 256 entries; 4 x 256 for chunks) to LDS
 GF2T_DEV void load_basis(u64 *dst, const u64 (*src)[256], int bytes) {
-    for (u32 i = threadIdx.x; i < (u32)bytes * 256; i += blockDim.x)
-        dst[i] = reinterpret_cast<const u64 *>(src)[i];
+    copy_lds(dst, src, (u32)bytes * 128);
 }
 GF2T_DEV u32 uniform32(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // One butterfly pass over the window of P (see BfPass): 2^RB units per
-// thread, RB levels, an exchange through LDS, and so on.
+// thread, RB levels, an exchange through LDS, and so on.  A block takes
+// every gridDim.x-th tile, so that the tables it copies to LDS (5 KB, and
+// 8 or 16 KB of a basis table) serve several tiles of 16 KB.
 template <int CLS, bool INV>
-__global__ __launch_bounds__(512) void k_bfly(u64 *__restrict__ f_, u64 f_stride, const BfPass P,
+__global__ __launch_bounds__(256) void k_bfly(u64 *__restrict__ f_, u64 f_stride, const BfPass P,
                                               const Operands ops, int in, int out) {
     constexpr int R = 1 << RB;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     MulLds &tab = *reinterpret_cast<MulLds *>(lds_raw);
-    u64 *basis = reinterpret_cast<u64 *>(lds_raw + sizeof(MulLds));
-    U4 *ex = reinterpret_cast<U4 *>(basis);
+    U4 *ex = reinterpret_cast<U4 *>(lds_raw + sizeof(MulLds));
+    u64 *basis = reinterpret_cast<u64 *>(ex + (P.w > RB ? 1u << P.tb : 0u));
     U4 *f = reinterpret_cast<U4 *>(f_ + (u64)blockIdx.y * f_stride);
     Operand o{};
     if (in == IO_CHUNKS || in == IO_LCH) o = operand(ops, blockIdx.y);
-    tab.load();
+    copy_lds(lds_raw, &g_tab, sizeof(MulLds) / 16);
     if (in != IO_UNITS) load_basis(basis, g_tab.emb, in == IO_PLAIN ? 8 : 4);
+    if (out == IO_PLAIN) load_basis(basis, g_tab.une, 8);   // never both
     __syncthreads();
     const u32 tid = threadIdx.x;
-    const BfTile T = bf_tile(P, blockIdx.x);
     const int ns = bf_stages(P);
     const Emb *emb = reinterpret_cast<const Emb *>(basis);
-    U4 x[R];
-    int s = INV ? ns - 1 : 0;
+    const u32 tiles = 1u << (P.m - 1 - P.tb);
+    for (u32 blk = blockIdx.x; blk < tiles; blk += gridDim.x) {
+        const BfTile T = bf_tile(P, blk);
+        U4 x[R];
+        int s = INV ? ns - 1 : 0;
 #pragma unroll
-    for (int r = 0; r < R; r++)
-        x[r] = load_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), in, o, emb);
-    bool gives = in != IO_UNITS;   // the basis table gives way to the exchange
+        for (int r = 0; r < R; r++)
+            x[r] = load_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), in, o, emb);
 #pragma nounroll
-    for (int k = 0;; k++) {
-        TwEnt W[RB];
-        bf_twiddles(P, T, s, tid, c_tw, W);
-        fft_stage<CLS, INV>(x, bf_active(P, s), W, tab);
-        if (k == ns - 1) break;
-        if (gives) __syncthreads();
-        gives = true;
+        for (int k = 0;; k++) {
+            TwEnt W[RB];
+            bf_twiddles(P, T, s, tid, c_tw, W);
+            fft_stage<CLS, INV>(x, bf_active(P, s), W, bf_zero(P, T, s), tab);
+            if (k == ns - 1) break;
+            __syncthreads();   // the last exchange is read
 #pragma unroll
-        for (int r = 0; r < R; r++) ex[bf_local(P, s, tid, r)] = x[r];
-        s += INV ? -1 : 1;
-        __syncthreads();
+            for (int r = 0; r < R; r++) ex[bf_local(P, s, tid, r)] = x[r];
+            s += INV ? -1 : 1;
+            __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; r++) x[r] = ex[bf_local(P, s, tid, r)];
+            for (int r = 0; r < R; r++) x[r] = ex[bf_local(P, s, tid, r)];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            store_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), x[r], out, emb);
     }
-    if (out == IO_PLAIN) {
-        __syncthreads();   // exchange (or embedding table) done with
-        load_basis(basis, g_tab.une, 8);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        store_unit(f, bf_unit(P, T, bf_local(P, s, tid, r)), x[r], out, emb);
 }
 
 // ---- the low levels
 constexpr u32 LO_UNITS = 64u << RB;              // per wave
-constexpr u32 LO_EXCH = (64u << RB) + (4u << RB);  // words of a wave's exchange plane
+// words of a wave's exchange plane, and of the two rows of units that the
+// waves of a pair hand over
+constexpr u32 LO_EXCH = 2 * 64 * 4;
+static_assert(LO_EXCH >= (64u << RB) + (4u << RB), "a padded plane of one word per unit");
 
-GF2T_DEV u32 lo_pad(u32 u) { return u + (u >> 4); }
+// (linear over disjoint bits, so a row's place is the lane's plus a constant)
+GF2T_HD constexpr u32 lo_pad(u32 u) { return u + (u >> 4); }
 // the wave's units from the layout of one stage to that of another, a word
 // of each unit at a time through the wave's own plane in LDS
-GF2T_DEV void lo_exchange(U4 *x, u32 lane, u32 *plane, int from, int to) {
+template <int FROM, int TO>
+GF2T_DEV void lo_exchange(U4 *x, u32 lane, u32 *plane) {
+    u32 *from = plane + lo_pad(lo_unit(FROM, lane, 0));
+    const u32 *to = plane + lo_pad(lo_unit(TO, lane, 0));
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int r = 0; r < (1 << RB); r++) plane[lo_pad(lo_unit(from, lane, r))] = x[r].w[p];
+        for (int r = 0; r < (1 << RB); r++) from[lo_pad((u32)r << lo_pos(FROM))] = x[r].w[p];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int r = 0; r < (1 << RB); r++) x[r].w[p] = plane[lo_pad(lo_unit(to, lane, r))];
+        for (int r = 0; r < (1 << RB); r++) x[r].w[p] = to[lo_pad((u32)r << lo_pos(TO))];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
+template <int S, int CLS, bool INV>
+GF2T_DEV void lo_stage(U4 *x, int m, u32 ubase, u32 lane, const MulLds &tab, const TwEnt *hi) {
+    TwEnt W[RB], W0;
+    lo_twiddles<S>(ubase, lane, c_tw, hi, W, W0);
+    if (INV && S == lo_stages() - 1) fft_level0<CLS, true>(x, W0, tab);
+    fft_stage<CLS, INV>(x, lo_active(m, S), W, false, tab);
+    if (!INV && S == lo_stages() - 1) fft_level0<CLS, false>(x, W0, tab);
+}
+static_assert(lo_stages() == 4, "the stages are spelled out below");
 template <int CA, int CB>
 GF2T_DEV void lo_forward(U4 *x, int m, u32 ubase, u32 lane, const MulLds &tab, const TwEnt *hi,
                          u32 *plane) {
-    TwEnt W[RB], W0;
-    lo_twiddles(ubase, 0, lane, c_tw, hi, W, W0);
-    fft_stage<CA, false>(x, lo_active(m, 0), W, tab);
-#pragma nounroll
-    for (int s = 1; s < lo_stages(); s++) {
-        lo_exchange(x, lane, plane, s - 1, s);
-        lo_twiddles(ubase, s, lane, c_tw, hi, W, W0);
-        fft_stage<CB, false>(x, lo_active(m, s), W, tab);
-    }
-    fft_level0<CB, false>(x, W0, tab);
+    lo_stage<0, CA, false>(x, m, ubase, lane, tab, hi);
+    lo_exchange<0, 1>(x, lane, plane);
+    lo_stage<1, CB, false>(x, m, ubase, lane, tab, hi);
+    lo_exchange<1, 2>(x, lane, plane);
+    lo_stage<2, CB, false>(x, m, ubase, lane, tab, hi);
+    lo_exchange<2, 3>(x, lane, plane);
+    lo_stage<3, CB, false>(x, m, ubase, lane, tab, hi);
 }
 template <int CA, int CB>
 GF2T_DEV void lo_inverse(U4 *x, int m, u32 ubase, u32 lane, const MulLds &tab, const TwEnt *hi,
                          u32 *plane) {
-    TwEnt W[RB], W0;
-    lo_twiddles(ubase, lo_stages() - 1, lane, c_tw, hi, W, W0);
-    fft_level0<CB, true>(x, W0, tab);
-#pragma nounroll
-    for (int s = lo_stages() - 1; s > 0; s--) {
-        lo_twiddles(ubase, s, lane, c_tw, hi, W, W0);
-        fft_stage<CB, true>(x, lo_active(m, s), W, tab);
-        lo_exchange(x, lane, plane, s, s - 1);
-    }
-    lo_twiddles(ubase, 0, lane, c_tw, hi, W, W0);
-    fft_stage<CA, true>(x, lo_active(m, 0), W, tab);
+    lo_stage<3, CB, true>(x, m, ubase, lane, tab, hi);
+    lo_exchange<3, 2>(x, lane, plane);
+    lo_stage<2, CB, true>(x, m, ubase, lane, tab, hi);
+    lo_exchange<2, 1>(x, lane, plane);
+    lo_stage<1, CB, true>(x, m, ubase, lane, tab, hi);
+    lo_exchange<1, 0>(x, lane, plane);
+    lo_stage<0, CA, true>(x, m, ubase, lane, tab, hi);
 }
-struct ProdLds {   // GF(2^32) basis tables
-    u32 d32[4][256], d5[4][256], b32[4][256];
-    GF2T_DEV void load() {
-        for (u32 i = threadIdx.x; i < 1024; i += blockDim.x) {
-            (&d32[0][0])[i] = (&g_tab.d32[0][0])[i];
-            (&d5[0][0])[i] = (&g_tab.d5[0][0])[i];
-            (&b32[0][0])[i] = (&g_tab.b32[0][0])[i];
-        }
-    }
-};
+GF2T_DEV U4 unit_select(bool c, const U4 &a, const U4 &b) {
+    return U4{{c ? a.w[0] : b.w[0], c ? a.w[1] : b.w[1], c ? a.w[2] : b.w[2],
+               c ? a.w[3] : b.w[3]}};
+}
 enum { LO_FWD = 0, LO_INV = 1, LO_MUL = 2 };
 // Levels 7..0 of a transform (LO_FWD, LO_INV), or, of two transforms, both
 // forward, their product and the inverse of it in one pass (LO_MUL: f and
-// g, into f).  A wave takes LO_UNITS consecutive units.
+// g, into f).  A wave takes LO_UNITS consecutive units; LO_MUL pairs two
+// waves, one per operand, which then multiply half of the units each, and
+// the first inverts (one wave for both operands took 164 registers instead
+// of about 100 and half as long again at sizes that do not fill the chip).
 template <int CA, int CB, int DIR>
 __global__ __launch_bounds__(256) void k_low(u64 *__restrict__ f_, u64 f_stride,
                                              const u64 *__restrict__ g_, int m,
                                              const Operands ops, u32 g_op, int in, int out) {
     constexpr int R = 1 << RB;
     constexpr int LAST = lo_stages() - 1;
+    constexpr bool MUL = DIR == LO_MUL;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     MulLds &tab = *reinterpret_cast<MulLds *>(lds_raw);
-    TwEnt *hi = reinterpret_cast<TwEnt *>(lds_raw + sizeof(MulLds));
-    ProdLds &pt = *reinterpret_cast<ProdLds *>(hi + 4);
-    unsigned char *rest = (unsigned char *)(hi + 4) + (DIR == LO_MUL ? sizeof(ProdLds) : 0);
-    u32 *plane = reinterpret_cast<u32 *>(rest) + (threadIdx.x >> 6) * LO_EXCH;
-    u64 *basis = reinterpret_cast<u64 *>(rest + (blockDim.x >> 6) * LO_EXCH * 4);
+    const ProdLds &pt = *reinterpret_cast<const ProdLds *>(lds_raw + sizeof(MulLds));
+    constexpr u32 TABS = sizeof(MulLds) + (MUL ? sizeof(ProdLds) : 0);
+    TwEnt *hi = reinterpret_cast<TwEnt *>(lds_raw + TABS);
+    const u32 wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    u32 *planes = reinterpret_cast<u32 *>(hi + 4);
+    u32 *plane = planes + wave * LO_EXCH;
+    u64 *basis = reinterpret_cast<u64 *>(planes + (blockDim.x >> 6) * LO_EXCH);
     const Emb *emb = reinterpret_cast<const Emb *>(basis);
-    U4 *f = reinterpret_cast<U4 *>(f_ + (u64)blockIdx.y * f_stride);
-    tab.load();
+    copy_lds(lds_raw, &g_tab, TABS / 16);
     if (threadIdx.x < 4) hi[threadIdx.x] = tw_of(g_tab.tw, threadIdx.x << 7);
-    if (DIR == LO_MUL) pt.load();
     if (in != IO_UNITS) load_basis(basis, g_tab.emb, in == IO_PLAIN ? 8 : 4);
     __syncthreads();
     const u32 units = 1u << (m - 1);
-    const u32 lane = threadIdx.x & 63;
-    const u32 ubase =
-        uniform32((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * LO_UNITS);
-    const bool act = ubase < units;   // whole wave
-    U4 x[R], y[R];
+    const u32 per = (blockDim.x >> 6) >> (MUL ? 1 : 0);   // runs of units per block
+    const bool second = MUL && (wave & 1);                // the wave of operand g
+    const u32 ubase = uniform32((blockIdx.x * per + (MUL ? wave >> 1 : wave)) * LO_UNITS);
+    const bool act = ubase < units;                       // whole wave
+    U4 *f = reinterpret_cast<U4 *>(f_ + (u64)blockIdx.y * f_stride);
+    U4 x[R];
     if (act) {
-#pragma nounroll
-        for (int op = 0; op < (DIR == LO_MUL ? 2 : 1); op++) {
-            if (DIR == LO_MUL) {
+        const U4 *src = second ? reinterpret_cast<const U4 *>(g_ + (u64)blockIdx.y * f_stride) : f;
+        Operand o{};
+        if (in == IO_CHUNKS || in == IO_LCH) o = operand(ops, blockIdx.y + (second ? g_op : 0));
 #pragma unroll
-                for (int r = 0; r < R; r++) y[r] = x[r];
-            }
-            const U4 *src = op ? reinterpret_cast<const U4 *>(g_ + (u64)blockIdx.y * f_stride) : f;
-            Operand o{};
-            if (in == IO_CHUNKS || in == IO_LCH) o = operand(ops, blockIdx.y + (op ? g_op : 0));
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const u32 i = ubase + lo_unit(0, lane, r);
-                x[r] = i < units ? load_unit(src, i, in, o, emb) : U4{{0, 0, 0, 0}};
-            }
-            if (DIR != LO_INV) lo_forward<CA, CB>(x, m, ubase, lane, tab, hi, plane);
+        for (int r = 0; r < R; r++) {
+            const u32 i = ubase + lo_unit(0, lane, r);
+            x[r] = i < units ? load_unit(src, i, in, o, emb) : U4{{0, 0, 0, 0}};
         }
-        if (DIR == LO_MUL) {
-            // one unit's product per round, the registers turning, so that
-            // the code is there once
-#pragma nounroll
-            for (int k = 0; k < R; k++) {
-                const U4 v = unit_mul(y[0], x[0], pt.d32, pt.d5, pt.b32);
-#pragma unroll
-                for (int r = 0; r + 1 < R; r++) {
-                    x[r] = x[r + 1];
-                    y[r] = y[r + 1];
-                }
-                x[R - 1] = v;
-            }
-        }
-        if (DIR == LO_FWD) lo_exchange(x, lane, plane, LAST, 0);   // to contiguous stores
-        if (DIR == LO_INV) lo_exchange(x, lane, plane, 0, LAST);
-        if (DIR != LO_FWD) lo_inverse<CA, CB>(x, m, ubase, lane, tab, hi, plane);
+        if (DIR != LO_INV) lo_forward<CA, CB>(x, m, ubase, lane, tab, hi, plane);
+        if (DIR == LO_FWD) lo_exchange<LAST, 0>(x, lane, plane);   // to contiguous stores
+        if (DIR == LO_INV) lo_exchange<0, LAST>(x, lane, plane);
     }
+    if (MUL) {
+        // rows 0 and 1 are multiplied by the first wave of a pair, 2 and 3
+        // by the second: each hands the other's rows over, then the second
+        // its products, through the planes (a unit is four words)
+        static_assert(R == 4 && LO_EXCH >= 2 * 64 * 4, "two rows fit a plane");
+        U4 *mine = reinterpret_cast<U4 *>(plane);
+        const U4 *other = reinterpret_cast<const U4 *>(planes + (wave ^ 1) * LO_EXCH);
+        __syncthreads();
+        mine[lane] = unit_select(second, x[0], x[2]);
+        mine[64 + lane] = unit_select(second, x[1], x[3]);
+        __syncthreads();
+        U4 y0 = other[lane], y1 = other[64 + lane];
+        U4 z0 = unit_select(second, x[2], x[0]), z1 = unit_select(second, x[3], x[1]);
+        __syncthreads();
+#pragma nounroll
+        for (int k = 0; k < 2; k++) {
+            const U4 v = unit_mul(z0, y0, pt.d32, pt.d5, pt.b32);
+            z0 = z1;
+            y0 = y1;
+            z1 = v;
+        }
+        if (second) {
+            mine[lane] = z0;
+            mine[64 + lane] = z1;
+        }
+        __syncthreads();
+        x[0] = z0;
+        x[1] = z1;
+        x[2] = other[lane];
+        x[3] = other[64 + lane];
+    }
+    if (DIR != LO_FWD && act && !second)
+        lo_inverse<CA, CB>(x, m, ubase, lane, tab, hi, plane);
     if (out == IO_PLAIN) {
         __syncthreads();
         load_basis(basis, g_tab.une, 8);
         __syncthreads();
     }
-    if (act) {
+    if (act && !second) {
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const u32 i = ubase + lo_unit(0, lane, r);
             if (i < units) store_unit(f, i, x[r], out, emb);
         }
     }
+}
+
+// --------------------------------------------------- small products
+// All chunk products of two operands, without a transform: c_k = sum of
+// a_i b_(k-i), carry-less, i over the shorter operand.  A block takes
+// SC_OUT outputs and SC_IN values of i, its four waves a quarter of them
+// each, a lane two outputs; the products of one bit class (see clmul32)
+// are XORed up as they come and the classes merged once at the end, so a
+// 32 x 32 product costs 16 multiply-adds and 12 XORs.  Block (t, c) writes
+// the part of the outputs [SC_OUT t, SC_OUT (t + 1)) that comes from the
+// i in [SC_IN c, SC_IN (c + 1)) to part[c][.].
+constexpr u32 SC_OUT = 128, SC_IN = 128;
+struct SchoolShape {
+    u32 na, nb;         // chunks, na <= nb
+    u32 nout, nparts;   // na + nb - 1 outputs; parts
+};
+// the parts that reach output tile t: c in [first, last]
+GF2T_HD u32 school_first(const SchoolShape &s, u32 t) {
+    const u32 k0 = t * SC_OUT;
+    return k0 >= s.nb + SC_IN - 1 ? (k0 - s.nb + 1 - (SC_IN - 1) + SC_IN - 1) / SC_IN : 0;
+}
+GF2T_HD u32 school_last(const SchoolShape &s, u32 t) { return t < s.nparts - 1 ? t : s.nparts - 1; }
+
+__global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, int swap,
+                                                const SchoolShape s, u64 *__restrict__ part,
+                                                u64 part_stride) {
+    static_assert(SC_OUT == 128 && SC_IN == 128, "two outputs per lane, 32 values per wave");
+    __shared__ u32 bs[SC_OUT + SC_IN];
+    __shared__ u64 sum[4][SC_OUT];
+    const u32 t = blockIdx.x, c = blockIdx.y, y = blockIdx.z;
+    if (c < school_first(s, t) || c > school_last(s, t)) return;   // whole block
+    const Operand oa = operand(ops, swap ? y + b_op : y), ob = operand(ops, swap ? y : y + b_op);
+    const int k0 = (int)(t * SC_OUT), i0 = (int)(c * SC_IN);
+    const int j0 = k0 - i0 - (int)(SC_IN - 1);   // b index of bs[0]
+    for (u32 x = threadIdx.x; x < SC_OUT + SC_IN - 1; x += 256) {
+        const int j = j0 + (int)x;
+        bs[x] = j >= 0 ? chunk(ob, (u64)j) : 0;
+    }
+    const u32 wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int iw = i0 + (int)wave * 32;
+    const u32 av = lane < 32 ? chunk(oa, (u64)iw + lane) : 0;
+    __syncthreads();
+    const u32 m0 = 0x11111111u;
+    u64 acc[2][4] = {};
+    const u32 at = lane + (SC_IN - 1) - wave * 32;   // bs index of output `lane`, i = iw
+#pragma unroll 2
+    for (int i = 0; i < 32; i++) {
+        const u32 a = __builtin_amdgcn_readlane(av, i);
+        const u64 a0 = a & m0, a1 = a & (m0 << 1), a2 = a & (m0 << 2), a3 = a & (m0 << 3);
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            const u32 b = bs[at - i + 64 * o];
+            const u64 b0 = b & m0, b1 = b & (m0 << 1), b2 = b & (m0 << 2), b3 = b & (m0 << 3);
+            acc[o][0] = xor3(acc[o][0], a0 * b0 + a1 * b3, a2 * b2) ^ (a3 * b1);
+            acc[o][1] = xor3(acc[o][1], a0 * b1 + a2 * b3, a1 * b0 + a3 * b2);
+            acc[o][2] = xor3(acc[o][2], a0 * b2 + a3 * b3, a1 * b1) ^ (a2 * b0);
+            acc[o][3] = xor3(xor3(acc[o][3], a0 * b3, a1 * b2), a2 * b1, a3 * b0);
+        }
+    }
+    const u64 q = 0x1111111111111111ULL;
+#pragma unroll
+    for (int o = 0; o < 2; o++)
+        sum[wave][lane + 64 * o] =
+            sel64(q, acc[o][0], sel64(q << 1, acc[o][1], sel64(q << 2, acc[o][2], acc[o][3])));
+    __syncthreads();
+    const u32 k = (u32)k0 + threadIdx.x;
+    if (threadIdx.x < SC_OUT && k < s.nout)
+        part[(u64)y * part_stride + (u64)c * s.nout + k] =
+            xor3(sum[0][threadIdx.x], sum[1][threadIdx.x], sum[2][threadIdx.x]) ^
+            sum[3][threadIdx.x];
+}
+// word k of the product: chunk coefficients 2k - 1, 2k and 2k + 1
+struct SchoolWords {
+    const u64 *part;
+    SchoolShape s;
+    GF2T_DEV u64 coef(u64 k) const {
+        if (k >= s.nout) return 0;
+        u64 v = 0;
+        const u32 t = (u32)k / SC_OUT, hi = school_last(s, t);
+        for (u32 c = school_first(s, t); c <= hi; c++) v ^= part[(u64)c * s.nout + k];
+        return v;
+    }
+    GF2T_DEV u64 operator()(size_t w) const {
+        const u64 k = 2 * (u64)w;
+        u64 v = coef(k) ^ (coef(k + 1) << 32);
+        if (w) v ^= coef(k - 1) >> 32;
+        return v;
+    }
+};
+// the product's words: a block adds up the parts of 2 SP_WORDS + 1 chunk
+// coefficients, four threads each, and writes SP_WORDS words
+constexpr u32 SP_WORDS = 32;
+__global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ part,
+                                                        const SchoolShape s,
+                                                        u64 *__restrict__ out, size_t owords) {
+    __shared__ u64 sum[4][2 * SP_WORDS + 1];   // coefficients k0 - 1 ..
+    const u32 w0 = blockIdx.x * SP_WORDS;
+    const u32 g = threadIdx.x & 3;
+    for (u32 x = threadIdx.x >> 2; x < 2 * SP_WORDS + 1; x += 64) {
+        u64 v = 0;
+        const u64 k = 2 * (u64)w0 + x;   // coefficient k - 1
+        if (k >= 1 && k - 1 < s.nout) {
+            const u32 t = (u32)(k - 1) / SC_OUT, hi = school_last(s, t);
+#pragma unroll 4
+            for (u32 c = school_first(s, t) + g; c <= hi; c += 4)
+                v ^= part[(u64)c * s.nout + (k - 1)];
+        }
+        sum[g][x] = v;
+    }
+    __syncthreads();
+    auto coef = [&](u32 x) { return xor3(sum[0][x], sum[1][x], sum[2][x]) ^ sum[3][x]; };
+    const u32 x = threadIdx.x;
+    if (x < SP_WORDS && w0 + x < owords)
+        out[w0 + x] = coef(2 * x + 1) ^ (coef(2 * x + 2) << 32) ^ (coef(2 * x) >> 32);
+}
+// the product folded mod x^r + x^s + 1 (s from svec where there is a batch)
+__global__ __launch_bounds__(256) void k_school_fold(const u64 *__restrict__ part, u64 part_stride,
+                                                     const SchoolShape s, u64 L,
+                                                     u64 *__restrict__ out, size_t nw,
+                                                     u64 o_stride, u64 r, u64 sv,
+                                                     const u64 *__restrict__ svec) {
+    const size_t w = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (w >= nw) return;
+    out[(u64)blockIdx.y * o_stride + w] =
+        fold_words(SchoolWords{part + (u64)blockIdx.y * part_stride, s}, L, r,
+                   svec ? svec[blockIdx.y] : sv, w);
 }
 
 // overlap-add in gather form: output word w collects chunks 2w-1, 2w, 2w+1
@@ -623,6 +732,9 @@ int ensure_basis() {
         }
         GF2T_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tab), tab, sizeof(FftTables)));
         GF2T_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_tw), tab->tw, sizeof(tab->tw)));
+        // the one kernel whose tile can pass 64 KiB of LDS (2^13 elements)
+        for (const void *k : {(const void *)k_conv_tile64<false>, (const void *)k_conv_tile64<true>})
+            GF2T_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024));
         g_basis.uploaded_dev = dev;
     }
     return GF2T_OK;
@@ -664,27 +776,21 @@ const cantor_host::ConvPlan &conv_plan64(int k) {
     }();
     return v[k];
 }
-TileArg tile_arg(const std::vector<cantor_host::TileOp> &ops, int T, bool inv) {
-    TileArg a{};
-    a.T = T;
-    a.nops = (int)ops.size();
-    for (int i = 0; i < a.nops; i++) {
-        const auto &op = ops[inv ? a.nops - 1 - i : i];
-        a.h[i] = (signed char)op.h;
-        a.pos[i] = (signed char)op.pos;
-    }
-    return a;
-}
 dim3 step_grid(const ConvStep &s, int k, unsigned nbatch, u32 &colblocks) {
     colblocks = (conv_full(s) + CONV_THREADS - 1) / CONV_THREADS;
     const u32 unit = 1u << s.ub;
     const u32 edges = unit < CONV_EDGE_RHO ? 1 : unit / CONV_EDGE_RHO;
     return dim3(colblocks + edges, 1u << (k - s.hb - s.K), nbatch);
 }
-size_t group_lds(const ConvGroup &g, size_t elem) {
-    return g.off && g.w <= 6 ? 0 : (((size_t)1 << g.tb) + ((size_t)1 << g.tb) / 64) * elem;
+size_t tile_lds(const ConvTile &t, size_t elem) {
+    const size_t n = (size_t)1 << (t.c + t.w);
+    return (n + n / 16) * elem;
 }
-unsigned tile_threads(int T) { return (unsigned)std::max(64, std::min(1024, 1 << (T - 1))); }
+dim3 tile_grid(const ConvTile &t, int k, unsigned nbatch) {
+    const int T = t.c + t.w;
+    return dim3(k > T ? 1u << (k - T) : 1u, nbatch);
+}
+dim3 tile_threads(const ConvTile &t) { return dim3(1u << (t.c + t.w - 4)); }
 
 // basis conversion of nbatch operands of at most 2^k chunks, into their
 // lch buffers; ran: whether anything was launched (k > 1)
@@ -692,9 +798,6 @@ int run_conv32(const Operands &ops, int k, unsigned nbatch, hipStream_t st, bool
     const cantor_host::ConvPlan &P = conv_plan32(k);
     ran = !P.empty();
     int first = 1;
-    if (!P.tile.empty())
-        hipLaunchKernelGGL(k_conv_tile32, dim3(1, nbatch), dim3(tile_threads(k)), (size_t)4 << k,
-                           st, ops, tile_arg(P.tile, k, false), first);
     for (const ConvStep &s : P.steps) {
         u32 cb;
         const dim3 g = step_grid(s, k, nbatch, cb);
@@ -706,9 +809,9 @@ int run_conv32(const Operands &ops, int k, unsigned nbatch, hipStream_t st, bool
         }
         first = 0;
     }
-    for (const ConvGroup &g : P.groups) {
-        hipLaunchKernelGGL(k_conv_group32, dim3(1u << (k - g.tb), nbatch), dim3(1u << (g.tb - 6)),
-                           group_lds(g, 4), st, ops, g, first);
+    for (const ConvTile &t : P.tiles) {
+        hipLaunchKernelGGL(k_conv_tile32, tile_grid(t, k, nbatch), tile_threads(t), tile_lds(t, 4),
+                           st, ops, t, first);
         first = 0;
     }
     GF2T_CHECK_LAUNCH("k_conv32");
@@ -727,23 +830,21 @@ int run_conv64(u64 *f, u64 stride, int m, unsigned nbatch, hipStream_t st) {
         default: hipLaunchKernelGGL((k_conv_step64<4, INV>), g, dim3(CONV_THREADS), 0, st, f, stride, s, cb); break;
         }
     };
-    auto group = [&](const ConvGroup &g) {
-        hipLaunchKernelGGL(k_conv_group64<INV>, dim3(1u << (m - g.tb), nbatch),
-                           dim3(1u << (g.tb - 6)), group_lds(g, 8), st, f, stride, g);
+    auto tile = [&](const ConvTile &t) {
+        hipLaunchKernelGGL(k_conv_tile64<INV>, tile_grid(t, m, nbatch), tile_threads(t),
+                           tile_lds(t, 8), st, f, stride, (u64)1 << m, t);
     };
-    if (!P.tile.empty())
-        hipLaunchKernelGGL(k_conv_tile64<INV>, dim3(1, nbatch), dim3(tile_threads(m)),
-                           (size_t)8 << m, st, f, stride, tile_arg(P.tile, m, INV));
     if (!INV) {
         for (const ConvStep &s : P.steps) step(s);
-        for (const ConvGroup &g : P.groups) group(g);
+        for (const ConvTile &t : P.tiles) tile(t);
     } else {
-        for (size_t i = P.groups.size(); i--;) group(P.groups[i]);
+        for (size_t i = P.tiles.size(); i--;) tile(P.tiles[i]);
         for (size_t i = P.steps.size(); i--;) step(P.steps[i]);
     }
     GF2T_CHECK_LAUNCH("k_conv64");
     return GF2T_OK;
 }
+constexpr u32 BF_BLOCKS = 2560;   // blocks of a butterfly launch: ten per CU
 // butterfly passes above the low eight levels, all of nbatch transforms
 // stride words apart
 std::vector<BfPass> passes_for(const gf2t_fft_plan &pl, unsigned nbatch) {
@@ -755,12 +856,12 @@ std::vector<BfPass> passes_for(const gf2t_fft_plan &pl, unsigned nbatch) {
 template <int CLS, bool INV>
 void launch_bfly(u64 *f, u64 stride, const BfPass &P, const Operands &ops, int in, int out,
                  unsigned nbatch, hipStream_t st) {
-    size_t body = P.w > RB ? ((size_t)16 << P.tb) : 0;
-    if (in == IO_PLAIN || out == IO_PLAIN) body = std::max<size_t>(body, 16384);
-    else if (in != IO_UNITS) body = std::max<size_t>(body, 8192);
-    hipLaunchKernelGGL((k_bfly<CLS, INV>), dim3(1u << (P.m - 1 - P.tb), nbatch),
-                       dim3(1u << (P.tb - RB)), sizeof(MulLds) + body, st, f, stride, P, ops, in,
-                       out);
+    size_t lds = sizeof(MulLds) + (P.w > RB ? ((size_t)16 << P.tb) : 0);
+    if (in == IO_PLAIN || out == IO_PLAIN) lds += 16384;
+    else if (in != IO_UNITS) lds += 8192;
+    const u32 tiles = 1u << (P.m - 1 - P.tb);
+    hipLaunchKernelGGL((k_bfly<CLS, INV>), dim3(std::min(tiles, std::max(1u, BF_BLOCKS / nbatch)), nbatch),
+                       dim3(1u << (P.tb - RB)), lds, st, f, stride, P, ops, in, out);
 }
 template <bool INV>
 void run_bfly(u64 *f, u64 stride, const BfPass &P, const Operands &ops, int in, int out,
@@ -774,9 +875,12 @@ void run_bfly(u64 *f, u64 stride, const BfPass &P, const Operands &ops, int in, 
 template <int DIR>
 void run_low(u64 *f, u64 stride, const u64 *g, int m, const Operands &ops, u32 g_op, int in,
                 int out, unsigned nbatch, hipStream_t st) {
-    const u32 waves = std::max<u32>(1, (1u << (m - 1)) / LO_UNITS);
-    const u32 wpb = (u64)waves * nbatch >= 4096 ? 4 : (u64)waves * nbatch >= 1024 ? 2 : 1;
-    const u32 blocks = (waves + wpb - 1) / wpb;
+    const u32 runs = std::max<u32>(1, (1u << (m - 1)) / LO_UNITS);
+    const u32 pair = DIR == LO_MUL ? 2 : 1;
+    // runs per block: more share the tables where the chip is full anyway
+    const u64 waves = (u64)runs * nbatch * pair;
+    const u32 rpb = waves >= 4096 ? 4 / pair : waves >= 1024 ? 2 / pair : 1;
+    const u32 blocks = (runs + rpb - 1) / rpb, wpb = rpb * pair;
     size_t lds = sizeof(MulLds) + 4 * sizeof(TwEnt) + (DIR == LO_MUL ? sizeof(ProdLds) : 0) +
                  wpb * LO_EXCH * 4;
     if (in == IO_PLAIN || out == IO_PLAIN) lds += 16384;
@@ -963,12 +1067,47 @@ extern "C" size_t gf2t_mul_out_words(uint64_t abits, uint64_t bbits) {
     return words_of(abits + bbits) + 1;
 }
 
+namespace {
+// Products of at most SC_WORK chunk pairs (and SC_OUTS outputs) are formed
+// without a transform (k_school).
+constexpr u64 SC_WORK = (u64)64 << 20, SC_OUTS = 65536;
+constexpr u32 SC_FOLD_PARTS = 4;
+bool school(u64 ca, u64 cb, u64 nbatch = 1) {
+    return ca && cb && ca + cb <= SC_OUTS && nbatch * ca * cb <= SC_WORK;
+}
+SchoolShape school_shape(u64 ca, u64 cb) {
+    SchoolShape s;
+    s.na = (u32)std::min(ca, cb);
+    s.nb = (u32)std::max(ca, cb);
+    s.nout = s.na + s.nb - 1;
+    s.nparts = (s.na + SC_IN - 1) / SC_IN;
+    return s;
+}
+// words of the parts, as a bound that grows with either operand also past
+// the products that use it (a workspace for larger operands serves smaller
+// ones): parts * outputs <= (na / SC_IN + 1)(na + nb) with na nb <= SC_WORK
+size_t school_words(u64 ca, u64 cb) {
+    const u64 na = std::min(ca, cb), nb = std::max(ca, cb);
+    const u64 most = 2 * SC_WORK / SC_IN + SC_OUTS;
+    const u64 a = std::min<u64>(na, SC_OUTS), b = std::min<u64>(nb, SC_OUTS);
+    return (size_t)std::min(most, (a / SC_IN + 1) * (a + b));
+}
+int run_school(const Operands &ops, u32 b_op, bool swap, const SchoolShape &s, u64 *part,
+               u64 part_stride, unsigned nbatch, hipStream_t st) {
+    hipLaunchKernelGGL(k_school, dim3((s.nout + SC_OUT - 1) / SC_OUT, s.nparts, nbatch), dim3(256),
+                       0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride);
+    GF2T_CHECK_LAUNCH("k_school");
+    return GF2T_OK;
+}
+}  // namespace
+
 extern "C" size_t gf2t_mul_workspace_bytes(uint64_t abits, uint64_t bbits) {
     u64 ca = (abits + 31) >> 5, cb = (bbits + 31) >> 5;
     if (!ca || !cb) return 0;
     int m = fft_m_for(ca + cb - 1);
     size_t n = (size_t)1 << m;
-    return (2 * n + gf2t_mul_out_words(abits, bbits) + 8) * sizeof(u64);
+    return (std::max(2 * n, school_words(ca, cb)) + gf2t_mul_out_words(abits, bbits) + 8) *
+           sizeof(u64);
 }
 
 namespace {
@@ -1013,11 +1152,15 @@ struct WrapArg {
     int noff;
     u32 off[15];    // 2^k for the proper bit-subsets k of mp
 };
-Wrap wrap_for(u64 ca, u64 cb) {
+// from 2^WRAP_MIN_M points (of all products of a batch together) up: below
+// that both products are a chain of launches as long as their work, and
+// one chain is faster than two (a 2^16-point product: 83 us, wrapped 221)
+constexpr int WRAP_MIN_M = 20;
+Wrap wrap_for(u64 ca, u64 cb, u64 nbatch = 1) {
     Wrap w;
     const u64 N = ca + cb - 1;
     const int m = fft_m_for(N);
-    if (m < 12 || m - 1 > FFT_MAX_M) return w;
+    if (m < 12 || m - 1 > FFT_MAX_M || (nbatch << (m - 1)) >> WRAP_MIN_M == 0) return w;
     const int mp = m - 1;
     const u64 n = (u64)1 << mp;
     if (N <= n) return w;
@@ -1039,13 +1182,13 @@ WrapArg wrap_arg(const Wrap &w) {
 }
 
 // chunk coefficient k < n + e of the wrapped product: R = C mod V (2^mp
-// coefficients), H = C_high
+// coefficients), H = C_high; hit: the offsets to look at
 GF2T_DEV u64 wrap_chunk(const u64 *__restrict__ R, const u64 *__restrict__ H, const WrapArg &w,
-                        u64 k) {
+                        u32 hit, u64 k) {
     if (k >= w.n) return H[k - w.n];
     u64 v = R[k];
-    for (int j = 0; j < w.noff; j++) {
-        const u64 o = w.off[j];
+    for (u32 h = hit; h; h &= h - 1) {
+        const u64 o = w.off[__builtin_ctz(h)];
         if (k >= o && k - o < w.e) v ^= H[k - o];
     }
     return v;
@@ -1058,16 +1201,22 @@ __global__ void k_overlap_add_wrap(const u64 *__restrict__ R, u64 r_stride,
                                    const u64 *__restrict__ H, u64 h_stride, const WrapArg w,
                                    size_t nchunks, u64 *__restrict__ out, size_t owords,
                                    u64 o_stride) {
-    size_t wd = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t w0 = (size_t)blockIdx.x * blockDim.x, wd = w0 + threadIdx.x;
+    // the offsets whose copy of C_high reaches the block's coefficients
+    // (most blocks: none)
+    const u64 k0 = w0 ? 2 * (u64)w0 - 1 : 0, k1 = 2 * (u64)(w0 + blockDim.x);
+    u32 hit = 0;
+    for (int j = 0; j < w.noff; j++)
+        if (k1 > w.off[j] && k0 < w.off[j] + w.e) hit |= 1u << j;
     if (wd >= owords) return;
     R += (u64)blockIdx.y * r_stride;
     H += (u64)blockIdx.y * h_stride;
     out += (u64)blockIdx.y * o_stride;
     size_t k = 2 * wd;
     u64 v = 0;
-    if (k < nchunks) v ^= wrap_chunk(R, H, w, k);
-    if (k + 1 < nchunks) v ^= wrap_chunk(R, H, w, k + 1) << 32;
-    if (wd && k - 1 < nchunks) v ^= wrap_chunk(R, H, w, k - 1) >> 32;
+    if (k < nchunks) v ^= wrap_chunk(R, H, w, hit, k);
+    if (k + 1 < nchunks) v ^= wrap_chunk(R, H, w, hit, k + 1) << 32;
+    if (wd && k - 1 < nchunks) v ^= wrap_chunk(R, H, w, hit, k - 1) >> 32;
     out[wd] = v;
 }
 
@@ -1083,6 +1232,18 @@ int mul_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 *dprod, voi
     }
     int rc = ensure_basis();
     if (rc) return rc;
+    if (school(ca, cb)) {
+        Operands two{};
+        two.op[0] = operand_of(da, abits, nullptr);
+        two.op[1] = operand_of(db, bbits, nullptr);
+        const SchoolShape s = school_shape(ca, cb);
+        rc = run_school(two, 1, ca > cb, s, (u64 *)dwork, 0, 1, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_school_product, dim3((unsigned)((ow + SP_WORDS - 1) / SP_WORDS)),
+                           dim3(256), 0, st, (const u64 *)dwork, s, dprod, ow);
+        GF2T_CHECK_LAUNCH("k_school_product");
+        return GF2T_OK;
+    }
     // the converted chunks of both operands, behind the two transforms
     // (where the product goes later, or the workspace's tail)
     const size_t n = (size_t)1 << m;
@@ -1134,6 +1295,35 @@ extern "C" int gf2t_mul(const uint64_t *da, uint64_t abits, const uint64_t *db, 
 extern "C" int gf2t_fold(const uint64_t *dsrc, uint64_t src_bits, uint64_t *dout, uint64_t r,
                          uint64_t s, void *stream);
 
+namespace {
+// the product in the workspace behind what mul_core uses of it, then its
+// fold; both operands have chunks
+int mulmod_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 r, u64 s, u64 *dout,
+                u64 *dwork, hipStream_t st) {
+    const u64 ca = (abits + 31) >> 5, cb = (bbits + 31) >> 5;
+    if (school(ca, cb)) {
+        const SchoolShape sh = school_shape(ca, cb);
+        if (sh.nparts <= SC_FOLD_PARTS) {   // few parts to add up: folded from them directly
+            Operands two{};
+            two.op[0] = operand_of(da, abits, nullptr);
+            two.op[1] = operand_of(db, bbits, nullptr);
+            int rc = run_school(two, 1, ca > cb, sh, dwork, 0, 1, st);
+            if (rc) return rc;
+            const size_t nw = words_of(r);
+            hipLaunchKernelGGL(k_school_fold, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st,
+                               (const u64 *)dwork, (u64)0, sh, abits + bbits - 1, dout, nw,
+                               (u64)0, r, s, (const u64 *)nullptr);
+            GF2T_CHECK_LAUNCH("k_school_fold");
+            return GF2T_OK;
+        }
+    }
+    u64 *prod = dwork + std::max((size_t)2 << fft_m_for(ca + cb - 1), school_words(ca, cb));
+    int rc = mul_core(da, abits, db, bbits, prod, dwork, st);
+    if (rc) return rc;
+    return gf2t_fold(prod, abits + bbits - 1, dout, r, s, st);
+}
+}  // namespace
+
 extern "C" int gf2t_mulmod(const uint64_t *da, uint64_t abits, const uint64_t *db,
                            uint64_t bbits, uint64_t r, uint64_t s, uint64_t *dout, void *dwork,
                            void *stream) {
@@ -1153,11 +1343,7 @@ extern "C" int gf2t_mulmod(const uint64_t *da, uint64_t abits, const uint64_t *d
     u64 ca = (abits + 31) >> 5, cb = (bbits + 31) >> 5;
     if (!ca || !cb)   // a zero operand: the workspace may be empty, dout is 0
         return zero_words(dout, words_of(r), (hipStream_t)stream);
-    size_t n = (size_t)1 << fft_m_for(ca + cb - 1);
-    u64 *prod = (u64 *)dwork + 2 * n;
-    int rc = mul_core(da, abits, db, bbits, prod, dwork, (hipStream_t)stream);
-    if (rc) return rc;
-    return gf2t_fold(prod, abits + bbits - 1, dout, r, s, stream);
+    return mulmod_core(da, abits, db, bbits, r, s, dout, (u64 *)dwork, (hipStream_t)stream);
 }
 
 // ------------------------------------------------ modmul without allocation
@@ -1254,11 +1440,7 @@ extern "C" int gf2t_mulmod_noalloc(const uint64_t *da, uint64_t abits, const uin
     }
     hipStream_t st = (hipStream_t)stream;
     if (!ca || !cb) return zero_words(dout, words_of(r), st);   // a zero operand
-    const size_t n = (size_t)1 << fft_m_for(ca + cb - 1);
-    u64 *prod = ptr + 2 * n;
-    int rc = mul_core(da, abits, db, bbits, prod, ptr, st);
-    if (rc) return rc;
-    return gf2t_fold(prod, abits + bbits - 1, dout, r, s, stream);
+    return mulmod_core(da, abits, db, bbits, r, s, dout, ptr, st);
 }
 
 // ------------------------------------------------- variable-size batch
@@ -1507,13 +1689,22 @@ extern "C" int gf2t_mulmod_slab(const uint64_t *da, size_t apitch, const uint64_
     Operands ops{};
     ops.group = (u32)n;
     ops.lstride = 2 * ppitch;
+    ops.sstride[0] = 2 * apitch;
+    ops.sstride[1] = 2 * bpitch;
     ops.op[0] = operand_of(da, r, prod);
     ops.op[1] = operand_of(db, r, (u32 *)prod + 2 * nw + 2, b_add_x ? 2u : 0u);
     const u64 ow = 2 * nw;   // product of two r-bit operands: 2r-1 bits
-    ops.sstride[0] = 2 * apitch;
-    ops.sstride[1] = 2 * bpitch;
+    const SchoolShape sh = school_shape(ca, ca);
+    if (sh.nparts <= 2 && school(ca, ca, (u64)n)) {   // the parts fit the transforms' space
+        rc = run_school(ops, (u32)n, false, sh, FA, 2 * N, (unsigned)n, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_school_fold, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st,
+                           FA, (u64)(2 * N), sh, 2 * r - 1, dout, nw, (u64)opitch, r, (u64)0, ds);
+        GF2T_CHECK_LAUNCH("k_school_fold");
+        return GF2T_OK;
+    }
     const int k = log2_ceil(ca);
-    const Wrap W = wrap_for(ca, ca);
+    const Wrap W = wrap_for(ca, ca, (u64)n);
     if (W.on) {
         // the wrapped product (see wrap_for): 2^mp-point transforms of both
         // operands and 2^ms-point transforms of their top e chunks, laid
@@ -1672,14 +1863,15 @@ namespace {
 // matrix transforms at F .. F + 3n left as they are.  A thread per unit.
 __global__ __launch_bounds__(256) void k_mat2n_pointwise(u64 *__restrict__ F, size_t n,
                                                          int npairs) {
-    __shared__ ProdLds pt;
-    pt.load();
+    __shared__ __align__(16) ProdLds pt;
+    copy_lds(&pt, g_tab.d32, sizeof(ProdLds) / 16);
     __syncthreads();
     const size_t units = n / 2;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     const Operand none{};
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < units; i += stride) {
         Half32 M[4], C[4];
+#pragma unroll
         for (int k = 0; k < 4; k++) {
             const U4 u = load_unit((const U4 *)(F + k * n), (u32)i, IO_UNITS, none, nullptr);
             M[k] = unit_to32(u, pt.d32);
@@ -1689,6 +1881,7 @@ __global__ __launch_bounds__(256) void k_mat2n_pointwise(u64 *__restrict__ F, si
             U4 *fa = (U4 *)(F + (4 + 2 * (size_t)p) * n), *fb = (U4 *)(F + (5 + 2 * (size_t)p) * n);
             const Half32 a = unit_to32(load_unit(fa, (u32)i, IO_UNITS, none, nullptr), pt.d32);
             const Half32 b = unit_to32(load_unit(fb, (u32)i, IO_UNITS, none, nullptr), pt.d32);
+#pragma unroll
             for (int o = 0; o < 2; o++) {
                 Acc64 E{0, 0}, G{0, 0};
                 acc_mul(E, a.v[0], a.v[1], M[2 * o].v[0], M[2 * o].v[1], C[2 * o].v[1]);

@@ -764,28 +764,36 @@ GF2T_HD u64 sq_delta_pairs(const SqConst &c) {
     return c.w2.off() >= c.w3.off() ? c.w2.off() - c.w3.off() : 0;
 }
 
-// 64-bit window of p (pw words) at bit pos, restricted to bits [lo, hi)
-GF2T_HD u64 pwin64(const u64 *p, size_t pw, u64 pos, u64 lo, u64 hi) {
+// 64-bit window of a bit array (p(k) is word k, zero beyond it) at bit pos,
+// restricted to bits [lo, hi)
+template <class Words>
+GF2T_HD u64 pwin64(const Words &p, u64 pos, u64 lo, u64 hi) {
     if (pos >= hi || pos + 64 <= lo) return 0;
-    u64 v = win64(p, pw, pos);
+    const unsigned sh = (unsigned)(pos & 63);
+    u64 v = p((size_t)(pos >> 6));
+    if (sh) v = (v >> sh) | (p((size_t)(pos >> 6) + 1) << (64 - sh));
     int lc = lo > pos ? (int)(lo - pos) : 0;
     int hc = (hi - pos) >= 64 ? 64 : (int)(hi - pos);
     return v & range_mask64(lc, hc);
 }
 
 // output word w of P mod x^r + x^s + 1 for a product P of L <= 2r-1 bits
-GF2T_HD u64 fold_word(const u64 *p, size_t pw, u64 L, u64 r, u64 s, size_t w) {
+template <class Words>
+GF2T_HD u64 fold_words(const Words &p, u64 L, u64 r, u64 s, size_t w) {
     u64 b = (u64)w << 6;
     u64 lim1 = L < r ? L : r;
-    u64 v = pwin64(p, pw, b, 0, lim1);
+    u64 v = pwin64(p, b, 0, lim1);
     if (L > r) {
         u64 t3 = L < 2 * r - s ? L : 2 * r - s;
-        v ^= pwin64(p, pw, b + r, r, L);
-        v ^= pwin64(p, pw, b + r - s, r, t3);
-        v ^= pwin64(p, pw, b + 2 * r - s, 2 * r - s, L);
-        v ^= pwin64(p, pw, b + 2 * r - 2 * s, 2 * r - s, L);
+        v ^= pwin64(p, b + r, r, L);
+        v ^= pwin64(p, b + r - s, r, t3);
+        v ^= pwin64(p, b + 2 * r - s, 2 * r - s, L);
+        v ^= pwin64(p, b + 2 * r - 2 * s, 2 * r - s, L);
     }
     return v;
+}
+GF2T_HD u64 fold_word(const u64 *p, size_t pw, u64 L, u64 r, u64 s, size_t w) {
+    return fold_words([=](size_t k) -> u64 { return k < pw ? p[k] : 0; }, L, r, s, w);
 }
 
 // ------------------------------------------------ sieve number theory

@@ -9,9 +9,10 @@
 static FftTables T;
 
 struct Tab {
-    Mul8 operator()(u32 v) const {
-        if (v > 255) abort();
-        return Mul8{T.mulA[v][0], T.mulA[v][1], T.mulA[v][2], T.mulA[v][3], T.mulB[v]};
+    Mul8 operator()(u32 off) const {
+        if (off > 255 * 16 || off % 16) abort();
+        const u32 *e = T.mulA[off / 16];
+        return Mul8{e[0], e[1], e[2], e[3], T.mulB[off / 16]};
     }
 };
 
@@ -49,7 +50,7 @@ static void step(std::vector<E> &f, const ConvStep &s, int k, bool inv) {
             for (int j = 0; j < s.K; j++) {
                 const int e = inv ? j : s.K - 1 - j;
                 for (u32 idx = 0; idx < (u32)(R * R / 2); idx++)
-                    conv_tile_op([&](u32 i) -> E & { return x.at(i); }, idx, s.K, e, inv);
+                    conv_edge_pair([&](u32 i) -> E & { return x.at(i); }, s.K, e, inv, idx);
             }
             for (int r = 0; r < R; r++)
                 for (int q = 0; q < R; q++) at(b, r, conv_edge(s, r, q, rho)) = x[r * R + q];
@@ -59,44 +60,40 @@ static void step(std::vector<E> &f, const ConvStep &s, int k, bool inv) {
         if (c != 1) abort();
     (void)k;
 }
-template <class E>
-static void tile(std::vector<E> &f, const std::vector<cantor_host::TileOp> &ops, bool inv) {
-    for (size_t o = 0; o < ops.size(); o++) {
-        const auto &op = ops[inv ? ops.size() - 1 - o : o];
-        for (u32 i = 0; i < f.size() / 2; i++)
-            conv_tile_op([&](u32 l) -> E & { return f.at(l); }, i, op.h, op.pos, inv);
-    }
-}
 template <class E, bool INV>
-static void group(std::vector<E> &f, const ConvGroup &g) {
-    const u32 n = 1u << g.tb, threads = n >> 6;
-    for (u32 blk = 0; blk < f.size() >> g.tb; blk++) {
-        std::vector<E> x(n);
-        const u64 base = group_base(g, blk);
-        for (u32 l = 0; l < n; l++) x[l] = f.at(base + group_mem(g, l));
-        const bool two = g.w > 6;
-        for (int s = 0; s < (two ? 3 : 1); s++)
-            for (u32 tid = 0; tid < threads; tid++) {
-                E y[64];
-                const int lay = s == 1;
-                for (int r = 0; r < 64; r++) y[r] = x.at(group_local(g, lay, tid, r));
-                if (s == 1) conv_group_low<INV>(y, g.w);
-                else if ((s == 0) != INV || !two) conv_group_first<INV>(y, g.w);
-                else conv_group_top<INV>(y, g.w);
-                for (int r = 0; r < 64; r++) x.at(group_local(g, lay, tid, r)) = y[r];
-            }
-        for (u32 l = 0; l < n; l++) f.at(base + group_mem(g, l)) = x[l];
+static void tile(std::vector<E> &f, const ConvTile &t, size_t n) {
+    const int T = t.c + t.w;
+    const u32 sz = 1u << T, threads = sz >> 4;
+    for (u32 blk = 0; blk == 0 || (size_t)blk < n >> T; blk++) {
+        std::vector<E> x(sz, 0);
+        const u64 base = tile_base(t, blk);
+        for (u32 l = 0; l < sz; l++)
+            if (base + tile_mem(t, l) < n) x[l] = f.at(base + tile_mem(t, l));
+        for (int i = 0; i < t.n; i++) {
+            const ConvStep &s = t.st[INV ? t.n - 1 - i : i];
+            std::vector<int> owner(sz, -1);   // no two threads touch one coefficient
+            for (u32 q = 0; q < threads; q++)
+                conv_tile_stage<INV, E>(
+                    [&](u32 l) -> E & {
+                        if (s.K != 1 && owner.at(l) >= 0 && owner[l] != (int)q) abort();
+                        owner.at(l) = (int)q;
+                        return x[l];
+                    },
+                    q, threads, s);
+        }
+        for (u32 l = 0; l < sz; l++)
+            if (base + tile_mem(t, l) < n) f.at(base + tile_mem(t, l)) = x[l];
+            else if (x[l]) abort();
     }
 }
 template <class E>
 static void convert(std::vector<E> &f, int k, int one, int tb, bool inv) {
     const cantor_host::ConvPlan P = cantor_host::conv_plan(k, one, tb);
-    if (!P.tile.empty()) tile(f, P.tile, inv);
     if (!inv) {
         for (auto &s : P.steps) step(f, s, k, false);
-        for (auto &g : P.groups) group<E, false>(f, g);
+        for (auto &t : P.tiles) tile<E, false>(f, t, f.size());
     } else {
-        for (size_t i = P.groups.size(); i--;) group<E, true>(f, P.groups[i]);
+        for (size_t i = P.tiles.size(); i--;) tile<E, true>(f, P.tiles[i], f.size());
         for (size_t i = P.steps.size(); i--;) step(f, P.steps[i], k, true);
     }
 }
@@ -105,7 +102,7 @@ template <int CLS>
 static void pass(std::vector<U4> &f, const BfPass &P, bool inv) {
     const u32 threads = 1u << (P.tb - RB);
     for (size_t blk = 0; blk < f.size() >> P.tb; blk++) {
-        const BfTile t = bf_tile(P, (u32)blk);
+        const BfTile T0 = bf_tile(P, (u32)blk), &t = T0;
         std::vector<U4> x((size_t)1 << P.tb);
         for (u32 l = 0; l < x.size(); l++) x[l] = f.at(bf_unit(P, t, l));
         const int ns = bf_stages(P);
@@ -116,8 +113,9 @@ static void pass(std::vector<U4> &f, const BfPass &P, bool inv) {
                 TwEnt W[RB];
                 for (int r = 0; r < (1 << RB); r++) y[r] = x.at(bf_local(P, s, tid, r));
                 bf_twiddles(P, t, s, tid, T.tw, W);
-                if (inv) fft_stage<CLS, true>(y, bf_active(P, s), W, Tab());
-                else fft_stage<CLS, false>(y, bf_active(P, s), W, Tab());
+                const bool zero = bf_zero(P, T0, s);
+                if (inv) fft_stage<CLS, true>(y, bf_active(P, s), W, zero, Tab());
+                else fft_stage<CLS, false>(y, bf_active(P, s), W, zero, Tab());
                 for (int r = 0; r < (1 << RB); r++) x.at(bf_local(P, s, tid, r)) = y[r];
             }
         }
@@ -140,17 +138,21 @@ static void low(std::vector<U4> &f, int m, bool inv) {
             const int s = inv ? ns - 1 - k : k;
             for (u32 lane = 0; lane < 64; lane++) {
                 U4 y[1 << RB];
-                TwEnt W[RB], W0;
+                TwEnt W[RB], W0{};
                 for (int r = 0; r < (1 << RB); r++) y[r] = x.at(lo_unit(s, lane, r));
-                lo_twiddles(base, s, lane, T.tw, hi, W, W0);
+                static_assert(lo_stages() == 4, "stages");
+                if (s == 0) lo_twiddles<0>(base, lane, T.tw, hi, W, W0);
+                if (s == 1) lo_twiddles<1>(base, lane, T.tw, hi, W, W0);
+                if (s == 2) lo_twiddles<2>(base, lane, T.tw, hi, W, W0);
+                if (s == 3) lo_twiddles<3>(base, lane, T.tw, hi, W, W0);
                 const int act = lo_active(m, s);
                 if (inv) {
                     if (s == ns - 1) fft_level0<CB, true>(y, W0, Tab());
-                    if (s) fft_stage<CB, true>(y, act, W, Tab());
-                    else fft_stage<CA, true>(y, act, W, Tab());
+                    if (s) fft_stage<CB, true>(y, act, W, false, Tab());
+                    else fft_stage<CA, true>(y, act, W, false, Tab());
                 } else {
-                    if (s) fft_stage<CB, false>(y, act, W, Tab());
-                    else fft_stage<CA, false>(y, act, W, Tab());
+                    if (s) fft_stage<CB, false>(y, act, W, false, Tab());
+                    else fft_stage<CA, false>(y, act, W, false, Tab());
                     if (s == ns - 1) fft_level0<CB, false>(y, W0, Tab());
                 }
                 for (int r = 0; r < (1 << RB); r++) x.at(lo_unit(s, lane, r)) = y[r];
