@@ -39,16 +39,6 @@ GF2T_HD u64 spread32(u32 v) {
     return x;
 }
 
-// 64-bit window [q, q+64) of a bit array of nw words (zeros beyond)
-GF2T_HD u64 win64(const u64 *a, size_t nw, u64 q) {
-    size_t w = (size_t)(q >> 6);
-    unsigned sh = (unsigned)(q & 63);
-    u64 lo = (w < nw) ? a[w] : 0;
-    if (!sh) return lo;
-    u64 hi = (w + 1 < nw) ? a[w + 1] : 0;
-    return (lo >> sh) | (hi << (64 - sh));
-}
-
 // mask of bit positions [lc, hc) within a 64-bit word; lc and hc may lie
 // anywhere (clamped to [0, 64]), and no shift count ever reaches 64
 GF2T_HD u64 range_mask64(int lc, int hc) {
@@ -516,6 +506,81 @@ template <bool W12 = false>
 GF2T_HD void square_fold_pair_fast(const u64 *in, const SqConst &C, size_t i, u64 &o0, u64 &o1) {
     square_fold_pair_fast_src(SqArrayT<W12>{in, C.nw}, C, i, o0, o1);
 }
+// The same for one pair at a time: window k at spread position P with only
+// the positions [lo, hi), and the pair from all five.  No branch and no
+// load waits for another, where square_fold_pair_src tests each window in
+// turn: a tile that straddles s, 2s or r then takes about as long as any
+// other (launches of few tiles took 9 to 13 us, their straddling tiles').
+template <class Src>
+GF2T_HD u64 sq_win_masked(const Src &src, int win, u64 P, u64 lo, u64 hi) {
+    const u64 q = (P + 1) >> 1;
+    const size_t w = (size_t)(q >> 6);
+    const u32 sh = (u32)(q & 63);
+    const int64_t k0 = (int64_t)((lo + 1) >> 1) - (int64_t)q, k1 = (int64_t)((hi + 1) >> 1) - (int64_t)q;
+    const int lc = k0 < 0 ? 0 : k0 > 64 ? 64 : (int)k0, hc = k1 < 0 ? 0 : k1 > 64 ? 64 : (int)k1;
+    return funnel64(src(win, w), src(win, w + (sh ? 1 : 0)), sh) & range_mask64(lc, hc);
+}
+template <class Src>
+GF2T_HD void square_fold_pair_masked(const Src &src, const SqConst &C, size_t i, u64 &o0, u64 &o1) {
+    const u64 b = (u64)i << 7, r = C.r, s = C.s;
+    const u64 v1 = sq_win_masked(src, 0, b, 0, r);
+    const u64 v2 = sq_win_masked(src, 1, b + r, r, 2 * r - 1);
+    const u64 v3 = sq_win_masked(src, 2, b + r - s, r, 2 * r - s);
+    const u64 v4 = sq_win_masked(src, 3, b + 2 * r - s, 2 * r - s, 2 * r - 1);
+    const u64 v5 = sq_win_masked(src, 4, b + 2 * r - 2 * s, 2 * r - s, 2 * r - 1);
+    const u64 m2 = (r & 1) ? ~0ULL : 0, m3 = ((r ^ s) & 1) ? ~0ULL : 0, m4 = (s & 1) ? ~0ULL : 0;
+    const u64 O = (v2 & m2) ^ (v3 & m3) ^ (v4 & m4);
+    const u64 E = v1 ^ v2 ^ v3 ^ v4 ^ v5 ^ O;
+    o0 = interleave32((u32)E, (u32)O);
+    o1 = interleave32((u32)(E >> 32), (u32)(O >> 32));
+}
+// Output pair i in any region, without a branch on it: all five windows,
+// each with the mask of its bits whose (even) spread position lies in the
+// window's clip range.  Addresses and masks do not change from one
+// squaring to the next, so a kernel that takes many keeps them.
+struct SqClip {
+    u32 q[5];       // 32-bit word of each window's first bit (0: nothing of it counts)
+    u32 m[5][2];    // the bits that count
+};
+GF2T_HD SqClip sq_clip(const SqConst &C, u64 i) {
+    const u64 b = i << 7, r = C.r, s = C.s;
+    const u64 P[5] = {b, b + r, b + r - s, b + 2 * r - s, b + 2 * r - 2 * s};
+    const u64 lo[5] = {0, r, r, 2 * r - s, 2 * r - s};
+    const u64 hi[5] = {r, 2 * r - 1, 2 * r - s, 2 * r - 1, 2 * r - 1};
+    SqClip c;
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const u64 q = (P[k] + 1) >> 1;
+        const int64_t k0 = (int64_t)((lo[k] + 1) >> 1) - (int64_t)q;
+        const int64_t k1 = (int64_t)((hi[k] + 1) >> 1) - (int64_t)q;
+        const u64 m = range_mask64(k0 < 0 ? 0 : k0 > 64 ? 64 : (int)k0,
+                                   k1 < 0 ? 0 : k1 > 64 ? 64 : (int)k1);
+        c.q[k] = m ? (u32)(q >> 5) : 0;
+        c.m[k][0] = (u32)m;
+        c.m[k][1] = (u32)(m >> 32);
+    }
+    return c;
+}
+// the pair from its clip; RP, SP the parities of r and s; need: the windows
+// any lane of the wave wants (uniform)
+template <int RP, int SP, class Src>
+GF2T_HD void sq_pair_clipped(const Src &src, const SqConst &C, const SqClip &c, u32 need, u64 &o0,
+                             u64 &o1) {
+    u32 E[2] = {0, 0}, O[2] = {0, 0};
+    const u32 sh[5] = {0, C.w2.sh, C.w3.sh, C.w4.sh, C.w5.sh};
+    const bool odd[5] = {false, RP != 0, (RP ^ SP) != 0, SP != 0, false};
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        if (!((need >> k) & 1)) continue;
+        u32 x, y, z;
+        src.raw3(k, c.q[k], sh[k], x, y, z);
+        u32 *A = odd[k] ? O : E;
+        A[0] ^= alignbit(y, x, sh[k]) & c.m[k][0];
+        A[1] ^= alignbit(z, y, sh[k]) & c.m[k][1];
+    }
+    o0 = interleave32(E[0], O[0]);
+    o1 = interleave32(E[1], O[1]);
+}
 // region shared by the pairs [i0, i1) (3: mixed or clipped)
 GF2T_HD int sq_tile_region(const SqConst &C, size_t i0, size_t i1) {
     return sq_region((u64)i0 << 7, (u64)i1 << 7, C.s, C.r);
@@ -552,9 +617,7 @@ GF2T_HD u64 sq2_p0(const SqConst &C, size_t i0, int k) { return ((u64)i0 + sq2_o
 // (sq_tile_region(C, p0, p0 + SQ2_GP) == 3)
 template <class Src>
 GF2T_HD void sq2_g_pair_clipped(const Src &F, const SqConst &C, u64 p, u64 &o0, u64 &o1) {
-    o0 = o1 = 0;
-    if (2 * p < C.nw) square_fold_pair_fast_src(F, C, (size_t)p, o0, o1);
-    if (2 * p + 1 >= C.nw) o1 = 0;
+    square_fold_pair_masked(F, C, (size_t)p, o0, o1);   // past the end: every mask empty
 }
 // the H phase reads G through the tile's window copies: window k's copy
 // holds G words from base_k = 2 p0_k on, at word at_k of the LDS area
@@ -649,19 +712,29 @@ GF2T_HD u32 sq2_col_start(const Sq2Chain &h, u32 c) {
 GF2T_HD u32 sq2_col_tiles(const Sq2Chain &h, u32 c) {
     return h.q + (sq2_col_start(h, c) < h.rm ? 1u : 0u);
 }
-inline Sq2Chain sq2_chain(const SqConst &C) {   // host
+inline Sq2Chain sq2_chain(const SqConst &C, u32 most = SQ2_CHAIN) {   // host
     Sq2Chain h;
     h.np = (u32)((C.nw + 1) / 2);
     const u32 d = C.w2.off() - C.w3.off();
     h.chained = d >= SQ2_CW;
     h.period = h.chained ? d : SQ2_TP;
     h.ncols = h.chained ? (d + SQ2_CW - 1) / SQ2_CW : 1u;
-    h.len = h.chained ? SQ2_CHAIN : 1u;
+    h.len = h.chained ? most : 1u;
     h.wlo = h.period / h.ncols;
     h.wrem = h.period % h.ncols;
     h.q = h.np / h.period;
     h.rm = h.np % h.period;
     return h;
+}
+// tiles of one residue
+inline u64 sq2_tiles(const Sq2Chain &h) { return (u64)h.ncols * sq2_col_tiles(h, 0); }
+// tiles per unit for a launch of `tiles` in all: a unit's tiles run one
+// after another, so units are shortened until the launch has SQ2_FULL of
+// them (eight blocks on each of 256 CUs)
+constexpr u64 SQ2_FULL = 2048;
+inline u32 sq2_chain_len(u64 tiles) {
+    const u64 n = tiles / SQ2_FULL;
+    return n < 1 ? 1u : n > SQ2_CHAIN ? SQ2_CHAIN : (u32)n;
 }
 // units of one residue (column 0 has the most tiles)
 inline u64 sq2_units(const Sq2Chain &h) {

@@ -24,6 +24,9 @@
 #include <numeric>
 #include <cstring>
 #include <cstdlib>
+#include <atomic>
+#include <mutex>
+#include <new>
 
 namespace {
 
@@ -43,10 +46,14 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square_fold(
     if (2 * i + 1 < c.nw) out[2 * i + 1] = o1;
 }
 
+__device__ __forceinline__ u32 uniform32(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+
 struct SqDesc {
     const u64 *in;
     u64 *out;
     SqConst c;
+    int odd;            // first launch: one squaring, where the others take two
+    int back;           // the chain ends in the scratch buffer (in, of an odd launch)
     const int *order;   // block -> tile (-1 idle), or null for identity
     Sq2Chain h;         // two-squaring tile layout
 };
@@ -102,7 +109,7 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square_fold_batch(
             const size_t i = t0 + (size_t)j * SQ_THREADS + threadIdx.x;
             if (i < np) {
                 u64 o0, o1;
-                square_fold_pair_fast<W12>(d.in, d.c, i, o0, o1);
+                square_fold_pair_masked(src, d.c, i, o0, o1);
                 store_pair<NT>(d.out, d.c.nw, i, o0, o1);
             }
         }
@@ -113,12 +120,12 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square_fold_batch(
 // One tile, the output pairs [i0, i1) (at most SQ2_TP): the G phase forms
 // the windows of pl.compute, one G pair per thread and window, into the
 // plan's LDS slots; the H phase then reads G through the window copies of
-// the plan.  LOADFIRST issues the loads of every window before any is
-// combined (a stand-alone tile); without it only windows 1 and 2, which
-// every tile forms, go first and the others are loaded as they are
-// formed, which keeps the work-unit loop at 56 VGPRs (7 waves per SIMD)
-// where the full load-first form needed 84.
-template <bool NT, bool W12, bool LOADFIRST = true>
+// the plan.  Only the loads of windows 1 and 2, which every tile forms, go
+// first; the others are loaded as they are formed, which keeps the
+// work-unit loop at 53 VGPRs (8 waves per SIMD) where loading every window
+// first needs 84 -- and gains nothing where tiles are few either (the 12
+// tiles of a 756839-bit residue: 176 us either way for 40 squarings).
+template <bool NT, bool W12>
 __device__ __forceinline__ void square2_run(const u64 *__restrict__ in, u64 *__restrict__ out,
                                             const SqConst &c, size_t i0, size_t i1, int treg,
                                             const Sq2Plan &pl, u64 *gw) {
@@ -132,10 +139,8 @@ __device__ __forceinline__ void square2_run(const u64 *__restrict__ in, u64 *__r
         const u64 p0 = pl.base[k] >> 1;
         greg[k] = ((pl.compute >> k) & 1) ? sq_tile_region(c, p0, p0 + SQ2_GP) : -1;
     }
-    // loads issued ahead of any combining: every window's (LOADFIRST), or
-    // those of windows 1 and 2, which every tile forms
 #pragma unroll
-    for (int k = 0; k < (LOADFIRST ? SQ2_WINS : 2); k++)
+    for (int k = 0; k < 2; k++)
         if (greg[k] >= 0 && greg[k] < 3)
             raw[k] = sq_raw_pair(fsrc, c, (u32)((pl.base[k] >> 1) + threadIdx.x), greg[k]);
 #pragma unroll
@@ -143,7 +148,7 @@ __device__ __forceinline__ void square2_run(const u64 *__restrict__ in, u64 *__r
         if (greg[k] < 0) continue;
         u64 o0, o1;
         if (greg[k] < 3) {
-            if (!LOADFIRST && k >= 2)
+            if (k >= 2)
                 raw[k] = sq_raw_pair(fsrc, c, (u32)((pl.base[k] >> 1) + threadIdx.x), greg[k]);
             sq_combine_pair(raw[k], c, greg[k], o0, o1);
         } else {
@@ -173,7 +178,7 @@ __device__ __forceinline__ void square2_run(const u64 *__restrict__ in, u64 *__r
             const size_t i = ib + (size_t)j * SQ_THREADS + threadIdx.x;
             if (i >= i0 && i < i1) {
                 u64 o0, o1;
-                square_fold_pair_fast_src(src, c, i, o0, o1);
+                square_fold_pair_masked(src, c, i, o0, o1);
                 store_pair<NT>(out, c.nw, i, o0, o1);
             }
         }
@@ -188,7 +193,7 @@ __device__ __forceinline__ void square2_tile(const u64 *__restrict__ in, u64 *__
     if (i0 >= np) return;   // whole block
     const size_t i1 = i0 + SQ2_TP < np ? i0 + SQ2_TP : np;
     const int treg = sq_tile_region(c, i0, i1);
-    square2_run<NT, W12, false>(in, out, c, i0, i1, treg, sq2_plan(c, i0, sq2_need(treg)), gw);
+    square2_run<NT, W12>(in, out, c, i0, i1, treg, sq2_plan(c, i0, sq2_need(treg)), gw);
 }
 // work unit u: its tiles one after another, each taking windows 3 and 5
 // from the copies of the tile before it where the plan says so
@@ -206,7 +211,7 @@ __device__ __forceinline__ void square2_unit(const u64 *__restrict__ in, u64 *__
         const int treg = sq_tile_region(c, i0, i1);
         const u32 need = sq2_need(treg);
         const Sq2Plan pl = sq2_chain_plan(c, h, i0, w.width, need, j - w.j0, prev_need, prev_base4);
-        square2_run<NT, W12, false>(in, out, c, i0, i1, treg, pl, gw);
+        square2_run<NT, W12>(in, out, c, i0, i1, treg, pl, gw);
         prev_need = need;
         prev_base4 = pl.base[3];
     }
@@ -222,6 +227,123 @@ k_square2_fold_batch(
     __shared__ __align__(16) u64 gw[SQ2_WINS * SQ2_LEN];
     const SqDesc d = desc[blockIdx.y];
     square2_unit<NT, W12>(d.in, d.out, d.c, d.h, blockIdx.x, gw);
+}
+// The same, and the residues marked odd advance by one squaring: the first
+// launch of a batch whose chains differ in length, so that every later one
+// advances all of its chains by two.
+template <bool NT, bool W12>
+__global__ __launch_bounds__(SQ_THREADS) void k_square12_fold_batch(
+        const SqDesc *__restrict__ desc) {
+    __shared__ __align__(16) u64 gw[SQ2_WINS * SQ2_LEN];
+    const SqDesc d = desc[blockIdx.y];
+    if (!d.odd) {
+        square2_unit<NT, W12>(d.in, d.out, d.c, d.h, blockIdx.x, gw);
+        return;
+    }
+    for (u32 i = blockIdx.x * SQ_THREADS + threadIdx.x; i < d.h.np; i += gridDim.x * SQ_THREADS) {
+        u64 o0, o1;
+        square_fold_pair_fast<W12>(d.in, d.c, i, o0, o1);
+        store_pair<NT>(d.out, d.c.nw, i, o0, o1);
+    }
+}
+
+// the values that ended in the scratch buffers, back to the residues: of
+// the entries `in` -> `out`, those marked back (one launch instead of a
+// device copy of 4 us for each)
+__global__ __launch_bounds__(SQ_THREADS) void k_batch_back(const SqDesc *__restrict__ desc) {
+    const SqDesc &d = desc[blockIdx.y];
+    if (!d.back) return;
+    typedef u64 v2u __attribute__((ext_vector_type(2)));
+    const u32 n2 = (u32)(d.c.nw / 2);   // 16-byte words (buffers are 16-byte aligned)
+    const v2u *in = (const v2u *)d.in;
+    v2u *out = (v2u *)d.out;
+    for (u32 i = blockIdx.x * SQ_THREADS + threadIdx.x; i < n2; i += gridDim.x * SQ_THREADS)
+        out[i] = in[i];
+    if ((d.c.nw & 1) && blockIdx.x == 0 && threadIdx.x == 0) d.out[d.c.nw - 1] = d.in[d.c.nw - 1];
+}
+
+// ---- whole chains of small residues
+// A residue whose two copies fit in LDS (r up to about 640,000) runs its
+// whole chain in one block, one squaring per barrier, between the copies:
+// no launch and no memory traffic per step.  Bounded by the issue of one
+// CU and the barrier: 0.85 us per squaring at 132049 bits and 2.2 us at
+// 640,000, where by launches two squarings took 9.5 us, all of it latency
+// (40 squarings: 191 -> 34 us, and 183 -> 90 us).  512 residues of 600,000
+// bits are 512 blocks, one per CU at a time: 276 us against 1085 us.
+constexpr int CH_THREADS = 1024;
+constexpr size_t CH_LDS = 160 * 1024;
+constexpr size_t CH_WORDS = CH_LDS / 16 - 2;   // words of a residue, at most
+constexpr u64 CH_STEPS = 4096;                 // squarings per launch, at most
+struct ChainDesc {
+    u64 *res;
+    SqConst c;
+    u64 steps;
+};
+struct SqLds {   // a residue's copy in LDS, two words past its end readable
+    const u32 *p;
+    __device__ void raw3(int, u32 q, u32, u32 &a, u32 &b, u32 &c) const {
+        a = p[q];
+        b = p[q + 1];
+        c = p[q + 2];
+    }
+};
+// `steps` squarings from cur, the copies changing places; K pairs per
+// thread, their window addresses and masks in registers
+template <int K, int RP, int SP>
+__device__ __forceinline__ u64 *chain_steps(u64 *cur, u64 *oth, const SqConst &c, u32 np, u32 steps,
+                                            const SqClip (&clip)[K], const u32 (&need)[K]) {
+    typedef u64 v2u __attribute__((ext_vector_type(2)));
+    const u32 nthr = blockDim.x, wave0 = uniform32(threadIdx.x & ~63u);
+    for (u32 k = 0; k < steps; k++) {
+        const SqLds src{(const u32 *)cur};
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            if (wave0 + j * nthr >= np) break;   // whole wave
+            u64 o0, o1;
+            sq_pair_clipped<RP, SP>(src, c, clip[j], need[j], o0, o1);
+            const u32 i = threadIdx.x + j * nthr;
+            if (i < np) *(v2u *)(oth + 2 * i) = v2u{o0, o1};
+        }
+        __syncthreads();
+        u64 *t = cur;
+        cur = oth;
+        oth = t;
+    }
+    return cur;
+}
+// list (or one, where list is null): one residue per block, at most
+// `most` squarings of its chain from squaring number `done` on
+template <int K>
+__global__ __launch_bounds__(CH_THREADS) void k_square_chain(const ChainDesc *__restrict__ list,
+                                                             const ChainDesc one, u64 done,
+                                                             u64 most) {
+    extern __shared__ __align__(16) u64 ch_lds[];
+    const ChainDesc d = list ? list[blockIdx.x] : one;
+    if (d.steps <= done) return;   // whole block
+    const u64 left = d.steps - done;
+    const u32 steps = (u32)(left < most ? left : most);
+    const u32 nw = (u32)d.c.nw, np = (nw + 1) / 2, nthr = blockDim.x;
+    u64 *cur = ch_lds, *oth = ch_lds + 2 * np + 2;
+    for (u32 w = threadIdx.x; w < nw; w += nthr) cur[w] = d.res[w];
+    SqClip clip[K];
+    u32 need[K];
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const u32 i = threadIdx.x + j * nthr;
+        clip[j] = sq_clip(d.c, i < np ? i : np);   // past the end: every mask empty
+        need[j] = 0;
+#pragma unroll
+        for (int k = 0; k < 5; k++)
+            if (__ballot((clip[j].m[k][0] | clip[j].m[k][1]) != 0)) need[j] |= 1u << k;
+    }
+    __syncthreads();
+    switch ((int)((d.c.r & 1) << 1) + (int)(d.c.s & 1)) {
+    case 0: cur = chain_steps<K, 0, 0>(cur, oth, d.c, np, steps, clip, need); break;
+    case 1: cur = chain_steps<K, 0, 1>(cur, oth, d.c, np, steps, clip, need); break;
+    case 2: cur = chain_steps<K, 1, 0>(cur, oth, d.c, np, steps, clip, need); break;
+    default: cur = chain_steps<K, 1, 1>(cur, oth, d.c, np, steps, clip, need); break;
+    }
+    for (u32 w = threadIdx.x; w < nw; w += nthr) d.res[w] = cur[w];
 }
 template <bool W12>
 __global__ __launch_bounds__(SQ_THREADS) void k_square2_fold(
@@ -262,11 +384,12 @@ struct Sq2SlabDesc {
 template <bool NT, bool W12>
 __global__ __launch_bounds__(SQ_THREADS) __attribute__((amdgpu_waves_per_eu(8))) void
 k_square2_fold_slab_u(const u64 *__restrict__ in, u64 *__restrict__ out, u64 pitch,
-                      const Sq2SlabDesc *__restrict__ desc, unsigned n, unsigned group) {
+                      const Sq2SlabDesc *__restrict__ desc, unsigned n, unsigned group, u32 len) {
     __shared__ __align__(16) u64 gw[SQ2_WINS * SQ2_LEN];
     const unsigned y = blockIdx.z * gridDim.y + blockIdx.y;
     if (y >= n) return;   // whole block
-    const Sq2SlabDesc d = desc[y / group];
+    Sq2SlabDesc d = desc[y / group];
+    if (d.h.len > len) d.h.len = len;   // a launch of few tiles: shorter units
     square2_unit<NT, W12>(in + (u64)y * pitch, out + (u64)y * pitch, d.c, d.h, blockIdx.x, gw);
 }
 
@@ -395,6 +518,32 @@ extern "C" int gf2t_square_fold(const uint64_t *din, uint64_t *dout, uint64_t r,
     return GF2T_OK;
 }
 
+namespace {
+// chains of n residues (list in device memory, or one) of at most nw words
+// and `steps` squarings, in LDS
+int run_chains(const ChainDesc *list, const ChainDesc &one, unsigned n, size_t nw, u64 steps,
+               hipStream_t st) {
+    const size_t np = (nw + 1) / 2, lds = 2 * (2 * np + 2) * 8;
+    const unsigned threads = (unsigned)std::min<size_t>(CH_THREADS, (np + 63) & ~(size_t)63);
+    const int K = (int)((np + threads - 1) / threads);   // 1..5
+    const auto kernel = K == 1 ? k_square_chain<1> : K == 2 ? k_square_chain<2>
+                        : K == 3 ? k_square_chain<3> : k_square_chain<5>;
+    // more than 64 KiB of LDS has to be allowed, once per kernel and device
+    static std::atomic<unsigned> allowed[64];
+    int dev = 0;
+    GF2T_HIP(hipGetDevice(&dev));
+    if (dev >= 64 || !((allowed[dev].load() >> K) & 1)) {
+        GF2T_HIP(hipFuncSetAttribute((const void *)kernel,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)CH_LDS));
+        if (dev < 64) allowed[dev].fetch_or(1u << K);
+    }
+    for (u64 k = 0; k < steps; k += CH_STEPS)
+        hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), lds, st, list, one, k, CH_STEPS);
+    GF2T_CHECK_LAUNCH("k_square_chain");
+    return GF2T_OK;
+}
+}  // namespace
+
 extern "C" int gf2t_square_fold_steps(uint64_t *dres, uint64_t *dtmp, uint64_t r,
                                       uint64_t s, uint64_t steps, void *stream) {
     if (!valid_rs(r, s) || !dres || !dtmp || dres == dtmp) {
@@ -404,9 +553,12 @@ extern "C" int gf2t_square_fold_steps(uint64_t *dres, uint64_t *dtmp, uint64_t r
     SqConst c = sq_const(r, s);
     size_t nw = c.nw;
     hipStream_t st = (hipStream_t)stream;
+    if (nw <= CH_WORDS && sq_fuse() && steps > 2)
+        return run_chains(nullptr, ChainDesc{dres, c, steps}, 1, nw, steps, st);
     u64 *a = dres, *b = dtmp;
     const bool fuse = sq_fuse(), w12 = sq_w12_ok(r);
-    const Sq2Chain h2 = sq2_chain(c);
+    const u64 tiles = sq2_tiles(sq2_chain(c));
+    const Sq2Chain h2 = sq2_chain(c, sq2_chain_len(tiles));
     const dim3 g2((unsigned)sq2_units(h2)), g1(blocks_for((nw + 1) / 2, SQ_THREADS));
     u64 launches = 0;
     for (u64 k = 0; k < steps; launches++) {
@@ -434,10 +586,11 @@ namespace {
 // descriptor and tile-order tables for the batched chain, cached and
 // grown on demand
 struct BatchScratch {
-    SqDesc *d = nullptr;
+    unsigned char *d = nullptr;   // cap bytes
     int *ord = nullptr;
     size_t cap = 0, ocap = 0;
     int dev = -1;
+    std::mutex mu;   // held by a call until its launches are done
 } g_batch;
 
 template <int PPT, bool W12>
@@ -448,6 +601,15 @@ void launch_batch(unsigned gx, unsigned active, const SqDesc *tab, hipStream_t s
     else
         hipLaunchKernelGGL((k_square_fold_batch<PPT, false, W12>), dim3(gx, active),
                            dim3(SQ_THREADS), 0, st, tab);
+}
+template <bool W12>
+void launch_batch12(unsigned gx, unsigned active, const SqDesc *tab, hipStream_t st) {
+    if (sq_nt())
+        hipLaunchKernelGGL((k_square12_fold_batch<true, W12>), dim3(gx, active), dim3(SQ_THREADS),
+                           0, st, tab);
+    else
+        hipLaunchKernelGGL((k_square12_fold_batch<false, W12>), dim3(gx, active), dim3(SQ_THREADS),
+                           0, st, tab);
 }
 template <bool W12>
 void launch_batch2(unsigned gx, unsigned active, const SqDesc *tab, hipStream_t st) {
@@ -604,23 +766,50 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     hipStream_t st = (hipStream_t)stream;
     int ppt, order;
     sq_tuning(ppt, order);
-    // order residues by remaining steps, longest first: the residues
-    // still active at step k are a prefix, so each launch covers exactly
-    // the live chains (uneven frontiers, per-s early exit)
-    std::vector<int> ord(n);
-    std::iota(ord.begin(), ord.end(), 0);
-    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return steps[a] > steps[b]; });
+    const bool fuse = sq_fuse();
     int dev = 0;
     GF2T_HIP(hipGetDevice(&dev));
-    size_t need = 2 * (size_t)n;
-    // per-residue tile orders
+    std::lock_guard<std::mutex> lock(g_batch.mu);
+    if (g_batch.dev != dev) {   // (what another device holds stays there)
+        g_batch.d = nullptr;
+        g_batch.ord = nullptr;
+        g_batch.cap = g_batch.ocap = 0;
+        g_batch.dev = dev;
+    }
+    // residues whose chain runs in LDS, and the others, by launches: those
+    // with most launches first, so that the residues still active at a
+    // launch are a prefix (uneven frontiers, per-s early exit)
+    std::vector<int> ord;
+    std::vector<ChainDesc> chains;
+    size_t chain_nw = 0;
+    u64 chain_steps = 0;
+    for (int i = 0; i < n; i++) {
+        const size_t nw = words_of(r[i]);
+        if (!steps[i]) continue;
+        if (fuse && nw <= CH_WORDS) {
+            chains.push_back(ChainDesc{dres[i], sq_const(r[i], s[i]), steps[i]});
+            chain_nw = std::max(chain_nw, nw);
+            chain_steps = std::max<u64>(chain_steps, steps[i]);
+        } else {
+            ord.push_back(i);
+        }
+    }
+    auto nlaunch = [&](int i) { return fuse ? (steps[i] + 1) / 2 : steps[i]; };
+    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return nlaunch(a) > nlaunch(b); });
+    std::stable_sort(chains.begin(), chains.end(), [](const ChainDesc &a, const ChainDesc &b) {
+        return a.steps * a.c.nw > b.steps * b.c.nw;
+    });
+    const int nl = (int)ord.size();
+    // descriptors of the launches (even, then odd ones), then the chains
+    const size_t chain_at = 2 * (size_t)nl * sizeof(SqDesc);
+    const size_t need = chain_at + chains.size() * sizeof(ChainDesc);
+    std::vector<size_t> ooff(nl, 0);
     std::vector<int> otab;
-    std::vector<size_t> ooff(n, 0);
-    size_t gx = 0;
+    size_t gx = 0, gx1 = 0;
     const u64 tile_pairs = (u64)SQ_THREADS * ppt;
-    for (int k = 0; k < n; k++) {
-        int i = ord[k];
-        SqConst c = sq_const(r[i], s[i]);
+    u64 tiles2 = 0;
+    for (int k = 0; k < nl; k++) {
+        SqConst c = sq_const(r[ord[k]], s[ord[k]]);
         u64 T = ((c.nw + 1) / 2 + tile_pairs - 1) / tile_pairs;
         if (order) {
             TileOrder o = tile_order(T, sq_delta_pairs(c), tile_pairs);
@@ -630,29 +819,21 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
         } else {
             gx = std::max<size_t>(gx, T);
         }
-    }
-    if (g_batch.dev != dev) {
-        g_batch = BatchScratch();
-        g_batch.dev = dev;
+        if (fuse) tiles2 += sq2_tiles(sq2_chain(c));
     }
     if (g_batch.cap < need) {
         if (g_batch.d) (void)hipFree(g_batch.d);
         g_batch.d = nullptr;
-        GF2T_HIP(hipMalloc(&g_batch.d, need * sizeof(SqDesc)));
+        g_batch.cap = 0;
+        GF2T_HIP(hipMalloc((void **)&g_batch.d, need));
         g_batch.cap = need;
-    }
-    if (order && g_batch.ocap < otab.size()) {
-        if (g_batch.ord) (void)hipFree(g_batch.ord);
-        g_batch.ord = nullptr;
-        GF2T_HIP(hipMalloc(&g_batch.ord, otab.size() * sizeof(int)));
-        g_batch.ocap = otab.size();
     }
     // a block index beyond a residue's own table must idle: pad each
     // residue's table to gx entries
-    if (order) {
-        std::vector<int> padded((size_t)n * gx, -1);
-        for (int k = 0; k < n; k++) {
-            size_t len = (k + 1 < n ? ooff[k + 1] : otab.size()) - ooff[k];
+    if (order && nl) {
+        std::vector<int> padded((size_t)nl * gx, -1);
+        for (int k = 0; k < nl; k++) {
+            size_t len = (k + 1 < nl ? ooff[k + 1] : otab.size()) - ooff[k];
             std::copy(otab.begin() + ooff[k], otab.begin() + ooff[k] + len,
                       padded.begin() + (size_t)k * gx);
         }
@@ -660,44 +841,58 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
         if (g_batch.ocap < otab.size()) {
             if (g_batch.ord) (void)hipFree(g_batch.ord);
             g_batch.ord = nullptr;
+            g_batch.ocap = 0;
             GF2T_HIP(hipMalloc(&g_batch.ord, otab.size() * sizeof(int)));
             g_batch.ocap = otab.size();
         }
         GF2T_HIP(hipMemcpyAsync(g_batch.ord, otab.data(), otab.size() * sizeof(int),
                                 hipMemcpyHostToDevice, st));
     }
-    std::vector<SqDesc> h(need);
-    for (int k = 0; k < n; k++) {
-        int i = ord[k];
-        SqConst c = sq_const(r[i], s[i]);
+    std::vector<unsigned char> h(need);
+    SqDesc *hd = (SqDesc *)h.data();
+    const u32 len2 = sq2_chain_len(tiles2);
+    u64 gx2 = 0;       // work units of the residue with the most
+    bool w12 = true;   // 12-byte window loads: no r of the launches a multiple of 64
+    bool odd = false;  // some chain has an odd number of squarings
+    bool back = false; // some chain ends in dtmp
+    for (int k = 0; k < nl; k++) {
+        const int i = ord[k];
+        const SqConst c = sq_const(r[i], s[i]);
         const int *ot = order ? g_batch.ord + (size_t)k * gx : nullptr;
-        const Sq2Chain h2 = sq2_chain(c);
-        h[k] = SqDesc{dres[i], dtmp[i], c, ot, h2};          // even steps
-        h[n + k] = SqDesc{dtmp[i], dres[i], c, ot, h2};      // odd steps
-    }
-    GF2T_HIP(hipMemcpyAsync(g_batch.d, h.data(), need * sizeof(SqDesc), hipMemcpyHostToDevice, st));
-    // Every launch advances all live chains together, by two squarings
-    // while each of them has two left, else by one; a chain leaves the
-    // prefix when its steps are done, after launches[k] launches (its
-    // value is in dtmp when that count is odd).
-    const bool fuse = sq_fuse();
-    u64 gx2 = 0;   // work units of the residue with the most
-    bool w12 = true;   // 12-byte window loads: no r of the batch a multiple of 64
-    for (int i = 0; i < n; i++) {
-        gx2 = std::max(gx2, sq2_units(sq2_chain(sq_const(r[i], s[i]))));
+        const Sq2Chain h2 = sq2_chain(c, len2);
+        const int od = fuse ? (int)(steps[i] & 1) : 0;
+        const int bk = (int)(nlaunch(i) & 1);
+        new (hd + k) SqDesc{dres[i], dtmp[i], c, od, bk, ot, h2};        // even launches
+        new (hd + nl + k) SqDesc{dtmp[i], dres[i], c, 0, bk, ot, h2};    // odd launches
+        odd = odd || od;
+        back = back || bk;
+        gx2 = std::max(gx2, sq2_units(h2));
         w12 = w12 && sq_w12_ok(r[i]);
+        gx1 = std::max<size_t>(gx1, ((c.nw + 1) / 2 + SQ_THREADS - 1) / SQ_THREADS);
     }
-    std::vector<u64> launches(n, 0);
-    int active = n;
-    u64 nl = 0;
-    for (u64 k = 0;; nl++) {
-        while (active > 0 && steps[ord[active - 1]] <= k) launches[--active] = nl;
-        if (!active) break;
-        const SqDesc *tab = g_batch.d + ((nl & 1) ? n : 0);
-        if (fuse && steps[ord[active - 1]] - k >= 2) {
+    if (!chains.empty()) std::memcpy(h.data() + chain_at, chains.data(), chains.size() * sizeof(ChainDesc));
+    if (need == 0) return GF2T_OK;   // no squaring to do
+    GF2T_HIP(hipMemcpyAsync(g_batch.d, h.data(), need, hipMemcpyHostToDevice, st));
+    if (!chains.empty()) {
+        int rc = run_chains((const ChainDesc *)(g_batch.d + chain_at), chains[0],
+                            (unsigned)chains.size(), chain_nw, chain_steps, st);
+        if (rc) return rc;
+    }
+    // Every launch advances all live chains together, by two squarings (by
+    // one in the first launch where a chain's length is odd); a chain's
+    // value is in dtmp after an odd number of launches.
+    const SqDesc *dd = (const SqDesc *)g_batch.d;
+    int active = nl;
+    for (u64 l = 0; active > 0; l++) {
+        const SqDesc *tab = dd + ((l & 1) ? nl : 0);
+        if (fuse && l == 0 && odd) {
+            // enough blocks for the one-squaring residues' pairs in a few rounds
+            const unsigned g = (unsigned)std::max<u64>(gx2, (gx1 + 7) / 8);
+            if (w12) launch_batch12<true>(g, active, tab, st);
+            else launch_batch12<false>(g, active, tab, st);
+        } else if (fuse) {
             if (w12) launch_batch2<true>((unsigned)gx2, active, tab, st);
             else launch_batch2<false>((unsigned)gx2, active, tab, st);
-            k += 2;
         } else {
             if (ppt == 4 && w12) launch_batch<4, true>((unsigned)gx, active, tab, st);
             else if (ppt == 4) launch_batch<4, false>((unsigned)gx, active, tab, st);
@@ -705,14 +900,13 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
             else if (ppt == 2) launch_batch<2, false>((unsigned)gx, active, tab, st);
             else if (w12) launch_batch<1, true>((unsigned)gx, active, tab, st);
             else launch_batch<1, false>((unsigned)gx, active, tab, st);
-            k += 1;
         }
+        while (active > 0 && nlaunch(ord[active - 1]) == l + 1) active--;
     }
+    if (back)
+        hipLaunchKernelGGL(k_batch_back, dim3((unsigned)std::min<size_t>((gx1 + 1) / 2, 1024), nl),
+                           dim3(SQ_THREADS), 0, st, dd + nl);
     GF2T_CHECK_LAUNCH("k_square_fold_batch");
-    for (int k = 0; k < n; k++)
-        if (launches[k] & 1)
-            GF2T_HIP(hipMemcpyAsync(dres[ord[k]], dtmp[ord[k]], words_of(r[ord[k]]) * 8,
-                                    hipMemcpyDeviceToDevice, st));
     // the host tables must outlive the async copies
     GF2T_HIP(hipStreamSynchronize(st));
     return GF2T_OK;
@@ -832,7 +1026,8 @@ extern "C" int gf2t_square2_fold_slab_g(const uint64_t *din, uint64_t *dout, siz
 struct gf2t_sq2_slab_plan {
     u64 r = 0;
     size_t cap = 0, ngroups = 0;
-    unsigned gx = 0;   // work units of the group with the most
+    unsigned gx[SQ2_CHAIN + 1] = {};   // work units of the group with the most, by unit length
+    u64 tiles = 0;                     // tiles of that group
     Sq2SlabDesc *d = nullptr;
     std::vector<Sq2SlabDesc> h;   // host copy (source of the last upload)
 };
@@ -852,16 +1047,20 @@ extern "C" int gf2t_sq2_slab_plan_set(gf2t_sq2_slab_plan *p, const uint64_t *hs,
     // the previous upload may still be in flight from h: let it finish
     // before h changes
     GF2T_HIP(hipStreamSynchronize((hipStream_t)stream));
-    unsigned gx = 0;
+    unsigned gx[SQ2_CHAIN + 1] = {};
+    u64 tiles = 0;
     for (size_t g = 0; g < ngroups; g++) {
         const SqConst c = sq_const(p->r, hs[g]);
         p->h[g] = Sq2SlabDesc{c, sq2_chain(c)};
-        gx = std::max(gx, (unsigned)sq2_units(p->h[g].h));
+        tiles = std::max(tiles, sq2_tiles(p->h[g].h));
+        for (u32 len = 1; len <= SQ2_CHAIN; len++)
+            gx[len] = std::max(gx[len], (unsigned)sq2_units(sq2_chain(c, len)));
     }
     GF2T_HIP(hipMemcpyAsync(p->d, p->h.data(), ngroups * sizeof(Sq2SlabDesc),
                             hipMemcpyHostToDevice, (hipStream_t)stream));
     p->ngroups = ngroups;
-    p->gx = gx;
+    std::copy(gx, gx + SQ2_CHAIN + 1, p->gx);
+    p->tiles = tiles;
     return GF2T_OK;
 }
 
@@ -912,21 +1111,22 @@ extern "C" int gf2t_square2_fold_slab_p(const gf2t_sq2_slab_plan *p, const uint6
     if (n == 0) return GF2T_OK;
     const unsigned gy = n < 65535 ? (unsigned)n : 65535u;
     const unsigned gz = (unsigned)((n + gy - 1) / gy);
-    const dim3 grid(p->gx, gy, gz);
+    const u32 len = sq2_chain_len(p->tiles * n);
+    const dim3 grid(p->gx[len], gy, gz);
     const bool w12 = sq_w12_ok(p->r), nt = sq_nt();
     hipStream_t st = (hipStream_t)stream;
     if (nt && w12)
         hipLaunchKernelGGL((k_square2_fold_slab_u<true, true>), grid, dim3(SQ_THREADS), 0, st, din,
-                           dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group);
+                           dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group, len);
     else if (nt)
         hipLaunchKernelGGL((k_square2_fold_slab_u<true, false>), grid, dim3(SQ_THREADS), 0, st,
-                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group);
+                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group, len);
     else if (w12)
         hipLaunchKernelGGL((k_square2_fold_slab_u<false, true>), grid, dim3(SQ_THREADS), 0, st,
-                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group);
+                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group, len);
     else
         hipLaunchKernelGGL((k_square2_fold_slab_u<false, false>), grid, dim3(SQ_THREADS), 0, st,
-                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group);
+                           din, dout, (u64)pitch, p->d, (unsigned)n, (unsigned)group, len);
     GF2T_CHECK_LAUNCH("k_square2_fold_slab_u");
     return GF2T_OK;
 }

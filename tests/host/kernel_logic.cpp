@@ -55,6 +55,61 @@ void kl_square_fold(const u64 *in, u64 *out, u64 r, u64 s) {
         if (2 * i + 1 < nw) out[2 * i + 1] = o1;
     }
 }
+// the chain kernel's pairs, wave by wave of 64: reads checked against the
+// LDS copy's 2 np + 2 words (what lies past the residue is poisoned)
+struct ChainSrc {
+    std::vector<u32> w;
+    void raw3(int, u32 q, u32 sh, u32 &a, u32 &b, u32 &c) const {
+        if (sh > 31) abort();
+        a = w.at(q);
+        b = w.at(q + 1);
+        c = w.at(q + 2);
+    }
+};
+void kl_square_fold_waves(const u64 *in, u64 *out, u64 r, u64 s) {
+    const SqConst c = sq_const(r, s);
+    const size_t np = (c.nw + 1) / 2;
+    ChainSrc src{std::vector<u32>(4 * np + 4, 0x5A5A5A5Au)};
+    for (size_t w = 0; w < c.nw; w++) {
+        src.w[2 * w] = (u32)in[w];
+        src.w[2 * w + 1] = (u32)(in[w] >> 32);
+    }
+    for (size_t iw = 0; iw < np; iw += 64) {
+        u32 need = 0;
+        for (size_t i = iw; i < iw + 64 && i < np; i++) {
+            const SqClip k = sq_clip(c, i);
+            for (int j = 0; j < 5; j++) need |= (k.m[j][0] | k.m[j][1]) ? 1u << j : 0;
+        }
+        for (size_t i = iw; i < iw + 64 && i < np; i++) {
+            const SqClip k = sq_clip(c, i);
+            u64 o0, o1;
+            if ((r & 1) && (s & 1)) sq_pair_clipped<1, 1>(src, c, k, need, o0, o1);
+            else if (r & 1) sq_pair_clipped<1, 0>(src, c, k, need, o0, o1);
+            else if (s & 1) sq_pair_clipped<0, 1>(src, c, k, need, o0, o1);
+            else sq_pair_clipped<0, 0>(src, c, k, need, o0, o1);
+            out[2 * i] = o0;
+            if (2 * i + 1 < c.nw) out[2 * i + 1] = o1;
+            else if (o1) abort();
+        }
+    }
+}
+// the two-squaring units at a given length
+void kl_square2_units_len(u64 r, u64 s, u32 len, u64 *tiles) {
+    const Sq2Chain h = sq2_chain(sq_const(r, s), len);
+    std::vector<unsigned char> hits(h.np);
+    for (u64 u = 0; u < sq2_units(h); u++) {
+        Sq2Unit w;
+        if (!sq2_unit(h, (u32)u, w)) continue;
+        if (w.j1 - w.j0 > len) abort();
+        for (u32 j = w.j0; j < w.j1; j++) {
+            const u32 i0 = w.start + j * h.period;
+            for (u32 i = i0; i < i0 + w.width && i < h.np; i++) hits[i]++;
+            ++*tiles;
+        }
+    }
+    for (unsigned char x : hits)
+        if (x != 1) abort();
+}
 void kl_square_fold_fast(const u64 *in, u64 *out, u64 r, u64 s) {
     SqConst c = sq_const(r, s);
     for (size_t i = 0; i < (c.nw + 1) / 2; i++) {

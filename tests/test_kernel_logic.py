@@ -23,6 +23,8 @@ def kl(tmp_path_factory):
     lib = C.CDLL(out)
     lib.kl_square_fold.argtypes = [P, P, C.c_uint64, C.c_uint64]
     lib.kl_square_fold_fast.argtypes = [P, P, C.c_uint64, C.c_uint64]
+    lib.kl_square_fold_waves.argtypes = [P, P, C.c_uint64, C.c_uint64]
+    lib.kl_square2_units_len.argtypes = [C.c_uint64, C.c_uint64, C.c_uint32, P]
     lib.kl_fold.argtypes = [P, C.c_uint64, P, C.c_uint64, C.c_uint64]
     lib.kl_square2_fold.argtypes = [P, P, C.c_uint64, C.c_uint64]
     lib.kl_square2_fold_units.argtypes = [P, P, C.c_uint64, C.c_uint64, P]
@@ -466,3 +468,28 @@ def test_wide_field_arithmetic(kl):
             assert kl.kl_inv64(a, M) * a % M == 1
     for d in range(3, 23):
         assert kl.kl_count_classes64(d) == O.count_irreducible(d), d
+
+
+@pytest.mark.parametrize("r", [5, 64, 127, 128, 129, 192, 1000, 4423, 8192, 8193, 66001])
+def test_chain_kernel_pairs(kl, r):
+    """One squaring as the LDS chain kernel forms it: five masked windows per
+    pair, those that no lane of a wave wants left out."""
+    rng = np.random.default_rng(r)
+    nw = O.words(r)
+    for s in sorted({1, 2, (r - 1) // 2, (r - 1) // 3 or 1, min(64, (r - 1) // 2),
+                     *[int(x) for x in rng.integers(1, (r - 1) // 2 + 1, 6)]}):
+        a = rng.integers(0, 2**64, nw, dtype=np.uint64)
+        if r & 63:
+            a[-1] &= np.uint64((1 << (r & 63)) - 1)
+        out = np.zeros(nw, np.uint64)
+        kl.kl_square_fold_waves(a.ctypes.data_as(P), out.ctypes.data_as(P), r, s)
+        assert np.array_equal(out, O.square_fold(a, r, s)), s
+
+
+@pytest.mark.parametrize("length", [1, 2, 3, 5, 7, 8])
+def test_two_squaring_units_cover_every_pair(kl, length):
+    """Work units of any length form every output pair once."""
+    for r, s in [(1048573, 500000), (1048573, 64127), (3021377, 1000001), (3021377, 70000)]:
+        tiles = np.zeros(1, np.uint64)
+        kl.kl_square2_units_len(r, s, length, tiles.ctypes.data_as(P))
+        assert tiles[0] > 0
