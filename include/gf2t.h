@@ -373,7 +373,7 @@ typedef struct gf2t_sieve_stats {
     uint64_t classes;         /* cyclotomic classes (= irreducibles of degree d) */
     uint64_t marking;         /* classes whose progression reaches s <= smax */
     uint64_t heavy;           /* progressions deferred to the heavy pass */
-    float ms_table, ms_classes, ms_heavy;
+    float ms_table, ms_classes, ms_heavy;   /* degrees of one launch share its time */
 } gf2t_sieve_stats;
 
 /* Mark every s in [1, smax] divisible by an irreducible of degree d in
@@ -392,7 +392,7 @@ typedef struct gf2t_sieve_stats {
 int gf2t_sieve(uint64_t r, int dmin, int dmax, uint64_t smax,
                uint64_t *dbest, gf2t_sieve_stats *stats);
 
-/* The sieve keeps its device tables (up to ~83 GB at dmax = 32) between
+/* The sieve keeps its device tables (7 GB at dmax = 32) between
  * calls; this frees them.  No reference counterpart. */
 int gf2t_sieve_release(void);
 

@@ -892,18 +892,41 @@ GF2T_HD u32 gcd32(u32 a, u32 b) {
     while (b) { u32 t = a % b; a = b; b = t; }
     return a;
 }
-// inverse of a modulo m (gcd(a, m) = 1, m >= 2), extended Euclid in u32
+// inverse of a modulo m (gcd(a, m) = 1, m >= 2), extended Euclid in u32:
+// the cofactors alternate in sign and never exceed m
 GF2T_HD u32 inv32(u32 a, u32 m) {
-    u32 r0 = m, r1 = a % m;
-    long long t0 = 0, t1 = 1;
+    u32 r0 = m, r1 = a % m, t0 = 0, t1 = 1;
+    bool plus = false;
     while (r1) {
-        u32 q = r0 / r1;
-        u32 r2 = r0 - q * r1;
-        long long t2 = t0 - (long long)q * t1;
+        const u32 q = r0 / r1, r2 = r0 - q * r1, t2 = t0 + q * t1;
         r0 = r1; r1 = r2; t0 = t1; t1 = t2;
+        plus = !plus;
     }
-    if (t0 < 0) t0 += m;
-    return (u32)t0;
+    return plus ? t0 : m - t0;
+}
+
+// The minimal polynomial of a sequence of linear complexity d over GF(2)
+// (Berlekamp-Massey on its first 2d terms, bit k = term k), or 0 if the
+// complexity is not d.
+GF2T_HD u64 minpoly_seq(u64 seq, int d) {
+    u64 C = 1, B = 1, W = 0;
+    int L = 0, m = 1;
+    for (int n = 0; n < 2 * d; n++) {
+        W = (W << 1) | ((seq >> n) & 1);           // bit j = a_{n-j}
+        if (!(__builtin_popcountll(C & W) & 1)) { m++; continue; }
+        u64 T = C;
+        C ^= B << m;
+        if (2 * L <= n) { L = n + 1 - L; B = T; m = 1; }
+        else m++;
+    }
+    if (L != d) return 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bitreverse64(C) >> (63 - d);
+#else
+    u64 mask = 0;
+    for (int k = 0; k <= d; k++) mask |= ((C >> (d - k)) & 1) << k;
+    return mask;
+#endif
 }
 
 // Minimal polynomial over GF(2) of beta in GF(2^d) (beta in no proper
@@ -921,18 +944,5 @@ GF2T_HD u64 minpoly_bm(u32 beta, u64 q, int d, u32 tmask) {
         seq |= (u64)(__builtin_popcount(pw & tmask) & 1) << k;
         pw = fmul(pw, beta, q, d);
     }
-    u64 C = 1, B = 1, W = 0;
-    int L = 0, m = 1;
-    for (int n = 0; n < 2 * d; n++) {
-        W = (W << 1) | ((seq >> n) & 1);           // bit j = a_{n-j}
-        if (!(__builtin_popcountll(C & W) & 1)) { m++; continue; }
-        u64 T = C;
-        C ^= B << m;
-        if (2 * L <= n) { L = n + 1 - L; B = T; m = 1; }
-        else m++;
-    }
-    if (L != d) return 0;
-    u64 mask = 0;
-    for (int k = 0; k <= d; k++) mask |= ((C >> (d - k)) & 1) << k;
-    return mask;
+    return minpoly_seq(seq, d);
 }

@@ -13,23 +13,28 @@
 // least mask (reference: src/sieve_ref.cpp:1-30, src/coarse_sieve.cu:
 // 237-299).
 //
-// Per degree, on the device:
-//   k_log_build   L[g^i] = i for all i < M (LFSR chain per lane, random
-//                 4-byte scatter: the HBM-bound part, 4*2^d bytes)
-//   k_lyndon_t    a run of 16 candidates j per thread, all rotations
-//                 compared, one output reservation per block: the class
-//                 representatives as a dense list
-//   k_zech        one lane per class: Zech log (one random gather) and the
-//                 progression; classes whose progression reaches s <= smax
-//                 are ballot-compacted into a queue (about 1.6% of them at
-//                 d = 32 for smax = 68,139,920)
-//   k_mark        one lane per queued class: minimal polynomial by
-//                 Berlekamp-Massey on Tr(beta^k), then the marks (inline up
-//                 to 1024, longer progressions to k_mark_heavy)
-//   k_mark_heavy  many blocks per heavy progression
-// The dense tables fit HBM for every d <= 32 (16 GiB at d = 32), so no
-// bucketed low-memory mode is needed on a 288 GB part.
+// Degrees up to 32 (class_log.hpp), on the device:
+//   k_classes     the class representatives (Lyndon words) as a dense list,
+//                 only below prefixes that can begin one
+//   k_class_log   one logarithm per class: T[least rotation of w(g^j)], a
+//                 table of 2^(d-2) words of which one in d/4 is written
+//   k_zech        per class: Zech logarithm (one random gather of T) and
+//                 the progression; classes whose progression reaches s <=
+//                 smax are ballot-compacted into a queue (about 1.6% of
+//                 them at d = 32 for smax = 68,139,920)
+//   k_mark        per queued class: minimal polynomial by Berlekamp-Massey
+//                 on Tr(beta^k), then the marks (inline up to 1024, longer
+//                 progressions to k_mark_heavy); degrees whose period M is
+//                 at most smax and below 2^16 mark one period instead, and
+//   k_sweep       takes every s through the periods once, lowest degree
+//                 first
+// A table of all 2^d logarithms (16 GiB at d = 32) took three radix
+// partition passes over 8-byte entries, 94 of 134 ms at degrees 2..32 over
+// 68,139,920 s; one logarithm per class needs none of them.  Several small
+// degrees run in one launch (blockIdx.y), and nothing waits for the host
+// until all degrees are done.
 #include "gf2t_internal.hpp"
+#include "class_log.hpp"
 #include "../../include/gf2t.h"
 #include <vector>
 #include <algorithm>
@@ -40,7 +45,6 @@ namespace {
 
 constexpr u64 INLINE_MARKS = 1024;
 constexpr u32 HEAVY_CAP = 1u << 22;
-constexpr int LOG_CHUNK = 64;
 
 struct Heavy {
     u64 s_first, n, key;
@@ -141,14 +145,15 @@ u64 irreducible_count(int d) {
 
 // Per-degree host constants, computed once per process: the smallest
 // primitive modulus q, the antilog tables g^k and g^(65536 k) (k < 2^16),
-// and the trace mask (bit i = Tr(x^i)).  The g^(65536 k) table steps by a
-// fixed multiplier, which is linear over GF(2): four 256-entry byte tables
-// make each step four lookups.
+// the byte maps of class_log.hpp, and the primes of M.  The g^(65536 k)
+// table steps by a fixed multiplier, which is linear over GF(2): four
+// 256-entry byte tables make each step four lookups.
+constexpr size_t DEG_TAB = 2 * 65536 + CL_MAP;   // words of a degree's tables
 struct DegHost {
     bool ready = false, trace_ok = false;
     u64 q = 0;
-    u32 tmask = 0;
-    std::vector<u32> lo, hi;
+    std::vector<u32> tab;   // g^k, g^(65536 k), byte maps
+    std::vector<SievePrime> primes;
 };
 std::mutex g_deg_mu;
 DegHost g_deg[33];
@@ -158,13 +163,13 @@ const DegHost &deg_host(int d) {
     DegHost &H = g_deg[d];
     if (H.ready) return H;
     H.q = primitive_poly(d);
-    H.lo.assign(65536, 0);
-    H.hi.assign(65536, 0);
+    H.tab.assign(DEG_TAB, 0);
     if (H.q) {
         const u64 q = H.q;
+        u32 *lo = H.tab.data(), *hi = lo + 65536;
         u64 a = 1;
         for (u64 k = 0; k < 65536; k++) {
-            H.lo[k] = (u32)a;
+            lo[k] = (u32)a;
             a <<= 1;
             if ((a >> d) & 1) a ^= q;
         }
@@ -177,49 +182,37 @@ const DegHost &deg_host(int d) {
             }
         u32 b = 1;
         for (u64 k = 0; k < 65536; k++) {
-            H.hi[k] = b;
+            hi[k] = b;
             b = T[0][b & 255] ^ T[1][(b >> 8) & 255] ^ T[2][(b >> 16) & 255] ^ T[3][b >> 24];
         }
-        H.trace_ok = true;
-        for (int i = 0; i < d; i++) {
-            u64 y = (u64)1 << i, acc = y;
-            for (int k = 1; k < d; k++) { y = hmulmod(y, y, q, d); acc ^= y; }
-            if (acc > 1) { H.trace_ok = false; break; }
-            H.tmask |= (u32)acc << i;
-        }
+        H.trace_ok = class_host::class_maps(q, d, hi + 65536);
+        const u64 M = ((u64)1 << d) - 1;
+        u64 ps[16];
+        const int np = hprimes(M, ps);
+        for (int i = 0; i < np; i++) H.primes.push_back(class_host::sieve_prime((u32)ps[i], M));
     }
     H.ready = true;
     return H;
 }
 
 // ---------------------------------------------------------- device side
-struct DegreeParams {
-    int d;
-    u64 M, q, rmod, smax;
-    u32 tmask;               // Tr(y) = parity(y & tmask)
-    const u32 *Alo, *Ahi;    // g^k and g^(k<<16), k < 2^16
+struct MarkRec {
+    u32 j, n, sf, pad;
 };
-
-GF2T_DEV u32 antilog(const DegreeParams &P, u64 e) {
-    if (P.d <= 16) return P.Alo[e];
-    return fmul(P.Ahi[e >> 16], P.Alo[e & 0xFFFF], P.q, P.d);
-}
-
-__global__ void k_log_build(DegreeParams P, u32 *__restrict__ L) {
-    u64 chunk = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    u64 i0 = chunk * LOG_CHUNK;
-    if (i0 >= P.M) return;
-    u32 a = antilog(P, i0);
-    const u32 top = 1u << (P.d - 1);
-    // (u32)q keeps the x^d term for d < 32 (it cancels the shifted-out
-    // bit) and drops it for d = 32 (the shift already discarded it)
-    const u32 qlow = (u32)P.q;
-    u64 iend = i0 + LOG_CHUNK < P.M ? i0 + LOG_CHUNK : P.M;
-    for (u64 i = i0; i < iend; i++) {
-        L[a] = (u32)i;
-        a = (a << 1) ^ ((a & top) ? qlow : 0u);
-    }
-}
+constexpr int SV_PRIMES = 8;     // primes of 2^d - 1, d <= 32: at most 6
+constexpr int PAT_MAX_D = 20;    // degrees that may mark one period
+struct SieveDeg {                // one degree of a launch (blockIdx.y)
+    int d, lb, np;               // lb: bits of a class word below its prefix
+    u32 M, rmod, ap;
+    u32 nprefix, per;            // prefixes, and how many a block takes
+    u64 q, smax, ncls, qcap;
+    const u32 *lo, *hi, *map;    // g^k, g^(k<<16), byte maps
+    u32 *surv, *T, *pat;         // pat: marks of one period, or null
+    MarkRec *queue;
+    unsigned long long *cnt;     // CN_*
+    SievePrime pr[SV_PRIMES];
+};
+enum { CN_SURV, CN_QUEUE, CN_HEAVY, CN_BAD, CN_N };
 
 // exclusive prefix sum of v over the block (blockDim.x = T), and the total;
 // wtot: T/64 words of LDS, free again after the caller's next barrier
@@ -264,153 +257,9 @@ __device__ void bucket_offsets(const unsigned *cnt, unsigned *off, unsigned nb, 
         }
 }
 
-// ---- log table by radix partition (d >= LP_MIN_D) --------------------
-// The direct build above scatters 4-byte stores over 4*2^d bytes.  For
-// large d the table is built in three coalesced passes instead:
-//   pass 1: each block generates E consecutive (g^i, i), sorts them in LDS
-//           by the top B1 bits of g^i and appends each bucket's run to
-//           that bucket's region (one cursor atomic per bucket per block);
-//   pass 2: the same by the next B2 bits, inside each level-1 bucket;
-//   pass 3: one block per sub-bucket of 2^LP_SB values places its entries
-//           into an LDS copy of that slice of L and writes it out whole.
-// Every value 1..2^d-1 occurs exactly once (g generates the group), so
-// every region's size is known in advance.  Entries are u64:
-// (g^i mod 2^(d-B1)) << 32 | i.
-constexpr int LP_MIN_D = 26;
-constexpr int LP_SB = 15;            // 2^15 values per placed slice (128 KiB)
-constexpr int LP_E = 16384;          // entries per block in passes 1 and 2
-constexpr int LP_T = 1024;           // threads per block in passes 1 and 2
-constexpr int LP_B1 = 9;            // level-1 partition bits (fewer when d - LP_SB is smaller)
-
-struct LpShape {
-    int B1, B2;                      // partition bits, level 1 and 2
-};
-
-__global__ __launch_bounds__(LP_T) void k_lp_part1(DegreeParams P, LpShape S,
-                                                   unsigned long long *__restrict__ out,
-                                                   unsigned *__restrict__ cursor,
-                                                   unsigned *__restrict__ bad) {
-    __shared__ unsigned cnt[1 << LP_B1], off[1 << LP_B1], gbase[1 << LP_B1], wtot[LP_T / 64];
-    __shared__ unsigned long long stage[LP_E];
-    const unsigned nb = 1u << S.B1;
-    const int shift = P.d - S.B1;
-    const u64 cap = (u64)1 << shift;
-    const u64 i0 = (u64)blockIdx.x * LP_E;
-    for (unsigned b = threadIdx.x; b < nb; b += LP_T) cnt[b] = 0;
-    __syncthreads();
-    // each thread: LP_E / LP_T consecutive exponents by the LFSR step a <- a*g
-    constexpr int PER = LP_E / LP_T;
-    const u64 my0 = i0 + (u64)threadIdx.x * PER;
-    unsigned rank[PER];
-    u32 av[PER];
-    const u32 top = 1u << (P.d - 1);
-    const u32 qlow = (u32)P.q;
-    u32 a = my0 < P.M ? antilog(P, my0) : 0;
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        av[k] = a;
-        rank[k] = 0;
-        if (my0 + k < P.M) rank[k] = atomicAdd(&cnt[a >> shift], 1u);
-        a = (a << 1) ^ ((a & top) ? qlow : 0u);
-    }
-    __syncthreads();
-    bucket_offsets<LP_T>(cnt, off, nb, wtot);
-    __syncthreads();
-    for (unsigned b = threadIdx.x; b < nb; b += LP_T)
-        gbase[b] = cnt[b] ? atomicAdd(&cursor[b], cnt[b]) : 0;
-#pragma unroll
-    for (int k = 0; k < PER; k++)
-        if (my0 + k < P.M)
-            stage[off[av[k] >> shift] + rank[k]] = ((unsigned long long)av[k] << 32) | (u32)(my0 + k);
-    __syncthreads();
-    const u64 nvalid = (i0 + LP_E <= P.M) ? LP_E : P.M - i0;
-    for (u64 k = threadIdx.x; k < nvalid; k += LP_T) {
-        unsigned long long e = stage[k];
-        u32 v = (u32)(e >> 32);
-        unsigned b = v >> shift;
-        u64 pos = (u64)gbase[b] + (k - off[b]);
-        if (pos >= cap) { atomicOr(bad, 4u); continue; }
-        out[(u64)b * cap + pos] = ((unsigned long long)(v & (u32)(cap - 1)) << 32) | (u32)e;
-    }
-}
-
-// level 2: inside level-1 bucket blockIdx.y, chunk blockIdx.x of LP_E
-// entries, by bits [LP_SB, LP_SB + B2) of the stored value
-__global__ __launch_bounds__(LP_T) void k_lp_part2(DegreeParams P, LpShape S,
-                                                   const unsigned long long *__restrict__ in,
-                                                   unsigned long long *__restrict__ out,
-                                                   unsigned *__restrict__ cursor,
-                                                   unsigned *__restrict__ bad) {
-    __shared__ unsigned cnt[512], off[512], gbase[512], wtot[LP_T / 64];
-    __shared__ unsigned long long stage[LP_E];
-    const unsigned nb2 = 1u << S.B2;
-    const u64 cap1 = (u64)1 << (P.d - S.B1);
-    const u64 cap2 = (u64)1 << LP_SB;
-    const unsigned b1 = blockIdx.y;
-    const u64 count = b1 ? cap1 : cap1 - 1;     // value 0 never occurs
-    const u64 k0 = (u64)blockIdx.x * LP_E;
-    if (k0 >= count) return;
-    const u64 nvalid = (k0 + LP_E <= count) ? LP_E : count - k0;
-    const unsigned long long *src = in + (u64)b1 * cap1 + k0;
-    for (unsigned b = threadIdx.x; b < nb2; b += LP_T) cnt[b] = 0;
-    __syncthreads();
-    constexpr int PER = LP_E / LP_T;
-    unsigned rank[PER];
-    unsigned long long ev[PER];
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        u64 idx = (u64)k * LP_T + threadIdx.x;
-        ev[k] = idx < nvalid ? src[idx] : 0;
-        rank[k] = idx < nvalid ? atomicAdd(&cnt[(unsigned)(ev[k] >> (32 + LP_SB)) & (nb2 - 1)], 1u) : 0;
-    }
-    __syncthreads();
-    bucket_offsets<LP_T>(cnt, off, nb2, wtot);
-    __syncthreads();
-    for (unsigned b = threadIdx.x; b < nb2; b += LP_T)
-        gbase[b] = cnt[b] ? atomicAdd(&cursor[(u64)b1 * nb2 + b], cnt[b]) : 0;
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        u64 idx = (u64)k * LP_T + threadIdx.x;
-        if (idx < nvalid) stage[off[(unsigned)(ev[k] >> (32 + LP_SB)) & (nb2 - 1)] + rank[k]] = ev[k];
-    }
-    __syncthreads();
-    for (u64 k = threadIdx.x; k < nvalid; k += LP_T) {
-        unsigned long long e = stage[k];
-        unsigned b = (unsigned)(e >> (32 + LP_SB)) & (nb2 - 1);
-        u64 pos = (u64)gbase[b] + (k - off[b]);
-        if (pos >= cap2) { atomicOr(bad, 4u); continue; }
-        out[((u64)b1 * nb2 + b) * cap2 + pos] = e;
-    }
-}
-
-// one block per slice z of 2^LP_SB values: L[z*2^LP_SB + v] for every v
-__global__ __launch_bounds__(1024) void k_lp_place(const unsigned long long *__restrict__ in,
-                                                   u32 *__restrict__ L) {
-    extern __shared__ u32 tile[];
-    const u64 cap = (u64)1 << LP_SB;
-    const unsigned z = blockIdx.x;
-    const u64 count = z ? cap : cap - 1;
-    const unsigned long long *src = in + (u64)z * cap;
-    if (z == 0 && threadIdx.x == 0) tile[0] = 0;
-    for (u64 k = threadIdx.x; k < count; k += blockDim.x) {
-        unsigned long long e = src[k];
-        tile[(u32)(e >> 32) & (u32)(cap - 1)] = (u32)e;
-    }
-    __syncthreads();
-    u32 *dst = L + (u64)z * cap;
-    for (u64 k = threadIdx.x; k < cap; k += blockDim.x) dst[k] = tile[k];
-}
-
-__global__ void k_fill_u32(unsigned *p, u64 n) {
+__global__ void k_fill_u32(unsigned *p, u64 n, unsigned v) {
     u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
-LpShape lp_shape(int d) {
-    LpShape S;
-    S.B1 = std::min(LP_B1, d - LP_SB);
-    S.B2 = d - LP_SB - S.B1;
-    return S;
+    if (i < n) p[i] = v;
 }
 
 // A Lyndon word of length >= 2 starts with 0 and ends with 1, so only the
@@ -468,103 +317,305 @@ unsigned lyndon_blocks(int d) {
     return (unsigned)std::min<u64>(chunks, 8192);
 }
 
-struct MarkRec {
-    u32 j, n, sf, pad;
-};
-
-// Phase 1, one lane per class: Zech logarithm (one random gather), the
-// progression s == s0 (mod n), and -- only for the few classes whose
-// progression reaches s <= smax -- a ballot-compacted queue entry, so the
-// expensive minimal polynomial below runs on dense waves.
 constexpr int ZC_T = 256, ZC_PER = 4;   // classes per thread per round
 
-__global__ __launch_bounds__(ZC_T) void k_zech(DegreeParams P, const u32 *__restrict__ surv,
-                                               u64 nsurv, const u32 *__restrict__ L,
-                                               MarkRec *__restrict__ queue,
-                                               unsigned long long *__restrict__ nqueue, u64 qcap) {
-    __shared__ unsigned wtot[ZC_T / 64];
-    __shared__ unsigned long long bbase;
-    const u32 M = (u32)P.M;
-    const u64 chunk = (u64)ZC_T * ZC_PER;
-    // a round: ZC_PER classes per thread, their table lookups all issued
-    // before any of the arithmetic, then one queue reservation per block
-    for (u64 c0 = (u64)blockIdx.x * chunk; c0 < nsurv; c0 += (u64)gridDim.x * chunk) {
-        u32 j[ZC_PER], a[ZC_PER], v[ZC_PER];
-        bool live[ZC_PER];
+// The classes of a degree: the Lyndon words of length d, which start with 0
+// and end with 1, as a list.  A word is a prefix and its low lb bits; a
+// block takes `per` prefixes, drops those that cannot begin a Lyndon word
+// (nine in ten at d = 32), and its waves try the odd words below the
+// others, 256 at a time.  Survivors gather in LDS, one output reservation
+// per 4096 or more.  Bounded by VALU issue (1.5 operations a rotation):
+// 0.7 ms at d = 32, where testing every odd word below 2^(d-1) took 6.0.
+constexpr int CS_T = 256, CS_LB = 11, CS_STAGE = 8192;
+__global__ __launch_bounds__(CS_T) void k_classes(const SieveDeg *__restrict__ degs) {
+    const SieveDeg &P = degs[blockIdx.y];
+    __shared__ u32 stage[CS_STAGE], list[CS_T];
+    __shared__ unsigned nlist, nstage;
+    __shared__ unsigned long long gpos;
+    const int d = P.d, lb = P.lb;
+    const u32 ap = P.ap, p0 = blockIdx.x * P.per;
+    if (p0 >= P.nprefix) return;   // whole block
+    if (threadIdx.x == 0) nlist = nstage = 0;
+    __syncthreads();
+    if (threadIdx.x < P.per && p0 + threadIdx.x < P.nprefix &&
+        lyndon_prefix(p0 + threadIdx.x, d - lb))
+        list[atomicAdd(&nlist, 1u)] = p0 + threadIdx.x;
+    __syncthreads();
+    const u32 n = nlist, ncand = 1u << (lb - 1);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (u32 r = 0; r < n; r += CS_T / 64) {
+        const u32 k = r + wave;
+        if (k < n) {
+            const u32 base = (__builtin_amdgcn_readfirstlane(list[k]) << lb) | 1;
+            for (u32 c0 = 0; c0 < ncand; c0 += 256) {
+                bool ok[4];
+                unsigned long long bal[4];
+                unsigned tot = 0;
 #pragma unroll
-        for (int q = 0; q < ZC_PER; q++) {
-            const u64 t = c0 + (u64)q * ZC_T + threadIdx.x;
-            live[q] = t < nsurv;
-            j[q] = live[q] ? surv[t] : 1u;
-        }
+                for (int q = 0; q < 4; q++) {
+                    const u32 c = c0 + 64 * q + lane;
+                    ok[q] = c < ncand && lyndon_word(base + 2 * c, d, ap);
+                    bal[q] = __ballot(ok[q]);
+                    tot += (unsigned)__popcll(bal[q]);
+                }
+                unsigned at = 0;
+                if (lane == 0) at = atomicAdd(&nstage, tot);
+                at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
-        for (int q = 0; q < ZC_PER; q++) {
-            const u64 u = mod_mersenne((u64)j[q] * P.rmod, P.d, P.M);
-            live[q] = live[q] && u;                    // u = 0: beta^r = 1, never a root
-            a[q] = antilog(P, u ? u : 1) ^ 1u;
-        }
-#pragma unroll
-        for (int q = 0; q < ZC_PER; q++) v[q] = live[q] ? L[a[q]] : 0u;   // Zech logarithms of u
-        unsigned keep = 0;
-        MarkRec rec[ZC_PER];
-#pragma unroll
-        for (int q = 0; q < ZC_PER; q++) {
-            rec[q] = MarkRec{0, 0, 0, 0};
-            if (!live[q]) continue;
-            const u32 gg = gcd32(j[q], M);
-            if (v[q] % gg) continue;
-            const u32 n = M / gg;
-            const u32 iv = inv32(j[q] / gg, n);
-            const u64 prod = (u64)iv * (v[q] / gg);
-            const u32 s0 = (u32)(gg == 1 ? mod_mersenne(prod, P.d, P.M) : prod % n);
-            const u32 sf = s0 ? s0 : n;
-            if (sf <= P.smax) {
-                keep |= 1u << q;
-                rec[q] = MarkRec{j[q], n, sf, 0};
+                for (int q = 0; q < 4; q++) {
+                    if (ok[q])
+                        stage[at + (unsigned)__popcll(bal[q] & ((1ULL << lane) - 1))] =
+                            base + 2 * (c0 + 64 * q + lane);
+                    at += (unsigned)__popcll(bal[q]);
+                }
             }
         }
-        unsigned total;
-        const unsigned pre = block_excl_scan<ZC_T>((unsigned)__popc(keep), &total, wtot);
-        if (threadIdx.x == 0) bbase = total ? atomicAdd(nqueue, (unsigned long long)total) : 0;
         __syncthreads();
-        u64 pos = bbase + pre;
+        const unsigned m = nstage;   // at most 4096 more per round
+        if (m > CS_STAGE - 4096 || (r + CS_T / 64 >= n && m)) {
+            if (threadIdx.x == 0) gpos = atomicAdd(P.cnt + CN_SURV, (unsigned long long)m);
+            __syncthreads();
+            for (unsigned i = threadIdx.x; i < m; i += CS_T)
+                if (gpos + i < P.ncls) P.surv[gpos + i] = stage[i];
+            if (threadIdx.x == 0) nstage = 0;
+        }
+        __syncthreads();
+    }
+}
+
+// the classes found, at most the list's length
+GF2T_DEV u64 class_count(const SieveDeg &P) {
+    const u64 n = P.cnt[CN_SURV];
+    return n < P.ncls ? n : P.ncls;
+}
+
+// T[class of g^j] = log of its least rotation, for every class.  Bounded by
+// the VALU (a carry-less product, 31 rotations at 4 operations) and the
+// antilog gathers while T stays in the caches, 16 ps a class up to d = 29;
+// at d = 32 by the scattered 4-byte stores, 4.2 ms.  The table of all
+// logarithms took 38 ms there.
+constexpr int CL_T = 256, CL_PER = 4;
+__global__ __launch_bounds__(CL_T) void k_class_log(const SieveDeg *__restrict__ degs) {
+    const SieveDeg &P = degs[blockIdx.y];
+    __shared__ u32 norm[2048];
+    const u64 n = class_count(P), chunk = (u64)CL_T * CL_PER;
+    if ((u64)blockIdx.x * chunk >= n) return;   // whole block
+    for (u32 i = threadIdx.x; i < 2048; i += CL_T) norm[i] = P.map[CL_NORM + i];
+    __syncthreads();
+    const int d = P.d;
+    for (u64 c0 = (u64)blockIdx.x * chunk; c0 < n; c0 += (u64)gridDim.x * chunk) {
+        u32 j[CL_PER], hi[CL_PER], lo[CL_PER];
 #pragma unroll
-        for (int q = 0; q < ZC_PER; q++)
+        for (int q = 0; q < CL_PER; q++) {
+            const u64 t = c0 + (u64)q * CL_T + threadIdx.x;
+            j[q] = t < n ? P.surv[t] : 0u;
+        }
+#pragma unroll
+        for (int q = 0; q < CL_PER; q++) {
+            hi[q] = P.hi[j[q] >> 16];
+            lo[q] = P.lo[j[q] & 0xFFFF];
+        }
+#pragma unroll
+        for (int q = 0; q < CL_PER; q++) {
+            const u64 t = c0 + (u64)q * CL_T + threadIdx.x;
+            int k;
+            const u32 m = least_rotation(periodic64(map8((const u32 *)norm, clmul32(hi[q], lo[q])), d), k);
+            if (t < n) P.T[class_index(m, d)] = rotl_d(j[q], k, d);
+        }
+    }
+}
+
+// Per class: Zech logarithm (one random gather), the progression
+// s == s0 (mod n), and -- only for the few classes whose progression
+// reaches s <= smax -- a queue entry, so that k_mark's minimal polynomials
+// run on dense waves.  A thread takes ZN_PER classes: their lookups are
+// overlapped, and one Euclid inverts the product of their units (three
+// products a class; a gcd, an inverse and two divisions a class before).
+// Bounded by the VALU and the gathers: 3.3 ms at d = 32, 5.6 before.
+constexpr int ZN_T = 256, ZN_PER = 8;
+__global__ __launch_bounds__(ZN_T) void k_zech(const SieveDeg *__restrict__ degs) {
+    const SieveDeg &P = degs[blockIdx.y];
+    __shared__ u32 norm[2048], zech[ZN_T * ZN_PER];
+    __shared__ unsigned wtot[ZN_T / 64];
+    __shared__ unsigned long long bbase;
+    const u64 n = class_count(P), chunk = (u64)ZN_T * ZN_PER;
+    if ((u64)blockIdx.x * chunk >= n) return;   // whole block
+    for (u32 i = threadIdx.x; i < 2048; i += ZN_T) norm[i] = P.map[CL_NORM + i];
+    __syncthreads();
+    const int d = P.d;
+    const u32 M = P.M;
+    for (u64 c0 = (u64)blockIdx.x * chunk; c0 < n; c0 += (u64)gridDim.x * chunk) {
+        // Zech logarithms, one class after another (all eight unrolled
+        // together took 256 VGPRs and scratch): a gather is on its way
+        // while the next class's rotation is found
+        u32 back = 0;   // the rotation still to be undone of the last gather
+        u32 got = 0;
+#pragma unroll 1
+        for (int q = 0; q <= ZN_PER; q++) {
+            u32 next = 0, nback = 0;
+            const u64 t = c0 + (u64)q * ZN_T + threadIdx.x;
+            if (q < ZN_PER && t < n) {
+                const u32 u = mulmod_mersenne(P.surv[t], P.rmod, d, M);   // beta^r = g^u, not 1: r is prime to M
+                // w(1) is all ones
+                const u32 w = map8((const u32 *)norm, clmul32(P.hi[u >> 16], P.lo[u & 0xFFFF])) ^ M;
+                int k;
+                next = P.T[class_index(least_rotation(periodic64(w, d), k), d)];
+                nback = (u32)(d - k);
+            }
+            if (q) zech[(q - 1) * ZN_T + threadIdx.x] = rotl_d(got, (int)back, d);
+            got = next;
+            back = nback;
+        }
+        u32 j[ZN_PER], v[ZN_PER];   // v: log(beta^r + 1)
+        unsigned live = 0;
+#pragma unroll
+        for (int q = 0; q < ZN_PER; q++) {
+            const u64 t = c0 + (u64)q * ZN_T + threadIdx.x;
+            live |= (unsigned)(t < n) << q;
+            j[q] = t < n ? P.surv[t] : 1u;
+            v[q] = zech[q * ZN_T + threadIdx.x];   // this thread's own
+        }
+        u32 un[ZN_PER], nn[ZN_PER], pre[ZN_PER];
+        live &= progressions(v, j, nn, un, M, P.pr, P.np);
+#pragma unroll
+        for (int q = 0; q < ZN_PER; q++)
+            pre[q] = q ? mulmod_mersenne(pre[q - 1], un[q], d, M) : un[q];
+        u32 inv = inv32(pre[ZN_PER - 1], M);
+        unsigned keep = 0;
+#pragma unroll
+        for (int q = ZN_PER - 1; q >= 0; q--) {
+            const u32 iv = q ? mulmod_mersenne(inv, pre[q - 1], d, M) : inv;
+            inv = mulmod_mersenne(inv, un[q], d, M);
+            u32 s0 = mulmod_mersenne(iv, v[q], d, M);
+            if (nn[q] != M) s0 %= nn[q];
+            v[q] = s0 ? s0 : nn[q];                              // first s >= 1
+            if (((live >> q) & 1) && v[q] <= P.smax) keep |= 1u << q;
+        }
+        unsigned total;
+        const unsigned before = block_excl_scan<ZN_T>((unsigned)__popc(keep), &total, wtot);
+        if (threadIdx.x == 0)
+            bbase = total ? atomicAdd(P.cnt + CN_QUEUE, (unsigned long long)total) : 0;
+        __syncthreads();
+        u64 pos = bbase + before;
+#pragma unroll
+        for (int q = 0; q < ZN_PER; q++)
             if ((keep >> q) & 1) {
-                if (pos < qcap) queue[pos] = rec[q];
+                if (pos < P.qcap) P.queue[pos] = MarkRec{j[q], nn[q], v[q], 0};
                 pos++;
             }
         __syncthreads();   // bbase and wtot are rewritten by the next round
     }
 }
 
-// Phase 2, one lane per queued class: minimal polynomial by
-// Berlekamp-Massey on the trace sequence, then the marks (inline up to
-// INLINE_MARKS, longer progressions to the heavy queue).
-__global__ void k_mark(DegreeParams P, const MarkRec *__restrict__ queue, u64 nq,
-                       unsigned long long *__restrict__ best, Heavy *__restrict__ heavy,
-                       unsigned *__restrict__ nheavy, unsigned *__restrict__ bad) {
-    u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nq) return;
-    const MarkRec rec = queue[t];
+// Per queued class: minimal polynomial, then the marks: of one period
+// (P.pat), inline up to INLINE_MARKS, or through the heavy queue (hcount
+// entries so far).  Bounded by the random read-modify-writes of best[]:
+// 0.16 ms at d = 32 and 0.30 ms at d = 28, where each class's 64 products
+// with a bit-serial reduction took 1.07 and 0.82.
+constexpr int MK_T = 256;
+__global__ __launch_bounds__(MK_T) void k_mark(const SieveDeg *__restrict__ degs,
+                                               unsigned long long *__restrict__ best,
+                                               Heavy *__restrict__ heavy,
+                                               unsigned long long *__restrict__ hcount) {
+    const SieveDeg &P = degs[blockIdx.y];
+    __shared__ u32 map[CL_MAP - CL_RED];
+    const u64 all = P.cnt[CN_QUEUE], nq = all < P.qcap ? all : P.qcap;
+    if ((u64)blockIdx.x * MK_T >= nq) return;   // whole block
+    for (u32 i = threadIdx.x; i < CL_MAP - CL_RED; i += MK_T) map[i] = P.map[CL_RED + i];
+    __syncthreads();
+    const u32 *red = map, *dual = map + (CL_DUAL - CL_RED);
     const int d = P.d;
-    u64 mask = minpoly_bm(antilog(P, rec.j), P.q, d, P.tmask);
-    if (mask == 0 || !((mask >> d) & 1) || !(mask & 1)) { atomicAdd(bad, 1u); return; }
-    unsigned long long key = ((unsigned long long)d << 48) | mask;
-    u64 n = rec.n, sf = rec.sf;
-    u64 count = (P.smax - sf) / n + 1;
-    if (count <= INLINE_MARKS) {
-        for (u64 s = sf; s <= P.smax; s += n)
-            if (best[s] > key) atomicMin(&best[s], key);
-    } else {
-        unsigned idx = atomicAdd(nheavy, 1u);
-        if (idx < HEAVY_CAP) heavy[idx] = Heavy{sf, n, key};
-        else atomicAdd(bad, 2u);
+    const u64 smax = P.smax;
+    for (u64 t = (u64)blockIdx.x * MK_T + threadIdx.x; t < nq; t += (u64)gridDim.x * MK_T) {
+        const MarkRec rec = P.queue[t];
+        const u32 beta = red_product(clmul32(P.hi[rec.j >> 16], P.lo[rec.j & 0xFFFF]), red, d);
+        const u64 mask = minpoly_seq(trace_sequence(beta, red, dual, d), d);
+        if (mask == 0 || !((mask >> d) & 1) || !(mask & 1)) {
+            atomicOr(P.cnt + CN_BAD, 1ULL);
+            continue;
+        }
+        const unsigned long long key = ((unsigned long long)d << 48) | mask;
+        const u64 n = rec.n, sf = rec.sf, count = (smax - sf) / n + 1;
+        if (count > INLINE_MARKS) atomicAdd(P.cnt + CN_HEAVY, 1ULL);
+        if (P.pat) {
+            for (u32 s = sf == n ? 0u : (u32)sf; s < P.M; s += (u32)n) atomicMin(&P.pat[s], (u32)mask);
+        } else if (count <= INLINE_MARKS) {
+            for (u64 s = sf; s <= smax; s += n)
+                if (best[s] > key) atomicMin(&best[s], key);
+        } else {
+            const u64 idx = atomicAdd(hcount, 1ULL);
+            if (idx < HEAVY_CAP) heavy[idx] = Heavy{sf, n, key};
+            else atomicOr(P.cnt + CN_BAD, 2ULL);
+        }
     }
 }
 
-__global__ void k_mark_heavy(const Heavy *__restrict__ heavy, unsigned nheavy, u64 smax,
-                             unsigned long long *__restrict__ best) {
+// Degrees lo..hi marked one period each (pat).  2^d - 1 divides 2^e - 1
+// where d divides e, so only the periods of the degrees e > hi / 2 are
+// needed: k_fold_periods takes the marks of e's divisors into e's table,
+// as keys d << 21 | mask, the lowest first.
+struct PeriodArgs {
+    const u32 *pat[PAT_MAX_D + 1];   // marks of degree d
+    u32 *tab[PAT_MAX_D / 2];         // tables of the degrees first..hi
+    int lo, hi, first;
+};
+__global__ void k_fold_periods(PeriodArgs A) {
+    const int e = A.first + (int)blockIdx.y;
+    const u32 M = (1u << e) - 1;
+    for (u32 x = blockIdx.x * blockDim.x + threadIdx.x; x < M; x += gridDim.x * blockDim.x) {
+        u32 key = ~0u;
+        for (int d = A.lo; d <= e; d++) {
+            if (e % d) continue;
+            const u32 m = A.pat[d][x % ((1u << d) - 1)];
+            if (m != ~0u) {
+                key = (u32)d << 21 | m;
+                break;
+            }
+        }
+        A.tab[blockIdx.y][x] = key;
+    }
+}
+// Every s through those tables: the least key is the least factor of the
+// degrees lo..hi.  One pass over best[], with its loads and stores, and
+// the tables' loads, in order: 0.7 ms for 68,139,920 s and degrees 2..20,
+// where marking the progressions one by one took 4.6.
+constexpr int SW_T = 256, SW_PER = 16;
+__global__ __launch_bounds__(SW_T) void k_sweep(PeriodArgs A, u64 smax,
+                                                unsigned long long *__restrict__ best) {
+    constexpr int N = PAT_MAX_D / 2;
+    __shared__ u32 base[N];   // the block's first s modulo each period
+    const u64 s0 = 1 + (u64)blockIdx.x * SW_T * SW_PER;
+    if (threadIdx.x < N && A.first + (int)threadIdx.x <= A.hi)
+        base[threadIdx.x] = (u32)(s0 % (((u64)1 << (A.first + threadIdx.x)) - 1));
+    __syncthreads();
+    u32 x[N];
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        if (A.first + i <= A.hi) x[i] = (base[i] + threadIdx.x) % ((1u << (A.first + i)) - 1);
+    for (int it = 0; it < SW_PER; it++) {
+        const u64 s = s0 + it * SW_T + threadIdx.x;
+        if (s > smax) return;
+        u32 key = ~0u;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if (A.first + i > A.hi) break;
+            const u32 M = (1u << (A.first + i)) - 1, m = A.tab[i][x[i]];
+            key = m < key ? m : key;
+            x[i] += SW_T % M;
+            x[i] = x[i] >= M ? x[i] - M : x[i];
+        }
+        if (key == ~0u) continue;
+        const unsigned long long k64 =
+            ((unsigned long long)(key >> 21) << 48) | (key & ((1u << 21) - 1));
+        if (best[s] > k64) best[s] = k64;
+    }
+}
+
+// nheavy: how many, or null and `known`
+__global__ void k_mark_heavy(const Heavy *__restrict__ heavy,
+                             const unsigned long long *__restrict__ count_at, unsigned known,
+                             u64 smax, unsigned long long *__restrict__ best) {
+    const unsigned nheavy = count_at ? (unsigned)(*count_at < HEAVY_CAP ? *count_at : HEAVY_CAP) : known;
     for (unsigned rec = blockIdx.y; rec < nheavy; rec += gridDim.y) {
         const Heavy h = heavy[rec];
         u64 count = (smax - h.s_first) / h.n + 1;
@@ -919,7 +970,8 @@ const WideHost &wide_host(int d) {
 }
 
 struct SieveWork {
-    DevBuf bL, bSurv, bQueue, bHeavy, bTab, bCnt, bP1, bP2, bCur;
+    DevBuf bClass, bHeavy, bTab, bCnt, bPat, bDegs;
+    u64 tab_ready = 0;   // degrees whose tables bTab holds
     DevBuf wP1, wTmp, wLlo, wLhi, wSurv, wQueue, wTab, wCur;   // degrees 33..34
 };
 std::mutex g_sw_mu;
@@ -930,11 +982,11 @@ SieveWork *g_sw = nullptr;   // never destroyed at exit: the runtime may be gone
 extern "C" int gf2t_sieve_release(void) {
     std::lock_guard<std::mutex> lk(g_sw_mu);
     if (g_sw) {
-        for (DevBuf *b : {&g_sw->bL, &g_sw->bSurv, &g_sw->bQueue, &g_sw->bHeavy, &g_sw->bTab,
-                          &g_sw->bCnt, &g_sw->bP1, &g_sw->bP2, &g_sw->bCur, &g_sw->wP1,
-                          &g_sw->wTmp, &g_sw->wLlo, &g_sw->wLhi, &g_sw->wSurv, &g_sw->wQueue,
-                          &g_sw->wTab, &g_sw->wCur})
+        for (DevBuf *b : {&g_sw->bClass, &g_sw->bHeavy, &g_sw->bTab, &g_sw->bCnt, &g_sw->bPat,
+                          &g_sw->bDegs, &g_sw->wP1, &g_sw->wTmp, &g_sw->wLlo, &g_sw->wLhi,
+                          &g_sw->wSurv, &g_sw->wQueue, &g_sw->wTab, &g_sw->wCur})
             b->release();
+        g_sw->tab_ready = 0;
     }
     return GF2T_OK;
 }
@@ -947,208 +999,214 @@ extern "C" uint64_t gf2t_primitive_poly(int d) {
 namespace {
 // per-degree phase timers, destroyed on every return path
 struct SieveEvents {
-    hipEvent_t e[4] = {};
+    hipEvent_t e[33][4] = {};
     ~SieveEvents() {
-        for (hipEvent_t x : e)
-            if (x) (void)hipEventDestroy(x);
+        for (auto &g : e)
+            for (hipEvent_t x : g)
+                if (x) (void)hipEventDestroy(x);
     }
-};
-
-// Device memory of the degrees <= 32: the log table, the two partition
-// buffers and the class / marking arrays of the largest degree.
-struct NarrowMem {
-    u32 *L;
-    unsigned long long *P1, *P2;
-    u32 *surv;
-    MarkRec *queue;
 };
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// The degree-<=32 arrays are carved out of the wide tables whenever those
-// are allocated (they are larger: 12 bytes per element of GF(2^33) against
-// 12 per element of GF(2^32) plus the class arrays), so a sieve to degree
-// 34 never holds both sets and never frees and reallocates between them.
-int narrow_mem(int dn, NarrowMem &m) {
+// Degrees that run in one launch: up to 20, 21..23, then each by itself (a degree-24 launch fills the card).  A launch waits for nothing
+// on the host, and costs about 5 us however little it does.
+int group_end(int d, int dmax) {
+    return std::min(dmax, d <= PAT_MAX_D ? PAT_MAX_D : d <= 23 ? 23 : d);
+}
+
+// bytes of a degree's class table, class list and marking queue
+struct NarrowBytes {
+    size_t T, surv, queue;
+    size_t all() const { return T + surv + queue; }
+};
+NarrowBytes narrow_bytes(int d) {
+    const u64 ncls = irreducible_count(d);
+    return {align256(((size_t)1 << (d - 2)) * 4), align256(ncls * 4), align256(ncls * sizeof(MarkRec))};
+}
+
+// The arrays of the largest group.  They are carved out of the wide log
+// table whenever that is allocated and large enough, so a sieve to degree
+// 34 never holds both.
+int narrow_mem(int dmin, int dmax, char *&mem) {
     SieveWork &W = *g_sw;
-    const size_t N = (size_t)1 << dn;
-    const u64 ncls = irreducible_count(dn);
-    const size_t lbytes = align256(N * sizeof(u32)), sbytes = align256((ncls + 64) * sizeof(u32));
-    const size_t qbytes = (ncls + 64) * sizeof(MarkRec);
-    const bool part = dn >= LP_MIN_D;
-    const size_t pbytes = part ? N * 8 : 0;
-    if (W.wP1.bytes >= 2 * pbytes && W.wLlo.bytes >= lbytes + sbytes + qbytes) {
-        char *l = (char *)W.wLlo.p;
-        m.L = (u32 *)l;
-        m.surv = (u32 *)(l + lbytes);
-        m.queue = (MarkRec *)(l + lbytes + sbytes);
-        m.P1 = (unsigned long long *)W.wP1.p;
-        m.P2 = (unsigned long long *)((char *)W.wP1.p + pbytes);
+    size_t bytes = 0;
+    for (int d = dmin; d <= dmax;) {
+        const int e = group_end(d, dmax);
+        size_t b = 0;
+        for (; d <= e; d++) b += narrow_bytes(d).all();
+        bytes = std::max(bytes, b);
+    }
+    if (W.wLlo.bytes >= bytes) {
+        mem = (char *)W.wLlo.p;
         return GF2T_OK;
     }
-    int rc;
-    if ((rc = W.bL.ensure(lbytes))) return rc;
-    if ((rc = W.bSurv.ensure(sbytes))) return rc;
-    if ((rc = W.bQueue.ensure(qbytes))) return rc;
-    if (part) {
-        if ((rc = W.bP1.ensure(pbytes))) return rc;
-        if (lp_shape(dn).B2 > 0 && (rc = W.bP2.ensure(pbytes))) return rc;
-    }
-    m.L = (u32 *)W.bL.p;
-    m.surv = (u32 *)W.bSurv.p;
-    m.queue = (MarkRec *)W.bQueue.p;
-    m.P1 = (unsigned long long *)W.bP1.p;
-    m.P2 = (unsigned long long *)W.bP2.p;
+    if (int rc = W.bClass.ensure(bytes)) return rc;
+    mem = (char *)W.bClass.p;
     return GF2T_OK;
 }
 
 // degrees dmin..dmax <= 32 (u32 field elements); g_sw_mu held by the caller
 int sieve_narrow(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
                  gf2t_sieve_stats *stats) {
-    DevBuf &bHeavy = g_sw->bHeavy, &bTab = g_sw->bTab, &bCnt = g_sw->bCnt, &bCur = g_sw->bCur;
-    int rc;
-    NarrowMem mem;
-    if ((rc = narrow_mem(dmax, mem))) return rc;
-    if (dmax >= LP_MIN_D) {
-        LpShape S = lp_shape(dmax);
-        if ((rc = bCur.ensure(((size_t)1 << (S.B1 + S.B2)) * 4 + (1 << LP_B1) * 4))) return rc;
-        static std::once_flag lds_once;
-        static hipError_t lds_err = hipSuccess;
-        std::call_once(lds_once, [] {
-            lds_err = hipFuncSetAttribute((const void *)k_lp_place,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)(((size_t)1 << LP_SB) * sizeof(u32)));
-        });
-        GF2T_HIP(lds_err);
-    }
-    if ((rc = bTab.ensure(2 * 65536 * sizeof(u32)))) return rc;
-    if ((rc = bHeavy.ensure((size_t)HEAVY_CAP * sizeof(Heavy)))) return rc;
-    if ((rc = bCnt.ensure(64))) return rc;
-    unsigned long long *cnt64 = (unsigned long long *)bCnt.p;   // [0] nsurv [1] nqueue
-    unsigned *cnt32 = (unsigned *)((char *)bCnt.p + 32);         // [0] nheavy [1] bad
-    u32 *Alo = (u32 *)bTab.p, *Ahi = Alo + 65536;
-    SieveEvents evs;
-    hipEvent_t(&ev)[4] = evs.e;
-    for (auto &e : ev) GF2T_HIP(hipEventCreate(&e));
-
-    int status = GF2T_OK;
-    for (int d = dmin; d <= dmax && status == GF2T_OK; d++) {
-        const u64 M = ((u64)1 << d) - 1;
+    SieveWork &W = *g_sw;
+    int status = GF2T_OK, rc;
+    // the degrees before the first that cannot be done
+    for (int d = dmin; d <= dmax; d++) {
+        const u64 M = ((u64)1 << d) - 1, rmod = r % M;
         const DegHost &H = deg_host(d);
-        const u64 q = H.q;
-        const u64 rmod = r % M;
-        if (!q || gcd_host(rmod ? rmod : M, M) != 1) {
+        if (!H.q || gcd_host(rmod ? rmod : M, M) != 1) {
             gf2t::set_error("gf2t_sieve: d=%d: gcd(r, 2^d-1) != 1, unsupported r", d);
             status = GF2T_EINVAL;
-            break;
-        }
-        if (!H.trace_ok) {
+        } else if (!H.trace_ok || H.primes.size() > SV_PRIMES) {
             gf2t::set_error("gf2t_sieve: d=%d: trace not in GF(2)", d);
             status = GF2T_EINTERNAL;
+        }
+        if (status != GF2T_OK) {
+            dmax = d - 1;
             break;
         }
-        GF2T_HIP(hipMemcpy(Alo, H.lo.data(), 65536 * 4, hipMemcpyHostToDevice));
-        GF2T_HIP(hipMemcpy(Ahi, H.hi.data(), 65536 * 4, hipMemcpyHostToDevice));
-        const u32 tmask = H.tmask;
-        DegreeParams P{d, M, q, rmod, smax, tmask, Alo, Ahi};
-
-        const u64 ncls = irreducible_count(d);
-        u32 *surv = mem.surv;
-        u32 *L = mem.L;
-        Heavy *heavy = (Heavy *)bHeavy.p;
-
-        GF2T_HIP(hipEventRecord(ev[0], 0));
-        if (d >= LP_MIN_D) {
-            const LpShape S = lp_shape(d);
-            const unsigned nb1 = 1u << S.B1, nb2 = 1u << S.B2;
-            unsigned *cur1 = (unsigned *)bCur.p, *cur2 = cur1 + (1 << LP_B1);
-            const u64 ncur = (1 << LP_B1) + (u64)nb1 * nb2;
-            hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((ncur + 255) / 256)), dim3(256), 0, 0,
-                               cur1, ncur);
-            hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, 0, cnt64, cnt32);
-            unsigned long long *p1 = mem.P1;
-            unsigned long long *p2 = S.B2 ? mem.P2 : p1;
-            hipLaunchKernelGGL(k_lp_part1, dim3((unsigned)((M + LP_E - 1) / LP_E)), dim3(LP_T), 0,
-                               0, P, S, p1, cur1, cnt32 + 1);
-            if (S.B2)
-                hipLaunchKernelGGL(k_lp_part2,
-                                   dim3((unsigned)((((u64)1 << (d - S.B1)) + LP_E - 1) / LP_E), nb1),
-                                   dim3(LP_T), 0, 0, P, S, p1, p2, cur2, cnt32 + 1);
-            hipLaunchKernelGGL(k_lp_place, dim3(nb1 * nb2), dim3(1024),
-                               ((size_t)1 << LP_SB) * sizeof(u32), 0, p2, L);
-            GF2T_CHECK_LAUNCH("log table partition");
-            unsigned chk[2];
-            GF2T_HIP(hipMemcpy(chk, cnt32, 8, hipMemcpyDeviceToHost));
-            if (chk[1]) {
-                gf2t::set_error("gf2t_sieve: d=%d: log table partition overflow", d);
-                status = GF2T_EINTERNAL;
-                break;
+    }
+    if (dmax < dmin) return status;
+    char *mem;
+    if ((rc = narrow_mem(dmin, dmax, mem))) return rc;
+    if ((rc = W.bTab.ensure(33 * DEG_TAB * sizeof(u32)))) return rc;
+    if ((rc = W.bHeavy.ensure((size_t)HEAVY_CAP * sizeof(Heavy)))) return rc;
+    if ((rc = W.bPat.ensure(((size_t)4 << PAT_MAX_D) * sizeof(u32)))) return rc;   // marks, tables
+    if ((rc = W.bDegs.ensure(33 * sizeof(SieveDeg)))) return rc;
+    if ((rc = W.bCnt.ensure(34 * CN_N * 8))) return rc;
+    u32 *tabs = (u32 *)W.bTab.p, *pats = (u32 *)W.bPat.p;
+    unsigned long long *cnt = (unsigned long long *)W.bCnt.p;   // by degree; then the heavy queue's
+    unsigned long long *hcount = cnt + 33 * CN_N;
+    Heavy *heavy = (Heavy *)W.bHeavy.p;
+    SieveDeg degs[33];
+    for (int d = dmin; d <= dmax;) {
+        char *at = mem;
+        for (const int e = group_end(d, dmax); d <= e; d++) {
+            const DegHost &H = deg_host(d);
+            u32 *tab = tabs + (size_t)d * DEG_TAB;
+            if (!((W.tab_ready >> d) & 1)) {
+                GF2T_HIP(hipMemcpy(tab, H.tab.data(), DEG_TAB * sizeof(u32), hipMemcpyHostToDevice));
+                W.tab_ready |= 1ULL << d;
             }
-        } else {
-            u64 nchunks = (M + LOG_CHUNK - 1) / LOG_CHUNK;
-            hipLaunchKernelGGL(k_log_build, dim3((unsigned)((nchunks + 255) / 256)), dim3(256), 0,
-                               0, P, L);
-            GF2T_CHECK_LAUNCH("k_log_build");
+            const NarrowBytes nb = narrow_bytes(d);
+            SieveDeg &P = degs[d];
+            P.d = d;
+            P.lb = std::min(CS_LB, d - 1);
+            P.np = (int)H.primes.size();
+            P.M = (u32)(((u64)1 << d) - 1);
+            P.rmod = (u32)(r % P.M);
+            P.ap = aperiodic_rotations(d);
+            P.nprefix = 1u << (d - P.lb - 1);
+            P.per = std::min<u32>(CS_T, std::max<u32>(4, P.nprefix / 2048));
+            P.q = H.q;
+            P.smax = smax;
+            P.ncls = P.qcap = irreducible_count(d);
+            P.lo = tab;
+            P.hi = tab + 65536;
+            P.map = tab + 2 * 65536;
+            P.T = (u32 *)at;
+            P.surv = (u32 *)(at + nb.T);
+            P.queue = (MarkRec *)(at + nb.T + nb.surv);
+            at += nb.all();
+            P.pat = d <= PAT_MAX_D && P.M <= smax ? pats + ((size_t)1 << d) : nullptr;
+            P.cnt = cnt + d * CN_N;
+            for (int i = 0; i < P.np; i++) P.pr[i] = H.primes[i];
         }
-        hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, 0, cnt64, cnt32);
-        GF2T_HIP(hipEventRecord(ev[1], 0));
-        hipLaunchKernelGGL(k_lyndon_t<u32>, dim3(lyndon_blocks(d)), dim3(LY_T), 0, 0, d, (u32)M,
-                           surv, cnt64, (u64)(ncls + 64));
-        GF2T_CHECK_LAUNCH("k_lyndon");
-        unsigned long long hs[2];
-        GF2T_HIP(hipMemcpy(hs, cnt64, 16, hipMemcpyDeviceToHost));
-        u64 nsurv = hs[0];
-        if (nsurv != ncls) {
-            gf2t::set_error("gf2t_sieve: d=%d: %llu classes, expected %llu", d,
-                            (unsigned long long)nsurv, (unsigned long long)ncls);
-            status = GF2T_EINTERNAL;
-            break;
-        }
-        MarkRec *queue = mem.queue;
-        if (nsurv) {
-            const u64 zb = std::min<u64>((nsurv + (u64)ZC_T * ZC_PER - 1) / ((u64)ZC_T * ZC_PER),
-                                         1u << 16);
-            hipLaunchKernelGGL(k_zech, dim3((unsigned)zb), dim3(ZC_T), 0, 0, P, surv, nsurv, L,
-                               queue, cnt64 + 1, (u64)(ncls + 64));
-            GF2T_CHECK_LAUNCH("k_zech");
-            GF2T_HIP(hipMemcpy(hs, cnt64, 16, hipMemcpyDeviceToHost));
-            u64 nq = std::min<u64>(hs[1], ncls + 64);
-            if (nq) {
-                hipLaunchKernelGGL(k_mark, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, 0, P,
-                                   queue, nq, (unsigned long long *)dbest, heavy, cnt32,
-                                   cnt32 + 1);
-                GF2T_CHECK_LAUNCH("k_mark");
+    }
+    SieveEvents evs;
+    hipEvent_t(&ev)[33][4] = evs.e;   // [first degree of a group]
+    if (stats)
+        for (int d = dmin; d <= dmax; d = group_end(d, dmax) + 1)
+            for (auto &e : ev[d]) GF2T_HIP(hipEventCreate(&e));
+    SieveDeg *ddegs = (SieveDeg *)W.bDegs.p;
+    GF2T_HIP(hipMemcpyAsync(ddegs + dmin, degs + dmin, (dmax - dmin + 1) * sizeof(SieveDeg),
+                            hipMemcpyHostToDevice, 0));
+    hipLaunchKernelGGL(k_fill_u32, dim3(2), dim3(256), 0, 0, (unsigned *)cnt, (u64)34 * CN_N * 2, 0u);
+    for (int d = dmin; d <= dmax;) {
+        const int e = group_end(d, dmax);
+        const unsigned ny = (unsigned)(e - d + 1);
+        const SieveDeg *g = ddegs + d;
+        u64 bc = 0, bl = 0, bz = 0, bm = 0;
+        PeriodArgs A{};
+        A.lo = d;
+        A.hi = d - 1;
+        for (int k = d; k <= e; k++) {
+            const SieveDeg &P = degs[k];
+            bc = std::max<u64>(bc, (P.nprefix + P.per - 1) / P.per);
+            bl = std::max<u64>(bl, (P.ncls + CL_T * CL_PER - 1) / (CL_T * CL_PER));
+            bz = std::max<u64>(bz, (P.ncls + ZN_T * ZN_PER - 1) / (ZN_T * ZN_PER));
+            bm = std::max<u64>(bm, (P.ncls + MK_T - 1) / MK_T);
+            if (P.pat) {
+                A.pat[k] = P.pat;
+                A.hi = k;
             }
         }
-        GF2T_HIP(hipEventRecord(ev[2], 0));
-        unsigned h32[2];
-        GF2T_HIP(hipMemcpy(h32, cnt32, 8, hipMemcpyDeviceToHost));
-        if (h32[1]) {
+        if (stats) GF2T_HIP(hipEventRecord(ev[d][0], 0));
+        hipLaunchKernelGGL(k_classes, dim3((unsigned)bc, ny), dim3(CS_T), 0, 0, g);
+        hipLaunchKernelGGL(k_class_log, dim3((unsigned)std::min<u64>(bl, 4096), ny), dim3(CL_T), 0, 0, g);
+        if (stats) GF2T_HIP(hipEventRecord(ev[d][1], 0));
+        hipLaunchKernelGGL(k_zech, dim3((unsigned)std::min<u64>(bz, 4096), ny), dim3(ZN_T), 0, 0, g);
+        const bool periods = A.hi >= A.lo;
+        if (periods) {
+            const u64 n = (u64)2 << A.hi;
+            hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, pats, n, ~0u);
+            A.first = std::max(A.lo, A.hi / 2 + 1);
+            for (int k = A.first; k <= A.hi; k++)
+                A.tab[k - A.first] = pats + ((size_t)2 << PAT_MAX_D) + ((size_t)1 << k);
+        }
+        hipLaunchKernelGGL(k_mark, dim3((unsigned)std::min<u64>(bm, 2048), ny), dim3(MK_T), 0, 0, g,
+                           (unsigned long long *)dbest, heavy, hcount);
+        if (stats) GF2T_HIP(hipEventRecord(ev[d][2], 0));
+        if (periods) {
+            const u64 n = ((u64)1 << A.hi) / 1024;
+            hipLaunchKernelGGL(k_fold_periods,
+                               dim3((unsigned)std::max<u64>(1, n), (unsigned)(A.hi - A.first + 1)),
+                               dim3(256), 0, 0, A);
+            hipLaunchKernelGGL(k_sweep, dim3((unsigned)((smax + SW_T * SW_PER - 1) / (SW_T * SW_PER))),
+                               dim3(SW_T), 0, 0, A, smax, (unsigned long long *)dbest);
+        }
+        hipLaunchKernelGGL(k_mark_heavy, dim3(64, 16), dim3(256), 0, 0, heavy, hcount, 0u, smax,
+                           (unsigned long long *)dbest);
+        if (e < dmax)   // the next group's heavy queue
+            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, 0, (unsigned *)hcount, (u64)2, 0u);
+        if (stats) GF2T_HIP(hipEventRecord(ev[d][3], 0));
+        GF2T_CHECK_LAUNCH("sieve degrees");
+        d = e + 1;
+    }
+    unsigned long long h[33 * CN_N];
+    GF2T_HIP(hipMemcpy(h, cnt, sizeof(h), hipMemcpyDeviceToHost));
+    for (int d = dmin; d <= dmax; d++) {
+        const unsigned long long *c = h + d * CN_N;
+        const SieveDeg &P = degs[d];
+        if (c[CN_SURV] != P.ncls) {
+            gf2t::set_error("gf2t_sieve: d=%d: %llu classes, expected %llu", d, c[CN_SURV],
+                            (unsigned long long)P.ncls);
+            return GF2T_EINTERNAL;
+        }
+        if (c[CN_BAD]) {
             gf2t::set_error("gf2t_sieve: d=%d: %s", d,
-                            (h32[1] & 1) ? "minimal polynomial not over GF(2)"
-                                         : "heavy queue overflow");
-            status = GF2T_EINTERNAL;
-            break;
+                            (c[CN_BAD] & 1) ? "minimal polynomial not over GF(2)"
+                                            : "heavy queue overflow");
+            return GF2T_EINTERNAL;
         }
-        unsigned nheavy = h32[0];
-        if (nheavy) {
-            unsigned gy = nheavy < 65535 ? nheavy : 65535;
-            hipLaunchKernelGGL(k_mark_heavy, dim3(64, gy), dim3(256), 0, 0, heavy, nheavy, smax,
-                               (unsigned long long *)dbest);
-            GF2T_CHECK_LAUNCH("k_mark_heavy");
-        }
-        GF2T_HIP(hipEventRecord(ev[3], 0));
-        GF2T_HIP(hipEventSynchronize(ev[3]));
-        if (stats) {
+    }
+    if (!stats) return status;
+    for (int d = dmin; d <= dmax;) {   // degrees that ran together share the time by their size
+        const int f = d, e = group_end(d, dmax);
+        float ms[3];
+        for (int i = 0; i < 3; i++) GF2T_HIP(hipEventElapsedTime(&ms[i], ev[f][i], ev[f][i + 1]));
+        for (; d <= e; d++) {
             gf2t_sieve_stats &S = stats[d];
+            const float part = (float)((double)((u64)1 << d) / (double)(((u64)2 << e) - ((u64)1 << f)));
             S.d = d;
-            S.q = q;
-            S.classes = nsurv;
-            S.marking = hs[1];
-            S.heavy = nheavy;
-            GF2T_HIP(hipEventElapsedTime(&S.ms_table, ev[0], ev[1]));
-            GF2T_HIP(hipEventElapsedTime(&S.ms_classes, ev[1], ev[2]));
-            GF2T_HIP(hipEventElapsedTime(&S.ms_heavy, ev[2], ev[3]));
+            S.q = degs[d].q;
+            S.classes = h[d * CN_N + CN_SURV];
+            S.marking = h[d * CN_N + CN_QUEUE];
+            S.heavy = h[d * CN_N + CN_HEAVY];
+            S.ms_table = ms[0] * part;
+            S.ms_classes = ms[1] * part;
+            S.ms_heavy = ms[2] * part;
         }
     }
     return status;
@@ -1180,7 +1238,7 @@ int wide_mem(int dmax) {
     const size_t n2 = (size_t)1 << std::max(0, dmax - W_B1 - W_SB);
     if ((rc = W.wCur.ensure((256 + n2) * 4))) return rc;
     if ((rc = W.bHeavy.ensure((size_t)HEAVY_CAP * sizeof(Heavy)))) return rc;
-    if ((rc = W.bCnt.ensure(64))) return rc;
+    if ((rc = W.bCnt.ensure(34 * CN_N * 8))) return rc;
     return GF2T_OK;
 }
 
@@ -1279,7 +1337,7 @@ int sieve_wide(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
             GF2T_HIP(hipEventRecord(ev[4 + 2 * sl], 0));
             // log table slice: partition pass 1 (this slice's buckets),
             // level-2 split per bucket, placement
-            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, 0, cur1, (u64)256);
+            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, 0, cur1, (u64)256, 0u);
             hipLaunchKernelGGL(k_w_part1, dim3((unsigned)((M + W_E - 1) / W_E)), dim3(W_T), 0, 0,
                                P, P1, cur1, cnt32 + 1, b0, (unsigned)nb);
             GF2T_CHECK_LAUNCH("k_w_part1");
@@ -1288,12 +1346,12 @@ int sieve_wide(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
             for (unsigned b1 = b0; b1 < b0 + (unsigned)nb; b1++) {
                 const u64 count = b1 ? cap1 : cap1 - 1;   // value 0 never occurs
                 unsigned long long *bk = P1 + (u64)(b1 - b0) * cap1;
-                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, 0, cur2, (u64)(1u << B2a));
+                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, 0, cur2, (u64)(1u << B2a), 0u);
                 hipLaunchKernelGGL(k_w_split, dim3((unsigned)((count + W_E - 1) / W_E), 1),
                                    dim3(WS_T), 0, 0, bk, cap1, count, W_SB + B2b, B2a, tmp, capA,
                                    cur2, cnt32 + 1);
                 hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)(((1u << B2) + 255) / 256)),
-                                   dim3(256), 0, 0, cur2, (u64)(1u << B2));
+                                   dim3(256), 0, 0, cur2, (u64)(1u << B2), 0u);
                 hipLaunchKernelGGL(k_w_split, dim3((unsigned)((capA + W_E - 1) / W_E), 1u << B2a),
                                    dim3(WS_T), 0, 0, tmp, capA, b1 ? capA : capA - 1, W_SB, B2b,
                                    bk, (u64)1 << W_SB, cur2, cnt32 + 1);
@@ -1341,8 +1399,8 @@ int sieve_wide(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
         const unsigned nheavy = h32[0];
         if (nheavy) {
             unsigned gy = nheavy < 65535 ? nheavy : 65535;
-            hipLaunchKernelGGL(k_mark_heavy, dim3(64, gy), dim3(256), 0, 0, heavy, nheavy, smax,
-                               (unsigned long long *)dbest);
+            hipLaunchKernelGGL(k_mark_heavy, dim3(64, gy), dim3(256), 0, 0, heavy, nullptr, nheavy,
+                               smax, (unsigned long long *)dbest);
             GF2T_CHECK_LAUNCH("k_mark_heavy");
         }
         GF2T_HIP(hipEventRecord(ev[3], 0));
@@ -1410,8 +1468,7 @@ extern "C" int gf2t_sieve(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_
     const int wf = g_wide_from;
     if (dmax >= 33) {
         // the degree-<=32 arrays live inside the wide tables from here on
-        for (DevBuf *b : {&g_sw->bL, &g_sw->bP1, &g_sw->bP2, &g_sw->bSurv, &g_sw->bQueue})
-            b->release();
+        g_sw->bClass.release();
         status = wide_mem(dmax);
     }
     if (status == GF2T_OK && dmin < wf)
