@@ -869,6 +869,130 @@ GF2T_HD u64 fold_word(const u64 *p, size_t pw, u64 L, u64 r, u64 s, size_t w) {
     return fold_words([=](size_t k) -> u64 { return k < pw ? p[k] : 0; }, L, r, s, w);
 }
 
+// --------------------------------------- 2^M-th powers by direct windows
+// F^(2^M) = sum of f_k x^(2^M k), 2^M k < 2^M r, is reduced by x^e ->
+// x^(e-r) + x^(e-r+s) until every exponent is below r.  A term that took
+// the first branch a - b times and the second b times lands on
+// v = e - a r + b s; all steps but the last have room whatever their
+// order, and the last has if it was a first branch (C(a-1, b) orders) or
+// v >= s (C(a-1, b-1) more).  So over GF(2)
+//   bit v of F^(2^M) mod T = sum over (a, b) of f[(v + a r - b s) / 2^M]
+// over the pairs with C(a, b) odd for v >= s, and C(a-1, b) odd for v < s,
+// where the division is exact and the index is below r.  For M = 3 that is
+// 27 pairs for small s and up to 41 as s nears r/2, a <= 15; a pair reaches
+// the bits v = c mod 2^M, c = -(a r - b s) mod 2^M, and 32 such bits in a
+// row are 32 consecutive coefficients of F: one shifted window.
+struct PowWin {
+    u32 kw, sh, cls;   // unit i: the 32 coefficients from 32 (i + kw) + sh on, to class cls
+    bool part;         // only the bits [lo, hi) of the range, from its first on
+    int lo, hi;
+};
+// the pair (a, b) over the output bits [V0, V1), V0 a multiple of 2^M 32;
+// false if it adds nothing there
+template <int M>
+GF2T_HD bool pow_window(u64 r, u64 s, u32 a, u32 b, u64 V0, u64 V1, PowWin &w) {
+    if (b > a) return false;
+    const bool up = (b & ~a) == 0, dn = a ? (b & ~(a - 1)) == 0 : true;
+    const int64_t off = (int64_t)(a * r) - (int64_t)(b * s);
+    int64_t hi = (int64_t)((r - 1) << M) - off + 1, lo = dn ? 0 : (int64_t)s;
+    const int64_t top = up ? (int64_t)r : (int64_t)s;
+    if (hi > top) hi = top;
+    w.part = lo > (int64_t)V0 || hi < (int64_t)V1;
+    lo = lo > (int64_t)V0 ? lo : (int64_t)V0;
+    hi = hi < (int64_t)V1 ? hi : (int64_t)V1;
+    if (!(up || dn) || lo >= hi) return false;
+    w.cls = (u32)(-off) & ((1u << M) - 1);
+    const u64 K = (u64)(off + w.cls) >> M;
+    w.kw = (u32)(K >> 5);
+    w.sh = (u32)(K & 31);
+    w.lo = (int)(lo - (int64_t)V0);
+    w.hi = (int)(hi - (int64_t)V0);
+    return true;
+}
+// of a window's 32 bits those that count, in the unit that starts `at`
+// bits into the range
+template <int M>
+GF2T_HD u32 pow_mask(int at, u32 cls, int lo, int hi) {
+    const int q = at + (int)cls - ((1 << M) - 1);
+    int k0 = (lo - q) >> M, k1 = (hi - q) >> M;
+    k0 = k0 < 0 ? 0 : k0 > 32 ? 32 : k0;
+    k1 = k1 < 0 ? 0 : k1 > 32 ? 32 : k1;
+    return (u32)(((u64)1 << k1) - ((u64)1 << (k0 < k1 ? k0 : k1)));
+}
+// x, y <- their bits at m from x and from y, and the bits above those
+template <int S>
+GF2T_HD void bit_swap(u32 &x, u32 &y, u32 m) {
+    const u32 t = sel_32(m, x, y << S);
+    y = sel_32(m, x >> S, y);
+    x = t;
+}
+// Order of a residue's output ranges of 2^16 bits: windows of one a differ
+// by multiples of s, so ranges about s apart read the same coefficients.
+// The ranges stand in ncol columns, s apart along each, and block x of the
+// launch takes them column by column, each eighth of that order on one XCD
+// (consecutive blocks go to different ones), whose L2 then holds what a
+// column shares.
+struct PowOrder {
+    u32 n, ncol, rows, per;   // ranges; columns; ranges of a column; blocks of an XCD
+};
+GF2T_HD PowOrder pow_order(u64 nw, u64 s) {
+    PowOrder o;
+    o.n = (u32)((nw + 1023) / 1024);
+    const u64 c = s >> 16;
+    o.ncol = c < 1 ? 1 : c > o.n ? o.n : (u32)c;
+    o.rows = (o.n + o.ncol - 1) / o.ncol;
+    o.per = (o.ncol * o.rows + 7) / 8;
+    return o;
+}
+// block x's range, or >= n for none
+GF2T_HD u32 pow_range(const PowOrder &o, u32 x) {
+    const u32 k = x >> 3, i = (x & 7) * o.per + k;
+    if (k >= o.per || i >= o.ncol * o.rows) return o.n;
+    return i % o.rows * o.ncol + i / o.rows;
+}
+// bytes of four words transposed: o[q] = byte q of w[0], w[1], w[2], w[3]
+GF2T_HD void byte_transpose(u32 w0, u32 w1, u32 w2, u32 w3, u32 (&o)[4]) {
+    const u32 a = perm8(w1, w0, 0x05010400u), b = perm8(w1, w0, 0x07030602u);
+    const u32 c = perm8(w3, w2, 0x05010400u), d = perm8(w3, w2, 0x07030602u);
+    o[0] = perm8(c, a, 0x05040100u);
+    o[1] = perm8(c, a, 0x07060302u);
+    o[2] = perm8(d, b, 0x05040100u);
+    o[3] = perm8(d, b, 0x07060302u);
+}
+// bit 2^M k + c of the 2^M words o = bit k of A[c]: bit transposes within
+// bytes, then bytes
+GF2T_HD void class_merge(u32 (&A)[8], u32 (&o)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) bit_swap<4>(A[i], A[i + 4], 0x0F0F0F0Fu);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (!(i & 2)) bit_swap<2>(A[i], A[i + 2], 0x33333333u);
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) bit_swap<1>(A[i], A[i + 1], 0x55555555u);
+    u32 lo[4], hi[4];
+    byte_transpose(A[0], A[1], A[2], A[3], lo);
+    byte_transpose(A[4], A[5], A[6], A[7], hi);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        o[2 * i] = lo[i];
+        o[2 * i + 1] = hi[i];
+    }
+}
+GF2T_HD void class_merge(u32 (&A)[4], u32 (&o)[4]) {
+    bit_swap<2>(A[0], A[2], 0x33333333u);
+    bit_swap<2>(A[1], A[3], 0x33333333u);
+    bit_swap<1>(A[0], A[1], 0x55555555u);
+    bit_swap<1>(A[2], A[3], 0x55555555u);
+    bit_swap<4>(A[0], A[1], 0x0F0F0F0Fu);
+    bit_swap<4>(A[2], A[3], 0x0F0F0F0Fu);
+    byte_transpose(A[0], A[2], A[1], A[3], o);
+}
+GF2T_HD void class_merge(u32 (&A)[2], u32 (&o)[2]) {
+    const u64 t = interleave32(A[0], A[1]);
+    o[0] = (u32)t;
+    o[1] = (u32)(t >> 32);
+}
+
 // ------------------------------------------------ sieve number theory
 // x mod M for M = 2^d - 1 (Mersenne folding)
 GF2T_HD u64 mod_mersenne(u64 x, int d, u64 M) {

@@ -52,10 +52,11 @@ struct SqDesc {
     const u64 *in;
     u64 *out;
     SqConst c;
-    int odd;            // first launch: one squaring, where the others take two
+    int m;              // squarings of the first launch; the others take two or three
     int back;           // the chain ends in the scratch buffer (in, of an odd launch)
     const int *order;   // block -> tile (-1 idle), or null for identity
     Sq2Chain h;         // two-squaring tile layout
+    PowOrder p;         // order of the ranges of F^8 windows
 };
 
 // output pair i (one 16-byte store when both words exist)
@@ -228,7 +229,7 @@ k_square2_fold_batch(
     const SqDesc d = desc[blockIdx.y];
     square2_unit<NT, W12>(d.in, d.out, d.c, d.h, blockIdx.x, gw);
 }
-// The same, and the residues marked odd advance by one squaring: the first
+// The same, and the residues with m = 1 advance by one squaring: the first
 // launch of a batch whose chains differ in length, so that every later one
 // advances all of its chains by two.
 template <bool NT, bool W12>
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square12_fold_batch(
         const SqDesc *__restrict__ desc) {
     __shared__ __align__(16) u64 gw[SQ2_WINS * SQ2_LEN];
     const SqDesc d = desc[blockIdx.y];
-    if (!d.odd) {
+    if (d.m == 2) {
         square2_unit<NT, W12>(d.in, d.out, d.c, d.h, blockIdx.x, gw);
         return;
     }
@@ -245,6 +246,220 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square12_fold_batch(
         square_fold_pair_fast<W12>(d.in, d.c, i, o0, o1);
         store_pair<NT>(d.out, d.c.nw, i, o0, o1);
     }
+}
+
+// ---- F^8 by direct windows: three squarings per launch
+// A block takes a range of units of 2^M words of 32 output bits.  Its list
+// of windows (pow_window: about 31 for M = 3, their shifts uniform) is
+// sorted by class and dealt to its waves in equal parts -- by class the
+// fullest wave had 7 of them -- and what a wave has of a class is XORed
+// into that class's words in LDS, which are then merged.  A tile of the
+// two-squaring kernel takes twice its arithmetic (165 VALU operations a
+// pair of words against 90, and copies in LDS) but reads each word about
+// once, where this reads it about four times, from the caches while they
+// hold the launch's residues: three squarings take 4.2 us where one launch
+// is all latency (756839 bits; two took 9), 14 us for one full-size residue
+// (two: 16), 92 us for 8 (two: 74) and 800 us for 64 (two: 480; these
+// exceed the 256 MiB cache).  So launches of up to PW_MOST ranges, 8
+// full-size residues, take this kernel.
+constexpr int PW_T = 512, PW_LIST = 128;
+template <int M, int U>
+constexpr u32 pw_units() { return 64u * U * (8 >> M); }
+// LDS word of unit x of a class, a range having `units`: with four units
+// per lane, by their place in the four and padded, so that neither the
+// lanes' XORs nor the merge's reads meet in a bank
+template <int U>
+__device__ __forceinline__ u32 pw_word(u32 x) {
+    return U == 4 ? (x >> 8) * 320 + (x & 3) * 80 + ((x & 255) >> 2) : x;
+}
+template <int M, int U>
+constexpr u32 pw_class_words() { return U == 4 ? pw_units<M, U>() / 256 * 320 : pw_units<M, U>(); }
+template <int M, int U>
+__device__ __forceinline__ void power_range(const u64 *__restrict__ in, u64 *__restrict__ out,
+                                            const SqConst &c, u32 blk, u32 *lds) {
+    typedef u32 v2u __attribute__((ext_vector_type(2), aligned(4)));
+    typedef u32 v4u __attribute__((ext_vector_type(4)));
+    typedef u32 v4a __attribute__((ext_vector_type(4), aligned(4)));
+    static_assert(U == 1 || U == 4, "units per lane");
+    constexpr int NC = 1 << M;
+    constexpr u32 UB = pw_units<M, U>(), UC = pw_class_words<M, U>();
+    const u32 nd = 2 * (u32)c.nw, i0 = blk * UB;
+    if ((u64)i0 * NC >= nd) return;   // whole block
+    u32 *acc = lds, *lk = lds + UC * NC, *li = lk + PW_LIST;
+    int *lo = (int *)(li + PW_LIST), *hi = lo + PW_LIST;
+    u32 *cnt = (u32 *)(hi + PW_LIST);   // [class], [8 + class]: whole, masked
+    if (threadIdx.x < 16) cnt[threadIdx.x] = 0;
+    for (u32 x = threadIdx.x; x < UC * NC; x += PW_T) acc[x] = 0;
+    __syncthreads();
+    PowWin w;
+    u32 rank = 0;
+    const bool got = threadIdx.x < 256 &&
+                     pow_window<M>(c.r, c.s, threadIdx.x >> 4, threadIdx.x & 15, (u64)i0 * NC * 32,
+                                   ((u64)i0 + UB) * NC * 32, w);
+    if (got) rank = atomicAdd(&cnt[w.cls + (w.part ? 8 : 0)], 1u);
+    __syncthreads();
+    u32 before = 0, nfull = 0, npart = 0;   // before this thread's pair in the list
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const u32 f = cnt[k], m = cnt[8 + k];
+        nfull += f;
+        npart += m;
+        if (got && k < (int)w.cls) before += w.part ? m : f;
+    }
+    if (got) {
+        const u32 at = before + rank + (w.part ? nfull : 0);
+        lk[at] = w.kw;
+        li[at] = w.sh | w.cls << 8;
+        lo[at] = w.lo;
+        hi[at] = w.hi;
+    }
+    __syncthreads();
+    nfull = uniform32(nfull);
+    npart = uniform32(npart);
+    const int lane = threadIdx.x & 63, wave = uniform32(threadIdx.x >> 6);
+    const u32 part = wave & (NC - 1), group = wave >> M;   // the waves of a group share its units
+    const u32 ub = i0 + group * 64 * U;
+    const GF2T_GLOBAL u32 *f = (const GF2T_GLOBAL u32 *)in;
+    u32 A[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) A[u] = 0;
+    u32 cls = 0;
+    auto flush = [&](u32 next) {   // A into class cls's words
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            atomicXor(&acc[cls * UC + pw_word<U>(group * 64 * U + (U == 4 ? 4 * lane + u : lane))], A[u]);
+            A[u] = 0;
+        }
+        cls = next;
+    };
+    const u32 f0 = part * nfull / NC, n = (part + 1) * nfull / NC - f0;   // at most 16
+    const u32 ek = lane < (int)n ? lk[f0 + lane] : 0, es = lane < (int)n ? li[f0 + lane] : 0;
+    constexpr int Q = 4;   // windows whose loads are in flight together
+    for (u32 q = 0; q < n; q += Q) {
+        v4u x[Q];
+        u32 y[Q], e[Q];
+#pragma unroll
+        for (int t = 0; t < Q; t++) {
+            if (q + t >= n) break;
+            e[t] = __builtin_amdgcn_readlane(es, (int)(q + t));
+            const GF2T_GLOBAL u32 *p = f + (size_t)ub + (u32)__builtin_amdgcn_readlane(ek, (int)(q + t));
+            // (of a window that ends on a word, the word after may lie
+            // past the residue)
+            const bool over = (e[t] & 31) != 0;
+            y[t] = 0;
+            if (U == 4) {
+                x[t] = *(const GF2T_GLOBAL v4a *)(p + 4 * lane);
+                if (over && lane == 63) y[t] = p[256];
+            } else if (over) {
+                const v2u v = *(const GF2T_GLOBAL v2u *)(p + lane);
+                x[t].x = v.x;
+                y[t] = v.y;
+            } else {
+                x[t].x = p[lane];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < Q; t++) {
+            if (q + t >= n) break;
+            if (e[t] >> 8 != cls) flush(e[t] >> 8);
+            const u32 sh = e[t] & 31;
+            const v4u v = x[t];
+            if (U == 4) {
+                // the next lane's first word (wave_shl:1), lane 63's its own y
+                const u32 nx = (u32)__builtin_amdgcn_update_dpp((int)y[t], (int)v.x, 0x130, 0xf, 0xf, false);
+                A[0] ^= alignbit(v.y, v.x, sh);
+                A[1 % U] ^= alignbit(v.z, v.y, sh);
+                A[2 % U] ^= alignbit(v.w, v.z, sh);
+                A[3 % U] ^= alignbit(nx, v.w, sh);
+            } else {
+                A[0] ^= alignbit(y[t], v.x, sh);
+            }
+        }
+    }
+    const u32 p0 = nfull + part * npart / NC, p1 = nfull + (part + 1) * npart / NC;
+    for (u32 at = p0; at < p1; at++) {
+        const u32 kw = uniform32(lk[at]), e = uniform32(li[at]);
+        const int l = (int)uniform32((u32)lo[at]), h = (int)uniform32((u32)hi[at]);
+        if (e >> 8 != cls) flush(e >> 8);
+        u32 x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const u64 j = (u64)ub + (U == 4 ? 4 * lane + u : lane) + kw;
+            x[u] = f[j < nd ? (u32)j : nd - 1];
+            y[u] = f[j + 1 < nd ? (u32)j + 1 : nd - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const u32 i = ub - i0 + (U == 4 ? 4 * lane + u : lane);
+            A[u] ^= alignbit(y[u], x[u], e & 31) & pow_mask<M>((int)(i * NC * 32), cls, l, h);
+        }
+    }
+    flush(0);
+    __syncthreads();
+    for (u32 k = wave * 64; k < UB; k += PW_T) {
+        const u32 i = i0 + k + lane;
+        u32 a[NC], o[NC];
+#pragma unroll
+        for (int t = 0; t < NC; t++) a[t] = acc[t * UC + pw_word<U>(k + lane)];
+        class_merge(a, o);
+        u32 *dst = (u32 *)out + (size_t)i * NC;
+        if ((u64)(i + 1) * NC <= nd) {
+            if (M == 1) {
+                *(u64 *)dst = ((u64)o[1] << 32) | o[0];
+            } else {
+#pragma unroll
+                for (int t = 0; t < NC; t += 4) *(v4u *)(dst + t) = v4u{o[t], o[t + 1], o[t + 2], o[t + 3]};
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < NC; t++)
+                if ((u64)i * NC + t < nd) dst[t] = o[t];
+        }
+    }
+}
+// ranges (2^16 output bits) of a launch
+inline u64 pow_ranges(size_t nw) { return (nw + 1023) / 1024; }
+constexpr u64 PW_FULL = 128;    // from which a block takes a range (U = 4)
+constexpr u64 PW_MOST = 16640;  // above which two squarings per launch are faster
+// ranges of a residue from which they run in columns: it exceeds the 4 MiB
+// L2 of an XCD (12 squarings of 8 residues of 44,497,001 bits: 174 us in
+// plain order, 150 us in columns; of 64 of 3,021,377 bits: 249 and 274)
+constexpr u64 PW_COLS = 512;
+template <int U>
+constexpr size_t pw_lds() { return (8 * pw_class_words<3, U>() + 4 * PW_LIST + 16) * 4; }
+
+// 2^m-th powers of a residue
+template <bool COLS>
+__device__ __forceinline__ u32 pw_block(const PowOrder &p) {
+    return COLS ? pow_range(p, blockIdx.x) : blockIdx.x;
+}
+template <int U, bool COLS>
+__global__ __launch_bounds__(PW_T) void k_power(const u64 *__restrict__ in, u64 *__restrict__ out,
+                                                const SqConst c, const PowOrder p, int m) {
+    __shared__ __align__(16) u32 lds[pw_lds<U>() / 4];
+    const u32 x = pw_block<COLS>(p);
+    if (m == 3) power_range<3, U>(in, out, c, x, lds);
+    else if (m == 2) power_range<2, U>(in, out, c, x, lds);
+    else power_range<1, U>(in, out, c, x, lds);
+}
+// of the residues of a batch (blockIdx.y); the first launch advances each
+// by d.m squarings, so that every later one takes three of all
+template <int U, bool COLS, bool FIRST>
+__global__ __launch_bounds__(PW_T) void k_power_batch(const SqDesc *__restrict__ desc) {
+    __shared__ __align__(16) u32 lds[pw_lds<U>() / 4];
+    const SqDesc &d = desc[blockIdx.y];
+    const u32 x = pw_block<COLS>(d.p);
+    if (!FIRST || d.m == 3) power_range<3, U>(d.in, d.out, d.c, x, lds);
+    else if (d.m == 2) power_range<2, U>(d.in, d.out, d.c, x, lds);
+    else power_range<1, U>(d.in, d.out, d.c, x, lds);
+}
+// blocks for 2^m-th powers of nw words
+template <int U, bool COLS>
+u64 power_blocks(size_t nw, int m, const PowOrder &p) {
+    static_assert(pw_units<3, 4>() * 256 == 65536 && pw_units<1, 4>() * 64 == 65536, "PowOrder");
+    if (COLS) return 8 * (u64)p.per;
+    const u64 units = (2 * (u64)nw + (1u << m) - 1) >> m, ub = 64ull * U * (8 >> m);
+    return (units + ub - 1) / ub;
 }
 
 // the values that ended in the scratch buffers, back to the residues: of
@@ -263,16 +478,20 @@ __global__ __launch_bounds__(SQ_THREADS) void k_batch_back(const SqDesc *__restr
 }
 
 // ---- whole chains of small residues
-// A residue whose two copies fit in LDS (r up to about 640,000) runs its
-// whole chain in one block, one squaring per barrier, between the copies:
-// no launch and no memory traffic per step.  Bounded by the issue of one
+// A residue whose two copies fit in LDS (r up to 655,232) runs its whole
+// chain in one block, one squaring per barrier, between the copies: no
+// launch and no memory traffic per step.  Bounded by the issue of one
 // CU and the barrier: 0.85 us per squaring at 132049 bits and 2.2 us at
 // 640,000, where by launches two squarings took 9.5 us, all of it latency
-// (40 squarings: 191 -> 34 us, and 183 -> 90 us).  512 residues of 600,000
+// (40 squarings: 191 -> 34 us, and 183 -> 90 us; by launches of three
+// squarings 57 us at any such size, so a few residues above 262,144 bits go
+// that way).  512 residues of 600,000
 // bits are 512 blocks, one per CU at a time: 276 us against 1085 us.
 constexpr int CH_THREADS = 1024;
 constexpr size_t CH_LDS = 160 * 1024;
 constexpr size_t CH_WORDS = CH_LDS / 16 - 2;   // words of a residue, at most
+constexpr size_t CH_ONE = 4096;                // of a few residues, at most
+constexpr int CH_FEW = 16;
 constexpr u64 CH_STEPS = 4096;                 // squarings per launch, at most
 struct ChainDesc {
     u64 *res;
@@ -553,21 +772,31 @@ extern "C" int gf2t_square_fold_steps(uint64_t *dres, uint64_t *dtmp, uint64_t r
     SqConst c = sq_const(r, s);
     size_t nw = c.nw;
     hipStream_t st = (hipStream_t)stream;
-    if (nw <= CH_WORDS && sq_fuse() && steps > 2)
+    if (nw <= CH_ONE && sq_fuse() && steps > 3)
         return run_chains(nullptr, ChainDesc{dres, c, steps}, 1, nw, steps, st);
     u64 *a = dres, *b = dtmp;
     const bool fuse = sq_fuse(), w12 = sq_w12_ok(r);
-    const u64 tiles = sq2_tiles(sq2_chain(c));
+    const PowOrder po = pow_order(nw, s);
+    const u64 ranges = pow_ranges(nw), tiles = sq2_tiles(sq2_chain(c));
     const Sq2Chain h2 = sq2_chain(c, sq2_chain_len(tiles));
     const dim3 g2((unsigned)sq2_units(h2)), g1(blocks_for((nw + 1) / 2, SQ_THREADS));
     u64 launches = 0;
     for (u64 k = 0; k < steps; launches++) {
-        if (fuse && steps - k >= 2) {
+        if (fuse && ranges > PW_MOST && steps - k >= 2) {
             if (w12)
                 hipLaunchKernelGGL(k_square2_fold<true>, g2, dim3(SQ_THREADS), 0, st, a, b, c, h2);
             else
                 hipLaunchKernelGGL(k_square2_fold<false>, g2, dim3(SQ_THREADS), 0, st, a, b, c, h2);
             k += 2;
+        } else if (fuse && ranges <= PW_MOST) {
+            const int m = (steps - k) % 3 ? (int)((steps - k) % 3) : 3;
+            auto launch = [&](auto kernel, u64 blocks) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(PW_T), 0, st, a, b, c, po, m);
+            };
+            if (ranges >= PW_COLS) launch(k_power<4, true>, power_blocks<4, true>(nw, m, po));
+            else if (ranges >= PW_FULL) launch(k_power<4, false>, power_blocks<4, false>(nw, m, po));
+            else launch(k_power<1, false>, power_blocks<1, false>(nw, m, po));
+            k += m;
         } else {
             if (w12)
                 hipLaunchKernelGGL(k_square_fold<true>, g1, dim3(SQ_THREADS), 0, st, a, b, c);
@@ -619,6 +848,13 @@ void launch_batch2(unsigned gx, unsigned active, const SqDesc *tab, hipStream_t 
     else
         hipLaunchKernelGGL((k_square2_fold_batch<false, W12>), dim3(gx, active),
                            dim3(SQ_THREADS), 0, st, tab);
+}
+template <int U, bool COLS>
+void launch_power(bool first, unsigned gx, unsigned active, const SqDesc *tab, hipStream_t st) {
+    if (first)
+        hipLaunchKernelGGL((k_power_batch<U, COLS, true>), dim3(gx, active), dim3(PW_T), 0, st, tab);
+    else
+        hipLaunchKernelGGL((k_power_batch<U, COLS, false>), dim3(gx, active), dim3(PW_T), 0, st, tab);
 }
 }  // namespace
 
@@ -783,10 +1019,13 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     std::vector<ChainDesc> chains;
     size_t chain_nw = 0;
     u64 chain_steps = 0;
+    int larger = 0;   // residues that fit in LDS, above CH_ONE
+    for (int i = 0; i < n; i++)
+        larger += steps[i] && words_of(r[i]) > CH_ONE && words_of(r[i]) <= CH_WORDS;
     for (int i = 0; i < n; i++) {
         const size_t nw = words_of(r[i]);
         if (!steps[i]) continue;
-        if (fuse && nw <= CH_WORDS) {
+        if (fuse && nw <= (larger < CH_FEW ? CH_ONE : CH_WORDS)) {
             chains.push_back(ChainDesc{dres[i], sq_const(r[i], s[i]), steps[i]});
             chain_nw = std::max(chain_nw, nw);
             chain_steps = std::max<u64>(chain_steps, steps[i]);
@@ -794,7 +1033,17 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
             ord.push_back(i);
         }
     }
-    auto nlaunch = [&](int i) { return fuse ? (steps[i] + 1) / 2 : steps[i]; };
+    u64 ranges = 0, most_ranges = 0, tiles2 = 0;   // of all residues by launches; of the largest
+    if (fuse)
+        for (int i : ord) {
+            const SqConst c = sq_const(r[i], s[i]);
+            ranges += pow_ranges(c.nw);
+            most_ranges = std::max(most_ranges, pow_ranges(c.nw));
+            tiles2 += sq2_tiles(sq2_chain(c));
+        }
+    // squarings per launch, and a chain's launches
+    const u64 per = !fuse ? 1 : ranges > PW_MOST ? 2 : 3;
+    auto nlaunch = [&](int i) { return (steps[i] + per - 1) / per; };
     std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return nlaunch(a) > nlaunch(b); });
     std::stable_sort(chains.begin(), chains.end(), [](const ChainDesc &a, const ChainDesc &b) {
         return a.steps * a.c.nw > b.steps * b.c.nw;
@@ -807,7 +1056,6 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     std::vector<int> otab;
     size_t gx = 0, gx1 = 0;
     const u64 tile_pairs = (u64)SQ_THREADS * ppt;
-    u64 tiles2 = 0;
     for (int k = 0; k < nl; k++) {
         SqConst c = sq_const(r[ord[k]], s[ord[k]]);
         u64 T = ((c.nw + 1) / 2 + tile_pairs - 1) / tile_pairs;
@@ -819,7 +1067,6 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
         } else {
             gx = std::max<size_t>(gx, T);
         }
-        if (fuse) tiles2 += sq2_tiles(sq2_chain(c));
     }
     if (g_batch.cap < need) {
         if (g_batch.d) (void)hipFree(g_batch.d);
@@ -850,23 +1097,32 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     }
     std::vector<unsigned char> h(need);
     SqDesc *hd = (SqDesc *)h.data();
+    const int shape = most_ranges >= PW_COLS ? 2 : ranges >= PW_FULL ? 1 : 0;
     const u32 len2 = sq2_chain_len(tiles2);
-    u64 gx2 = 0;       // work units of the residue with the most
+    u64 gx2 = 0;            // work units of the residue with the most
+    u64 gx3 = 0, gxf = 0;   // its blocks of F^8 windows, and in the first launch
+    bool odd = false;       // some chain's first launch takes fewer than the others
     bool w12 = true;   // 12-byte window loads: no r of the launches a multiple of 64
-    bool odd = false;  // some chain has an odd number of squarings
     bool back = false; // some chain ends in dtmp
     for (int k = 0; k < nl; k++) {
         const int i = ord[k];
         const SqConst c = sq_const(r[i], s[i]);
         const int *ot = order ? g_batch.ord + (size_t)k * gx : nullptr;
         const Sq2Chain h2 = sq2_chain(c, len2);
-        const int od = fuse ? (int)(steps[i] & 1) : 0;
+        const PowOrder po = pow_order(c.nw, c.s);
+        const int m = (int)(steps[i] % per ? steps[i] % per : per);
         const int bk = (int)(nlaunch(i) & 1);
-        new (hd + k) SqDesc{dres[i], dtmp[i], c, od, bk, ot, h2};        // even launches
-        new (hd + nl + k) SqDesc{dtmp[i], dres[i], c, 0, bk, ot, h2};    // odd launches
-        odd = odd || od;
+        new (hd + k) SqDesc{dres[i], dtmp[i], c, m, bk, ot, h2, po};        // even launches
+        new (hd + nl + k) SqDesc{dtmp[i], dres[i], c, (int)per, bk, ot, h2, po};   // odd launches
+        odd = odd || m != (int)per;
         back = back || bk;
         gx2 = std::max(gx2, sq2_units(h2));
+        auto blocks = [&](int m) {
+            return shape == 2 ? power_blocks<4, true>(c.nw, m, po)
+                   : shape == 1 ? power_blocks<4, false>(c.nw, m, po) : power_blocks<1, false>(c.nw, m, po);
+        };
+        gx3 = std::max(gx3, blocks(3));
+        gxf = std::max(gxf, blocks(m));
         w12 = w12 && sq_w12_ok(r[i]);
         gx1 = std::max<size_t>(gx1, ((c.nw + 1) / 2 + SQ_THREADS - 1) / SQ_THREADS);
     }
@@ -878,19 +1134,25 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
                             (unsigned)chains.size(), chain_nw, chain_steps, st);
         if (rc) return rc;
     }
-    // Every launch advances all live chains together, by two squarings (by
-    // one in the first launch where a chain's length is odd); a chain's
-    // value is in dtmp after an odd number of launches.
+    // Every launch advances all live chains together, by `per` squarings (in
+    // the first by what a chain's length leaves over); a chain's value is in
+    // dtmp after an odd number of launches.
     const SqDesc *dd = (const SqDesc *)g_batch.d;
     int active = nl;
     for (u64 l = 0; active > 0; l++) {
         const SqDesc *tab = dd + ((l & 1) ? nl : 0);
-        if (fuse && l == 0 && odd) {
+        const bool first = l == 0 && odd;
+        if (per == 3) {
+            const unsigned g = (unsigned)(first ? gxf : gx3);
+            if (shape == 2) launch_power<4, true>(first, g, active, tab, st);
+            else if (shape == 1) launch_power<4, false>(first, g, active, tab, st);
+            else launch_power<1, false>(first, g, active, tab, st);
+        } else if (per == 2 && first) {
             // enough blocks for the one-squaring residues' pairs in a few rounds
             const unsigned g = (unsigned)std::max<u64>(gx2, (gx1 + 7) / 8);
             if (w12) launch_batch12<true>(g, active, tab, st);
             else launch_batch12<false>(g, active, tab, st);
-        } else if (fuse) {
+        } else if (per == 2) {
             if (w12) launch_batch2<true>((unsigned)gx2, active, tab, st);
             else launch_batch2<false>((unsigned)gx2, active, tab, st);
         } else {

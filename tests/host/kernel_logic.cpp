@@ -1,6 +1,7 @@
 // Host build of the kernels' arithmetic (mersenne_trinomial_amd/csrc/
 // gf2t_arith.hpp) for CPU checks against the oracle.  Test code only.
 #include "gf2t_arith.hpp"
+#include <algorithm>
 #include <stdlib.h>
 #include <vector>
 
@@ -45,6 +46,41 @@ struct CheckedArray {
     }
 };
 
+// F^(2^M) by direct windows, as k_power takes it: ranges of `units` units,
+// every pair (a, b); -> the most windows of one range
+template <int M>
+static int power_windows(const u64 *in, u64 *out, u64 r, u64 s, u32 units) {
+    const u32 nd = 2 * (u32)((r + 63) / 64), per = 1u << M;   // dwords; dwords per unit
+    const u32 *f = (const u32 *)in;
+    u32 *o = (u32 *)out;
+    const u64 nunits = (nd + per - 1) / per;
+    int most = 0;
+    for (u64 i0 = 0; i0 < nunits; i0 += units) {
+        std::vector<PowWin> ws;
+        for (u32 t = 0; t < 256; t++) {
+            PowWin w;
+            if (pow_window<M>(r, s, t >> 4, t & 15, (i0 << M) * 32, ((i0 + units) << M) * 32, w)) ws.push_back(w);
+        }
+        most = std::max(most, (int)ws.size());
+        for (u64 i = i0; i < i0 + units && i < nunits; i++) {
+            u32 A[1 << M] = {}, q[1 << M];
+            for (const PowWin &w : ws) {
+                const u64 at = i + w.kw;
+                if (!w.part) {
+                    if (at + (w.sh ? 1 : 0) >= nd) return -1;   // a read past the residue
+                    A[w.cls] ^= w.sh ? alignbit(f[at + 1], f[at], w.sh) : f[at];
+                } else {
+                    const u32 x = f[std::min<u64>(at, nd - 1)], y = f[std::min<u64>(at + 1, nd - 1)];
+                    A[w.cls] ^= alignbit(y, x, w.sh) &
+                                pow_mask<M>((int)((i - i0) << M) * 32, w.cls, w.lo, w.hi);
+                }
+            }
+            class_merge(A, q);
+            for (u32 k = 0; k < per && per * i + k < nd; k++) o[per * i + k] = q[k];
+        }
+    }
+    return most;
+}
 extern "C" {
 void kl_square_fold(const u64 *in, u64 *out, u64 r, u64 s) {
     size_t nw = (size_t)((r + 63) >> 6);
@@ -276,5 +312,20 @@ u64 kl_count_classes_all(int d) {
     u64 n = 0;
     for (u64 j = 1; j < M; j++) n += is_lyndon32((u32)j, d, M);
     return n;
+}
+// how often block x of a residue's launch takes range i: 1 for all, or 0
+int kl_power_order(u64 nw, u64 s) {
+    const PowOrder o = pow_order(nw, s);
+    std::vector<int> hit(o.n, 0);
+    for (u32 x = 0; x < 8 * o.per; x++) {
+        const u32 i = pow_range(o, x);
+        if (i < o.n) hit[i]++;
+    }
+    return std::all_of(hit.begin(), hit.end(), [](int h) { return h == 1; });
+}
+int kl_power_windows(int M, const u64 *in, u64 *out, u64 r, u64 s, u32 units) {
+    return M == 1 ? power_windows<1>(in, out, r, s, units)
+           : M == 2 ? power_windows<2>(in, out, r, s, units)
+                    : power_windows<3>(in, out, r, s, units);
 }
 }

@@ -53,10 +53,13 @@ BATCHES = [
     [(756839, 1, 1), (756839, 378419, 2), (756839, 3000, 3), (700032, 350015, 0)],
     [(3021377, 1510688, 7), (859433, 288477, 6), (132049, 2, 9), (44497, 22248, 5000)],
     [(859433, 7, 2), (859433, 429716, 2)],
+    [(6972593, 3486296, 4), (65536 * 16, 65535, 3), (65536 * 16 + 64, 65537, 5), (859433, 1, 7)],
+    [(37156667, 18578333, 4), (859433, 3, 2)],
+    [(37156667, 5, 3), (43112609, 9000000, 5), (3021377, 77, 1)],
 ]
 
 
-@pytest.mark.parametrize("cases", BATCHES, ids=["edge", "odd", "mixed", "even"])
+@pytest.mark.parametrize("cases", BATCHES, ids=["edge", "odd", "mixed", "even", "ranges", "columns", "columns-odd"])
 def test_batch_edges(eng, cases):
     from mersenne_trinomial_amd._capi import check, lib
     from mersenne_trinomial_amd.device import DeviceBuffer
@@ -73,3 +76,33 @@ def test_batch_edges(eng, cases):
                                      kk.ctypes.data_as(P), n, None))
     for (r, s, k), a, b in zip(cases, ins, bufs):
         assert np.array_equal(b.download(O.words(r)), O.square_fold_steps(a, r, s, k)), (r, s, k)
+
+
+@pytest.mark.parametrize("s", [1, 8, 65536, 11000000, 18578333])
+@pytest.mark.parametrize("k", [1, 2, 4])
+def test_windows_in_columns(eng, s, k):
+    r = 37156667   # more than an XCD's L2: ranges in columns s apart
+    a = rand_res(np.random.default_rng(s), r)
+    assert np.array_equal(eng.square_fold(a, r, s, k), O.square_fold_steps(a, r, s, k))
+
+
+def test_two_squaring_launches_above_the_windows_bound(eng):
+    """A batch of more ranges than F^8 windows are used for: two squarings
+    per launch, one in the first for the odd chain."""
+    from mersenne_trinomial_amd._capi import check, lib
+    from mersenne_trinomial_amd.device import DeviceBuffer
+    r, n = 136279841, 9
+    rng = np.random.default_rng(9)
+    svals = [474, 1, 68139920, 40000001, 3, 65536, 30000000, 1000003, 9]
+    steps = [4, 3, 2, 1, 4, 5, 3, 0, 2]
+    ins = [rand_res(rng, r) for _ in range(n)]
+    bufs = [DeviceBuffer.from_array(a) for a in ins]
+    tmps = [DeviceBuffer.words(O.words(r)) for _ in range(n)]
+    P = C.POINTER(C.c_uint64)
+    rr, ss, kk = (np.array(v, dtype=np.uint64) for v in ([r] * n, svals, steps))
+    check(lib.gf2t_square_fold_batch((C.c_void_p * n)(*[b.ptr for b in bufs]),
+                                     (C.c_void_p * n)(*[t.ptr for t in tmps]),
+                                     rr.ctypes.data_as(P), ss.ctypes.data_as(P),
+                                     kk.ctypes.data_as(P), n, None))
+    for s, k, a, b in zip(svals, steps, ins, bufs):
+        assert np.array_equal(b.download(O.words(r)), O.square_fold_steps(a, r, s, k)), (s, k)

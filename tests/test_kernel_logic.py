@@ -493,3 +493,32 @@ def test_two_squaring_units_cover_every_pair(kl, length):
         tiles = np.zeros(1, np.uint64)
         kl.kl_square2_units_len(r, s, length, tiles.ctypes.data_as(P))
         assert tiles[0] > 0
+
+
+def test_power_windows(kl):
+    """F^2, F^4 and F^8 by direct windows against repeated squaring: every s
+    of small r, s at its ends and r at word edges; no read past the residue
+    outside the masked windows, and at most 128 windows a range."""
+    kl.kl_power_windows.restype = C.c_int
+    kl.kl_power_windows.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint32]
+    cases = [(r, s) for r in (3, 5, 31, 64, 65, 129) for s in range(1, (r + 1) // 2)]
+    cases += [(r, s) for r in (1000, 1024, 4096, 9689, 20011, 65536)
+              for s in (1, 2, 31, 64, 177, r // 7, r // 4, r // 3, 2 * r // 5, (r - 1) // 2 - 1, (r - 1) // 2)]
+    rng = np.random.default_rng(8)
+    for r, s in cases:
+        a = rng.integers(0, 2**64, O.words(r), dtype=np.uint64)
+        if r & 63:
+            a[-1] &= np.uint64((1 << (r & 63)) - 1)
+        for M in (1, 2, 3):
+            want = O.square_fold_steps(a, r, s, M)
+            for units in (1, 2, 7, 64):
+                got = np.zeros_like(a)
+                most = kl.kl_power_windows(M, a.ctypes.data, got.ctypes.data, r, s, units)
+                assert 0 < most <= 128 and np.array_equal(got, want), (r, s, M, units, most)
+
+
+def test_power_order_takes_every_range_once(kl):
+    kl.kl_power_order.argtypes = [C.c_uint64, C.c_uint64]
+    for r in (3, 65536, 65537, 3021377, 44497001, 136279841):
+        for s in sorted({1, 65535, 65536, 65537, 200000, r // 9, r // 5, r // 3, (r - 1) // 2} & set(range(1, (r + 1) // 2))):
+            assert kl.kl_power_order(O.words(r), s), (r, s)
