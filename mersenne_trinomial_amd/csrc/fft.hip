@@ -517,12 +517,49 @@ __global__ __launch_bounds__(256) void k_low(u64 *__restrict__ f_, u64 f_stride,
 // are XORed up as they come and the classes merged once at the end, so a
 // 32 x 32 product costs 16 multiply-adds and 12 XORs.  Block (t, c) writes
 // the part of the outputs [SC_OUT t, SC_OUT (t + 1)) that comes from the
-// i in [SC_IN c, SC_IN (c + 1)) to part[c][.].
-constexpr u32 SC_OUT = 128, SC_IN = 128;
+// i in [SC_IN c, SC_IN (c + 1)) to part[c][.].  Bounded by the multiply-adds
+// (a quarter of the VALU rate).
+//
+// From SC_KARA chunks on, two levels of Karatsuba's splitting by the
+// chunks' index: of even, odd and all (summed) chunks, and of each again,
+// nine products of a quarter of the length stand for sixteen.  The operand
+// sums are formed as the chunks are read, and the products are put together
+// by k_school_kara.  Two 132049-bit operands: 24 us, of which one product
+// of all chunks took 27; 262,144 bits: 48 and 72 us; below SC_KARA chunks
+// the nine are no faster (60,000 bits: 12.6 and 12.2 us).
+constexpr u32 SC_OUT = 128, SC_IN = 128, SC_KARA = 1024;
 struct SchoolShape {
-    u32 na, nb;         // chunks, na <= nb
+    u32 na, nb;         // chunks (of a quarter where split), na <= nb
     u32 nout, nparts;   // na + nb - 1 outputs; parts
+    u32 np;             // products: 1, or 9 where split
 };
+// of product p, whether the chunks r mod 4 are in its operands: p / 3 picks
+// by the index's bit 0 (0: even, 1: odd, 2: both), p % 3 by its bit 1
+GF2T_HD bool kara_picks(u32 p, u32 r) {
+    const u32 u = p / 3, v = p % 3;
+    return (u == 2 || u == (r & 1)) && (v == 2 || v == (r >> 1));
+}
+// chunk i of an operand of product p, 0 below the first and past the last;
+// its loads do not wait for one another
+GF2T_DEV u32 school_chunk(const Operand &o, u32 np, u32 p, int i) {
+    if (np == 1) return i >= 0 ? chunk(o, (u64)i) : 0;
+    u32 w[4], v = 0;
+    const u32 n = (u32)o.n;
+#pragma unroll
+    for (u32 r = 0; r < 4; r++) {
+        const u32 k = i >= 0 ? 4 * (u32)i + r : 0;
+        w[r] = o.src[k < n ? k : n - 1];
+    }
+#pragma unroll
+    for (u32 r = 0; r < 4; r++) {
+        const u32 k = 4 * (u32)i + r;
+        u32 x = w[r];
+        x &= k == n - 1 ? o.mask : ~0u;
+        x ^= k == 0 ? o.xor0 : 0u;
+        v ^= i >= 0 && k < n && kara_picks(p, r) ? x : 0u;
+    }
+    return v;
+}
 // the parts that reach output tile t: c in [first, last]
 GF2T_HD u32 school_first(const SchoolShape &s, u32 t) {
     const u32 k0 = t * SC_OUT;
@@ -533,21 +570,19 @@ GF2T_HD u32 school_last(const SchoolShape &s, u32 t) { return t < s.nparts - 1 ?
 __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, int swap,
                                                 const SchoolShape s, u64 *__restrict__ part,
                                                 u64 part_stride) {
-    static_assert(SC_OUT == 128 && SC_IN == 128, "two outputs per lane, 32 values per wave");
+    static_assert(SC_OUT == 128 && SC_IN == 128, "two outputs per lane, 32 values per wave, a b per thread");
     __shared__ u32 bs[SC_OUT + SC_IN];
     __shared__ u64 sum[4][SC_OUT];
-    const u32 t = blockIdx.x, c = blockIdx.y, y = blockIdx.z;
+    const u32 c = blockIdx.y, t = c + blockIdx.x, y = blockIdx.z / s.np, p = blockIdx.z % s.np;
     if (c < school_first(s, t) || c > school_last(s, t)) return;   // whole block
     const Operand oa = operand(ops, swap ? y + b_op : y), ob = operand(ops, swap ? y : y + b_op);
     const int k0 = (int)(t * SC_OUT), i0 = (int)(c * SC_IN);
     const int j0 = k0 - i0 - (int)(SC_IN - 1);   // b index of bs[0]
-    for (u32 x = threadIdx.x; x < SC_OUT + SC_IN - 1; x += 256) {
-        const int j = j0 + (int)x;
-        bs[x] = j >= 0 ? chunk(ob, (u64)j) : 0;
-    }
     const u32 wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int iw = i0 + (int)wave * 32;
-    const u32 av = lane < 32 ? chunk(oa, (u64)iw + lane) : 0;
+    const u32 bv = school_chunk(ob, s.np, p, j0 + (int)threadIdx.x);
+    const u32 av = lane < 32 ? school_chunk(oa, s.np, p, iw + (int)lane) : 0;
+    bs[threadIdx.x] = bv;
     __syncthreads();
     const u32 m0 = 0x11111111u;
     u64 acc[2][4] = {};
@@ -574,7 +609,7 @@ __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, in
     __syncthreads();
     const u32 k = (u32)k0 + threadIdx.x;
     if (threadIdx.x < SC_OUT && k < s.nout)
-        part[(u64)y * part_stride + (u64)c * s.nout + k] =
+        part[(u64)y * part_stride + (u64)(p * s.nparts + c) * s.nout + k] =
             xor3(sum[0][threadIdx.x], sum[1][threadIdx.x], sum[2][threadIdx.x]) ^
             sum[3][threadIdx.x];
 }
@@ -620,6 +655,45 @@ __global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ 
     auto coef = [&](u32 x) { return xor3(sum[0][x], sum[1][x], sum[2][x]) ^ sum[3][x]; };
     const u32 x = threadIdx.x;
     if (x < SP_WORDS && w0 + x < owords)
+        out[w0 + x] = coef(2 * x + 1) ^ (coef(2 * x + 2) << 32) ^ (coef(2 * x) >> 32);
+}
+// The same from nine products: those of the index's bit 1 first,
+//   e_2h = E_h + O_(h-1), e_(2h+1) = S_h + E_h + O_h
+// (E, O, S: the products of even, odd and all), then those of bit 0 in the
+// same way.  A block adds up the parts of the 17 coefficients of each that
+// its words need.
+__global__ __launch_bounds__(256) void k_school_kara(const u64 *__restrict__ part,
+                                                     const SchoolShape s, u64 *__restrict__ out,
+                                                     size_t owords) {
+    constexpr int H = 2 * SP_WORDS / 4 + 1;
+    __shared__ u64 sum[9][H];
+    const u32 w0 = blockIdx.x * SP_WORDS;
+    if (threadIdx.x < 9 * H) {
+        const u32 p = threadIdx.x / H, x = threadIdx.x % H;
+        const u32 h = w0 / 2 + x - 1;   // coefficient; none before the first
+        u64 v = 0;
+        if (w0 / 2 + x >= 1 && h < s.nout) {
+            const u32 t = h / SC_OUT, hi = school_last(s, t);
+#pragma unroll 4
+            for (u32 c = school_first(s, t); c <= hi; c++)
+                v ^= part[(u64)(p * s.nparts + c) * s.nout + h];
+        }
+        sum[p][x] = v;
+    }
+    __syncthreads();
+    // coefficient w0 - 1 + l of the product of bit 0's choice u
+    auto half = [&](int u, int l) -> u64 {
+        const u64(*q)[H] = &sum[3 * u];
+        if (l & 1) return q[0][(l + 1) / 2] ^ q[1][(l - 1) / 2];
+        return xor3(q[2][l / 2], q[0][l / 2], q[1][l / 2]);
+    };
+    // coefficient 2 w0 - 1 + x
+    auto coef = [&](int x) -> u64 {
+        if (x & 1) return half(0, (x + 1) / 2) ^ half(1, (x - 1) / 2);
+        return xor3(half(2, x / 2), half(0, x / 2), half(1, x / 2));
+    };
+    const int x = (int)threadIdx.x;
+    if (x < (int)SP_WORDS && w0 + x < owords)
         out[w0 + x] = coef(2 * x + 1) ^ (coef(2 * x + 2) << 32) ^ (coef(2 * x) >> 32);
 }
 // the product folded mod x^r + x^s + 1 (s from svec where there is a batch)
@@ -1069,33 +1143,45 @@ extern "C" size_t gf2t_mul_out_words(uint64_t abits, uint64_t bbits) {
 
 namespace {
 // Products of at most SC_WORK chunk pairs (and SC_OUTS outputs) are formed
-// without a transform (k_school).
-constexpr u64 SC_WORK = (u64)64 << 20, SC_OUTS = 65536;
+// without a transform (k_school): 320,000 bits squared take 67 us so and
+// 70 us by transforms, which at 360,000 are ahead, 71 to 78 us.
+constexpr u64 SC_WORK = (u64)100 << 20, SC_OUTS = 65536;
 constexpr u32 SC_FOLD_PARTS = 4;
 bool school(u64 ca, u64 cb, u64 nbatch = 1) {
     return ca && cb && ca + cb <= SC_OUTS && nbatch * ca * cb <= SC_WORK;
 }
 SchoolShape school_shape(u64 ca, u64 cb) {
     SchoolShape s;
-    s.na = (u32)std::min(ca, cb);
-    s.nb = (u32)std::max(ca, cb);
+    u64 na = std::min(ca, cb), nb = std::max(ca, cb);
+    s.np = na >= SC_KARA ? 9 : 1;
+    if (s.np == 9) {
+        na = (na + 3) / 4;
+        nb = (nb + 3) / 4;
+    }
+    s.na = (u32)na;
+    s.nb = (u32)nb;
     s.nout = s.na + s.nb - 1;
     s.nparts = (s.na + SC_IN - 1) / SC_IN;
     return s;
 }
 // words of the parts, as a bound that grows with either operand also past
 // the products that use it (a workspace for larger operands serves smaller
-// ones): parts * outputs <= (na / SC_IN + 1)(na + nb) with na nb <= SC_WORK
+// ones): parts * outputs <= (na / SC_IN + 1)(na + nb), or a quarter of each
+// nine times, with na nb <= SC_WORK
 size_t school_words(u64 ca, u64 cb) {
     const u64 na = std::min(ca, cb), nb = std::max(ca, cb);
-    const u64 most = 2 * SC_WORK / SC_IN + SC_OUTS;
+    const u64 most = 9 * ((2 * SC_WORK + 4 * SC_OUTS) / (4 * SC_IN) + SC_OUTS + 4) / 4;
     const u64 a = std::min<u64>(na, SC_OUTS), b = std::min<u64>(nb, SC_OUTS);
-    return (size_t)std::min(most, (a / SC_IN + 1) * (a + b));
+    if (a < SC_KARA) return (size_t)std::min(most, (a / SC_IN + 1) * (a + b));
+    return (size_t)std::min(most, 9 * (a / (4 * SC_IN) + 1) * ((a + b) / 4 + 1));
 }
 int run_school(const Operands &ops, u32 b_op, bool swap, const SchoolShape &s, u64 *part,
                u64 part_stride, unsigned nbatch, hipStream_t st) {
-    hipLaunchKernelGGL(k_school, dim3((s.nout + SC_OUT - 1) / SC_OUT, s.nparts, nbatch), dim3(256),
-                       0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride);
+    // part c reaches the outputs [SC_IN c, SC_IN (c + 1) + nb - 1): the tiles
+    // from c on, as tiles and parts are of one length
+    static_assert(SC_IN == SC_OUT, "tiles of a part");
+    hipLaunchKernelGGL(k_school, dim3((SC_IN - 1 + s.nb + SC_OUT - 1) / SC_OUT, s.nparts, nbatch * s.np),
+                       dim3(256), 0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride);
     GF2T_CHECK_LAUNCH("k_school");
     return GF2T_OK;
 }
@@ -1239,8 +1325,9 @@ int mul_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 *dprod, voi
         const SchoolShape s = school_shape(ca, cb);
         rc = run_school(two, 1, ca > cb, s, (u64 *)dwork, 0, 1, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_school_product, dim3((unsigned)((ow + SP_WORDS - 1) / SP_WORDS)),
-                           dim3(256), 0, st, (const u64 *)dwork, s, dprod, ow);
+        hipLaunchKernelGGL(s.np == 1 ? k_school_product : k_school_kara,
+                           dim3((unsigned)((ow + SP_WORDS - 1) / SP_WORDS)), dim3(256), 0, st,
+                           (const u64 *)dwork, s, dprod, ow);
         GF2T_CHECK_LAUNCH("k_school_product");
         return GF2T_OK;
     }
@@ -1303,7 +1390,7 @@ int mulmod_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 r, u64 s
     const u64 ca = (abits + 31) >> 5, cb = (bbits + 31) >> 5;
     if (school(ca, cb)) {
         const SchoolShape sh = school_shape(ca, cb);
-        if (sh.nparts <= SC_FOLD_PARTS) {   // few parts to add up: folded from them directly
+        if (sh.np == 1 && sh.nparts <= SC_FOLD_PARTS) {   // few parts to add up: folded from them directly
             Operands two{};
             two.op[0] = operand_of(da, abits, nullptr);
             two.op[1] = operand_of(db, bbits, nullptr);
@@ -1467,23 +1554,28 @@ GF2T_DEV int find_seg(const PairSeg *__restrict__ sg, int np, u64 i) {
 }
 
 // phase 0: overlap-add FA into prod; 1: fold prod into out.  total = sum
-// of the pairs' element counts for the phase.
-__global__ void k_pairs_grouped(const PairSeg *__restrict__ sg, int np, u64 total, int phase,
-                                u64 r) {
-    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (; i < total; i += stride) {
-        const PairSeg &S = sg[find_seg(sg, np, i)];
-        const u64 k = i - S.start;
-        if (phase == 0) {
-            const u64 c = 2 * k;
-            u64 v = 0;
-            if (c < S.nch) v ^= S.fa[c];
-            if (c + 1 < S.nch) v ^= S.fa[c + 1] << 32;
-            if (k && c - 1 < S.nch) v ^= S.fa[c - 1] >> 32;
-            S.prod[k] = v;
-        } else {
-            S.out[k] = fold_word(S.prod, S.pw, S.L, r, S.s, k);
+// of the pairs' element counts for the phase.  A block takes PG_RUN
+// consecutive elements and finds the first one's pair once; the pairs after
+// it are few (a search per element took two thirds of the time).
+constexpr u32 PG_RUN = 2048;
+__global__ __launch_bounds__(256) void k_pairs_grouped(const PairSeg *__restrict__ sg, int np,
+                                                       u64 total, int phase, u64 r) {
+    const u64 i0 = (u64)blockIdx.x * PG_RUN, i1 = i0 + PG_RUN < total ? i0 + PG_RUN : total;
+    for (int p = find_seg(sg, np, i0); p < np && sg[p].start < i1; p++) {
+        const PairSeg S = sg[p];
+        const u64 end = p + 1 < np && sg[p + 1].start < i1 ? sg[p + 1].start : i1;
+        for (u64 i = (S.start > i0 ? S.start : i0) + threadIdx.x; i < end; i += 256) {
+            const u64 k = i - S.start;
+            if (phase == 0) {
+                const u64 c = 2 * k;
+                u64 v = 0;
+                if (c < S.nch) v ^= S.fa[c];
+                if (c + 1 < S.nch) v ^= S.fa[c + 1] << 32;
+                if (k && c - 1 < S.nch) v ^= S.fa[c - 1] >> 32;
+                S.prod[k] = v;
+            } else {
+                S.out[k] = fold_word(S.prod, S.pw, S.L, r, S.s, k);
+            }
         }
     }
 }
@@ -1635,8 +1727,8 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     }
     for (int ph = 0; ph < 2; ph++)
         hipLaunchKernelGGL(k_pairs_grouped,
-                           dim3((unsigned)std::min<u64>((total[ph] + 255) / 256, 65536)),
-                           dim3(256), 0, st, dseg + ph * np, np, total[ph], ph, (u64)r);
+                           dim3((unsigned)((total[ph] + PG_RUN - 1) / PG_RUN)), dim3(256), 0, st,
+                           dseg + ph * np, np, total[ph], ph, (u64)r);
     GF2T_CHECK_LAUNCH("gf2t_mulmod_batch");
     return GF2T_OK;
 }
@@ -1695,7 +1787,7 @@ extern "C" int gf2t_mulmod_slab(const uint64_t *da, size_t apitch, const uint64_
     ops.op[1] = operand_of(db, r, (u32 *)prod + 2 * nw + 2, b_add_x ? 2u : 0u);
     const u64 ow = 2 * nw;   // product of two r-bit operands: 2r-1 bits
     const SchoolShape sh = school_shape(ca, ca);
-    if (sh.nparts <= 2 && school(ca, ca, (u64)n)) {   // the parts fit the transforms' space
+    if (sh.np == 1 && sh.nparts <= 2 && school(ca, ca, (u64)n)) {   // the parts fit the transforms' space
         rc = run_school(ops, (u32)n, false, sh, FA, 2 * N, (unsigned)n, st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_school_fold, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st,
