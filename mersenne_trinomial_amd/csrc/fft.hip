@@ -1238,24 +1238,29 @@ struct WrapArg {
     int noff;
     u32 off[15];    // 2^k for the proper bit-subsets k of mp
 };
-// from 2^WRAP_MIN_M points (of all products of a batch together) up: below
-// that both products are a chain of launches as long as their work, and
-// one chain is faster than two (a 2^16-point product: 83 us, wrapped 221)
-constexpr int WRAP_MIN_M = 20;
+// Wrapping pays where the 2^mp points it saves (of all products of a batch
+// together) take longer than the top product: its chain of launches, as
+// long as WRAP_CHAIN points, and a fourth more than its own points, as a
+// smaller transform uses the chip less.  2^20 + 2^19 points take 328 us and
+// 2^21 take 284, 2^21 + 2^20 486 and 2^22 443, but 2^22 + 2^21 738 and 2^23
+// 745, and 2^23 + 2^18 940 against 1420.
+constexpr u64 WRAP_CHAIN = 900000;
 Wrap wrap_for(u64 ca, u64 cb, u64 nbatch = 1) {
     Wrap w;
     const u64 N = ca + cb - 1;
     const int m = fft_m_for(N);
-    if (m < 12 || m - 1 > FFT_MAX_M || (nbatch << (m - 1)) >> WRAP_MIN_M == 0) return w;
+    if (m < 12 || m - 1 > FFT_MAX_M) return w;
     const int mp = m - 1;
     const u64 n = (u64)1 << mp;
     if (N <= n) return w;
     const u64 e = N - n;
     if (e > n / 4 || ca > n || cb > n || e >= ca || e >= cb) return w;
+    const int ms = fft_m_for(2 * e - 1);
+    if (nbatch * n < WRAP_CHAIN + 5 * (nbatch << ms) / 4) return w;
     w.on = true;
     w.mp = mp;
     w.e = e;
-    w.ms = fft_m_for(2 * e - 1);
+    w.ms = ms;
     return w;
 }
 WrapArg wrap_arg(const Wrap &w) {
