@@ -428,11 +428,15 @@ __global__ __launch_bounds__(CL_T) void k_class_log(const SieveDeg *__restrict__
 // Per class: Zech logarithm (one random gather), the progression
 // s == s0 (mod n), and -- only for the few classes whose progression
 // reaches s <= smax -- a queue entry, so that k_mark's minimal polynomials
-// run on dense waves.  A thread takes ZN_PER classes: their lookups are
+// run on dense waves.  A thread takes PER classes (8, or 2 where there are
+// too few to fill the chip and a launch is as long as one thread: 24 us
+// and 13 for the degrees up to 20, but 38 and 80 at degree 25): their
+// lookups are
 // overlapped, and one Euclid inverts the product of their units (three
 // products a class; a gcd, an inverse and two divisions a class before).
 // Bounded by the VALU and the gathers: 3.3 ms at d = 32, 5.6 before.
-constexpr int ZN_T = 256, ZN_PER = 8;
+constexpr int ZN_T = 256;
+template <int ZN_PER>
 __global__ __launch_bounds__(ZN_T) void k_zech(const SieveDeg *__restrict__ degs) {
     const SieveDeg &P = degs[blockIdx.y];
     __shared__ u32 norm[2048], zech[ZN_T * ZN_PER];
@@ -557,6 +561,7 @@ __global__ __launch_bounds__(MK_T) void k_mark(const SieveDeg *__restrict__ degs
 struct PeriodArgs {
     const u32 *pat[PAT_MAX_D + 1];   // marks of degree d
     u32 *tab[PAT_MAX_D / 2];         // tables of the degrees first..hi
+    u32 divs[PAT_MAX_D / 2];         // bit d: d divides that degree, and was marked
     int lo, hi, first;
 };
 __global__ void k_fold_periods(PeriodArgs A) {
@@ -564,8 +569,8 @@ __global__ void k_fold_periods(PeriodArgs A) {
     const u32 M = (1u << e) - 1;
     for (u32 x = blockIdx.x * blockDim.x + threadIdx.x; x < M; x += gridDim.x * blockDim.x) {
         u32 key = ~0u;
-        for (int d = A.lo; d <= e; d++) {
-            if (e % d) continue;
+        for (u32 w = A.divs[blockIdx.y]; w; w &= w - 1) {
+            const int d = __builtin_ctz(w);
             const u32 m = A.pat[d][x % ((1u << d) - 1)];
             if (m != ~0u) {
                 key = (u32)d << 21 | m;
@@ -579,12 +584,14 @@ __global__ void k_fold_periods(PeriodArgs A) {
 // degrees lo..hi.  One pass over best[], with its loads and stores, and
 // the tables' loads, in order: 0.7 ms for 68,139,920 s and degrees 2..20,
 // where marking the progressions one by one took 4.6.
-constexpr int SW_T = 256, SW_PER = 16;
-__global__ __launch_bounds__(SW_T) void k_sweep(PeriodArgs A, u64 smax,
+// A thread takes `per` values of s, fewer where they would leave the chip
+// idle (66,024 values: 36 us at 16 each, 5.6 us at one).
+constexpr int SW_T = 256;
+__global__ __launch_bounds__(SW_T) void k_sweep(PeriodArgs A, u64 smax, u32 per,
                                                 unsigned long long *__restrict__ best) {
     constexpr int N = PAT_MAX_D / 2;
     __shared__ u32 base[N];   // the block's first s modulo each period
-    const u64 s0 = 1 + (u64)blockIdx.x * SW_T * SW_PER;
+    const u64 s0 = 1 + (u64)blockIdx.x * SW_T * per;
     if (threadIdx.x < N && A.first + (int)threadIdx.x <= A.hi)
         base[threadIdx.x] = (u32)(s0 % (((u64)1 << (A.first + threadIdx.x)) - 1));
     __syncthreads();
@@ -592,7 +599,7 @@ __global__ __launch_bounds__(SW_T) void k_sweep(PeriodArgs A, u64 smax,
 #pragma unroll
     for (int i = 0; i < N; i++)
         if (A.first + i <= A.hi) x[i] = (base[i] + threadIdx.x) % ((1u << (A.first + i)) - 1);
-    for (int it = 0; it < SW_PER; it++) {
+    for (u32 it = 0; it < per; it++) {
         const u64 s = s0 + it * SW_T + threadIdx.x;
         if (s > smax) return;
         u32 key = ~0u;
@@ -1127,7 +1134,7 @@ int sieve_narrow(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
         const int e = group_end(d, dmax);
         const unsigned ny = (unsigned)(e - d + 1);
         const SieveDeg *g = ddegs + d;
-        u64 bc = 0, bl = 0, bz = 0, bm = 0;
+        u64 bc = 0, bl = 0, bm = 0, most = 0;
         PeriodArgs A{};
         A.lo = d;
         A.hi = d - 1;
@@ -1135,7 +1142,7 @@ int sieve_narrow(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
             const SieveDeg &P = degs[k];
             bc = std::max<u64>(bc, (P.nprefix + P.per - 1) / P.per);
             bl = std::max<u64>(bl, (P.ncls + CL_T * CL_PER - 1) / (CL_T * CL_PER));
-            bz = std::max<u64>(bz, (P.ncls + ZN_T * ZN_PER - 1) / (ZN_T * ZN_PER));
+            most = std::max(most, P.ncls);
             bm = std::max<u64>(bm, (P.ncls + MK_T - 1) / MK_T);
             if (P.pat) {
                 A.pat[k] = P.pat;
@@ -1146,14 +1153,20 @@ int sieve_narrow(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
         hipLaunchKernelGGL(k_classes, dim3((unsigned)bc, ny), dim3(CS_T), 0, 0, g);
         hipLaunchKernelGGL(k_class_log, dim3((unsigned)std::min<u64>(bl, 4096), ny), dim3(CL_T), 0, 0, g);
         if (stats) GF2T_HIP(hipEventRecord(ev[d][1], 0));
-        hipLaunchKernelGGL(k_zech, dim3((unsigned)std::min<u64>(bz, 4096), ny), dim3(ZN_T), 0, 0, g);
+        const u64 zper = most >= ((u64)8 * ZN_T * 64) ? 8 : 2;
+        const dim3 gz((unsigned)std::min<u64>((most + ZN_T * zper - 1) / (ZN_T * zper), 4096), ny);
+        if (zper == 8) hipLaunchKernelGGL(k_zech<8>, gz, dim3(ZN_T), 0, 0, g);
+        else hipLaunchKernelGGL(k_zech<2>, gz, dim3(ZN_T), 0, 0, g);
         const bool periods = A.hi >= A.lo;
         if (periods) {
             const u64 n = (u64)2 << A.hi;
             hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, pats, n, ~0u);
             A.first = std::max(A.lo, A.hi / 2 + 1);
-            for (int k = A.first; k <= A.hi; k++)
+            for (int k = A.first; k <= A.hi; k++) {
+                for (int j = A.lo; j <= k; j++)
+                    if (k % j == 0) A.divs[k - A.first] |= 1u << j;
                 A.tab[k - A.first] = pats + ((size_t)2 << PAT_MAX_D) + ((size_t)1 << k);
+            }
         }
         hipLaunchKernelGGL(k_mark, dim3((unsigned)std::min<u64>(bm, 2048), ny), dim3(MK_T), 0, 0, g,
                            (unsigned long long *)dbest, heavy, hcount);
@@ -1163,8 +1176,9 @@ int sieve_narrow(uint64_t r, int dmin, int dmax, uint64_t smax, uint64_t *dbest,
             hipLaunchKernelGGL(k_fold_periods,
                                dim3((unsigned)std::max<u64>(1, n), (unsigned)(A.hi - A.first + 1)),
                                dim3(256), 0, 0, A);
-            hipLaunchKernelGGL(k_sweep, dim3((unsigned)((smax + SW_T * SW_PER - 1) / (SW_T * SW_PER))),
-                               dim3(SW_T), 0, 0, A, smax, (unsigned long long *)dbest);
+            const u32 per = (u32)std::min<u64>(16, smax / (SW_T * 2048) + 1);
+            hipLaunchKernelGGL(k_sweep, dim3((unsigned)((smax + SW_T * per - 1) / (SW_T * per))),
+                               dim3(SW_T), 0, 0, A, smax, per, (unsigned long long *)dbest);
         }
         hipLaunchKernelGGL(k_mark_heavy, dim3(64, 16), dim3(256), 0, 0, heavy, hcount, 0u, smax,
                            (unsigned long long *)dbest);
