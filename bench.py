@@ -506,7 +506,7 @@ def c4_measure(args):
 
 def mode_fft24(args):
     """Only 2^24-point transforms (forward then inverse, --steps times each)
-    on one buffer, for rocprofv3 counter runs of k_fft_pass at the size of
+    on one buffer, for rocprofv3 counter runs of the transform kernels at the size of
     the full 136279841-bit product."""
     from mersenne_trinomial_amd import device
     from mersenne_trinomial_amd._capi import check, lib

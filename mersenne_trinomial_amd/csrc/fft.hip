@@ -12,8 +12,8 @@
 //   2. butterflies, level L on index bit L: e1 = g + W(t) h, e2 = e1 + h
 //      with W(t) = sum_{bits k of t} b[k+1], t = index >> (L+1); forward
 //      L = m-1 down to 0.  Elements are in the tower basis of cantor.hpp,
-//      two to a unit of four words; a thread holds 16 units and takes four
-//      levels between two exchanges through LDS, so a pass over memory
+//      two to a unit of four words; a thread holds four units and takes two
+//      levels between two exchanges through LDS; a pass over memory
 //      takes eight levels.
 #include "gf2t_internal.hpp"
 #include "cantor.hpp"
