@@ -1172,8 +1172,10 @@ size_t school_words(u64 ca, u64 cb) {
     const u64 na = std::min(ca, cb), nb = std::max(ca, cb);
     const u64 most = 9 * ((2 * SC_WORK + 4 * SC_OUTS) / (4 * SC_IN) + SC_OUTS + 4) / 4;
     const u64 a = std::min<u64>(na, SC_OUTS), b = std::min<u64>(nb, SC_OUTS);
-    if (a < SC_KARA) return (size_t)std::min(most, (a / SC_IN + 1) * (a + b));
-    return (size_t)std::min(most, 9 * (a / (4 * SC_IN) + 1) * ((a + b) / 4 + 1));
+    const u64 one = std::min<u64>(a, SC_KARA - 1);
+    u64 words = (one / SC_IN + 1) * (one + b);
+    if (a >= SC_KARA) words = std::max(words, 9 * (a / (4 * SC_IN) + 1) * ((a + b) / 4 + 1));
+    return (size_t)std::min(most, words);
 }
 int run_school(const Operands &ops, u32 b_op, bool swap, const SchoolShape &s, u64 *part,
                u64 part_stride, unsigned nbatch, hipStream_t st) {
