@@ -352,7 +352,7 @@ def mode_squaring(args):
                                      kk.ctypes.data_as(P64), n, None))
     e1.record()
     ms = e0.elapsed_ms(e1)
-    kernel, launches, per = chain_launches(args.chain_steps, args.sq_fuse != 0)
+    kernel, launches, per = chain_launches(args.chain_steps, args.sq_fuse != 0, args.residues)
     launch_ms = ms / (args.chain_steps / per)
     gbs = 16 * nw * n / (launch_ms * 1e-3) / 1e9
     print(json.dumps({"mode": "squaring", "residues": n, "steps": args.chain_steps,
@@ -786,10 +786,13 @@ def apply_tuning(args):
         check(lib.gf2t_tune(key.encode(), int(val)))
 
 
-def chain_launches(steps: int, fuse: bool):
-    """(kernel, launches) of a chain of `steps` squarings: with fusion,
-    steps // 2 two-squaring launches (plus one single launch for an odd
-    count, which the roofline line does not cover)."""
+def chain_launches(steps: int, fuse: bool, residues: int):
+    """(kernel, launches, squarings per launch) of a batch's chain of `steps`
+    squarings at r = 136279841: with fusion, three per launch up to eight
+    residues, else steps // 2 two-squaring launches (a launch that takes what
+    is left over is not covered by the roofline line)."""
+    if fuse and residues <= 8 and steps >= 3:
+        return "k_power_batch", steps // 3, 3
     if fuse and steps >= 2:
         return "k_square2_fold_batch", steps // 2, 2
     return "k_square_fold_batch", steps, 1
@@ -909,7 +912,7 @@ def main():
         print("c4: 64 seeded Cantor products, folded", file=sys.stderr, flush=True)
         c4 = c4_measure(args)
 
-    kernel, launches, per = chain_launches(args.chain_steps, args.sq_fuse != 0)
+    kernel, launches, per = chain_launches(args.chain_steps, args.sq_fuse != 0, args.residues)
     launch_ms = float(np.mean(chain_ms)) / (args.chain_steps / per)
     bytes_per_launch = 16 * nw * n
     achieved = bytes_per_launch / (launch_ms * 1e-3) / 1e9

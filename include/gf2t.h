@@ -116,9 +116,10 @@ int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dtmp,
 
 /* Tuning knobs of the kernels (the autotuner's handle; the reference
  * reads GF2C_* environment variables, src/gf2_cantor_cuda.h:24-61):
- *   "sq_fuse"  1 = two squarings per launch in gf2t_square_fold_steps and
- *              gf2t_square_fold_batch while every live chain has two
- *              steps left; 0 = one squaring per launch
+ *   "sq_fuse"  1 = several squarings per launch in gf2t_square_fold_steps
+ *              and gf2t_square_fold_batch (whole chains of small residues,
+ *              three up to about eight full-size ones, two above); 0 = one
+ *              squaring per launch
  *   "sq_ppt"   output pairs per lane in the one-step batched squaring
  *              (1, 2, 4)
  *   "sq_order" 1 = XCD-aware tile order in the one-step batched squaring,
