@@ -697,6 +697,27 @@ inline std::vector<BfPass> bf_passes(int m, int tile) {
     }
     return v;
 }
+// The transforms of a launch are the rows of its grid, which has at most
+// 65535, and a product has two of them: the pairs of one chain of launches.
+constexpr unsigned MAX_PAIRS = 32767;
+// the pairs j of a batch by their transform size m[j] (0: no transform), the
+// largest first, at most MAX_PAIRS to a group
+struct SizeGroup {
+    int m;
+    std::vector<int> pairs;
+};
+inline std::vector<SizeGroup> size_groups(const std::vector<int> &m) {
+    std::vector<SizeGroup> v;
+    for (int k = 31; k >= 1; k--) {
+        const size_t first = v.size();
+        for (int j = 0; j < (int)m.size(); j++) {
+            if (m[j] != k) continue;
+            if (v.size() == first || v.back().pairs.size() == MAX_PAIRS) v.push_back(SizeGroup{k, {}});
+            v.back().pairs.push_back(j);
+        }
+    }
+    return v;
+}
 // the subfield class of a window's twiddles: 8, 16 or 32
 inline int bf_class(const BfPass &P) {
     const int bits = P.m - 1 - P.a;

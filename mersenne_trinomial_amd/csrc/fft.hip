@@ -1006,6 +1006,7 @@ int run_inverse(const gf2t_fft_plan &pl, u64 *f, u64 stride, unsigned nbatch, bo
 // most 2^k chunks): transforms at f + y stride and g + y stride, the
 // product's coefficients modulo the vanishing polynomial of the 2^m
 // points at f + y stride, in the polynomial basis.  g - f = nbatch stride.
+// nbatch is at most MAX_PAIRS.
 int run_product(const gf2t_fft_plan &pl, u64 *f, u64 stride, const Operands &ops, int k,
                 unsigned nbatch, hipStream_t st) {
     int in;
@@ -1589,13 +1590,8 @@ __global__ __launch_bounds__(256) void k_pairs_grouped(const PairSeg *__restrict
 
 // Pairs of one transform size run as one chain of launches, their A
 // transforms side by side and the B transforms behind them.
-struct BatchGroup {
-    int m;
-    std::vector<int> pairs;
-    size_t f;   // word offset of the group's transforms
-};
 struct BatchLayout {
-    std::vector<BatchGroup> groups;
+    std::vector<cantor_host::SizeGroup> groups;
     std::vector<size_t> fa, prod;   // word offsets of each pair's A transform and product
     std::vector<int> m;
     size_t desc_off = 0, words = 0;
@@ -1608,17 +1604,11 @@ BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
         u64 ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
         L.m.push_back((ca && cb) ? fft_m_for(ca + cb - 1) : 0);
     }
+    L.groups = cantor_host::size_groups(L.m);
     size_t off = 0;
-    for (int m = FFT_MAX_M; m >= 1; m--) {
-        BatchGroup g{m, {}, off};
-        for (int j = 0; j < n; j++)
-            if (L.m[j] == m) {
-                L.fa[j] = off + (g.pairs.size() << m);
-                g.pairs.push_back(j);
-            }
-        if (g.pairs.empty()) continue;
-        off += 2 * g.pairs.size() << m;
-        L.groups.push_back(g);
+    for (const cantor_host::SizeGroup &g : L.groups) {
+        for (size_t i = 0; i < g.pairs.size(); i++) L.fa[g.pairs[i]] = off + (i << g.m);
+        off += 2 * g.pairs.size() << g.m;
     }
     for (int j = 0; j < n; j++) {
         L.prod.push_back(off);
@@ -1668,7 +1658,7 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     u64 *W = (u64 *)dwork;
     // the operands, group by group: the A's, then the B's
     std::vector<Operand> opv;
-    for (const BatchGroup &g : L.groups)
+    for (const cantor_host::SizeGroup &g : L.groups)
         for (int o = 0; o < 2; o++)
             for (int j : g.pairs) {
                 u32 *lch = (u32 *)(W + L.prod[j]);
@@ -1721,14 +1711,14 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     const Operand *dop = (const Operand *)dd;
     const PairSeg *dseg = (const PairSeg *)(dd + ob);
     size_t first = 0;
-    for (const BatchGroup &g : L.groups) {
+    for (const cantor_host::SizeGroup &g : L.groups) {
         const unsigned cnt = (unsigned)g.pairs.size();
         u64 most = 1;
         for (int j : g.pairs)
             most = std::max(most, std::max((abits[j] + 31) >> 5, (bbits[j] + 31) >> 5));
         Operands ops{};
         ops.list = dop + first;
-        rc = run_product(plan_for(g.m), W + g.f, (u64)1 << g.m, ops, log2_ceil(most), cnt, st);
+        rc = run_product(plan_for(g.m), W + L.fa[g.pairs[0]], (u64)1 << g.m, ops, log2_ceil(most), cnt, st);
         if (rc) return rc;
         first += 2 * cnt;
     }
@@ -1804,27 +1794,39 @@ extern "C" int gf2t_mulmod_slab(const uint64_t *da, size_t apitch, const uint64_
     }
     const int k = log2_ceil(ca);
     const Wrap W = wrap_for(ca, ca, (u64)n);
-    if (W.on) {
-        // the wrapped product (see wrap_for): 2^mp-point transforms of both
-        // operands and 2^ms-point transforms of their top e chunks, laid
-        // out inside the 2 N n words an unwrapped product uses
-        const size_t np = (size_t)1 << W.mp, ns = (size_t)1 << W.ms;
-        u64 *TA = FA + 2 * np * n;
-        rc = run_product(plan_for(W.mp), FA, np, ops, k, (unsigned)n, st);
-        if (rc) return rc;
-        // top chunks [ca - e, ca); chunk 0 (where b_add_x adds x) is not among them
-        Operands top = ops;
-        for (int g = 0; g < 2; g++) top.op[g] = operand_range(ops.op[g], ca - W.e, W.e);
-        rc = run_product(plan_for(W.ms), TA, ns, top, log2_ceil(W.e), (unsigned)n, st);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_overlap_add_wrap, dim3((unsigned)((ow + 255) / 256), n), dim3(256), 0,
-                           st, FA, (u64)np, TA + (W.e - 1), (u64)ns, wrap_arg(W),
-                           (size_t)(2 * ca - 1), prod, (size_t)ow, (u64)ppitch);
-    } else {
-        rc = run_product(plan_for(m), FA, N, ops, k, (unsigned)n, st);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), n), dim3(256), 0, st,
-                           FA, (size_t)(2 * ca - 1), prod, (size_t)ow, (u64)N, (u64)ppitch);
+    // MAX_PAIRS residues at a time, through the same transforms' space
+    for (unsigned i0 = 0; i0 < (unsigned)n; i0 += cantor_host::MAX_PAIRS) {
+        const unsigned cnt = std::min((unsigned)n - i0, cantor_host::MAX_PAIRS);
+        Operands part = ops;
+        part.group = cnt;
+        for (int g = 0; g < 2; g++) {
+            part.op[g].src += i0 * ops.sstride[g];
+            part.op[g].lch += i0 * ops.lstride;
+        }
+        u64 *pr = prod + i0 * ppitch;
+        if (W.on) {
+            // the wrapped product (see wrap_for): 2^mp-point transforms of
+            // both operands and 2^ms-point transforms of their top e chunks,
+            // laid out inside the 2 N words a residue of an unwrapped product
+            // uses
+            const size_t np = (size_t)1 << W.mp, ns = (size_t)1 << W.ms;
+            u64 *TA = FA + 2 * np * cnt;
+            rc = run_product(plan_for(W.mp), FA, np, part, k, cnt, st);
+            if (rc) return rc;
+            // top chunks [ca - e, ca); chunk 0 (where b_add_x adds x) is not among them
+            Operands top = part;
+            for (int g = 0; g < 2; g++) top.op[g] = operand_range(part.op[g], ca - W.e, W.e);
+            rc = run_product(plan_for(W.ms), TA, ns, top, log2_ceil(W.e), cnt, st);
+            if (rc) return rc;
+            hipLaunchKernelGGL(k_overlap_add_wrap, dim3((unsigned)((ow + 255) / 256), cnt),
+                               dim3(256), 0, st, FA, (u64)np, TA + (W.e - 1), (u64)ns, wrap_arg(W),
+                               (size_t)(2 * ca - 1), pr, (size_t)ow, (u64)ppitch);
+        } else {
+            rc = run_product(plan_for(m), FA, N, part, k, cnt, st);
+            if (rc) return rc;
+            hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), cnt), dim3(256), 0,
+                               st, FA, (size_t)(2 * ca - 1), pr, (size_t)ow, (u64)N, (u64)ppitch);
+        }
     }
     hipLaunchKernelGGL(k_fold_slab, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st, prod,
                        (size_t)ow, (u64)ppitch, 2 * r - 1, dout, (u64)opitch, nw, r, ds);

@@ -1,0 +1,20 @@
+// The host rules of the products' launches (cantor.hpp), for CPU checks.
+// Test code only.
+#include "cantor.hpp"
+
+extern "C" {
+unsigned pr_max_pairs() { return cantor_host::MAX_PAIRS; }
+// group[j], place[j]: of pair j (-1: none); size[g]: transform size of group g
+int pr_groups(const int *m, int n, int *group, int *place, int *size) {
+    const auto v = cantor_host::size_groups(std::vector<int>(m, m + n));
+    for (int j = 0; j < n; j++) group[j] = place[j] = -1;
+    for (size_t g = 0; g < v.size(); g++) {
+        size[g] = v[g].m;
+        for (size_t i = 0; i < v[g].pairs.size(); i++) {
+            group[v[g].pairs[i]] = (int)g;
+            place[v[g].pairs[i]] = (int)i;
+        }
+    }
+    return (int)v.size();
+}
+}
