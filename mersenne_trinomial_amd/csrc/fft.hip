@@ -1399,6 +1399,10 @@ int mulmod_core(const u64 *da, u64 abits, const u64 *db, u64 bbits, u64 r, u64 s
     if (school(ca, cb)) {
         const SchoolShape sh = school_shape(ca, cb);
         if (sh.np == 1 && sh.nparts <= SC_FOLD_PARTS) {   // few parts to add up: folded from them directly
+            if (r >= (1ULL << 34)) {   // what gf2t_fold, passed by here, takes
+                gf2t::set_error("gf2t_mulmod: need r < 2^34");
+                return GF2T_EINVAL;
+            }
             Operands two{};
             two.op[0] = operand_of(da, abits, nullptr);
             two.op[1] = operand_of(db, bbits, nullptr);
