@@ -421,10 +421,30 @@ __device__ __forceinline__ void power_range(const u64 *__restrict__ in, u64 *__r
 inline u64 pow_ranges(size_t nw) { return (nw + 1023) / 1024; }
 constexpr u64 PW_FULL = 128;    // from which a block takes a range (U = 4)
 constexpr u64 PW_MOST = 16640;  // above which two squarings per launch are faster
+constexpr u64 PW_SHORT = 13500;  // above which they are for some short chains
 // ranges of a residue from which they run in columns: it exceeds the 4 MiB
 // L2 of an XCD (12 squarings of 8 residues of 44,497,001 bits: 174 us in
 // plain order, 150 us in columns; of 64 of 3,021,377 bits: 249 and 274)
 constexpr u64 PW_COLS = 512;
+// Squarings per launch.  Where a launch's residues and their copies no
+// longer fit the 256 MiB cache, one of three squarings takes a fourth longer
+// than one of two, and the copy back after an odd number of launches three
+// fourths of that: chains of up to 4, 7 and 8 squarings are shorter by two
+// (7 squarings of 8 residues of 136,279,841 bits: 274 us, by three 318; of 6
+// residues: 224, by three 220).  two, three: the chains' costs, each times
+// its residue's length.
+inline u64 pow_cost(u64 steps, u64 per) {
+    const u64 l = (steps + per - 1) / per;
+    return (per == 3 ? 5 : 4) * l + 3 * (l & 1);
+}
+inline int pow_per(u64 ranges, u64 two, u64 three) {
+    return ranges > PW_MOST || (ranges > PW_SHORT && two <= three) ? 2 : 3;
+}
+// A single squaring by windows is as long as three where residues come from
+// memory: from PW_COLS ranges on the one-squaring kernels take it
+// (136,279,841 bits: 18.6 us against 20.5, s = 1 15.9 against 20.1;
+// 20,000,003 bits: 8.7 against 7.8).
+inline bool pow_one(u64 ranges) { return ranges < PW_COLS; }
 template <int U>
 constexpr size_t pw_lds() { return (8 * pw_class_words<3, U>() + 4 * PW_LIST + 16) * 4; }
 
@@ -780,16 +800,18 @@ extern "C" int gf2t_square_fold_steps(uint64_t *dres, uint64_t *dtmp, uint64_t r
     const u64 ranges = pow_ranges(nw), tiles = sq2_tiles(sq2_chain(c));
     const Sq2Chain h2 = sq2_chain(c, sq2_chain_len(tiles));
     const dim3 g2((unsigned)sq2_units(h2)), g1(blocks_for((nw + 1) / 2, SQ_THREADS));
+    const int per = !fuse ? 1 : pow_per(ranges, pow_cost(steps, 2), pow_cost(steps, 3));
     u64 launches = 0;
     for (u64 k = 0; k < steps; launches++) {
-        if (fuse && ranges > PW_MOST && steps - k >= 2) {
+        // by three: what is left over first
+        const int m = per == 3 && (steps - k) % 3 ? (int)((steps - k) % 3) : per;
+        if (per == 2 && steps - k >= 2) {
             if (w12)
                 hipLaunchKernelGGL(k_square2_fold<true>, g2, dim3(SQ_THREADS), 0, st, a, b, c, h2);
             else
                 hipLaunchKernelGGL(k_square2_fold<false>, g2, dim3(SQ_THREADS), 0, st, a, b, c, h2);
             k += 2;
-        } else if (fuse && ranges <= PW_MOST) {
-            const int m = (steps - k) % 3 ? (int)((steps - k) % 3) : 3;
+        } else if (per == 3 && (m > 1 || pow_one(ranges))) {
             auto launch = [&](auto kernel, u64 blocks) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(PW_T), 0, st, a, b, c, po, m);
             };
@@ -1034,15 +1056,18 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
         }
     }
     u64 ranges = 0, most_ranges = 0, tiles2 = 0;   // of all residues by launches; of the largest
+    u64 two = 0, three = 0;   // their costs by two and by three squarings a launch
     if (fuse)
         for (int i : ord) {
             const SqConst c = sq_const(r[i], s[i]);
             ranges += pow_ranges(c.nw);
             most_ranges = std::max(most_ranges, pow_ranges(c.nw));
+            two += c.nw * pow_cost(steps[i], 2);
+            three += c.nw * pow_cost(steps[i], 3);
             tiles2 += sq2_tiles(sq2_chain(c));
         }
     // squarings per launch, and a chain's launches
-    const u64 per = !fuse ? 1 : ranges > PW_MOST ? 2 : 3;
+    const u64 per = !fuse ? 1 : (u64)pow_per(ranges, two, three);
     auto nlaunch = [&](int i) { return (steps[i] + per - 1) / per; };
     std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return nlaunch(a) > nlaunch(b); });
     std::stable_sort(chains.begin(), chains.end(), [](const ChainDesc &a, const ChainDesc &b) {
@@ -1102,6 +1127,7 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     u64 gx2 = 0;            // work units of the residue with the most
     u64 gx3 = 0, gxf = 0;   // its blocks of F^8 windows, and in the first launch
     bool odd = false;       // some chain's first launch takes fewer than the others
+    bool ones = per > 1;    // every chain's takes one
     bool w12 = true;   // 12-byte window loads: no r of the launches a multiple of 64
     bool back = false; // some chain ends in dtmp
     for (int k = 0; k < nl; k++) {
@@ -1115,6 +1141,7 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
         new (hd + k) SqDesc{dres[i], dtmp[i], c, m, bk, ot, h2, po};        // even launches
         new (hd + nl + k) SqDesc{dtmp[i], dres[i], c, (int)per, bk, ot, h2, po};   // odd launches
         odd = odd || m != (int)per;
+        ones = ones && m == 1;
         back = back || bk;
         gx2 = std::max(gx2, sq2_units(h2));
         auto blocks = [&](int m) {
@@ -1142,7 +1169,14 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
     for (u64 l = 0; active > 0; l++) {
         const SqDesc *tab = dd + ((l & 1) ? nl : 0);
         const bool first = l == 0 && odd;
-        if (per == 3) {
+        if (per == 1 || (l == 0 && ones && !(per == 3 && pow_one(most_ranges)))) {
+            if (ppt == 4 && w12) launch_batch<4, true>((unsigned)gx, active, tab, st);
+            else if (ppt == 4) launch_batch<4, false>((unsigned)gx, active, tab, st);
+            else if (ppt == 2 && w12) launch_batch<2, true>((unsigned)gx, active, tab, st);
+            else if (ppt == 2) launch_batch<2, false>((unsigned)gx, active, tab, st);
+            else if (w12) launch_batch<1, true>((unsigned)gx, active, tab, st);
+            else launch_batch<1, false>((unsigned)gx, active, tab, st);
+        } else if (per == 3) {
             const unsigned g = (unsigned)(first ? gxf : gx3);
             if (shape == 2) launch_power<4, true>(first, g, active, tab, st);
             else if (shape == 1) launch_power<4, false>(first, g, active, tab, st);
@@ -1152,16 +1186,9 @@ extern "C" int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dt
             const unsigned g = (unsigned)std::max<u64>(gx2, (gx1 + 7) / 8);
             if (w12) launch_batch12<true>(g, active, tab, st);
             else launch_batch12<false>(g, active, tab, st);
-        } else if (per == 2) {
+        } else {
             if (w12) launch_batch2<true>((unsigned)gx2, active, tab, st);
             else launch_batch2<false>((unsigned)gx2, active, tab, st);
-        } else {
-            if (ppt == 4 && w12) launch_batch<4, true>((unsigned)gx, active, tab, st);
-            else if (ppt == 4) launch_batch<4, false>((unsigned)gx, active, tab, st);
-            else if (ppt == 2 && w12) launch_batch<2, true>((unsigned)gx, active, tab, st);
-            else if (ppt == 2) launch_batch<2, false>((unsigned)gx, active, tab, st);
-            else if (w12) launch_batch<1, true>((unsigned)gx, active, tab, st);
-            else launch_batch<1, false>((unsigned)gx, active, tab, st);
         }
         while (active > 0 && nlaunch(ord[active - 1]) == l + 1) active--;
     }
