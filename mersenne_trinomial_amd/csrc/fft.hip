@@ -567,6 +567,11 @@ GF2T_HD u32 school_first(const SchoolShape &s, u32 t) {
 }
 GF2T_HD u32 school_last(const SchoolShape &s, u32 t) { return t < s.nparts - 1 ? t : s.nparts - 1; }
 
+// FULL: a product split in nine, whose tiles are full but for a few (the
+// tests below cost two 320,000-bit operands 2%).  The others skip what a tile has past their operands or outside its triangle:
+// a slab of 4096 residues of 89 bits takes 23 us instead of 130, one of
+// 20,000 of 3071 bits 473 (620 by transforms).
+template <bool FULL>
 __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, int swap,
                                                 const SchoolShape s, u64 *__restrict__ part,
                                                 u64 part_stride) {
@@ -587,18 +592,37 @@ __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, in
     const u32 m0 = 0x11111111u;
     u64 acc[2][4] = {};
     const u32 at = lane + (SC_IN - 1) - wave * 32;   // bs index of output `lane`, i = iw
-#pragma unroll 2
-    for (int i = 0; i < 32; i++) {
+    auto term = [&](int i, int o) {
         const u32 a = __builtin_amdgcn_readlane(av, i);
         const u64 a0 = a & m0, a1 = a & (m0 << 1), a2 = a & (m0 << 2), a3 = a & (m0 << 3);
-#pragma unroll
-        for (int o = 0; o < 2; o++) {
-            const u32 b = bs[at - i + 64 * o];
-            const u64 b0 = b & m0, b1 = b & (m0 << 1), b2 = b & (m0 << 2), b3 = b & (m0 << 3);
-            acc[o][0] = xor3(acc[o][0], a0 * b0 + a1 * b3, a2 * b2) ^ (a3 * b1);
-            acc[o][1] = xor3(acc[o][1], a0 * b1 + a2 * b3, a1 * b0 + a3 * b2);
-            acc[o][2] = xor3(acc[o][2], a0 * b2 + a3 * b3, a1 * b1) ^ (a2 * b0);
-            acc[o][3] = xor3(xor3(acc[o][3], a0 * b3, a1 * b2), a2 * b1, a3 * b0);
+        const u32 b = bs[at - i + 64 * o];
+        const u64 b0 = b & m0, b1 = b & (m0 << 1), b2 = b & (m0 << 2), b3 = b & (m0 << 3);
+        acc[o][0] = xor3(acc[o][0], a0 * b0 + a1 * b3, a2 * b2) ^ (a3 * b1);
+        acc[o][1] = xor3(acc[o][1], a0 * b1 + a2 * b3, a1 * b0 + a3 * b2);
+        acc[o][2] = xor3(acc[o][2], a0 * b2 + a3 * b3, a1 * b1) ^ (a2 * b0);
+        acc[o][3] = xor3(xor3(acc[o][3], a0 * b3, a1 * b2), a2 * b1, a3 * b0);
+    };
+    // the wave's values that there are (an odd last one and a 0), and those
+    // 64 of its outputs that any of them reaches
+    const int i1 = FULL ? 0 : (int)uniform32((u32)iw);
+    const int left = (int)s.na - i1, ni = FULL || left > 32 ? 32 : left;
+    auto reached = [&](int k) { return FULL || (k + 63 >= i1 && k < i1 + ni - 1 + (int)s.nb); };
+    if (reached(k0) && reached(k0 + 64)) {
+        for (int i = 0; i < ni; i += 2) {
+            term(i, 0);
+            term(i, 1);
+            term(i + 1, 0);
+            term(i + 1, 1);
+        }
+    } else if (reached(k0)) {
+        for (int i = 0; i < ni; i += 2) {
+            term(i, 0);
+            term(i + 1, 0);
+        }
+    } else if (reached(k0 + 64)) {
+        for (int i = 0; i < ni; i += 2) {
+            term(i, 1);
+            term(i + 1, 1);
         }
     }
     const u64 q = 0x1111111111111111ULL;
@@ -1148,9 +1172,13 @@ namespace {
 // 70 us by transforms, which at 360,000 are ahead, 71 to 78 us.
 constexpr u64 SC_WORK = (u64)100 << 20, SC_OUTS = 65536;
 constexpr u32 SC_FOLD_PARTS = 4;
-bool school(u64 ca, u64 cb, u64 nbatch = 1) {
-    return ca && cb && ca + cb <= SC_OUTS && nbatch * ca * cb <= SC_WORK;
-}
+// Chunk pairs of a slab of products of two parts up to which it takes no
+// transforms either (4423 bits: 42 us against 51 for 512 residues, 72 against
+// 60 for 1000; 8190 bits: 35 against 48 for 256, 59 against 52 for 512).
+// Products of one part never take any (4090 bits: 15 against 34 us for one
+// residue, 818 against 1000 for 32,767).
+constexpr u64 SC_SLAB = 1 << 24;
+bool school(u64 ca, u64 cb) { return ca && cb && ca + cb <= SC_OUTS && ca * cb <= SC_WORK; }
 SchoolShape school_shape(u64 ca, u64 cb) {
     SchoolShape s;
     u64 na = std::min(ca, cb), nb = std::max(ca, cb);
@@ -1183,7 +1211,8 @@ int run_school(const Operands &ops, u32 b_op, bool swap, const SchoolShape &s, u
     // part c reaches the outputs [SC_IN c, SC_IN (c + 1) + nb - 1): the tiles
     // from c on, as tiles and parts are of one length
     static_assert(SC_IN == SC_OUT, "tiles of a part");
-    hipLaunchKernelGGL(k_school, dim3((SC_IN - 1 + s.nb + SC_OUT - 1) / SC_OUT, s.nparts, nbatch * s.np),
+    hipLaunchKernelGGL(s.np == 1 ? k_school<false> : k_school<true>,
+                       dim3((SC_IN - 1 + s.nb + SC_OUT - 1) / SC_OUT, s.nparts, nbatch * s.np),
                        dim3(256), 0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride);
     GF2T_CHECK_LAUNCH("k_school");
     return GF2T_OK;
@@ -1788,7 +1817,7 @@ extern "C" int gf2t_mulmod_slab(const uint64_t *da, size_t apitch, const uint64_
     ops.op[1] = operand_of(db, r, (u32 *)prod + 2 * nw + 2, b_add_x ? 2u : 0u);
     const u64 ow = 2 * nw;   // product of two r-bit operands: 2r-1 bits
     const SchoolShape sh = school_shape(ca, ca);
-    if (sh.np == 1 && sh.nparts <= 2 && school(ca, ca, (u64)n)) {   // the parts fit the transforms' space
+    if (sh.np == 1 && (sh.nparts == 1 || (sh.nparts == 2 && n * ca * ca <= SC_SLAB))) {   // the parts fit the transforms' space
         rc = run_school(ops, (u32)n, false, sh, FA, 2 * N, (unsigned)n, st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_school_fold, dim3((unsigned)((nw + 255) / 256), n), dim3(256), 0, st,
