@@ -252,11 +252,10 @@ int gf2t_mulmod_noalloc(const uint64_t *da, uint64_t abits, const uint64_t *db,
 /* n products of different sizes, each folded: dout[j] (nw words) =
  * a_j * b_j mod x^r + x^s[j] + 1 (da, db, dout: host arrays of device
  * pointers; abits, bbits, s: host arrays), with dwork of
- * gf2t_mulmod_batch_workspace_bytes(n, abits, bbits) bytes.  Every pair
- * keeps its own transform size, and the batch runs as one set of
- * launches: the i-th pass of every pair's forward (inverse) transforms is
- * one grouped launch, and the pointwise products, overlap-adds and folds
- * are one launch each.  Synchronous with respect to the host only for
+ * gf2t_mulmod_batch_workspace_bytes(n, abits, bbits) bytes.  The
+ * smaller pairs are multiplied without transforms, all in one launch; the
+ * others by size, the pairs of one size sharing a chain of launches; the
+ * overlap-adds and folds of all are one launch each.  Synchronous with respect to the host only for
  * its small descriptor upload.  No reference counterpart: the reference
  * multiplies one pair at a time (gf2x_fft_mul_buf,
  * src/gf2_cantor_engine.h:207-229). */

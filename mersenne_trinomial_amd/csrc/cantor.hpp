@@ -718,6 +718,27 @@ inline std::vector<SizeGroup> size_groups(const std::vector<int> &m) {
     }
     return v;
 }
+// Of a batch of pairs of ca[j] and cb[j] chunks and transform sizes m[j],
+// those formed without transforms, all in one launch: whole sizes, the
+// smallest first, while their chunk pairs are at most DIRECT_PAIRS together.
+// A size by transforms is a chain of launches of its own, 40 to 60 us however
+// few its pairs; 2^25 chunk pairs take about 50 us (eight pairs of 2^15 ..
+// 2^22 bits: 464 us, 586 all by transforms; one pair of 132,049 bits: 46 and
+// 91), and where there are more the transforms' fewer operations count (64
+// pairs of 44,497 bits: 80 us by transforms).
+constexpr size_t DIRECT_PAIRS = (size_t)1 << 25;
+constexpr int DIRECT_MAX_M = 15;   // of at most 2^15 + 1 chunks
+inline std::vector<char> direct_pairs(const std::vector<int> &m, const std::vector<u64> &ca,
+                                      const std::vector<u64> &cb) {
+    u64 work[DIRECT_MAX_M + 1] = {}, all = 0;
+    for (size_t j = 0; j < m.size(); j++)
+        if (m[j] && m[j] <= DIRECT_MAX_M) work[m[j]] += ca[j] * cb[j];
+    int most = 0;
+    while (most < DIRECT_MAX_M && all + work[most + 1] <= DIRECT_PAIRS) all += work[++most];
+    std::vector<char> v(m.size());
+    for (size_t j = 0; j < m.size(); j++) v[j] = m[j] && m[j] <= most;
+    return v;
+}
 // the subfield class of a window's twiddles: 8, 16 or 32
 inline int bf_class(const BfPass &P) {
     const int bits = P.m - 1 - P.a;

@@ -567,20 +567,43 @@ GF2T_HD u32 school_first(const SchoolShape &s, u32 t) {
 }
 GF2T_HD u32 school_last(const SchoolShape &s, u32 t) { return t < s.nparts - 1 ? t : s.nparts - 1; }
 
-// FULL: a product split in nine, whose tiles are full but for a few (the
-// tests below cost two 320,000-bit operands 2%).  The others skip what a tile has past their operands or outside its triangle:
-// a slab of 4096 residues of 89 bits takes 23 us instead of 130, one of
-// 20,000 of 3071 bits 473 (620 by transforms).
-template <bool FULL>
+// products of any sizes without a transform: one of them, and a block for
+// each of their tiles that has work (of the product's words: t its run of
+// SP_WORDS)
+struct SchoolJob {
+    Operand a, b;   // a the shorter
+    SchoolShape s;
+    u64 *part, *out;
+    u64 owords;
+};
+struct SchoolBlock {
+    u32 job;
+    unsigned short t, c;
+};
+// SC_JOBS: of a list of jobs, else of the operands y and b_op + y (swapped
+// if y is the longer).  SC_FULL: a product split in nine, whose tiles are
+// full but for a few (the tests below cost two 320,000-bit operands 2%).  The
+// others skip what a tile has past their operands or outside its triangle: a
+// slab of 4096 residues of 89 bits takes 23 us instead of 130, one of 20,000
+// of 3071 bits 473 (620 by transforms).
+enum { SC_SLACK = 0, SC_FULL = 1, SC_JOBS = 2 };
+template <int FORM>
 __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, int swap,
-                                                const SchoolShape s, u64 *__restrict__ part,
-                                                u64 part_stride) {
+                                                const SchoolShape shape, u64 *__restrict__ part,
+                                                u64 part_stride, const SchoolJob *__restrict__ jobs,
+                                                const SchoolBlock *__restrict__ blocks) {
     static_assert(SC_OUT == 128 && SC_IN == 128, "two outputs per lane, 32 values per wave, a b per thread");
+    constexpr bool FULL = FORM == SC_FULL, JOBS = FORM == SC_JOBS;
     __shared__ u32 bs[SC_OUT + SC_IN];
     __shared__ u64 sum[4][SC_OUT];
-    const u32 c = blockIdx.y, t = c + blockIdx.x, y = blockIdx.z / s.np, p = blockIdx.z % s.np;
-    if (c < school_first(s, t) || c > school_last(s, t)) return;   // whole block
-    const Operand oa = operand(ops, swap ? y + b_op : y), ob = operand(ops, swap ? y : y + b_op);
+    const SchoolBlock blk = JOBS ? blocks[blockIdx.x] : SchoolBlock{};
+    const SchoolShape s = JOBS ? jobs[blk.job].s : shape;
+    const u32 c = JOBS ? blk.c : blockIdx.y, t = JOBS ? blk.t : c + blockIdx.x;
+    const u32 y = JOBS ? 0 : blockIdx.z / s.np, p = JOBS ? 0 : blockIdx.z % s.np;
+    if (!JOBS && (c < school_first(s, t) || c > school_last(s, t))) return;   // whole block
+    const Operand oa = JOBS ? jobs[blk.job].a : operand(ops, swap ? y + b_op : y);
+    const Operand ob = JOBS ? jobs[blk.job].b : operand(ops, swap ? y : y + b_op);
+    if (JOBS) part = jobs[blk.job].part;
     const int k0 = (int)(t * SC_OUT), i0 = (int)(c * SC_IN);
     const int j0 = k0 - i0 - (int)(SC_IN - 1);   // b index of bs[0]
     const u32 wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -655,14 +678,12 @@ struct SchoolWords {
         return v;
     }
 };
-// the product's words: a block adds up the parts of 2 SP_WORDS + 1 chunk
-// coefficients, four threads each, and writes SP_WORDS words
+// the product's words from w0 on: a block adds up the parts of 2 SP_WORDS + 1
+// chunk coefficients, four threads each, and writes SP_WORDS words
 constexpr u32 SP_WORDS = 32;
-__global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ part,
-                                                        const SchoolShape s,
-                                                        u64 *__restrict__ out, size_t owords) {
+GF2T_DEV void school_product(const u64 *__restrict__ part, const SchoolShape &s, u32 w0,
+                             u64 *__restrict__ out, size_t owords) {
     __shared__ u64 sum[4][2 * SP_WORDS + 1];   // coefficients k0 - 1 ..
-    const u32 w0 = blockIdx.x * SP_WORDS;
     const u32 g = threadIdx.x & 3;
     for (u32 x = threadIdx.x >> 2; x < 2 * SP_WORDS + 1; x += 64) {
         u64 v = 0;
@@ -680,6 +701,18 @@ __global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ 
     const u32 x = threadIdx.x;
     if (x < SP_WORDS && w0 + x < owords)
         out[w0 + x] = coef(2 * x + 1) ^ (coef(2 * x + 2) << 32) ^ (coef(2 * x) >> 32);
+}
+__global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ part,
+                                                        const SchoolShape s,
+                                                        u64 *__restrict__ out, size_t owords) {
+    school_product(part, s, blockIdx.x * SP_WORDS, out, owords);
+}
+// of a job's blocks number t is its words' run of SP_WORDS
+__global__ __launch_bounds__(256) void k_school_products(const SchoolJob *__restrict__ jobs,
+                                                         const SchoolBlock *__restrict__ blocks) {
+    const SchoolBlock b = blocks[blockIdx.x];
+    const SchoolJob &j = jobs[b.job];
+    school_product(j.part, j.s, b.t * SP_WORDS, j.out, j.owords);
 }
 // The same from nine products: those of the index's bit 1 first,
 //   e_2h = E_h + O_(h-1), e_(2h+1) = S_h + E_h + O_h
@@ -1179,10 +1212,10 @@ constexpr u32 SC_FOLD_PARTS = 4;
 // residue, 818 against 1000 for 32,767).
 constexpr u64 SC_SLAB = 1 << 24;
 bool school(u64 ca, u64 cb) { return ca && cb && ca + cb <= SC_OUTS && ca * cb <= SC_WORK; }
-SchoolShape school_shape(u64 ca, u64 cb) {
+SchoolShape school_shape(u64 ca, u64 cb, bool split = true) {
     SchoolShape s;
     u64 na = std::min(ca, cb), nb = std::max(ca, cb);
-    s.np = na >= SC_KARA ? 9 : 1;
+    s.np = split && na >= SC_KARA ? 9 : 1;
     if (s.np == 9) {
         na = (na + 3) / 4;
         nb = (nb + 3) / 4;
@@ -1211,9 +1244,10 @@ int run_school(const Operands &ops, u32 b_op, bool swap, const SchoolShape &s, u
     // part c reaches the outputs [SC_IN c, SC_IN (c + 1) + nb - 1): the tiles
     // from c on, as tiles and parts are of one length
     static_assert(SC_IN == SC_OUT, "tiles of a part");
-    hipLaunchKernelGGL(s.np == 1 ? k_school<false> : k_school<true>,
+    hipLaunchKernelGGL(s.np == 1 ? k_school<SC_SLACK> : k_school<SC_FULL>,
                        dim3((SC_IN - 1 + s.nb + SC_OUT - 1) / SC_OUT, s.nparts, nbatch * s.np),
-                       dim3(256), 0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride);
+                       dim3(256), 0, st, ops, b_op, swap ? 1 : 0, s, part, part_stride,
+                       (const SchoolJob *)nullptr, (const SchoolBlock *)nullptr);
     GF2T_CHECK_LAUNCH("k_school");
     return GF2T_OK;
 }
@@ -1573,10 +1607,9 @@ extern "C" int gf2t_mulmod_noalloc(const uint64_t *da, uint64_t abits, const uin
 
 // ------------------------------------------------- variable-size batch
 // gf2t_mulmod_batch: products of different sizes, each folded mod
-// x^r + x^s_j + 1, in one set of launches: the i-th forward (inverse) pass
-// of every product that has one shares a grouped launch, and the
-// pointwise products, overlap-adds and folds of all pairs are one launch
-// each.  Each product keeps its own transform size and tile.
+// x^r + x^s_j + 1.  The smaller sizes are formed without transforms, all in
+// one launch; of the others the pairs of one size share a chain of launches;
+// the overlap-adds and folds of all pairs are one launch each.
 namespace {
 struct PairSeg {       // one pair's part of a flat grouped launch over elements
     const u64 *fa;
@@ -1595,13 +1628,15 @@ GF2T_DEV int find_seg(const PairSeg *__restrict__ sg, int np, u64 i) {
 }
 
 // phase 0: overlap-add FA into prod; 1: fold prod into out.  total = sum
-// of the pairs' element counts for the phase.  A block takes PG_RUN
+// of the pairs' element counts for the phase.  A block takes `run`
 // consecutive elements and finds the first one's pair once; the pairs after
-// it are few (a search per element took two thirds of the time).
-constexpr u32 PG_RUN = 2048;
+// it are few (a search per element took two thirds of the time).  Runs of up
+// to 2048 elements, shorter where that fills the chip: 200 pairs of 18 words
+// were two blocks that took their 114 pairs one after another, 529 us in all.
+u32 pairs_run(u64 total) { return (u32)std::max<u64>(8, std::min<u64>(2048, total / 1024)); }
 __global__ __launch_bounds__(256) void k_pairs_grouped(const PairSeg *__restrict__ sg, int np,
-                                                       u64 total, int phase, u64 r) {
-    const u64 i0 = (u64)blockIdx.x * PG_RUN, i1 = i0 + PG_RUN < total ? i0 + PG_RUN : total;
+                                                       u64 total, u32 run, int phase, u64 r) {
+    const u64 i0 = (u64)blockIdx.x * run, i1 = i0 + run < total ? i0 + run : total;
     for (int p = find_seg(sg, np, i0); p < np && sg[p].start < i1; p++) {
         const PairSeg S = sg[p];
         const u64 end = p + 1 < np && sg[p + 1].start < i1 ? sg[p + 1].start : i1;
@@ -1625,31 +1660,55 @@ __global__ __launch_bounds__(256) void k_pairs_grouped(const PairSeg *__restrict
 // transforms side by side and the B transforms behind them.
 struct BatchLayout {
     std::vector<cantor_host::SizeGroup> groups;
-    std::vector<size_t> fa, prod;   // word offsets of each pair's A transform and product
+    std::vector<size_t> fa, prod;   // word offsets of each pair's A transform (or parts) and product
     std::vector<int> m;
+    std::vector<char> school;
     size_t desc_off = 0, words = 0;
 };
 
+// The words grow with each pair's operands, and with the number of pairs:
+// every pair has its transforms' space, whatever its route, and the parts of
+// those that take none lie in theirs together and 2 SC_BATCH / SC_IN words
+// more: parts * outputs <= (ca / SC_IN + 1)(ca + cb) for ca <= cb.
 BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
     BatchLayout L;
     L.fa.resize(n);
+    std::vector<u64> ca(n), cb(n);
     for (int j = 0; j < n; j++) {
-        u64 ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
-        L.m.push_back((ca && cb) ? fft_m_for(ca + cb - 1) : 0);
+        ca[j] = (abits[j] + 31) >> 5;
+        cb[j] = (bbits[j] + 31) >> 5;
+        L.m.push_back((ca[j] && cb[j]) ? fft_m_for(ca[j] + cb[j] - 1) : 0);
     }
-    L.groups = cantor_host::size_groups(L.m);
-    size_t off = 0;
+    L.school = cantor_host::direct_pairs(L.m, ca, cb);
+    std::vector<int> m = L.m;
+    size_t off = 0, space = 0, blocks = 0;
+    for (int j = 0; j < n; j++) {
+        if (!m[j]) continue;
+        space += (size_t)2 << m[j];
+        blocks += 3 * (ca[j] + cb[j]) / SC_IN + 4 + (ca[j] + cb[j]) / (2 * SP_WORDS) + 2;
+        if (L.school[j]) m[j] = 0;
+    }
+    L.groups = cantor_host::size_groups(m);
     for (const cantor_host::SizeGroup &g : L.groups) {
         for (size_t i = 0; i < g.pairs.size(); i++) L.fa[g.pairs[i]] = off + (i << g.m);
         off += 2 * g.pairs.size() << g.m;
     }
+    for (int j = 0; j < n; j++) {
+        if (!L.school[j]) continue;
+        const SchoolShape s = school_shape(ca[j], cb[j], false);
+        L.fa[j] = off;
+        off += (size_t)s.nparts * s.nout;
+    }
+    off = space + 2 * cantor_host::DIRECT_PAIRS / SC_IN;
     for (int j = 0; j < n; j++) {
         L.prod.push_back(off);
         // the product, and before it both operands' converted chunks
         off += (gf2t_mul_out_words(abits[j], bbits[j]) + 4 + 31) & ~(size_t)31;
     }
     L.desc_off = off;
-    const size_t desc = (size_t)n * 2 * (sizeof(Operand) + sizeof(PairSeg)) + 256;
+    blocks += cantor_host::DIRECT_PAIRS / (SC_IN * SC_IN);
+    const size_t desc = (size_t)n * 2 * (sizeof(Operand) + sizeof(PairSeg)) +
+                        (size_t)n * sizeof(SchoolJob) + blocks * sizeof(SchoolBlock) + 256;
     L.words = off + (desc + 7) / 8 + 32;
     return L;
 }
@@ -1689,7 +1748,26 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
     hipStream_t st = (hipStream_t)stream;
     const BatchLayout L = batch_layout(n, abits, bbits);
     u64 *W = (u64 *)dwork;
-    // the operands, group by group: the A's, then the B's
+    // products without a transform, and the operands of the others, group
+    // by group: the A's, then the B's
+    std::vector<SchoolJob> jobs;
+    std::vector<SchoolBlock> blocks;
+    for (int j = 0; j < n; j++) {
+        if (!L.school[j]) continue;
+        const u64 ca = (abits[j] + 31) >> 5, cb = (bbits[j] + 31) >> 5;
+        SchoolJob q{operand_of(da[j], abits[j], nullptr), operand_of(db[j], bbits[j], nullptr),
+                    school_shape(ca, cb, false), W + L.fa[j], W + L.prod[j],
+                    gf2t_mul_out_words(abits[j], bbits[j])};
+        if (ca > cb) std::swap(q.a, q.b);
+        for (u32 t = 0; t * SC_OUT < q.s.nout; t++)
+            for (u32 c = school_first(q.s, t); c <= school_last(q.s, t); c++)
+                blocks.push_back(SchoolBlock{(u32)jobs.size(), (unsigned short)t, (unsigned short)c});
+        jobs.push_back(q);
+    }
+    const size_t nblocks = blocks.size();   // and then those of the products
+    for (u32 j = 0; j < jobs.size(); j++)
+        for (u32 t = 0; t * SP_WORDS < jobs[j].owords; t++)
+            blocks.push_back(SchoolBlock{j, (unsigned short)t, 0});
     std::vector<Operand> opv;
     for (const cantor_host::SizeGroup &g : L.groups)
         for (int o = 0; o < 2; o++)
@@ -1722,27 +1800,41 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
         p.L = abits[j] + bbits[j] - 1;
         p.s = s[j];
         const u64 cnt[2] = {ow, (u64)nw};
-        for (int ph = 0; ph < 2; ph++) {
+        for (int ph = L.school[j] ? 1 : 0; ph < 2; ph++) {
             p.start = total[ph];
             total[ph] += cnt[ph];
             seg[ph].push_back(p);
         }
     }
-    const int np = n - nz;
-    if (np == 0) return GF2T_OK;
-    // descriptors: the operands, then the two segment tables
-    const size_t ob = opv.size() * sizeof(Operand);
-    std::vector<unsigned char> host(ob + 2 * np * sizeof(PairSeg));
-    std::memcpy(host.data(), opv.data(), ob);
-    for (int ph = 0; ph < 2; ph++)
-        std::memcpy(host.data() + ob + ph * np * sizeof(PairSeg), seg[ph].data(),
-                    np * sizeof(PairSeg));
+    if (nz == n) return GF2T_OK;
+    // descriptors: the jobs and their blocks, the operands, then the two
+    // segment tables
+    std::vector<unsigned char> host;
+    auto put = [&](const void *v, size_t bytes) {
+        const size_t at = host.size();
+        host.resize(at + bytes);
+        if (bytes) std::memcpy(host.data() + at, v, bytes);
+        return at;
+    };
+    const size_t oj = put(jobs.data(), jobs.size() * sizeof(SchoolJob));
+    const size_t ok = put(blocks.data(), blocks.size() * sizeof(SchoolBlock));
+    const size_t oo = put(opv.data(), opv.size() * sizeof(Operand));
+    const size_t os[2] = {put(seg[0].data(), seg[0].size() * sizeof(PairSeg)),
+                          put(seg[1].data(), seg[1].size() * sizeof(PairSeg))};
     unsigned char *dd = (unsigned char *)(W + L.desc_off);
     dd = (unsigned char *)(((uintptr_t)dd + 255) & ~(uintptr_t)255);
     GF2T_HIP(hipMemcpyAsync(dd, host.data(), host.size(), hipMemcpyHostToDevice, st));
     GF2T_HIP(hipStreamSynchronize(st));   // `host` is a pageable local buffer
-    const Operand *dop = (const Operand *)dd;
-    const PairSeg *dseg = (const PairSeg *)(dd + ob);
+    const Operand *dop = (const Operand *)(dd + oo);
+    if (!blocks.empty()) {
+        const SchoolJob *dj = (const SchoolJob *)(dd + oj);
+        const SchoolBlock *db = (const SchoolBlock *)(dd + ok);
+        hipLaunchKernelGGL(k_school<SC_JOBS>, dim3((unsigned)nblocks), dim3(256), 0, st, Operands{},
+                           0u, 0, SchoolShape{}, (u64 *)nullptr, (u64)0, dj, db);
+        hipLaunchKernelGGL(k_school_products, dim3((unsigned)(blocks.size() - nblocks)), dim3(256), 0,
+                           st, dj, db + nblocks);
+        GF2T_CHECK_LAUNCH("k_school_products");
+    }
     size_t first = 0;
     for (const cantor_host::SizeGroup &g : L.groups) {
         const unsigned cnt = (unsigned)g.pairs.size();
@@ -1755,10 +1847,13 @@ extern "C" int gf2t_mulmod_batch(int n, const uint64_t *const *da, const uint64_
         if (rc) return rc;
         first += 2 * cnt;
     }
-    for (int ph = 0; ph < 2; ph++)
-        hipLaunchKernelGGL(k_pairs_grouped,
-                           dim3((unsigned)((total[ph] + PG_RUN - 1) / PG_RUN)), dim3(256), 0, st,
-                           dseg + ph * np, np, total[ph], ph, (u64)r);
+    for (int ph = 0; ph < 2; ph++) {
+        if (!total[ph]) continue;
+        const u32 run = pairs_run(total[ph]);
+        hipLaunchKernelGGL(k_pairs_grouped, dim3((unsigned)((total[ph] + run - 1) / run)), dim3(256),
+                           0, st, (const PairSeg *)(dd + os[ph]), (int)seg[ph].size(), total[ph], run,
+                           ph, (u64)r);
+    }
     GF2T_CHECK_LAUNCH("gf2t_mulmod_batch");
     return GF2T_OK;
 }

@@ -1,5 +1,6 @@
 // The host rules of the products' launches (cantor.hpp), for CPU checks.
 // Test code only.
+#include <algorithm>
 #include "cantor.hpp"
 
 extern "C" {
@@ -17,4 +18,11 @@ int pr_groups(const int *m, int n, int *group, int *place, int *size) {
     }
     return (int)v.size();
 }
+// v[j]: pair j is formed without transforms
+void pr_direct(const int *m, const u64 *ca, const u64 *cb, int n, char *v) {
+    const auto d = cantor_host::direct_pairs(std::vector<int>(m, m + n), std::vector<u64>(ca, ca + n),
+                                             std::vector<u64>(cb, cb + n));
+    std::copy(d.begin(), d.end(), v);
+}
+u64 pr_direct_pairs() { return cantor_host::DIRECT_PAIRS; }
 }

@@ -35,3 +35,48 @@ def test_groups_fit_a_grid(pr, n, sizes):
         mine = np.flatnonzero(group == g)
         assert 1 <= mine.size <= most and np.all(m[mine] == size[g])
         assert np.array_equal(place[mine], np.arange(mine.size))
+
+
+def size_of(ca, cb):
+    m = 1
+    while (1 << m) < ca + cb - 1:
+        m += 1
+    return m if ca and cb else 0
+
+
+def test_direct_pairs(pr):
+    """Whole sizes from the smallest on, as long as their chunk pairs together
+    are within the limit."""
+    most = C.c_uint64(0)
+    pr.pr_direct_pairs.restype = C.c_uint64
+    most = pr.pr_direct_pairs()
+    rng = np.random.default_rng(1)
+    for _ in range(200):
+        n, hi = int(rng.integers(1, 200)), rng.uniform(2, 18)
+        ca, cb = (np.floor(2 ** rng.uniform(0, hi, n)).astype(np.uint64) for _ in range(2))
+        ca[rng.random(n) < 0.1] = 0
+        m = np.array([size_of(int(a), int(b)) for a, b in zip(ca, cb)], np.int32)
+        v = np.zeros(n, np.int8)
+        pr.pr_direct(m.ctypes.data_as(C.c_void_p), ca.ctypes.data_as(C.c_void_p),
+                     cb.ctypes.data_as(C.c_void_p), n, v.ctypes.data_as(C.c_void_p))
+        work = (ca * cb).astype(object)
+        assert work[v == 1].sum() <= most and np.all(m[v == 1] > 0) and np.all(m[v == 1] <= 15)
+        rest = m[(v == 0) & (m > 0)]
+        if rest.size and rest.min() <= 15:   # the next size would pass the limit
+            assert np.all(m[v == 1] < rest.min())
+            assert work[v == 1].sum() + work[m == rest.min()].sum() > most
+
+
+def test_batch_workspace_grows():
+    """A batch's workspace serves every batch of fewer or shorter pairs."""
+    from mersenne_trinomial_amd._capi import lib
+    rng = np.random.default_rng(2)
+    U = lambda v: (C.c_uint64 * len(v))(*[int(x) for x in v])
+    size = lambda a, b: lib.gf2t_mulmod_batch_workspace_bytes(len(a), U(a), U(b))
+    for _ in range(300):
+        n, hi = int(rng.integers(1, 60)), rng.uniform(3, 23)
+        a, b = (np.floor(2 ** rng.uniform(0, hi, n)) for _ in range(2))
+        keep = rng.random(n) < 0.7
+        keep[0] = True
+        fa, fb = (np.floor(v * np.where(rng.random(n) < 0.5, 1, rng.random(n))) for v in (a, b))
+        assert size(fa[keep], fb[keep]) <= size(a, b)
