@@ -219,6 +219,52 @@ __global__ __launch_bounds__(512) void k_conv_tile64(u64 *__restrict__ f, u64 f_
     conv_tile_block<INV>(ElemIo{f + (u64)blockIdx.y * f_stride, n}, t, lds64);
 }
 
+// ------------------------------------------------------ small transforms
+// A whole transform of up to 2^FFT_SMALL points in one block, in the
+// polynomial basis: the conversion's one tile, then the butterflies with
+// GF(2^64) products.  Such a transform is all latency: by the kernels below
+// it is two or three launches, each of which first copies up to 37 KB of
+// tables (2^2 points: 10.3 us and 3.0 here, 2^8 16.8 and 9.5, 2^10 21.8 and
+// 15.0; 2^11, two elements a thread, 25.5 and 24).
+constexpr int FFT_SMALL = 10;
+struct SmallFft {
+    int m;
+    u64 b[FFT_SMALL];   // W(t) = sum of b[k] over the bits k of t
+    ConvTile t;
+};
+template <bool INV>
+__global__ __launch_bounds__(1 << (FFT_SMALL - 1)) void k_fft_small(u64 *__restrict__ f,
+                                                                    const SmallFft A) {
+    __shared__ u64 lds[(1 << FFT_SMALL) + (1 << (FFT_SMALL - 4))];
+    auto x = [&](u32 i) -> u64 & { return lds[conv_pad(i)]; };
+    const u32 n = 1u << A.m, tile = n < 16 ? 16 : n, q = threadIdx.x, nthr = blockDim.x;
+    for (u32 i = q; i < tile; i += nthr) x(i) = i < n ? f[i] : 0;
+    __syncthreads();
+    auto convert = [&] {
+        for (int i = 0; i < A.t.n; i++) {
+            if (q < tile / 16) conv_tile_stage<INV, u64>(x, q, tile / 16, A.t.st[INV ? A.t.n - 1 - i : i]);
+            __syncthreads();
+        }
+    };
+    if (!INV) convert();
+    for (int i = 0; i < A.m; i++) {
+        const int L = INV ? i : A.m - 1 - i;
+        for (u32 k = q; k < n / 2; k += nthr) {
+            const u32 t = k >> L, at = k + (t << L);
+            u64 g = x(at), h = x(at + (1u << L)), w = 0;
+            for (int j = 0; j < A.m - 1 - L; j++) w ^= (t >> j) & 1 ? A.b[j] : 0;
+            if (INV) h ^= g;
+            if (L < A.m - 1) g ^= gf64_mul(w, h);
+            if (!INV) h ^= g;
+            x(at) = g;
+            x(at + (1u << L)) = h;
+        }
+        __syncthreads();
+    }
+    if (INV) convert();
+    for (u32 i = q; i < n; i += nthr) f[i] = x(i);
+}
+
 // ------------------------------------------------------------ butterflies
 // n 16-byte words from memory to LDS, four loads in flight per thread
 GF2T_DEV void copy_lds(void *dst_, const void *src_, u32 n) {
@@ -1162,9 +1208,23 @@ extern "C" int gf2t_fft_plan_destroy(gf2t_fft_plan *plan) {
     return GF2T_OK;
 }
 
+namespace {
+template <bool INV>
+int run_small(u64 *f, int m, hipStream_t st) {
+    SmallFft A{};
+    A.m = m;
+    for (int k = 0; k < m - 1; k++) A.b[k] = g_basis.b[k + 1];
+    if (m > 1) A.t = conv_plan64(m).tiles[0];
+    hipLaunchKernelGGL(k_fft_small<INV>, dim3(1), dim3(m > 7 ? 1u << (m - 1) : 64u), 0, st, f, A);
+    GF2T_CHECK_LAUNCH("k_fft_small");
+    return GF2T_OK;
+}
+}  // namespace
+
 extern "C" int gf2t_fft_plan_passes(const gf2t_fft_plan *plan, int *fwd_passes, int *inv_passes) {
     if (!plan) return GF2T_EINVAL;
-    const size_t n = conv_plan64(plan->m).launches() + passes_for(*plan, 1).size() + 1;
+    const size_t n = plan->m <= FFT_SMALL
+                         ? 1 : conv_plan64(plan->m).launches() + passes_for(*plan, 1).size() + 1;
     if (fwd_passes) *fwd_passes = (int)n;
     if (inv_passes) *inv_passes = (int)n;
     return GF2T_OK;
@@ -1175,6 +1235,7 @@ extern "C" int gf2t_fft_fwd(const gf2t_fft_plan *plan, uint64_t *df, void *strea
     int rc = ensure_basis();
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
+    if (plan->m <= FFT_SMALL) return run_small<false>(df, plan->m, st);
     rc = run_conv64<false>(df, 0, plan->m, 1, st);
     if (rc) return rc;
     const Operands none{};
@@ -1192,6 +1253,7 @@ extern "C" int gf2t_fft_inv(const gf2t_fft_plan *plan, uint64_t *df, void *strea
     if (!plan || !df) return GF2T_EINVAL;
     int rc = ensure_basis();
     if (rc) return rc;
+    if (plan->m <= FFT_SMALL) return run_small<true>(df, plan->m, (hipStream_t)stream);
     return run_inverse(*plan, df, 0, 1, true, IO_PLAIN, (hipStream_t)stream);
 }
 
