@@ -627,12 +627,14 @@ struct SchoolBlock {
     unsigned short t, c;
 };
 // SC_JOBS: of a list of jobs, else of the operands y and b_op + y (swapped
-// if y is the longer).  SC_FULL: a product split in nine, whose tiles are
+// if y is the longer).  SC_MAT: the operands are a matrix m0..m3 and vector
+// pairs (see gf2t_mat2n_host), product y = 4 pair + 2 o + h of entry 2 o + h
+// and element h.  SC_FULL: a product split in nine, whose tiles are
 // full but for a few (the tests below cost two 320,000-bit operands 2%).  The
 // others skip what a tile has past their operands or outside its triangle: a
 // slab of 4096 residues of 89 bits takes 23 us instead of 130, one of 20,000
 // of 3071 bits 473 (620 by transforms).
-enum { SC_SLACK = 0, SC_FULL = 1, SC_JOBS = 2 };
+enum { SC_SLACK = 0, SC_FULL = 1, SC_JOBS = 2, SC_MAT = 3 };
 template <int FORM>
 __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, int swap,
                                                 const SchoolShape shape, u64 *__restrict__ part,
@@ -647,8 +649,10 @@ __global__ __launch_bounds__(256) void k_school(const Operands ops, u32 b_op, in
     const u32 c = JOBS ? blk.c : blockIdx.y, t = JOBS ? blk.t : c + blockIdx.x;
     const u32 y = JOBS ? 0 : blockIdx.z / s.np, p = JOBS ? 0 : blockIdx.z % s.np;
     if (!JOBS && (c < school_first(s, t) || c > school_last(s, t))) return;   // whole block
-    const Operand oa = JOBS ? jobs[blk.job].a : operand(ops, swap ? y + b_op : y);
-    const Operand ob = JOBS ? jobs[blk.job].b : operand(ops, swap ? y : y + b_op);
+    const u32 ya = FORM == SC_MAT ? y & 3 : y;
+    const u32 yb = FORM == SC_MAT ? 4 + 2 * (y >> 2) + (y & 1) : y + b_op;
+    const Operand oa = JOBS ? jobs[blk.job].a : operand(ops, swap ? yb : ya);
+    const Operand ob = JOBS ? jobs[blk.job].b : operand(ops, swap ? ya : yb);
     if (JOBS) part = jobs[blk.job].part;
     const int k0 = (int)(t * SC_OUT), i0 = (int)(c * SC_IN);
     const int j0 = k0 - i0 - (int)(SC_IN - 1);   // b index of bs[0]
@@ -724,9 +728,11 @@ struct SchoolWords {
         return v;
     }
 };
-// the product's words from w0 on: a block adds up the parts of 2 SP_WORDS + 1
-// chunk coefficients, four threads each, and writes SP_WORDS words
+// the words from w0 on of a product, or of the sum of SUMS: a block adds up
+// the parts of 2 SP_WORDS + 1 chunk coefficients, four threads each, and
+// writes SP_WORDS words
 constexpr u32 SP_WORDS = 32;
+template <int SUMS>
 GF2T_DEV void school_product(const u64 *__restrict__ part, const SchoolShape &s, u32 w0,
                              u64 *__restrict__ out, size_t owords) {
     __shared__ u64 sum[4][2 * SP_WORDS + 1];   // coefficients k0 - 1 ..
@@ -736,9 +742,11 @@ GF2T_DEV void school_product(const u64 *__restrict__ part, const SchoolShape &s,
         const u64 k = 2 * (u64)w0 + x;   // coefficient k - 1
         if (k >= 1 && k - 1 < s.nout) {
             const u32 t = (u32)(k - 1) / SC_OUT, hi = school_last(s, t);
+#pragma unroll
+            for (u32 j = 0; j < SUMS; j++)
 #pragma unroll 4
-            for (u32 c = school_first(s, t) + g; c <= hi; c += 4)
-                v ^= part[(u64)c * s.nout + (k - 1)];
+                for (u32 c = school_first(s, t) + g; c <= hi; c += 4)
+                    v ^= part[(u64)(j * s.nparts + c) * s.nout + (k - 1)];
         }
         sum[g][x] = v;
     }
@@ -751,14 +759,22 @@ GF2T_DEV void school_product(const u64 *__restrict__ part, const SchoolShape &s,
 __global__ __launch_bounds__(256) void k_school_product(const u64 *__restrict__ part,
                                                         const SchoolShape s,
                                                         u64 *__restrict__ out, size_t owords) {
-    school_product(part, s, blockIdx.x * SP_WORDS, out, owords);
+    school_product<1>(part, s, blockIdx.x * SP_WORDS, out, owords);
+}
+// output y of a matrix-vector product, the sum of two (SC_MAT)
+__global__ __launch_bounds__(256) void k_school_mat(const u64 *__restrict__ part,
+                                                    const SchoolShape s, u64 *__restrict__ out,
+                                                    size_t owords) {
+    const u32 y = blockIdx.y;
+    school_product<2>(part + (u64)y * 2 * s.nparts * s.nout, s, blockIdx.x * SP_WORDS,
+                      out + y * owords, owords);
 }
 // of a job's blocks number t is its words' run of SP_WORDS
 __global__ __launch_bounds__(256) void k_school_products(const SchoolJob *__restrict__ jobs,
                                                          const SchoolBlock *__restrict__ blocks) {
     const SchoolBlock b = blocks[blockIdx.x];
     const SchoolJob &j = jobs[b.job];
-    school_product(j.part, j.s, b.t * SP_WORDS, j.out, j.owords);
+    school_product<1>(j.part, j.s, b.t * SP_WORDS, j.out, j.owords);
 }
 // The same from nine products: those of the index's bit 1 first,
 //   e_2h = E_h + O_(h-1), e_(2h+1) = S_h + E_h + O_h
@@ -2186,6 +2202,15 @@ __global__ __launch_bounds__(256) void k_mat2n_pointwise(u64 *__restrict__ F, si
 }
 }  // namespace
 
+// Matrix-vector products of up to MAT_PAIRS chunk pairs are formed without
+// transforms, whose chain of eight launches (five below 2^9 points) is as
+// long however few points it has: two pairs of 64 bits take 18 us and 37 by
+// transforms, of 16,000 bits 26 and 87, of 65,000 bits (2^25) 66 and 96.  One
+// product at a time is faster so up to 2^26 (one pair of 131,000 bits: 95 and
+// 101), but 15 full-size gcds at once, whose products share the chip, take
+// 4.45 s with that line and 4.2 with this one (4.39 by transforms alone).
+namespace { constexpr u64 MAT_PAIRS = (u64)1 << 25; }
+
 extern "C" int gf2t_mat2n_host(const uint64_t *const hm[4], const uint64_t mbits[4], int npairs,
                                const uint64_t *const *hv, const uint64_t *vbits,
                                uint64_t *const *hout, size_t outw) {
@@ -2234,11 +2259,15 @@ extern "C" int gf2t_mat2n_host(const uint64_t *const hm[4], const uint64_t mbits
         stage += (in_w[i] + 3) & ~(size_t)3;
     }
     lchw = stage;   // the converted chunks of every operand
-    rc = hm_reserve(hc, nt * n + nv * ow + stage + lchw + 64, std::max(stage, nv * ow));
+    // the transforms, or two products' parts for each output
+    const SchoolShape sh = school_shape(cm, cv, false);
+    const bool direct = cm + cv <= SC_OUTS && 4 * npairs * cm * cv <= MAT_PAIRS;
+    const size_t space = direct ? (size_t)2 * nv * sh.nparts * sh.nout : nt * n;
+    rc = hm_reserve(hc, space + nv * ow + stage + lchw + 64, std::max(stage, nv * ow));
     if (rc) return rc;
     hipStream_t st = hc.st;
     u64 *F = hc.dbuf;                         // nt transforms, n words apart
-    u64 *dout = F + nt * n, *dstage = dout + nv * ow;
+    u64 *dout = F + space, *dstage = dout + nv * ow;
     // the operands, 32-byte aligned, in one pinned buffer and one copy
     Operands pk{};
     u64 *lch = dstage + stage;
@@ -2262,16 +2291,25 @@ extern "C" int gf2t_mat2n_host(const uint64_t *const hm[4], const uint64_t mbits
     } else if (off) {
         GF2T_HIP(hipMemcpyAsync(dstage, hc.hbuf, off * 8, hipMemcpyHostToDevice, st));
     }
-    int in;
-    rc = run_forward(plan, F, n, pk, log2_ceil(std::max(cm, cv)), (unsigned)nt, true, st, in);
-    if (rc) return rc;
-    unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_mat2n_pointwise, dim3(blocks), dim3(256), 0, st, F, n, npairs);
-    rc = run_inverse(plan, F + 4 * n, n, (unsigned)nv, true, IO_UNITS, st);
-    if (rc) return rc;
-    size_t nch = (size_t)(cm + cv - 1);
-    hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), nv), dim3(256), 0, st,
-                       F + 4 * n, nch, dout, ow, (u64)n, (u64)ow);
+    if (direct) {
+        hipLaunchKernelGGL(k_school<SC_MAT>, dim3((SC_IN - 1 + sh.nb + SC_OUT - 1) / SC_OUT, sh.nparts, 2 * nv),
+                           dim3(256), 0, st, pk, 0u, cm > cv ? 1 : 0, sh, F,
+                           (u64)sh.nparts * sh.nout, (const SchoolJob *)nullptr,
+                           (const SchoolBlock *)nullptr);
+        hipLaunchKernelGGL(k_school_mat, dim3((unsigned)((ow + SP_WORDS - 1) / SP_WORDS), nv),
+                           dim3(256), 0, st, F, sh, dout, ow);
+    } else {
+        int in;
+        rc = run_forward(plan, F, n, pk, log2_ceil(std::max(cm, cv)), (unsigned)nt, true, st, in);
+        if (rc) return rc;
+        unsigned blocks = (unsigned)std::min<size_t>((n / 2 + 255) / 256, 2048);
+        hipLaunchKernelGGL(k_mat2n_pointwise, dim3(blocks), dim3(256), 0, st, F, n, npairs);
+        rc = run_inverse(plan, F + 4 * n, n, (unsigned)nv, true, IO_UNITS, st);
+        if (rc) return rc;
+        size_t nch = (size_t)(cm + cv - 1);
+        hipLaunchKernelGGL(k_overlap_add, dim3((unsigned)((ow + 255) / 256), nv), dim3(256), 0, st,
+                           F + 4 * n, nch, dout, ow, (u64)n, (u64)ow);
+    }
     GF2T_CHECK_LAUNCH("gf2t_mat2n_host");
     if (!zc) GF2T_HIP(hipMemcpyAsync(hc.hbuf, dout, nv * ow * 8, hipMemcpyDeviceToHost, st));
     GF2T_HIP(hipStreamSynchronize(st));
