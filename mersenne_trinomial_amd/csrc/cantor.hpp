@@ -697,6 +697,60 @@ inline std::vector<BfPass> bf_passes(int m, int tile) {
     }
     return v;
 }
+constexpr int FFT_MAX_M = 27;
+// a transform's size for that many coefficients
+inline int fft_m_for(u64 nchunks_total) {
+    int m = 1;
+    while (((u64)1 << m) < nchunks_total) m++;
+    return m;
+}
+// Wrapped products.  A product whose N = ca + cb - 1 chunk coefficients lie just above a
+// power of two, 2^mp < N <= 2^mp + 2^mp/4, runs on 2^mp-point transforms
+// instead of 2^(mp+1), plus a product at most half that size.  The 2^mp
+// points are the span of the first mp Cantor basis elements, whose
+// vanishing polynomial is
+//     V(X) = sum over k with bits(k) inside bits(mp) of X^(2^k)
+// (V_{i+1} = V_i^2 + V_i, since V_i(b_i) = 1 for the Cantor basis; the
+// binomial coefficients mod 2 follow Lucas).  So pointwise products and
+// the inverse give C mod V.  The e = N - 2^mp top coefficients
+// C_high = C div X^(2^mp) come from the product of the top e chunks of
+// each operand (pairs i + j >= 2^mp only involve those), a 2^ms-point
+// product.  V's next term below X^(2^mp) is at most X^(2^(mp-1)), and
+// deg C_high < e <= 2^(mp-2), so C div V = C_high and
+//     C = (C mod V) + C_high * (V - X^(2^mp)) + C_high * X^(2^mp):
+// C_high is XORed into the low coefficients at each offset 2^k, k a
+// proper bit-subset of mp, and forms the coefficients from 2^mp up.
+struct Wrap {
+    bool on = false;
+    int mp = 0, ms = 0;
+    u64 e = 0;
+};
+// Wrapping pays where the 2^mp points it saves (of all products of a batch
+// together) take longer than the top product: its chain of launches, as
+// long as WRAP_CHAIN points, and a fourth more than its own points, as a
+// smaller transform uses the chip less.  Wrapped and not, 2^20 coefficients
+// and a 32nd more take 265 and 268 us, a 16th more 284 and 268; 2^21 and an
+// eighth 439 and 419; 2^22 and an eighth 645 and 721, and a quarter 743 and
+// 717; 2^23 and a 64th 928 and 1352.
+constexpr u64 WRAP_CHAIN = 900000;
+inline Wrap wrap_for(u64 ca, u64 cb, u64 nbatch = 1) {
+    Wrap w;
+    const u64 N = ca + cb - 1;
+    const int m = fft_m_for(N);
+    if (m < 12 || m - 1 > FFT_MAX_M) return w;
+    const int mp = m - 1;
+    const u64 n = (u64)1 << mp;
+    if (N <= n) return w;
+    const u64 e = N - n;
+    if (e > n / 4 || ca > n || cb > n || e >= ca || e >= cb) return w;
+    const int ms = fft_m_for(2 * e - 1);
+    if (nbatch * n < WRAP_CHAIN + 5 * (nbatch << ms) / 4) return w;
+    w.on = true;
+    w.mp = mp;
+    w.e = e;
+    w.ms = ms;
+    return w;
+}
 // The transforms of a launch are the rows of its grid, which has at most
 // 65535, and a product has two of them: the pairs of one chain of launches.
 constexpr unsigned MAX_PAIRS = 32767;

@@ -25,4 +25,12 @@ void pr_direct(const int *m, const u64 *ca, const u64 *cb, int n, char *v) {
     std::copy(d.begin(), d.end(), v);
 }
 u64 pr_direct_pairs() { return cantor_host::DIRECT_PAIRS; }
+// whether products of ca x cb chunks wrap, and the sizes
+int pr_wrap(u64 ca, u64 cb, u64 nbatch, int *mp, int *ms, u64 *e) {
+    const auto w = cantor_host::wrap_for(ca, cb, nbatch);
+    *mp = w.mp;
+    *ms = w.ms;
+    *e = w.e;
+    return w.on;
+}
 }

@@ -6,6 +6,8 @@ import subprocess
 import numpy as np
 import pytest
 
+import wrapped_shapes as W
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "mersenne_trinomial_amd", "csrc")
 
@@ -80,3 +82,24 @@ def test_batch_workspace_grows():
         keep[0] = True
         fa, fb = (np.floor(v * np.where(rng.random(n) < 0.5, 1, rng.random(n))) for v in (a, b))
         assert size(fa[keep], fb[keep]) <= size(a, b)
+
+
+def wrap(pr, ca, cb, n):
+    mp, ms, e = C.c_int(), C.c_int(), C.c_uint64()
+    pr.pr_wrap.argtypes = [C.c_uint64] * 3 + [C.c_void_p] * 3
+    on = pr.pr_wrap(ca, cb, n, C.addressof(mp), C.addressof(ms), C.addressof(e))
+    return bool(on), mp.value, ms.value, e.value
+
+
+@pytest.mark.parametrize("mp,e,ca,on", W.PRODUCTS)
+def test_wrapped_products(pr, mp, e, ca, on):
+    """The shapes that the GPU tests run lie where they are meant to."""
+    got = wrap(pr, ca, W.other(mp, e, ca), 1)
+    assert got[0] == on
+    if on:   # the transforms fit those of an ordinary product
+        assert got[1] == mp and got[3] == e and 2 * e - 1 <= 1 << got[2] and got[2] < mp
+
+
+@pytest.mark.parametrize("r,n,on", W.SLABS)
+def test_wrapped_slabs(pr, r, n, on):
+    assert wrap(pr, W.chunks(r), W.chunks(r), n)[0] == on
