@@ -154,10 +154,12 @@ int gf2t_square_fold_batch(uint64_t *const *dres, uint64_t *const *dtmp,
  * PCLMULQDQ where the CPU also has AVX-512 VPCLMULQDQ (read once). */
 int gf2t_tune(const char *key, int64_t value);
 /* The value a knob has now (the default until set): the keys above, and
- * "fft_tile_<m>" -- the butterfly passes of the 2^m-point transforms use
- * tiles of at most 2^T elements, T in 6..13 (set with
- * gf2t_tune("fft_tile_<m>", T), 0 = the default: 13, or m where that is
- * less).  A smaller tile spreads a small transform over more workgroups; the reference's split knobs are gf2c_taylor_lv / gf2c_bfly_lv
+ * "fft_tile_<m>" -- of the 2^m-point transforms, the butterfly passes of
+ * fewer than eight levels take tiles of at most 2^T elements (T in 6..13, set
+ * with gf2t_tune("fft_tile_<m>", T); 0 = the default, 13, or m where that is
+ * less): 2^11 at the most, smaller where a launch would not fill the chip.
+ * Passes of eight levels have tiles of 2^11 elements whatever T.  The
+ * reference's split knobs are gf2c_taylor_lv / gf2c_bfly_lv
  * (src/gf2_cantor_cuda.h:24-61).  The autotuner (mersenne_trinomial_amd/
  * autotune.py) measures these and installs its choices. */
 int gf2t_tune_get(const char *key, int64_t *value);

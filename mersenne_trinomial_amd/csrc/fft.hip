@@ -30,8 +30,8 @@
 namespace {
 
 using cantor_host::FFT_MAX_M;
-constexpr int FFT_TILE_BITS = 13;   // largest tile: 8192 elements
-constexpr int FFT_MIN_TILE_BITS = 6;
+// of the knobs fft_tile_<m> (see passes_for) and fft_low_bits (no effect)
+constexpr int FFT_TILE_BITS = 13, FFT_MIN_TILE_BITS = 6;
 constexpr int FFT_LOW_BITS = 4;
 constexpr int PACK_LIST = 12;   // four matrix entries + four vector pairs
 constexpr int CONV_ONE_TILE = 13;   // largest conversion done in one tile
@@ -1041,7 +1041,8 @@ constexpr u32 BF_BLOCKS = 2560;   // blocks of a butterfly launch: ten per CU
 // butterfly passes above the low eight levels, all of nbatch transforms
 // stride words apart
 std::vector<BfPass> passes_for(const gf2t_fft_plan &pl, unsigned nbatch) {
-    // smaller tiles until the launch fills the chip
+    // tiles of at most 2^(T - 1) units (2^(8 + RB), as the eight levels of a
+    // whole window always have), smaller until the launch fills the chip
     int tile = std::min(8 + RB, std::max(pl.T - 1, 6));
     while (tile > 6 + RB && ((((u64)1 << (pl.m - 1)) >> tile) * nbatch) < 1024) tile--;
     return cantor_host::bf_passes(pl.m, tile);
@@ -1162,8 +1163,9 @@ using cantor_host::fft_m_for;
 
 }  // namespace
 
-// gf2t_tune("fft_tile_<m>", T): butterfly tiles of at most 2^T elements
-// (6..13) for 2^m-point transforms from now on; 0 restores the default.
+// gf2t_tune("fft_tile_<m>", T): tiles of at most 2^T elements (6..13) in the
+// butterfly passes of fewer than eight levels of 2^m-point transforms from
+// now on; 0 restores the default.
 // Plans already made keep theirs.
 int gf2t_fft_set_tile_bits(int m, int64_t T) {
     if (m < 1 || m > FFT_MAX_M || (T != 0 && (T < FFT_MIN_TILE_BITS || T > FFT_TILE_BITS))) {
