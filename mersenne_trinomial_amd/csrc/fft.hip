@@ -19,7 +19,6 @@
 #include "cantor.hpp"
 #include "../../include/gf2t.h"
 #include <vector>
-#include <map>
 #include <mutex>
 #include <condition_variable>
 #include <cstring>
@@ -42,7 +41,7 @@ __device__ FftTables g_tab;
 
 // One operand of a transform: n 32-bit chunks at src (the last masked to
 // mask, xor0 XORed into the first), and the buffer its converted
-// coefficients go to (16-byte aligned).
+// coefficients go to (8-byte aligned: they are read two at a time).
 struct Operand {
     const u32 *src;
     u32 *lch;

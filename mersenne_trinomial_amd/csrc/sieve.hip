@@ -24,8 +24,8 @@
 //                 them at d = 32 for smax = 68,139,920)
 //   k_mark        per queued class: minimal polynomial by Berlekamp-Massey
 //                 on Tr(beta^k), then the marks (inline up to 1024, longer
-//                 progressions to k_mark_heavy); degrees whose period M is
-//                 at most smax and below 2^16 mark one period instead, and
+//                 progressions to k_mark_heavy); degrees up to 20 whose
+//                 period M is at most smax mark one period instead, and
 //   k_sweep       takes every s through the periods once, lowest degree
 //                 first
 // A table of all 2^d logarithms (16 GiB at d = 32) took three radix

@@ -253,15 +253,20 @@ __global__ __launch_bounds__(SQ_THREADS) void k_square12_fold_batch(
 // of windows (pow_window: about 31 for M = 3, their shifts uniform) is
 // sorted by class and dealt to its waves in equal parts -- by class the
 // fullest wave had 7 of them -- and what a wave has of a class is XORed
-// into that class's words in LDS, which are then merged.  A tile of the
-// two-squaring kernel takes twice its arithmetic (165 VALU operations a
-// pair of words against 90, and copies in LDS) but reads each word about
-// once, where this reads it about four times, from the caches while they
+// into that class's words in LDS, which are then merged.  For three
+// squarings that is 216 VALU operations a pair of words in all, the list
+// among them (0.5 per cycle per CU: not the issue limit), where a tile of the
+// two-squaring kernel takes 174 for two and copies in LDS; but a tile reads
+// each word about once, this about four times, from the caches while they
 // hold the launch's residues: three squarings take 4.2 us where one launch
 // is all latency (756839 bits; two took 9), 14 us for one full-size residue
-// (two: 16), 92 us for 8 (two: 74) and 800 us for 64 (two: 480; these
-// exceed the 256 MiB cache).  So launches of up to PW_MOST ranges, 8
-// full-size residues, take this kernel.
+// (two: 16), 92 us for 8 (two: 74) and 800 us for 64 (two: 455).  Past the
+// 256 MiB cache, which eight full-size residues and their copies fill, two
+// at a time are faster: 12 squarings of 8, 9, 16 and 32 of them take 396,
+// 497, 871 and 1712 us by three and 469, 460, 729 and 1370 by two, 24 of 24
+// and 26 residues of 44,497,001 bits 724 and 916 by three and 860 of the 26
+// by two.  (Residues small enough to run in rows, 13,466,917 bits, keep the
+// threes faster a little longer: 96 of them 874 us against 970.)
 constexpr int PW_T = 512, PW_LIST = 128;
 template <int M, int U>
 constexpr u32 pw_units() { return 64u * U * (8 >> M); }
@@ -442,8 +447,8 @@ inline int pow_per(u64 ranges, u64 two, u64 three) {
 }
 // A single squaring by windows is as long as three where residues come from
 // memory: from PW_COLS ranges on the one-squaring kernels take it
-// (136,279,841 bits: 18.6 us against 20.5, s = 1 15.9 against 20.1;
-// 20,000,003 bits: 8.7 against 7.8).
+// (136,279,841 bits: 19.1 us against 20.4, s = 1 17.1 against 19.7; below,
+// 20,000,003 bits: 8.7 against 7.7).
 inline bool pow_one(u64 ranges) { return ranges < PW_COLS; }
 template <int U>
 constexpr size_t pw_lds() { return (8 * pw_class_words<3, U>() + 4 * PW_LIST + 16) * 4; }
@@ -503,10 +508,14 @@ __global__ __launch_bounds__(SQ_THREADS) void k_batch_back(const SqDesc *__restr
 // launch and no memory traffic per step.  Bounded by the issue of one
 // CU and the barrier: 0.85 us per squaring at 132049 bits and 2.2 us at
 // 640,000, where by launches two squarings took 9.5 us, all of it latency
-// (40 squarings: 191 -> 34 us, and 183 -> 90 us; by launches of three
-// squarings 57 us at any such size, so a few residues above 262,144 bits go
-// that way).  512 residues of 600,000
-// bits are 512 blocks, one per CU at a time: 276 us against 1085 us.
+// (40 squarings: 191 -> 34 us, and 183 -> 90 us).  By launches of three
+// squarings 40 take about 57 us at any such size, and a few squarings less
+// (6 of 262,144 bits 8.2 us against 12.4, 40 56 against 54), so residues above
+// CH_ONE words go that way unless there are CH_FEW of them: a batch of 16 of
+// 300,000 bits takes 63 us in LDS and 83 by launches (40 squarings, upload
+// and wait among them), 16 of 640,000 135 and 120, 32 of them 136 and 173, and
+// of 64 137 and 202.  512 residues of 600,000 bits are 512 blocks, one per CU
+// at a time: 276 us against 1085 us.
 constexpr int CH_THREADS = 1024;
 constexpr size_t CH_LDS = 160 * 1024;
 constexpr size_t CH_WORDS = CH_LDS / 16 - 2;   // words of a residue, at most
