@@ -1700,8 +1700,8 @@ struct BatchLayout {
 
 // The words grow with each pair's operands, and with the number of pairs:
 // every pair has its transforms' space, whatever its route, and the parts of
-// those that take none lie in theirs together and 2 SC_BATCH / SC_IN words
-// more: parts * outputs <= (ca / SC_IN + 1)(ca + cb) for ca <= cb.
+// those that take none lie in theirs together and 2 / SC_IN words more for
+// each chunk pair: parts * outputs <= (ca / SC_IN + 1)(ca + cb) for ca <= cb.
 BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
     BatchLayout L;
     L.fa.resize(n);
@@ -1713,10 +1713,12 @@ BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
     }
     L.school = cantor_host::direct_pairs(L.m, ca, cb);
     std::vector<int> m = L.m;
-    size_t off = 0, space = 0, blocks = 0;
+    size_t off = 0, space = 0, blocks = 0, direct = 0;
     for (int j = 0; j < n; j++) {
         if (!m[j]) continue;
         space += (size_t)2 << m[j];
+        direct = std::min(cantor_host::DIRECT_PAIRS,
+                          direct + std::min<size_t>(cantor_host::DIRECT_PAIRS, ca[j] * cb[j]));
         blocks += 3 * (ca[j] + cb[j]) / SC_IN + 4 + (ca[j] + cb[j]) / (2 * SP_WORDS) + 2;
         if (L.school[j]) m[j] = 0;
     }
@@ -1731,14 +1733,14 @@ BatchLayout batch_layout(int n, const uint64_t *abits, const uint64_t *bbits) {
         L.fa[j] = off;
         off += (size_t)s.nparts * s.nout;
     }
-    off = space + 2 * cantor_host::DIRECT_PAIRS / SC_IN;
+    off = (space + 2 * direct / SC_IN + 31) & ~(size_t)31;
     for (int j = 0; j < n; j++) {
         L.prod.push_back(off);
         // the product, and before it both operands' converted chunks
         off += (gf2t_mul_out_words(abits[j], bbits[j]) + 4 + 31) & ~(size_t)31;
     }
     L.desc_off = off;
-    blocks += cantor_host::DIRECT_PAIRS / (SC_IN * SC_IN);
+    blocks += direct / (SC_IN * SC_IN);
     const size_t desc = (size_t)n * 2 * (sizeof(Operand) + sizeof(PairSeg)) +
                         (size_t)n * sizeof(SchoolJob) + blocks * sizeof(SchoolBlock) + 256;
     L.words = off + (desc + 7) / 8 + 32;
