@@ -6,11 +6,10 @@ What it searches (the reference times its transform variants and picks
 its block size the same way, src/tsfactor.cu:1986-1989 and auto_m
 :2093-2114):
 
-- fft_tile_<m>: the tile of the Cantor transform's LDS passes, 2^T
-  elements for T in 6..13, per transform size 2^m.  Small tiles spread a
-  small transform over more workgroups but need more passes.  Timed on
-  the product shape the half-gcd's device service runs most: a batch of
-  six transforms (four matrix entries and two vectors), here as three
+- fft_tile_<m>: the tile of the Cantor transform's butterfly passes of
+  fewer than eight levels, at most 2^T elements, per transform size 2^m.
+  Most sizes of T give the same passes, so another than the default is
+  chosen only where it is faster by more than runs differ.  Timed on three
   two-operand products back to back on one stream.
 - the batched squaring knobs sq_fuse / sq_nt / sq_order / sq_ppt, timed
   on the deep scan's residue shape at the given r.
@@ -68,6 +67,14 @@ def _time_ms(fn, reps: int) -> float:
     return e0.elapsed_ms(e1) / reps
 
 
+def pick(times: dict, default):
+    """The key with the least time, but the default unless that is 3% faster."""
+    best = min(times, key=times.get)
+    if default in times and times[best] > 0.97 * times[default]:
+        return default
+    return best
+
+
 def tune_fft(ms, tiles, reps: int = 5):
     """For each transform size 2^m, the tile bits with the least time for
     three products whose transforms have 2^m points."""
@@ -92,7 +99,7 @@ def tune_fft(ms, tiles, reps: int = 5):
                 continue
             tune_set(f"fft_tile_{m}", T)
             times[T] = _time_ms(run, reps)
-        best = min(times, key=times.get)
+        best = pick(times, default)
         tune_set(f"fft_tile_{m}", best)
         out[m] = {"default": default, "default_ms": times.get(default), "chosen": best,
                   "chosen_ms": times[best], "ms": {T: round(v, 4) for T, v in times.items()}}
